@@ -78,8 +78,13 @@ struct Tiles {
   int max_rec = 0, max_mrec = 0;  // records per tile (plain, matrix-core padded)
   int ncolors = 0;
   const int *node0 = nullptr;     // [n_tiles + 1]
-  const int *ext_ptr = nullptr;   // [n_tiles + 1] non-owned slots
-  const int *ext = nullptr;       // global node (>= 0) or -(hanging + 1)
+  // slots: owned, then the hanging ones (accumulated first) by their parents
+  // (a, b, c, d): two of weight 1/2 (c = -1) or four of weight 1/4, then the
+  // halo nodes
+  const int *extd_ptr = nullptr;  // [n_tiles + 1]
+  const int4 *extd = nullptr;
+  const int *ext_ptr = nullptr;   // [n_tiles + 1]
+  const int *ext = nullptr;       // global node
   const int *nacc_dep = nullptr;  // [n_tiles] accumulated hanging slots
   const int *el_ptr = nullptr;    // [n_tiles + 1]
   const TileElem *el = nullptr;
@@ -88,12 +93,10 @@ struct Tiles {
   TileElem *el32 = nullptr;
   const int *el_elem = nullptr;  // element of each record
   int n_rec = 0;
-  const int *comb_ptr = nullptr;  // [n_nodes + 1] owned node <- hanging slots
-  const int *comb_slot = nullptr; // local slot in the owning tile
-  const float *comb_w = nullptr;
-  const int *dep_ptr = nullptr;
-  const int *dep_conn = nullptr;
-  const float *dep_w = nullptr;
+  // owned node <- hanging slots of its tile, groups of four packed entries:
+  // LDS position | 2^16 (weight 1/2) or 2^17 (weight 1/4), 0 pads
+  const int *comb_ptr = nullptr;  // [n_nodes + 1] in groups
+  const uint4 *comb = nullptr;
   const uint8_t *bcmask = nullptr;
   // matrix-core (FP32) form: per tile and wave, records of the elements
   // touching the wave's share of the nodes, in batches of 16 of one colour

@@ -69,6 +69,34 @@ __device__ __forceinline__ void load_node(int e, const T *__restrict__ x,
   }
 }
 
+// Value of a hanging node from its packed parents (a, b, c, d): two parents
+// of weight 1/2 (c < 0) or four of weight 1/4, clamped dofs zero.  The four
+// loads go out together (the pair form loads its parents twice), so a hanging
+// node costs two dependent memory round trips, its record and its parents,
+// in place of the ten or so of the constraint-list loop of load_node; the
+// sums are the same, term by term.
+template <class T>
+__device__ __forceinline__ void load_dep(const int4 p, const T *__restrict__ x,
+                                         const uint8_t *__restrict__ bcmask, T v[3]) {
+  const bool two = p.z < 0;
+  const int g[4] = {p.x, p.y, two ? p.x : p.z, two ? p.y : p.w};
+  Vec3<T> u[4];
+  uint8_t m[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) u[k] = load_vec3(x + 3 * (size_t)g[k]);
+#pragma unroll
+  for (int k = 0; k < 4; k++) m[k] = bcmask[g[k]];
+  const T w = two ? T(0.5) : T(0.25);
+  v[0] = v[1] = v[2] = T(0);
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const bool on = k < 2 || !two;
+    if (on && !(m[k] & 1)) v[0] += w * u[k].a;
+    if (on && !(m[k] & 2)) v[1] += w * u[k].b;
+    if (on && !(m[k] & 4)) v[2] += w * u[k].c;
+  }
+}
+
 template <class T>
 __global__ __launch_bounds__(WG_ELEMS) void k_elem_apply(
     const int *__restrict__ wg_node_ptr, const int *__restrict__ wg_nodes,
@@ -1223,15 +1251,13 @@ void launch_dinv_dots(int64_t n, const double *dinv, double *y, const double *x,
 // ---------------------------------------------------------------------------
 // owner-tile apply: one pass, final values of the owned nodes, fused epilogue
 
-// stage x of the tile's slots into LDS (owned nodes in place, halo nodes with
-// hanging-node interpolation, clamped dofs zero) and zero the accumulators;
-// S floats per node (S = 4 pads each node to 16 bytes with a zero)
+// stage x of the tile's slots into LDS (owned nodes in place, then the
+// hanging slots from their packed parents extd_l, then the halo nodes ext_l,
+// clamped dofs zero) and zero the accumulators; S values per node
 template <class T, int S, int NT = TILE_THREADS, int SY = S>
-__device__ __forceinline__ void tile_stage(int n0, int nown, const int *__restrict__ ext_l, int next,
-                                           int nacc, const int *__restrict__ dep_ptr,
-                                           const int *__restrict__ dep_conn,
-                                           const float *__restrict__ dep_w,
-                                           const uint8_t *__restrict__ bcmask,
+__device__ __forceinline__ void tile_stage(int n0, int nown, const int4 *__restrict__ extd_l,
+                                           int ndep, const int *__restrict__ ext_l, int nhalo,
+                                           int nacc, const uint8_t *__restrict__ bcmask,
                                            const T *__restrict__ x, T *xs, T *ys) {
   const int tid = threadIdx.x;
   constexpr int VN = 2, VH = 2;
@@ -1241,20 +1267,14 @@ __device__ __forceinline__ void tile_stage(int n0, int nown, const int *__restri
     xs[q + 1] = b;
     xs[q + 2] = c;
   };
-  // halo node g of slot nown + i: independent nodes load directly (masked),
-  // hanging ones are interpolated from their parents
-  auto put_halo = [&](int i, int g, const Vec3<T> &w, uint8_t m) {
-    T v[3] = {(m & 1) ? T(0) : w.a, (m & 2) ? T(0) : w.b, (m & 4) ? T(0) : w.c};
-    if (g < 0) load_node<T>(g, x, dep_ptr, dep_conn, dep_w, bcmask, v);
-    put(nown + i, v[0], v[1], v[2]);
-  };
+  const int h0 = nown + ndep;  // first halo slot
   // First rounds: the halo node indices, then the owned values (one 12-byte
   // load and one mask byte per node) and the halo values all go out before
   // any is used; indices are clamped into the tile, so the loads are
   // unconditional.
   int gf[VH];
 #pragma unroll
-  for (int k = 0; k < VH; k++) gf[k] = next > 0 ? ext_l[min(tid + k * NT, next - 1)] : 0;
+  for (int k = 0; k < VH; k++) gf[k] = nhalo > 0 ? ext_l[min(tid + k * NT, nhalo - 1)] : 0;
   Vec3<T> vo[VN], vh[VH];
   uint8_t mo[VN], mh[VH];
 #pragma unroll
@@ -1265,9 +1285,8 @@ __device__ __forceinline__ void tile_stage(int n0, int nown, const int *__restri
   }
 #pragma unroll
   for (int k = 0; k < VH; k++) {
-    const int gg = gf[k] >= 0 ? gf[k] : 0;
-    vh[k] = load_vec3(x + 3 * (size_t)gg);
-    mh[k] = bcmask[gg];
+    vh[k] = load_vec3(x + 3 * (size_t)gf[k]);
+    mh[k] = bcmask[gf[k]];
   }
 #pragma unroll
   for (int k = 0; k < VN; k++)
@@ -1276,7 +1295,20 @@ __device__ __forceinline__ void tile_stage(int n0, int nown, const int *__restri
           (mo[k] & 4) ? T(0) : vo[k].c);
 #pragma unroll
   for (int k = 0; k < VH; k++)
-    if (tid + k * NT < next) put_halo(tid + k * NT, gf[k], vh[k], mh[k]);
+    if (tid + k * NT < nhalo)
+      put(h0 + tid + k * NT, (mh[k] & 1) ? T(0) : vh[k].a, (mh[k] & 2) ? T(0) : vh[k].b,
+          (mh[k] & 4) ? T(0) : vh[k].c);
+  // hanging slots; the next round's records load before this round's parents
+  if (ndep > 0) {
+    int4 pn = extd_l[min(tid, ndep - 1)];
+    for (int i = tid; i < ndep; i += NT) {
+      const int4 p = pn;
+      pn = extd_l[min(i + NT, ndep - 1)];
+      T v[3];
+      load_dep<T>(p, x, bcmask, v);
+      put(nown + i, v[0], v[1], v[2]);
+    }
+  }
   // further rounds (tiles of more than two nodes or halo slots per thread)
   for (int j0 = tid + VN * NT; j0 < nown; j0 += VN * NT) {
 #pragma unroll
@@ -1291,22 +1323,21 @@ __device__ __forceinline__ void tile_stage(int n0, int nown, const int *__restri
         put(j0 + k * NT, (mo[k] & 1) ? T(0) : vo[k].a, (mo[k] & 2) ? T(0) : vo[k].b,
             (mo[k] & 4) ? T(0) : vo[k].c);
   }
-  for (int i0 = tid + VH * NT; i0 < next; i0 += VH * NT) {
+  for (int i0 = tid + VH * NT; i0 < nhalo; i0 += VH * NT) {
     int g[VH];
 #pragma unroll
-    for (int k = 0; k < VH; k++) g[k] = ext_l[min(i0 + k * NT, next - 1)];
+    for (int k = 0; k < VH; k++) g[k] = ext_l[min(i0 + k * NT, nhalo - 1)];
 #pragma unroll
     for (int k = 0; k < VH; k++) {
-      const int gg = g[k] >= 0 ? g[k] : 0;
-      vh[k] = load_vec3(x + 3 * (size_t)gg);
-      mh[k] = bcmask[gg];
+      vh[k] = load_vec3(x + 3 * (size_t)g[k]);
+      mh[k] = bcmask[g[k]];
     }
 #pragma unroll
     for (int k = 0; k < VH; k++)
-      if (i0 + k * NT < next) put_halo(i0 + k * NT, g[k], vh[k], mh[k]);
+      if (i0 + k * NT < nhalo)
+        put(h0 + i0 + k * NT, (mh[k] & 1) ? T(0) : vh[k].a, (mh[k] & 2) ? T(0) : vh[k].b,
+            (mh[k] & 4) ? T(0) : vh[k].c);
   }
-  if (S == 4)
-    for (int i = tid; i < ((nown + next + 7) & ~7); i += NT) xs[4 * i + 3] = T(0);
   // accumulators: SY * round8(nacc) values, a multiple of 16 bytes starting
   // 16-byte aligned, cleared 16 bytes at a time
   uint4 *y16 = reinterpret_cast<uint4 *>(ys);
@@ -1347,8 +1378,8 @@ __device__ __forceinline__ EpiIn<T> epi_load(int node, const uint8_t *__restrict
 
 template <class T, int MODE, int S, int NT = TILE_THREADS, bool SPLIT = false, int SX = S>
 __device__ __forceinline__ void tile_finish(
-    int t, int n0, int nown, const int *__restrict__ comb_ptr, const int *__restrict__ comb_slot,
-    const float *__restrict__ comb_w, const uint8_t *__restrict__ bcmask, const T *xs, const T *ys,
+    int t, int n0, int nown, const int *__restrict__ comb_ptr, const uint4 *__restrict__ comb,
+    const uint8_t *__restrict__ bcmask, const T *xs, const T *ys,
     const T *__restrict__ x, const T *__restrict__ b, T *__restrict__ y, T *__restrict__ x_out,
     T *__restrict__ d, const T *__restrict__ dinv, double ca, double cc, int cflags,
     double *__restrict__ partials, double *red, int pstride = 0, bool hang = true) {
@@ -1369,6 +1400,15 @@ __device__ __forceinline__ void tile_finish(
 #pragma unroll
     for (int u = 0; u < 2; u++)
       ein[u] = epi_load<T, MODE>(n0 + min(i0 + u * NT, nown - 1), bcmask, x, b, d, dinv, cflags);
+    int cj[2][2] = {{0, 0}, {0, 0}};
+    if (hang) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int node = n0 + min(i0 + u * NT, nown - 1);
+        cj[u][0] = comb_ptr[node];
+        cj[u][1] = comb_ptr[node + 1];
+      }
+    }
 #pragma unroll
     for (int u = 0; u < 2; u++) {
       const int i = i0 + u * NT;
@@ -1382,13 +1422,20 @@ __device__ __forceinline__ void tile_finish(
       const T wv[3] = {e.w.a, e.w.b, e.w.c}, xv[3] = {e.x.a, e.x.b, e.x.c};
       const uint8_t m = e.m;
       T a[3] = {ys[pi], ys[pi + 1], ys[pi + 2]};
-      const int j0 = hang ? comb_ptr[node] : 0, j1 = hang ? comb_ptr[node + 1] : 0;
-      for (int j = j0; j < j1; j++) {
-        const int sl = comb_slot[j];
-        const T w = (T)comb_w[j];
-        a[0] += w * ys[S * sl];
-        a[1] += w * ys[S * sl + 1];
-        a[2] += w * ys[S * sl + 2];
+      // hanging slots that depend on the node, four packed entries a load
+      // (entry: slot, plus 2^16 for weight 1/2 or 2^17 for 1/4; 0 pads)
+      for (int j = cj[u][0]; j < cj[u][1]; j++) {
+        const uint4 q = comb[j];
+        const uint32_t en[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          if (en[k] >> 16) {
+            const int sl = S * (int)(en[k] & 0xffff);
+            const T w = (en[k] >> 17) ? T(0.25) : T(0.5);
+            a[0] += w * ys[sl];
+            a[1] += w * ys[sl + 1];
+            a[2] += w * ys[sl + 2];
+          }
       }
       T yo[3], dno[3];
 #pragma unroll
@@ -1603,9 +1650,8 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
     const int *__restrict__ node0, const int *__restrict__ ext_ptr, const int *__restrict__ ext,
     const int *__restrict__ nacc_dep, const int *__restrict__ el_ptr,
     const uint2 *__restrict__ el, int ncolors, const int *__restrict__ comb_ptr,
-    const int *__restrict__ comb_slot, const float *__restrict__ comb_w,
-    const int *__restrict__ dep_ptr, const int *__restrict__ dep_conn,
-    const float *__restrict__ dep_w, const uint8_t *__restrict__ bcmask,
+    const uint4 *__restrict__ comb, const int *__restrict__ extd_ptr,
+    const int4 *__restrict__ extd, const uint8_t *__restrict__ bcmask,
     const T *__restrict__ K0, const T *__restrict__ s_elem, const T *__restrict__ x,
     const T *__restrict__ b, T *__restrict__ y, T *__restrict__ x_out, T *__restrict__ d,
     const T *__restrict__ dinv, double ca, double cc, int cflags, double *__restrict__ partials,
@@ -1631,8 +1677,9 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
     if (partials) partials += (int64_t)blockIdx.y * gridDim.x;
   }
   const int n0 = node0[t], nown = node0[t + 1] - n0;
-  const int e0 = ext_ptr[t], next = ext_ptr[t + 1] - e0;
-  const int nslot = nown + next;
+  const int e0 = ext_ptr[t], nhalo = ext_ptr[t + 1] - e0;
+  const int d0 = extd_ptr[t], ndep = extd_ptr[t + 1] - d0;
+  const int nslot = nown + ndep + nhalo;
   const int nacc = nown + nacc_dep[t];
   T *xs = reinterpret_cast<T *>(smem_raw);
   T *ys = xs + SX * ((nslot + 7) & ~7);
@@ -1644,8 +1691,7 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
     w1 = el[3 * (size_t)(q0 + tid) + 1];
     w2 = el[3 * (size_t)(q0 + tid) + 2];
   }
-  tile_stage<T, SX, NT, S>(n0, nown, ext + e0, next, nacc, dep_ptr, dep_conn, dep_w,
-                                     bcmask, x, xs, ys);
+  tile_stage<T, SX, NT, S>(n0, nown, extd + d0, ndep, ext + e0, nhalo, nacc, bcmask, x, xs, ys);
   __syncthreads();
   for (int r0 = 0; r0 < nel; r0 += NT) {
     const int k = r0 + tid;
@@ -1706,9 +1752,9 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
       __syncthreads();
     }
   }
-  tile_finish<T, MODE, S, NT, false, SX>(t, n0, nown, comb_ptr, comb_slot, comb_w,
-                                                   bcmask, xs, ys, x, b, y, x_out, d, dinv, ca,
-                                                   cc, cflags, partials, red, 0, nacc > nown);
+  tile_finish<T, MODE, S, NT, false, SX>(t, n0, nown, comb_ptr, comb, bcmask, xs, ys, x, b, y,
+                                         x_out, d, dinv, ca, cc, cflags, partials, red, 0,
+                                         nacc > nown);
 }
 
 // ---------------------------------------------------------------------------
@@ -1766,11 +1812,10 @@ __device__ __forceinline__ void put_planes(uint2 *ph, int np, int pos, float vx,
   ph[pos + 2 * np] = make_uint2(l0, l1);
 }
 
-__device__ __forceinline__ void tile_stage_planes(int n0, int nown, const int *__restrict__ ext_l,
-                                                  int next, int nacc, int np,
-                                                  const int *__restrict__ dep_ptr,
-                                                  const int *__restrict__ dep_conn,
-                                                  const float *__restrict__ dep_w,
+__device__ __forceinline__ void tile_stage_planes(int n0, int nown,
+                                                  const int4 *__restrict__ extd_l, int ndep,
+                                                  const int *__restrict__ ext_l, int nhalo,
+                                                  int nacc, int np,
                                                   const uint8_t *__restrict__ bcmask,
                                                   const float *__restrict__ x, uint2 *ph,
                                                   float *ys) {
@@ -1794,10 +1839,17 @@ __device__ __forceinline__ void tile_stage_planes(int n0, int nown, const int *_
                    (mk[k] & 4) ? 0.0f : v[k][2]);
     }
   }
-  for (int i = tid; i < next; i += TILE_THREADS) {
+  for (int i = tid; i < ndep; i += TILE_THREADS) {
     float v[3];
-    load_node<float>(ext_l[i], x, dep_ptr, dep_conn, dep_w, bcmask, v);
+    load_dep<float>(extd_l[i], x, bcmask, v);
     put_planes(ph, np, tile_pos(nown + i), v[0], v[1], v[2]);
+  }
+  for (int i = tid; i < nhalo; i += TILE_THREADS) {
+    const int g = ext_l[i];
+    const Vec3<float> u = load_vec3(x + 3 * (size_t)g);
+    const uint8_t m = bcmask[g];
+    put_planes(ph, np, tile_pos(nown + ndep + i), (m & 1) ? 0.0f : u.a, (m & 2) ? 0.0f : u.b,
+               (m & 4) ? 0.0f : u.c);
   }
   for (int i = tid; i < 4 * ((nacc + 7) & ~7); i += TILE_THREADS) ys[i] = 0.0f;
 }
@@ -1807,9 +1859,8 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma(
     const int *__restrict__ node0, const int *__restrict__ ext_ptr, const int *__restrict__ ext,
     const int *__restrict__ nacc_dep, const int *__restrict__ mb_ptr,
     const uint32_t *__restrict__ mel, int ncolors, const uint4 *__restrict__ afrag,
-    const int *__restrict__ comb_ptr, const int *__restrict__ comb_slot,
-    const float *__restrict__ comb_w, const int *__restrict__ dep_ptr,
-    const int *__restrict__ dep_conn, const float *__restrict__ dep_w,
+    const int *__restrict__ comb_ptr, const uint4 *__restrict__ comb,
+    const int *__restrict__ extd_ptr, const int4 *__restrict__ extd,
     const uint8_t *__restrict__ bcmask, const float *__restrict__ s_elem,
     const float *__restrict__ x, const float *__restrict__ b, float *__restrict__ y,
     float *__restrict__ x_out, float *__restrict__ d, const float *__restrict__ dinv, double ca,
@@ -1831,8 +1882,9 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma(
   }
   const int en = lane & 15, g = lane >> 4;
   const int n0 = node0[t], nown = node0[t + 1] - n0;
-  const int e0 = ext_ptr[t], next = ext_ptr[t + 1] - e0;
-  const int nslot = nown + next;
+  const int e0 = ext_ptr[t], nhalo = ext_ptr[t + 1] - e0;
+  const int d0 = extd_ptr[t], ndep = extd_ptr[t + 1] - d0;
+  const int nslot = nown + ndep + nhalo;
   const int nacc = nown + nacc_dep[t];
   // LDS: x as three bf16 planes of np nodes (8 bytes per node each), then
   // the FP32 accumulators (16 bytes per node)
@@ -1860,7 +1912,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma(
   if (bb0 < bb1) load_rec(bb0, r0);
   if (bb0 + 1 < bb1) load_rec(bb0 + 1, r1);
   if (bb0 + 2 < bb1) load_rec(bb0 + 2, r2);
-  tile_stage_planes(n0, nown, ext + e0, next, nacc, np, dep_ptr, dep_conn, dep_w, bcmask, x, ph, ys);
+  tile_stage_planes(n0, nown, extd + d0, ndep, ext + e0, nhalo, nacc, np, bcmask, x, ph, ys);
   // A fragments of K0: [class][part hi, mid, lo][row block][lane]
   Frag a[3][2];
   if (SINGLE_CLASS) {
@@ -1958,7 +2010,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma(
   if (bt + 2 < bb1) step(bt + 2, r2, r3, r1, B0, B1);
   __syncthreads();
   tile_finish<float, MODE, 4, TILE_THREADS, true>(
-      t, n0, nown, comb_ptr, comb_slot, comb_w, bcmask, reinterpret_cast<const float *>(ph), ys, x,
+      t, n0, nown, comb_ptr, comb, bcmask, reinterpret_cast<const float *>(ph), ys, x,
       b, y, x_out, d, dinv, ca, cc, cflags, partials, red, np);
 }
 
@@ -1977,9 +2029,8 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma32(
     const int *__restrict__ node0, const int *__restrict__ ext_ptr, const int *__restrict__ ext,
     const int *__restrict__ nacc_dep, const int *__restrict__ mb_ptr,
     const uint32_t *__restrict__ mel, const float *__restrict__ afrag32,
-    const int *__restrict__ comb_ptr, const int *__restrict__ comb_slot,
-    const float *__restrict__ comb_w, const int *__restrict__ dep_ptr,
-    const int *__restrict__ dep_conn, const float *__restrict__ dep_w,
+    const int *__restrict__ comb_ptr, const uint4 *__restrict__ comb,
+    const int *__restrict__ extd_ptr, const int4 *__restrict__ extd,
     const uint8_t *__restrict__ bcmask, const float *__restrict__ x, const float *__restrict__ b,
     float *__restrict__ y, float *__restrict__ x_out, float *__restrict__ d,
     const float *__restrict__ dinv, double ca, double cc, int cflags,
@@ -2000,8 +2051,9 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma32(
   }
   const int en = lane & 15, g = lane >> 4;
   const int n0 = node0[t], nown = node0[t + 1] - n0;
-  const int e0 = ext_ptr[t], next = ext_ptr[t + 1] - e0;
-  const int nslot = nown + next;
+  const int e0 = ext_ptr[t], nhalo = ext_ptr[t + 1] - e0;
+  const int d0 = extd_ptr[t], ndep = extd_ptr[t + 1] - d0;
+  const int nslot = nown + ndep + nhalo;
   const int nacc = nown + nacc_dep[t];
   float *xs = reinterpret_cast<float *>(smem_raw);
   float *ys = xs + 3 * ((nslot + 7) & ~7);
@@ -2029,7 +2081,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma32(
   if (bb0 < bb1) load_rec(bb0, r0);
   if (bb0 + 1 < bb1) load_rec(bb0 + 1, r1);
   if (bb0 + 2 < bb1) load_rec(bb0 + 2, r2);
-  tile_stage<float, 3, TILE_THREADS, 4>(n0, nown, ext + e0, next, nacc, dep_ptr, dep_conn, dep_w,
+  tile_stage<float, 3, TILE_THREADS, 4>(n0, nown, extd + d0, ndep, ext + e0, nhalo, nacc,
                                         bcmask, x, xs, ys);
   // A fragments: [class][row block][step][lane]
   float a[2][6];
@@ -2122,7 +2174,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma32(
   if (bt + 1 < bb1) step(bt + 1, r1, r2, r0, B1, B0);
   if (bt + 2 < bb1) step(bt + 2, r2, r3, r1, B0, B1);
   __syncthreads();
-  tile_finish<float, MODE, 4, TILE_THREADS, false, 3>(t, n0, nown, comb_ptr, comb_slot, comb_w,
+  tile_finish<float, MODE, 4, TILE_THREADS, false, 3>(t, n0, nown, comb_ptr, comb,
                                                       bcmask, xs, ys, x, b, y, x_out, d, dinv, ca,
                                                       cc, cflags, partials, red);
 }
@@ -2145,7 +2197,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
   hipLaunchKernelGGL((k_tile_apply_mfma32<M, S>), grid, dim3(TILE_THREADS), sh3, st, tl.node0,  \
                      tl.ext_ptr, tl.ext, tl.nacc_dep, tl.mb_ptr,                                \
                      reinterpret_cast<const uint32_t *>(tl.mel), tl.afrag32, tl.comb_ptr,       \
-                     tl.comb_slot, tl.comb_w, tl.dep_ptr, tl.dep_conn, tl.dep_w, tl.bcmask,     \
+                     tl.comb, tl.extd_ptr, tl.extd, tl.bcmask,     \
                      (const float *)x, (const float *)b, (float *)y, (float *)xo, (float *)d,    \
                      (const float *)dinv, g.ca, g.cc, g.cflags, g.partials, vs, tl.run)
 #define TMRX_MTILE32B(M)    \
@@ -2171,7 +2223,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
   hipLaunchKernelGGL((k_tile_apply_mfma<M, S>), grid, dim3(TILE_THREADS), sh4, st,               \
                      tl.node0, tl.ext_ptr, tl.ext, tl.nacc_dep, tl.mb_ptr,                       \
                      reinterpret_cast<const uint32_t *>(tl.mel), tl.ncolors, tl.afrag, tl.comb_ptr, \
-                     tl.comb_slot, tl.comb_w, tl.dep_ptr, tl.dep_conn, tl.dep_w, tl.bcmask,      \
+                     tl.comb, tl.extd_ptr, tl.extd, tl.bcmask,      \
                      (const float *)s_elem, (const float *)x, (const float *)b, (float *)y,      \
                      (float *)xo, (float *)d, (const float *)dinv, g.ca, g.cc, g.cflags,          \
                      g.partials, vs, tl.run)
@@ -2203,7 +2255,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
   hipLaunchKernelGGL((k_tile_apply<T, M, S, N, NTH>), grid, dim3(NTH), sh, st, tl.node0,          \
                      tl.ext_ptr, tl.ext, tl.nacc_dep, tl.el_ptr,                                  \
                      reinterpret_cast<const uint2 *>(recs), tl.ncolors, tl.comb_ptr,              \
-                     tl.comb_slot, tl.comb_w, tl.dep_ptr, tl.dep_conn, tl.dep_w, tl.bcmask, K0,   \
+                     tl.comb, tl.extd_ptr, tl.extd, tl.bcmask, K0,   \
                      s_elem, x, b, y, xo, d, dinv, g.ca, g.cc, g.cflags, g.partials, vs, tl.run)
 #define TMRX_TILE(M, S)                    \
   if (tl.threads == 512) {                 \

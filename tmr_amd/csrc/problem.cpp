@@ -595,20 +595,26 @@ int Problem::build_tiles(int l) {
     for (int e = 0; e < ne; e++)
       for (int a = 0; a < 8; a++) iel[fill[xid(L.conn[8 * e + a])]++] = e;
   }
-  // parent -> hanging nodes
+  // parent -> hanging nodes.  A hanging node of a trilinear mesh sits in the
+  // middle of a coarser edge (two parents, 1/2) or face (four, 1/4); the
+  // kernels' packed records hold nothing else.
   std::vector<int> pptr(n + 1, 0), pdep;
-  std::vector<float> pw;
+  for (int d = 0; d < nd; d++) {
+    const int np = dptr[d + 1] - dptr[d];
+    bool ok = np == 2 || np == 4;
+    for (int j = dptr[d]; ok && j < dptr[d + 1]; j++) ok = dw[j] * np == 1.0 && dconn[j] >= 0;
+    if (!ok) {
+      last_error = "problem: a hanging node is not the mean of two or four nodes";
+      return -1;
+    }
+  }
   for (int j = 0; j < (nd ? dptr[nd] : 0); j++) pptr[dconn[j] + 1]++;
   for (int i = 0; i < n; i++) pptr[i + 1] += pptr[i];
   pdep.resize(pptr[n]);
-  pw.resize(pptr[n]);
   {
     std::vector<int> fill(pptr.begin(), pptr.end() - 1);
     for (int d = 0; d < nd; d++)
-      for (int j = dptr[d]; j < dptr[d + 1]; j++) {
-        pdep[fill[dconn[j]]] = d;
-        pw[fill[dconn[j]]++] = (float)dw[j];
-      }
+      for (int j = dptr[d]; j < dptr[d + 1]; j++) pdep[fill[dconn[j]]++] = d;
   }
   // tiles never straddle two independent components
   std::vector<int> tstart;
@@ -619,11 +625,11 @@ int Problem::build_tiles(int l) {
   }
   tstart.push_back(n);
   const int ntiles = (int)tstart.size() - 1;
-  std::vector<int> node0(ntiles + 1), ext_ptr{0}, ext, nacc(ntiles), el_ptr{0};
+  std::vector<int> node0(ntiles + 1), ext_ptr{0}, ext, extd_ptr{0}, extd, nacc(ntiles), el_ptr{0};
   std::vector<TileElem> els, mel;
   std::vector<int> mb_ptr((size_t)ntiles * (MFMA_WAVES + 1), 0);
-  std::vector<int> comb_ptr(n + 1, 0), comb_slot;
-  std::vector<float> comb_w;
+  std::vector<int> comb_ptr(n + 1, 0);
+  std::vector<uint32_t> comb;
   std::vector<int> stamp_n(n + nd, -1), slot(n + nd, 0), stamp_e(ne, -1);
   std::vector<uint32_t> col;
   int max_slots = 0, max_acc = 0, ncolors = 0, max_mrec = 0, max_rec = 0;
@@ -662,8 +668,22 @@ int Problem::build_tiles(int l) {
     for (int p = n0; p < n1; p++) add_elems(p);
     for (int d : rdeps) add_elems(n + d);
     std::sort(tel.begin(), tel.end());
-    for (int d : rdeps) ext.push_back(-(d + 1));
+    auto put_dep = [&](int d) {
+      const int *p = &dconn[dptr[d]];
+      const bool two = dptr[d + 1] - dptr[d] == 2;
+      for (int k = 0; k < 4; k++) extd.push_back(two && k > 1 ? -1 : p[k]);
+    };
+    for (int d : rdeps) put_dep(d);
     int ns = na;
+    // hanging slots first, so that a wave stages one kind of slot
+    for (int e : tel)
+      for (int a = 0; a < 8; a++) {
+        const int g = L.conn[8 * e + a];
+        if (g >= 0 || stamp_n[xid(g)] == t) continue;
+        stamp_n[xid(g)] = t;
+        slot[xid(g)] = ns++;
+        put_dep(-g - 1);
+      }
     const size_t el0 = els.size();
     for (int e : tel) {
       TileElem te{};
@@ -769,6 +789,7 @@ int Problem::build_tiles(int l) {
     }
     nacc[t] = (int)rdeps.size();
     ext_ptr.push_back((int)ext.size());
+    extd_ptr.push_back((int)(extd.size() / 4));
     el_ptr.push_back((int)els.size());
     max_slots = std::max(max_slots, ns);
     max_acc = std::max(max_acc, na);
@@ -779,10 +800,12 @@ int Problem::build_tiles(int l) {
     }
     for (int p = n0; p < n1; p++) {
       for (int j = pptr[p]; j < pptr[p + 1]; j++) {
-        comb_slot.push_back(tile_pos(slot[n + pdep[j]]));
-        comb_w.push_back(pw[j]);
+        const int d = pdep[j];
+        const uint32_t code = dptr[d + 1] - dptr[d] == 2 ? 1u << 16 : 1u << 17;
+        comb.push_back((uint32_t)tile_pos(slot[n + d]) | code);
       }
-      comb_ptr[p + 1] = (int)comb_slot.size();
+      while (comb.size() % 4) comb.push_back(0u);
+      comb_ptr[p + 1] = (int)(comb.size() / 4);
     }
   }
   node0[ntiles] = n;
@@ -797,15 +820,13 @@ int Problem::build_tiles(int l) {
       return -1;
     }
   }
-  if (comb_slot.empty()) {
-    comb_slot.push_back(0);
-    comb_w.push_back(0.0f);
-  }
+  if (comb.empty()) comb.assign(4, 0u);
+  if (extd.empty()) extd.assign(4, 0);
   if (ext.empty()) ext.push_back(0);
   if (L.t_node0.upload(node0) || L.t_ext_ptr.upload(ext_ptr) || L.t_ext.upload(ext) ||
       L.t_nacc.upload(nacc) || L.t_el_ptr.upload(el_ptr) || L.t_el.upload(els) ||
-      L.t_comb_ptr.upload(comb_ptr) || L.t_comb_slot.upload(comb_slot) ||
-      L.t_comb_w.upload(comb_w) || L.t_mb_ptr.upload(mb_ptr) || L.t_mel.upload(mel)) {
+      L.t_extd_ptr.upload(extd_ptr) || L.t_extd.upload(extd) ||
+      L.t_comb_ptr.upload(comb_ptr) || L.t_comb.upload(comb) || L.t_mb_ptr.upload(mb_ptr) || L.t_mel.upload(mel)) {
     last_error = "problem: device allocation failed";
     return -1;
   }
@@ -836,11 +857,9 @@ int Problem::build_tiles(int l) {
   T.el_ptr = L.t_el_ptr.p;
   T.el = L.t_el.p;
   T.comb_ptr = L.t_comb_ptr.p;
-  T.comb_slot = L.t_comb_slot.p;
-  T.comb_w = L.t_comb_w.p;
-  T.dep_ptr = L.dep_ptr.p;
-  T.dep_conn = L.dep_conn.p;
-  T.dep_w = L.dep_w.p;
+  T.comb = reinterpret_cast<const uint4 *>(L.t_comb.p);
+  T.extd_ptr = L.t_extd_ptr.p;
+  T.extd = reinterpret_cast<const int4 *>(L.t_extd.p);
   T.bcmask = L.d_bcmask.p;
   T.mb_ptr = L.t_mb_ptr.p;
   T.mel = L.t_mel.p;

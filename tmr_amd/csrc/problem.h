@@ -143,10 +143,10 @@ struct Level {
   DevArray<int> t_mb_ptr;
   DevArray<TileElem> t_mel;
   DevArray<int> t_mel_elem;
-  DevArray<int> t_node0, t_ext_ptr, t_ext, t_nacc, t_el_ptr, t_comb_ptr, t_comb_slot;
+  DevArray<int> t_node0, t_ext_ptr, t_ext, t_extd_ptr, t_extd, t_nacc, t_el_ptr, t_comb_ptr;
+  DevArray<uint32_t> t_comb;
   DevArray<TileElem> t_el, t_el32;
   DevArray<int> t_el_elem;
-  DevArray<float> t_comb_w;
   Tiles tiles;
   // transfer to the next coarser level (P: rows = this level's nodes)
   DevArray<int> P_ptr, P_col, R_ptr, R_col;
