@@ -1,0 +1,46 @@
+"""Owner tiles over their sizes and FP32 operator forms: the product against
+the oracle's FP64 operator on forests with and without hanging nodes."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as po
+from tmr_amd import solver, workloads
+
+pytestmark = pytest.mark.gpu
+
+Q, K0 = 3.0, 1e-6
+
+
+@pytest.fixture(scope="module")
+def meshes():
+    out = {}
+    for name, (forests, rho, _) in (
+            ("adaptive", workloads.adaptive(seed=5, base_level=2, max_level=4, nlevels=2)),
+            ("cube", workloads.cube_l4(2))):
+        orc = po.from_forest(forests[0], [("fixed", 7)])
+        orc.assemble(rho ** Q + K0)
+        prob = solver.Problem(forests, q=Q, k0=K0, bcs=[("fixed", 7)])
+        prob.set_design(rho)
+        x = np.random.default_rng(3).standard_normal(prob.ndof)
+        out[name] = (prob, x, orc.matvec(x))
+    return out
+
+
+# 64: many small tiles; 100: ends inside a wave; 512: several rounds per
+# thread; 800: tiles of 512 threads
+@pytest.mark.parametrize("tile", [0, 64, 100, 512, 800])
+@pytest.mark.parametrize("name", ["adaptive", "cube"])
+def test_product_over_tile_sizes_and_forms(name, tile, meshes):
+    prob, x, ref = meshes[name]
+    if tile:
+        prob.set_tiling(tile)
+    print(name, tile, prob.tile_info(0), flush=True)
+    # FP64 to rounding; plain FP32 sums of about 80 terms; three bf16 parts
+    # keep 24 bits of each operand but drop products below 2^-16
+    for form, precision, bound in ((0, 0, 1e-13), (0, 1, 1e-5), (1, 1, 1e-4), (2, 1, 1e-5)):
+        prob.set_fp32_form(form)
+        y = prob.apply(x, precision=precision)
+        e = np.linalg.norm(y - ref) / np.linalg.norm(ref)
+        print("  form %d precision %d: %.2e" % (form, precision, e), flush=True)
+        assert e < bound
+    prob.set_fp32_form(0)

@@ -34,6 +34,22 @@ static int coarse_tile_nodes(int fine_tile, int n_nodes) {
   return t;
 }
 
+// Owner-tile size of the finest level until autotune or set_tiling chooses
+// one.  A tile's element phase is a chain of colour phases behind barriers,
+// so the chip wants at least a thousand tiles before tiles grow (their halo
+// shrinks with size).  Per PCG iteration, FP32 / FP64 V-cycle: adaptive
+// 880,983 nodes 979 / 1278 us at 256, 977 / 1319 at 128, 1097 / 1478 at 512;
+// adaptive 167,384 nodes 381 / 414 at 128, 424 / 505 at 512; adaptive 32,858
+// nodes 252 / 245 at 96, 321 / 322 at 512; box 545,025 nodes 359 / 378 at
+// 256, 351 / 395 at 512.  Very large uniform levels amortise 1024-node tiles
+// (4,276,737 nodes: 582 us of finest-level launches an iteration against 695
+// at 256); with hanging nodes those would not fit in LDS.
+static int default_tile_nodes(int n_nodes, bool hanging) {
+  if (!hanging && n_nodes >= 2048 * 1024) return 1024;
+  if (n_nodes >= 1000 * 256) return 256;
+  return n_nodes >= 500 * 128 ? 128 : 96;
+}
+
 void Problem::drop_graphs() {
   for (int k = 0; k < 2; k++)
     if (gexec_[k]) {
@@ -320,7 +336,8 @@ int Problem::init(int nlevels, Forest **forests, const Material &mat, int nbcs,
     L.cls.resize(octs.size());
     for (size_t e = 0; e < octs.size(); e++) L.cls[e] = block_cls[l][octs[e].block];
     if (build_level(l, nbcs, names, dof_masks)) return -1;
-    if (l > 0) L.tile_nodes = coarse_tile_nodes(levels_[0].tile_nodes, L.n_nodes);
+    L.tile_nodes = l > 0 ? coarse_tile_nodes(TILE_NODES, L.n_nodes)
+                         : default_tile_nodes(L.n_nodes, L.n_dep > 0);
     if (build_tiles(l)) return -1;
   }
   for (int l = 0; l + 1 < nlevels; l++)
@@ -731,12 +748,12 @@ int Problem::build_tiles(int l) {
     std::stable_sort(els.begin() + el0, els.end(), [](const TileElem &a, const TileElem &b) {
       return a.color != b.color ? a.color < b.color : a.mask > b.mask;
     });
-    // matrix-core batches: each of the MFMA_WAVES waves owns a contiguous
-    // share of the owned nodes (and the hanging nodes whose first owned
+    // matrix-core batches (when a matrix-core form has been asked for): each
+    // of the MFMA_WAVES waves owns a contiguous share of the owned nodes (and the hanging nodes whose first owned
     // parent it owns) and takes every element touching them, with the rows
     // of those corners only; per wave, records are coloured over its
     // corners and (colour, class) groups are padded to 16 records
-    {
+    if (mfma_tiles_) {
       auto wave_of = [&](int pos) {
         const int sl = tile_pos(pos);  // tile_pos is an involution
         return sl < nown ? sl / qw : (sl < na ? rdep_wave[sl - nown] : -1);
@@ -794,7 +811,7 @@ int Problem::build_tiles(int l) {
     max_slots = std::max(max_slots, ns);
     max_acc = std::max(max_acc, na);
     max_rec = std::max(max_rec, (int)(els.size() - el0));
-    {
+    if (mfma_tiles_) {
       const int *cp = &mb_ptr[(size_t)t * (MFMA_WAVES + 1)];
       max_mrec = std::max(max_mrec, 16 * (cp[MFMA_WAVES] - cp[0]));
     }
@@ -814,8 +831,8 @@ int Problem::build_tiles(int l) {
     std::vector<int> na_t(ntiles);
     for (int t = 0; t < ntiles; t++) na_t[t] = node0[t + 1] - node0[t] + nacc[t];
     std::string err;
-    if (check_tile_schedule(ntiles, el_ptr.data(), els.data(), na_t.data(), MFMA_WAVES,
-                            mb_ptr.data(), mel.data(), err)) {
+    if (check_tile_schedule(ntiles, el_ptr.data(), els.data(), na_t.data(),
+                            mfma_tiles_ ? MFMA_WAVES : 0, mb_ptr.data(), mel.data(), err)) {
       last_error = "problem: tile schedule check failed: " + err;
       return -1;
     }
@@ -874,7 +891,7 @@ int Problem::build_tiles(int l) {
   }
   T.afrag = reinterpret_cast<const uint4 *>(afrag_.p);
   T.afrag32 = afrag32_.p;
-  T.use_mfma = true;
+  T.use_mfma = mfma_tiles_;
   return 0;
 }
 
@@ -1147,8 +1164,9 @@ int Problem::set_design(const double *rho, int n, bool on_device) {
                           Cc.d_lev.p, Cc.s64.p, Cc.s32.p, st_);
   }
   for (auto &L : levels_) {
-    launch_rec_scale(L.tiles.n_mrec, L.tiles.mel_elem, L.s32.p,
-                     reinterpret_cast<uint32_t *>(L.tiles.mel), st_);
+    if (fp32_mfma_)
+      launch_rec_scale(L.tiles.n_mrec, L.tiles.mel_elem, L.s32.p,
+                       reinterpret_cast<uint32_t *>(L.tiles.mel), st_);
     launch_rec_scale(L.tiles.n_rec, L.tiles.el_elem, L.s32.p,
                      reinterpret_cast<uint32_t *>(L.tiles.el32), st_);
   }
@@ -2451,11 +2469,29 @@ int Problem::set_tiling(int tile_nodes) {
   return 0;
 }
 
+// The matrix-core batches of every level's tiles are only built once a
+// matrix-core form is asked for.
+int Problem::ensure_mfma_tiles() {
+  if (mfma_tiles_) return 0;
+  mfma_tiles_ = true;
+  for (size_t l = 0; l < levels_.size(); l++)
+    if (build_tiles((int)l)) return -1;
+  return 0;
+}
+
 int Problem::set_fp32_form(int form) {
   if (form < 0 || form > 2) {
     last_error = "set_fp32_form: form must be 0 (vector ALUs), 1 (matrix cores, bf16 split) or 2 "
                  "(matrix cores, FP32 inputs)";
     return -1;
+  }
+  if (form != 0) {
+    if (ensure_mfma_tiles()) return -1;
+    // set_design keeps their scales current only while a matrix-core form is on
+    if (have_design_ && design_mode_ == 0)
+      for (auto &L : levels_)
+        launch_rec_scale(L.tiles.n_mrec, L.tiles.mel_elem, L.s32.p,
+                         reinterpret_cast<uint32_t *>(L.tiles.mel), st_);
   }
   fp32_mfma_ = form != 0;
   fp32_mfma_in32_ = form == 2;
@@ -2500,6 +2536,7 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
   HIPCHK(hipEventCreate(&e1));
   const bool keep_valu = fp32_valu_, keep_mfma = fp32_mfma_, keep_in32 = fp32_mfma_in32_;
   fp32_valu_ = false;
+  mfma_tiles_ = true;  // every form is timed
   int dev = 0, max_lds = 0;
   HIPCHK(hipGetDevice(&dev));
   HIPCHK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));

@@ -124,7 +124,7 @@ struct Level {
   // nodes [seg_node0[s], seg_node0[s+1]) belong to component s, owner
   // tiles [seg_tile[s], seg_tile[s+1]) hold them
   std::vector<int> seg_node0, seg_tile;
-  int tile_nodes = TILE_NODES;  // owner-tile size (autotuned)
+  int tile_nodes = TILE_NODES;  // owner-tile size
   // host copies
   std::vector<int16_t> lev;
   std::vector<int> cls;
@@ -435,7 +435,13 @@ class Problem {
   double last_stress_sum_ = 0.0;
   hipStream_t st_ = nullptr;
   bool fp32_valu_ = false;  // FP32 operator on the vector ALUs
-  bool fp32_mfma_ = true;   // autotuned: FP32 operator on the matrix cores
+  // FP32 operator on the matrix cores.  The vector ALUs are the default: the
+  // autotuner has chosen them on every workload (finest-level Chebyshev step,
+  // 512-node tiles, vector / bf16 split / FP32 MFMA: 4.2M-hex box 114 / 189 /
+  // 202 us; adaptive 1.2M hex 106 / 175 us for the first two).
+  bool fp32_mfma_ = false;
+  bool mfma_tiles_ = false;      // tiles carry matrix-core batches
+  int ensure_mfma_tiles();
   bool fp32_mfma_in32_ = false;  // ... with FP32 inputs (else bf16 three-way split)
   int timing_ = 0;  // mask of the timed launch modes (bit m = AsmMode m)
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_pool_;
