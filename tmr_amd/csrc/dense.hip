@@ -1,478 +1,428 @@
-// Coarsest-level direct solve on the GPU: blocked FP64 Cholesky A = L L^T of
-// a dense symmetric matrix and the explicit inverse A^-1 = L^-T L^-1 (the
-// coarse solve of every V-cycle is then one GEMV, launch_dense_solve).
-// Replaces TACSMg's direct coarse solve (src/TMR_RefinementTools.cpp:83-86).
+// Coarsest-level direct solve on the GPU.  Replaces TACSMg's direct coarse
+// solve (src/TMR_RefinementTools.cpp:83-86).
 //
-// Matrices are row-major mp x mp with mp a multiple of DB (padding rows and
-// columns hold the identity), processed in DB x DB blocks:
-//   Cholesky (right-looking): factor block (k,k); solve the panel below it;
-//     update the trailing lower blocks;
-//   L^-1 = X: X[i][i] = L[i][i]^-1 and, right-looking over k,
-//     X[i][j] = -X[i][i] sum_{k=j}^{i-1} L[i][k] X[k][j];
-//   A^-1 = X^T X, lower blocks then mirrored, written into the m x m result.
+// Explicit inverses of dense SPD matrices, many at once, by blocked
+// Gauss-Jordan: step k turns every 64 x 64 block of A into
+//   A_kk <- P = A_kk^-1,  A_kj <- P A_kj,  A_ik <- -A_ik P,
+//   A_ij <- A_ij - A_ik (P A_kj),
+// and after the last block A holds A^-1.  No pivoting: the pivots are those
+// of the Cholesky factorisation of an SPD matrix.  A step is one launch over
+// all blocks of all matrices, from one buffer to the other, and the
+// workgroup that produces block (k + 1, k + 1) also inverts it, so that a
+// matrix of nb blocks takes nb + 1 launches.  What bounds it at the sizes of
+// a coarse level is that chain: the 64 dependent pivots of a block (in
+// registers, one barrier each) and the launch, not the arithmetic (FP64
+// matrix cores).  It replaced blocked Cholesky, L^-1 and L^-T L^-1 (about
+// five launches a block column, 54 us of them for the diagonal factor in
+// LDS).
+//
+// Matrices of coarse_schur_min dofs and more are first split by
+// substructuring (coarse.cpp): leaves D_i, separator S,
+//   W_i^T = E_i^T D_i^-1,  S <- S - sum_i E_i^T W_i,
+// all products through k_gemm_nt, and the solve goes through D_i^-1, W_i and
+// S^-1 (k_coarse_rows).
 #include <hip/hip_runtime.h>
-#include <rocblas/rocblas.h>
 
 #include "kernels.h"
 
 namespace tmrx {
 
-constexpr int DB = 64;  // block size
-constexpr int DT = 256;  // threads per workgroup
-
-// factor the diagonal block k in LDS; *bad = 1 on a non-positive pivot
-__global__ void __launch_bounds__(DT) k_potrf_diag(double *__restrict__ W, int mp, int k,
-                                                   int *bad) {
-  __shared__ double a[DB][DB + 1];
-  const int tid = threadIdx.x;
-  double *blk = W + (size_t)(k * DB) * mp + k * DB;
-  for (int t = tid; t < DB * DB; t += DT) a[t / DB][t % DB] = blk[(size_t)(t / DB) * mp + t % DB];
-  __syncthreads();
-  for (int j = 0; j < DB; j++) {
-    const double d = a[j][j];
-    __syncthreads();
-    if (!(d > 0.0)) {
-      if (tid == 0) atomicOr(bad, 1);
-      return;
-    }
-    const double s = sqrt(d);
-    if (tid == 0) a[j][j] = s;
-    for (int i = j + 1 + tid; i < DB; i += DT) a[i][j] /= s;
-    __syncthreads();
-    // trailing update of the lower part: a[i][l] -= a[i][j] a[l][j], j < l <= i
-    // (thread: row i = tid / 4, columns l = j + 1 + tid % 4, step 4)
-    {
-      const int i = tid >> 2;
-      if (i > j) {
-        const double aij = a[i][j];
-        for (int l = j + 1 + (tid & 3); l <= i; l += 4) a[i][l] -= aij * a[l][j];
-      }
-    }
-    __syncthreads();
-  }
-  for (int t = tid; t < DB * DB; t += DT) {
-    const int i = t / DB, l = t % DB;
-    blk[(size_t)i * mp + l] = l <= i ? a[i][l] : 0.0;
-  }
-}
-
-// rows below block k: x L_kk^T = a, one row per thread
-__global__ void __launch_bounds__(DT) k_trsm_panel(double *__restrict__ W, int mp, int k) {
-  __shared__ double L[DB][DB + 1];
-  const int tid = threadIdx.x;
-  const double *lk = W + (size_t)(k * DB) * mp + k * DB;
-  for (int t = tid; t < DB * DB; t += DT) L[t / DB][t % DB] = lk[(size_t)(t / DB) * mp + t % DB];
-  __syncthreads();
-  const int r = (k + 1) * DB + blockIdx.x * DT + tid;
-  if (r >= mp) return;
-  double *row = W + (size_t)r * mp + k * DB;
-  double x[DB];
-#pragma unroll
-  for (int j = 0; j < DB; j++) x[j] = row[j];
-#pragma unroll
-  for (int j = 0; j < DB; j++) {
-    double v = x[j];
-#pragma unroll
-    for (int t = 0; t < j; t++) v -= x[t] * L[j][t];
-    x[j] = v / L[j][j];
-  }
-#pragma unroll
-  for (int j = 0; j < DB; j++) row[j] = x[j];
-}
-
-// C[I][J] -= A[I][k] A[J][k]^T for the trailing lower blocks I >= J > k
-__global__ void __launch_bounds__(DT) k_syrk_trailing(double *__restrict__ W, int mp, int k) {
-  __shared__ double PI[DB][DB + 1], PJ[DB][DB + 1];
-  // lower-triangle tile index -> (I, J) over the T = nblk - k - 1 trailing blocks
-  const int t = blockIdx.x;
-  int I = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
-  while ((I + 1) * (I + 2) / 2 <= t) I++;
-  while (I * (I + 1) / 2 > t) I--;
-  const int J = t - I * (I + 1) / 2;
-  const int bi = (k + 1 + I) * DB, bj = (k + 1 + J) * DB, bk = k * DB;
-  const int tid = threadIdx.x;
-  for (int q = tid; q < DB * DB; q += DT) {
-    PI[q / DB][q % DB] = W[(size_t)(bi + q / DB) * mp + bk + q % DB];
-    PJ[q / DB][q % DB] = W[(size_t)(bj + q / DB) * mp + bk + q % DB];
-  }
-  __syncthreads();
-  // 4 x 4 outputs per thread
-  const int r0 = (tid / 16) * 4, c0 = (tid % 16) * 4;
-  double acc[4][4] = {};
-  for (int kk = 0; kk < DB; kk++) {
-    double a[4], b[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      a[u] = PI[r0 + u][kk];
-      b[u] = PJ[c0 + u][kk];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) acc[u][v] += a[u] * b[v];
-  }
-#pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) W[(size_t)(bi + r0 + u) * mp + bj + c0 + v] -= acc[u][v];
-}
-
-// X[i][i] = L[i][i]^-1 (lower) for every diagonal block i = blockIdx.x:
-// column c solves L x = e_c
-__global__ void __launch_bounds__(DB) k_trtri_diag(const double *__restrict__ W,
-                                                   double *__restrict__ X, int mp) {
-  __shared__ double L[DB][DB + 1];
-  const int i = blockIdx.x;
-  const int tid = threadIdx.x;
-  const size_t o = (size_t)(i * DB) * mp + i * DB;
-  for (int t = tid; t < DB * DB; t += DB) L[t / DB][t % DB] = W[o + (size_t)(t / DB) * mp + t % DB];
-  __syncthreads();
-  const int c = tid;
-  double x[DB];
-#pragma unroll
-  for (int r = 0; r < DB; r++) {
-    double v = r == c ? 1.0 : 0.0;
-#pragma unroll
-    for (int t = 0; t < r; t++) v -= L[r][t] * x[t];
-    x[r] = r < c ? 0.0 : v / L[r][r];
-  }
-#pragma unroll
-  for (int r = 0; r < DB; r++) X[o + (size_t)r * mp + c] = x[r];
-}
-
-// zero the strictly lower blocks of X (the accumulators of the right-looking
-// inverse below)
-__global__ void k_trtri_zero(int mp, double *__restrict__ X) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)mp * mp) return;
-  const int r = (int)(t / mp), c = (int)(t % mp);
-  if (r / DB > c / DB) X[t] = 0.0;
-}
-
-// Right-looking L^-1, step k: every block (i, j), i > k >= j, takes
-// X[i][j] -= L[i][k] X[k][j]; row k + 1 has then received all its terms and
-// is finished in the same pass, X[k+1][j] = X[k+1][k+1] X[k+1][j].  After
-// step k rows 0..k+1 are final, so each step is one launch of
-// (nblk - 1 - k) (k + 1) independent block products.
-__global__ void __launch_bounds__(DT) k_trtri_step(const double *__restrict__ W,
-                                                   double *__restrict__ X, int mp, int k) {
-  __shared__ double A[DB][DB + 1], B[DB][DB + 1];
-  const int t = blockIdx.x;
-  const int i = k + 1 + t / (k + 1), j = t % (k + 1);
-  const int tid = threadIdx.x;
-  const int r0 = (tid / 16) * 4, c0 = (tid % 16) * 4;
-  for (int q = tid; q < DB * DB; q += DT) {
-    A[q / DB][q % DB] = W[(size_t)(i * DB + q / DB) * mp + k * DB + q % DB];
-    B[q / DB][q % DB] = X[(size_t)(k * DB + q / DB) * mp + j * DB + q % DB];
-  }
-  __syncthreads();
-  double acc[4][4];
-#pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-      acc[u][v] = X[(size_t)(i * DB + r0 + u) * mp + j * DB + c0 + v];
-  for (int kk = 0; kk < DB; kk++) {
-    double a[4], b[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      a[u] = A[r0 + u][kk];
-      b[u] = B[kk][c0 + u];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) acc[u][v] -= a[u] * b[v];
-  }
-  if (i != k + 1) {
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) X[(size_t)(i * DB + r0 + u) * mp + j * DB + c0 + v] = acc[u][v];
-    return;
-  }
-  // the last term of row k + 1: X[k+1][j] = X[k+1][k+1] acc
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) B[r0 + u][c0 + v] = acc[u][v];
-  for (int q = tid; q < DB * DB; q += DT)
-    A[q / DB][q % DB] = X[(size_t)(i * DB + q / DB) * mp + i * DB + q % DB];
-  __syncthreads();
-  double out[4][4] = {};
-  for (int kk = 0; kk < DB; kk++) {
-    double a[4], b[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      a[u] = A[r0 + u][kk];
-      b[u] = B[kk][c0 + u];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) out[u][v] += a[u] * b[v];
-  }
-#pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) X[(size_t)(i * DB + r0 + u) * mp + j * DB + c0 + v] = out[u][v];
-}
-
-// A^-1[I][J] = sum_{k >= I} X[k][I]^T X[k][J] for I >= J (X lower); the m x m
-// result (row-major) takes both the block and its mirror
-__global__ void __launch_bounds__(DT) k_gram(const double *__restrict__ X, int mp, int nblk,
-                                             int m, double *__restrict__ out) {
-  __shared__ double A[DB][DB + 1], B[DB][DB + 1];
-  const int t = blockIdx.x;
-  int I = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
-  while ((I + 1) * (I + 2) / 2 <= t) I++;
-  while (I * (I + 1) / 2 > t) I--;
-  const int J = t - I * (I + 1) / 2;
-  const int tid = threadIdx.x;
-  const int r0 = (tid / 16) * 4, c0 = (tid % 16) * 4;
-  double acc[4][4] = {};
-  for (int k = I; k < nblk; k++) {
-    __syncthreads();
-    for (int q = tid; q < DB * DB; q += DT) {
-      A[q / DB][q % DB] = X[(size_t)(k * DB + q / DB) * mp + I * DB + q % DB];
-      B[q / DB][q % DB] = X[(size_t)(k * DB + q / DB) * mp + J * DB + q % DB];
-    }
-    __syncthreads();
-    for (int kk = 0; kk < DB; kk++) {
-      double a[4], b[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        a[u] = A[kk][r0 + u];
-        b[u] = B[kk][c0 + u];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) acc[u][v] += a[u] * b[v];
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int r = I * DB + r0 + u, c = J * DB + c0 + v;
-      if (r < m && c < m) {
-        out[(size_t)r * m + c] = acc[u][v];
-        out[(size_t)c * m + r] = acc[u][v];
-      }
-    }
-}
-
-// zero the dense matrix, identity on the padding rows (r >= m)
-__global__ void k_dense_fill(int64_t total, int mp, int m, double *__restrict__ W) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= total) return;
-  const int r = (int)(t / mp), c = (int)(t % mp);
-  W[t] = (r >= m && r == c) ? 1.0 : 0.0;
-}
-
-// one thread per block of the component's block rows
-__global__ void k_bsr_scatter(const int *__restrict__ col, const double *__restrict__ val, int n0,
-                              int k0, int k1, const int *__restrict__ rowof, int mp,
-                              double *__restrict__ W) {
-  const int k = k0 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= k1) return;
-  const int i = rowof[k] - n0, j = col[k] - n0;
-  const double *v = val + 9 * (size_t)k;
-  for (int p = 0; p < 3; p++)
-    for (int q = 0; q < 3; q++) W[(size_t)(3 * i + p) * mp + 3 * j + q] = v[3 * p + q];
-}
-
-// ---------------------------------------------------------------------------
-// Large matrices (m >= DENSE_BIG): the same factorisation by recursive
-// halving at multiples of 256, with 256 x 256 diagonal blocks factored and
-// inverted by the kernels above (as matrices of their own) and everything
-// else in plain FP64 GEMMs (rocBLAS), large enough to fill the device:
-//   cholinv(A) = (L, X = L^-1): for A = [A11 .; A21 A22],
-//     (L11, X11) = cholinv(A11); L21 = A21 X11^T; A22 -= L21 L21^T;
-//     (L22, X22) = cholinv(A22); X21 = -X22 (L21 X11);
-//   gram(c) = the lower part of X[c:, c:]^T X[c:, c:] (X lower), by halving
-//     the block columns: G22 = gram(second half), G21 = X22^T X21 over all
-//     rows below, G11 = gram(first half).
-// The factor and the inverse live in W and X; A21 is parked in the free
-// block of X where X21 goes, and L21 X11 (transposed) in the unused upper
-// block of W, so no GEMM works in place.
-constexpr int DS = 256;          // diagonal block of the recursion
-constexpr int DENSE_BIG = 2048;  // matrices from this size take this path
-constexpr int GRAM_LEAF = 1024;  // gram: blocks up to this size in one GEMM
-
-// out (m x m) = the lower part of G (mp x mp, row-major) and its mirror
-__global__ void k_dense_mirror(const double *__restrict__ G, int mp, int m, double *__restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)m * m) return;
-  const int r = (int)(t / m), c = (int)(t % m);
-  out[t] = r >= c ? G[(size_t)r * mp + c] : G[(size_t)c * mp + r];
-}
-
 namespace {
 
-// row-major C (M x N) = alpha op(A) op(B) + beta C on a column-major GEMM:
-// C^T = op(B)^T op(A)^T
-bool gemm_rm(rocblas_handle h, bool ta, bool tb, int M, int N, int K, double alpha,
-             const double *A, int lda, const double *B, int ldb, double beta, double *C,
-             int ldc) {
-  if (M <= 0 || N <= 0) return true;
-  return rocblas_dgemm(h, tb ? rocblas_operation_transpose : rocblas_operation_none,
-                       ta ? rocblas_operation_transpose : rocblas_operation_none, N, M, K, &alpha,
-                       B, ldb, A, lda, &beta, C, ldc) == rocblas_status_success;
+constexpr int DB = 64;   // block size
+constexpr int DT = 256;  // threads per workgroup
+// LDS leading dimensions of the matrix-core operands (doubles): rows of a
+// half wave's 16 x 2 read fall into distinct banks
+constexpr int LDA = 66;  // read as [row][k]
+constexpr int LDB = 80;  // read as [k][col]
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// wave w of four takes the 32 x 32 quadrant (w / 2, w % 2) of a 64 x 64
+// product over 64 inner indices: acc += A B, A[row][k] with leading dimension
+// LDA, B[k][col] with LDB, or (NT) B[col][k] with LDA
+template <bool NT>
+__device__ __forceinline__ void quad_product(const double *A, const double *B, f64x4 acc[2][2]) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int r = 32 * (w >> 1) + (lane & 15), c = 32 * (w & 1) + (lane & 15), g = lane >> 4;
+#pragma unroll 4
+  for (int k = 0; k < DB; k += 4) {
+    double a[2], b[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      a[u] = A[(r + 16 * u) * LDA + k + g];
+      b[u] = NT ? B[(c + 16 * u) * LDA + k + g] : B[(k + g) * LDB + c + 16 * u];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int v = 0; v < 2; v++)
+        acc[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[v], acc[u][v], 0, 0, 0);
+  }
+}
+// row and column in the 64 x 64 block of element e of acc[u][v]
+__device__ __forceinline__ int quad_row(int u, int e) {
+  return 32 * (threadIdx.x >> 7) + 16 * u + 4 * e + ((threadIdx.x & 63) >> 4);
+}
+__device__ __forceinline__ int quad_col(int v) {
+  return 32 * ((threadIdx.x >> 6) & 1) + 16 * v + (threadIdx.x & 15);
 }
 
-bool copy2d(double *dst, int ldd, const double *src, int lds, int rows, int cols, hipStream_t st) {
-  return hipMemcpy2DAsync(dst, sizeof(double) * ldd, src, sizeof(double) * lds,
-                          sizeof(double) * cols, rows, hipMemcpyDeviceToDevice, st) == hipSuccess;
+// 64 x 64 block (leading dimension ld) into LDS
+template <int LD>
+__device__ __forceinline__ void stage_block(const double *__restrict__ src, int64_t ld, double *dst) {
+#pragma unroll
+  for (int t = threadIdx.x; t < DB * DB; t += DT) dst[(t >> 6) * LD + (t & 63)] = src[(t >> 6) * ld + (t & 63)];
 }
 
-struct Dense {
-  rocblas_handle h;
-  hipStream_t st;
-  double *W, *X, *D, *Xs;  // D, Xs: DS x DS work of the diagonal blocks
-  int ld;
-  int *bad;
-  double *at(double *M, int r, int c) const { return M + (size_t)r * ld + c; }
-
-  // L (lower) and L^-1 of the DS x DS block at (o, o)
-  bool leaf(int o) {
-    const int nblk = DS / DB;
-    if (!copy2d(D, DS, at(W, o, o), ld, DS, DS, st)) return false;
-    for (int k = 0; k < nblk; k++) {
-      hipLaunchKernelGGL(k_potrf_diag, dim3(1), dim3(DT), 0, st, D, DS, k, bad);
-      const int rows = DS - (k + 1) * DB;
-      if (rows > 0) {
-        hipLaunchKernelGGL(k_trsm_panel, dim3((rows + DT - 1) / DT), dim3(DT), 0, st, D, DS, k);
-        const int T = nblk - k - 1;
-        hipLaunchKernelGGL(k_syrk_trailing, dim3(T * (T + 1) / 2), dim3(DT), 0, st, D, DS, k);
+// in-place inverse of the SPD block in `blk` (LDS, leading dimension LDA),
+// written to out (row-major 64 x 64): a 4 x 4 piece per thread in registers,
+// the pivot row and column through LDS (buf: 256 doubles, two sets in turn,
+// so one barrier a pivot)
+__device__ __forceinline__ void invert_block(const double *blk, double *buf, double *__restrict__ out,
+                                             int *bad) {
+  const int tr = threadIdx.x >> 4, tc = threadIdx.x & 15;
+  double a[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) a[i][j] = blk[(4 * tr + i) * LDA + 4 * tc + j];
+  bool neg = false;
+  for (int kb = 0; kb < DB / 4; kb++) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      double *row = buf + 128 * (q & 1), *col = row + 64;
+      if (tr == kb)
+#pragma unroll
+        for (int j = 0; j < 4; j++) row[4 * tc + j] = a[q][j];
+      if (tc == kb)
+#pragma unroll
+        for (int i = 0; i < 4; i++) col[4 * tr + i] = a[i][q];
+      __syncthreads();
+      const double p = row[4 * kb + q];
+      double rv[4], cv[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) rv[j] = row[4 * tc + j];
+#pragma unroll
+      for (int i = 0; i < 4; i++) cv[i] = col[4 * tr + i];
+      if (!(p > 0.0)) neg = true;
+      // 1 / p by two Newton steps from the hardware estimate: the division's
+      // range scaling would lengthen every pivot's chain
+      double d = __builtin_amdgcn_rcp(p);
+      d = __builtin_fma(__builtin_fma(-p, d, 1.0), d, d);
+      d = __builtin_fma(__builtin_fma(-p, d, 1.0), d, d);
+#pragma unroll
+      for (int j = 0; j < 4; j++) rv[j] *= d;
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) a[i][j] = __builtin_fma(-cv[i], rv[j], a[i][j]);
+      if (tr == kb)
+#pragma unroll
+        for (int j = 0; j < 4; j++) a[q][j] = rv[j];
+      if (tc == kb) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[i][q] = -d * cv[i];
+        if (tr == kb) a[q][q] = d;
       }
     }
-    if (!copy2d(at(W, o, o), ld, D, DS, DS, DS, st)) return false;
-    if (hipMemsetAsync(Xs, 0, sizeof(double) * DS * DS, st) != hipSuccess) return false;
-    hipLaunchKernelGGL(k_trtri_diag, dim3(nblk), dim3(DB), 0, st, D, Xs, DS);
-    for (int k = 0; k + 1 < nblk; k++)
-      hipLaunchKernelGGL(k_trtri_step, dim3((nblk - 1 - k) * (k + 1)), dim3(DT), 0, st, D, Xs, DS,
-                         k);
-    return copy2d(at(X, o, o), ld, Xs, DS, DS, DS, st);
   }
+  if (neg && threadIdx.x == 0) atomicOr(bad, 1);
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) out[(4 * tr + i) * DB + 4 * tc + j] = a[i][j];
+}
 
-  // L and X = L^-1 of the n x n diagonal block at (o, o), n a multiple of DS
-  bool cholinv(int o, int n) {
-    if (n == DS) return leaf(o);
-    const int n1 = DS * ((n / DS) / 2), n2 = n - n1, o2 = o + n1;
-    if (!cholinv(o, n1)) return false;
-    // L21 = A21 X11^T (A21 parked in X21's place)
-    if (!copy2d(at(X, o2, o), ld, at(W, o2, o), ld, n2, n1, st)) return false;
-    if (!gemm_rm(h, false, true, n2, n1, n1, 1.0, at(X, o2, o), ld, at(X, o, o), ld, 0.0,
-                 at(W, o2, o), ld))
-      return false;
-    // A22 -= L21 L21^T, lower part, in up to four strips of block rows
-    const int hs = DS * (((n2 / DS) + 3) / 4);
-    for (int s0 = o2; s0 < o2 + n2; s0 += hs) {
-      const int s1 = s0 + hs < o2 + n2 ? s0 + hs : o2 + n2;
-      if (!gemm_rm(h, false, true, s1 - s0, s1 - o2, n1, -1.0, at(W, s0, o), ld, at(W, o2, o), ld,
-                   1.0, at(W, s0, o2), ld))
-        return false;
-    }
-    if (!cholinv(o2, n2)) return false;
-    // X21 = -X22 (L21 X11): (L21 X11)^T = X11^T L21^T into the upper block
-    if (!gemm_rm(h, true, true, n1, n2, n1, 1.0, at(X, o, o), ld, at(W, o2, o), ld, 0.0,
-                 at(W, o, o2), ld))
-      return false;
-    return gemm_rm(h, false, true, n2, n1, n2, -1.0, at(X, o2, o2), ld, at(W, o, o2), ld, 0.0,
-                   at(X, o2, o), ld);
+// problem of block b: last p with tile0[p] <= b
+__device__ __forceinline__ int find_prob(const int *__restrict__ tile0, int n, int b) {
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int m = (lo + hi + 1) >> 1;
+    if (tile0[m] <= b)
+      lo = m;
+    else
+      hi = m - 1;
   }
-
-  // lower part of X[o:end, o:o+n]^T X[o:end, o:o+n] into W[o:o+n, o:o+n]
-  bool gram(int o, int n, int end) {
-    if (n <= GRAM_LEAF)
-      return gemm_rm(h, true, false, n, n, end - o, 1.0, at(X, o, o), ld, at(X, o, o), ld, 0.0,
-                     at(W, o, o), ld);
-    const int n1 = DS * ((n / DS) / 2), n2 = n - n1, o2 = o + n1;
-    if (!gram(o2, n2, end)) return false;
-    if (!gemm_rm(h, true, false, n2, n1, end - o2, 1.0, at(X, o2, o2), ld, at(X, o2, o), ld, 0.0,
-                 at(W, o2, o), ld))
-      return false;
-    return gram(o, n1, end);
-  }
-};
-
-// workspace: D (DS^2), Xs (DS^2)
-bool dense_inverse_big(rocblas_handle h, double *W, double *X, double *ws, int m, double *out,
-                       int *bad, hipStream_t st) {
-  const int mp = dense_padded(m);
-  if (rocblas_set_stream(h, st) != rocblas_status_success) return false;
-  if (hipMemsetAsync(X, 0, sizeof(double) * mp * mp, st) != hipSuccess) return false;
-  Dense dn{h, st, W, X, ws, ws + DS * DS, mp, bad};
-  if (!dn.cholinv(0, mp)) return false;
-  // the factor is no longer needed: A^-1 = X^T X into W
-  if (!dn.gram(0, mp, mp)) return false;
-  const int64_t tot = (int64_t)m * m;
-  hipLaunchKernelGGL(k_dense_mirror, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, W, mp,
-                     m, out);
-  return true;
+  return lo;
 }
 
 }  // namespace
 
-void *dense_blas_create() {
-  rocblas_handle h = nullptr;
-  if (rocblas_create_handle(&h) != rocblas_status_success) return nullptr;
-  return h;
+// identity on the padding rows of every matrix
+__global__ void k_gj_pad(const GJProb *__restrict__ pr, double *A0, double *A1) {
+  const GJProb p = pr[blockIdx.x];
+  const int ld = DB * p.nblk, i = p.n + threadIdx.x;
+  double *A = ((p.nblk & 1) ? A1 : A0) + p.off;
+  if (i < ld) A[(size_t)i * ld + i] = 1.0;
 }
 
-void dense_blas_destroy(void *h) {
-  if (h) (void)rocblas_destroy_handle(static_cast<rocblas_handle>(h));
+__global__ __launch_bounds__(DT) void k_gj_first(const GJProb *__restrict__ pr, const double *A0,
+                                                 const double *A1, double *__restrict__ dinv,
+                                                 int *bad) {
+  __shared__ double blk[DB * LDA], buf[256];
+  const GJProb p = pr[blockIdx.x];
+  stage_block<LDA>(((p.nblk & 1) ? A1 : A0) + p.off, DB * p.nblk, blk);
+  __syncthreads();
+  invert_block(blk, buf, dinv + (size_t)2 * DB * DB * blockIdx.x, bad);
 }
 
-int dense_padded(int m) {
-  return m >= DENSE_BIG ? (m + DS - 1) / DS * DS : (m + DB - 1) / DB * DB;
+__global__ __launch_bounds__(DT) void k_gj_step(int k, int nprob, const GJProb *__restrict__ pr,
+                                                const int *__restrict__ tile0, double *A0,
+                                                double *A1, double *dinv, int *bad) {
+  __shared__ double sa[DB * LDA], sb[DB * LDB];
+  const int q = find_prob(tile0, nprob, blockIdx.x);
+  const GJProb p = pr[q];
+  const int nb = p.nblk, t = blockIdx.x - tile0[q], i = t / nb, j = t % nb;
+  const int64_t ld = DB * nb;
+  const double *src = (((nb - k) & 1) ? A1 : A0) + p.off;
+  double *dst = (((nb - k - 1) & 1) ? A1 : A0) + p.off;
+  const double *P = dinv + (size_t)DB * DB * (2 * q + (k & 1));
+  double *out = dst + (int64_t)DB * i * ld + DB * j;
+  if (i == k && j == k) {
+    for (int s = threadIdx.x; s < DB * DB; s += DT) out[(s >> 6) * ld + (s & 63)] = P[s];
+    return;
+  }
+  const double *Aik = src + (int64_t)DB * i * ld + DB * k;
+  const double *Akj = src + (int64_t)DB * k * ld + DB * j;
+  f64x4 acc[2][2] = {};
+  if (j == k) {
+    stage_block<LDA>(Aik, ld, sa);
+    stage_block<LDB>(P, DB, sb);
+  } else {
+    stage_block<LDA>(P, DB, sa);
+    stage_block<LDB>(Akj, ld, sb);
+  }
+  __syncthreads();
+  quad_product<false>(sa, sb, acc);
+  if (i == k || j == k) {
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int v = 0; v < 2; v++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          out[quad_row(u, e) * ld + quad_col(v)] = i == k ? acc[u][v][e] : -acc[u][v][e];
+    return;
+  }
+  // A_ij - A_ik (P A_kj)
+  const double *Aij = src + (int64_t)DB * i * ld + DB * j;
+  f64x4 o[2][2];
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[u][v][e] = Aij[quad_row(u, e) * ld + quad_col(v)];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        sb[quad_row(u, e) * LDB + quad_col(v)] = -acc[u][v][e];
+      }
+  stage_block<LDA>(Aik, ld, sa);
+  __syncthreads();
+  quad_product<false>(sa, sb, o);
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) out[quad_row(u, e) * ld + quad_col(v)] = o[u][v][e];
+  if (i != k + 1 || j != k + 1) return;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) sa[quad_row(u, e) * LDA + quad_col(v)] = o[u][v][e];
+  __syncthreads();
+  invert_block(sa, sb, dinv + (size_t)DB * DB * (2 * q + ((k + 1) & 1)), bad);
 }
 
-size_t dense_workspace(int m) { return m < DENSE_BIG ? 0 : 2 * (size_t)DS * DS; }
-
-int launch_dense_inverse_big(void *blas, double *W, double *X, double *ws, int m, double *out,
-                             int *bad, hipStream_t st) {
-  if (m < DENSE_BIG || !blas || !ws) return -1;
-  if (!dense_inverse_big(static_cast<rocblas_handle>(blas), W, X, ws, m, out, bad, st)) return -1;
+void launch_gj_inverse(const GJProb *pr, const int *tile0, int nprob, const int *active,
+                       const int *tiles, int nsteps, double *A0, double *A1, double *dinv,
+                       int *bad, hipStream_t st) {
+  if (nprob == 0) return;
+  hipLaunchKernelGGL(k_gj_pad, dim3(nprob), dim3(DB), 0, st, pr, A0, A1);
+  hipLaunchKernelGGL(k_gj_first, dim3(nprob), dim3(DT), 0, st, pr, A0, A1, dinv, bad);
+  for (int k = 0; k < nsteps; k++)
+    hipLaunchKernelGGL(k_gj_step, dim3(tiles[k]), dim3(DT), 0, st, k, active[k], pr, tile0, A0, A1,
+                       dinv, bad);
   TMRX_LAUNCH_CHECK();
-  return 0;
 }
 
-void launch_dense_inverse(double *W, double *X, int m, double *out, int *bad, hipStream_t st) {
-  const int mp = dense_padded(m), nblk = mp / DB;
+// C = A B^T per problem (row-major, dimensions multiples of 64), and C^T into
+// a second array where ct >= 0
+__global__ __launch_bounds__(DT) void k_gemm_nt(int nprob, const GemmProb *__restrict__ pr,
+                                                const int *__restrict__ tile0,
+                                                const double *__restrict__ A,
+                                                const double *__restrict__ B,
+                                                double *__restrict__ C, double *__restrict__ Ct) {
+  __shared__ double sa[DB * LDA], sb[DB * LDA];
+  const int q = find_prob(tile0, nprob, blockIdx.x);
+  const GemmProb p = pr[q];
+  const int t = blockIdx.x - tile0[q], nj = p.N / DB, i = t / nj, j = t % nj;
+  const double *a = A + p.a + (int64_t)DB * i * p.K, *b = B + p.b + (int64_t)DB * j * p.K;
+  f64x4 acc[2][2] = {};
+  for (int k = 0; k < p.K; k += DB) {
+    __syncthreads();
+    stage_block<LDA>(a + k, p.K, sa);
+    stage_block<LDA>(b + k, p.K, sb);
+    __syncthreads();
+    quad_product<true>(sa, sb, acc);
+  }
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int r = DB * i + quad_row(u, e), c = DB * j + quad_col(v);
+        C[p.c + (int64_t)r * p.N + c] = acc[u][v][e];
+        if (p.ct >= 0) Ct[p.ct + (int64_t)c * p.M + r] = acc[u][v][e];
+      }
+}
+
+void launch_gemm_nt(int nprob, int ntiles, const GemmProb *pr, const int *tile0, const double *A,
+                    const double *B, double *C, double *Ct, hipStream_t st) {
+  if (ntiles == 0) return;
+  hipLaunchKernelGGL(k_gemm_nt, dim3(ntiles), dim3(DT), 0, st, nprob, pr, tile0, A, B, C, Ct);
+  TMRX_LAUNCH_CHECK();
+}
+
+// BSR block k into the dense arrays: buf[which[k]] + dst[k], leading
+// dimension ld[k] (which 255: dropped)
+__global__ void k_coarse_scatter(int nnzb, const double *__restrict__ val,
+                                 const uint8_t *__restrict__ which, const int64_t *__restrict__ dst,
+                                 const int *__restrict__ ld, double *A0, double *A1, double *Et) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= nnzb || which[k] == 255) return;
+  double *o = (which[k] == 0 ? A0 : which[k] == 1 ? A1 : Et) + dst[k];
+  const double *v = val + 9 * (size_t)k;
+  const int64_t l = ld[k];
+  for (int p = 0; p < 3; p++)
+    for (int q = 0; q < 3; q++) o[p * l + q] = v[3 * p + q];
+}
+
+void launch_coarse_scatter(int nnzb, const double *val, const uint8_t *which, const int64_t *dst,
+                           const int *ld, double *A0, double *A1, double *Et, hipStream_t st) {
+  if (nnzb == 0) return;
+  hipLaunchKernelGGL(k_coarse_scatter, dim3((nnzb + 255) / 256), dim3(256), 0, st, nnzb, val, which,
+                     dst, ld, A0, A1, Et);
+  TMRX_LAUNCH_CHECK();
+}
+
+// S[a][b] -= sum_i C_i[loc_i(a)][loc_i(b)] in leaf order, C_i (ldc_i wide)
+// holding 3 x 3 blocks of the separator nodes next to leaf i
+__global__ void k_schur_sum(int m, int lds, int nleaf, const int *__restrict__ loc,
+                            const int64_t *__restrict__ coff, const int *__restrict__ ldc,
+                            const double *__restrict__ C, double *__restrict__ S) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (int64_t)m * m) return;
+  const int a = (int)(t / m), b = (int)(t % m), ns = m / 3;
+  double s = S[(int64_t)a * lds + b];
+  for (int i = 0; i < nleaf; i++) {
+    const int la = loc[(int64_t)i * ns + a / 3], lb = loc[(int64_t)i * ns + b / 3];
+    if (la < 0 || lb < 0) continue;
+    s -= C[coff[i] + (int64_t)(3 * la + a % 3) * ldc[i] + 3 * lb + b % 3];
+  }
+  S[(int64_t)a * lds + b] = s;
+}
+
+void launch_schur_sum(int m, int lds, int nleaf, const int *loc, const int64_t *coff,
+                      const int *ldc, const double *C, double *S, hipStream_t st) {
   if (m == 0) return;
-  for (int k = 0; k < nblk; k++) {
-    hipLaunchKernelGGL(k_potrf_diag, dim3(1), dim3(DT), 0, st, W, mp, k, bad);
-    const int rows = mp - (k + 1) * DB;
-    if (rows > 0) {
-      hipLaunchKernelGGL(k_trsm_panel, dim3((rows + DT - 1) / DT), dim3(DT), 0, st, W, mp, k);
-      const int T = nblk - k - 1;
-      hipLaunchKernelGGL(k_syrk_trailing, dim3(T * (T + 1) / 2), dim3(DT), 0, st, W, mp, k);
+  const int64_t n = (int64_t)m * m;
+  hipLaunchKernelGGL(k_schur_sum, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m, lds, nleaf,
+                     loc, coff, ldc, C, S);
+  TMRX_LAUNCH_CHECK();
+}
+
+// One stage of the substructured solve, one wave per row: s = sum over the
+// row's segments of M[a + j] v[idx[j]], FP64.
+//   stage 1: v = b; leaf rows tmp = s, separator rows tmp = b[dof] - s
+//   stage 2: v = tmp; x[dof] = xs[pos] = s
+//   stage 3: v = xs; x[dof] = tmp[pos] - s
+template <class T, class TA, int STAGE>
+__global__ __launch_bounds__(256) void k_coarse_rows(int nrows, const CoarseRow *__restrict__ rows,
+                                                     const CoarseSeg *__restrict__ segs,
+                                                     const int *__restrict__ idx,
+                                                     const TA *__restrict__ M,
+                                                     const T *__restrict__ b, T *__restrict__ x,
+                                                     double *__restrict__ tmp,
+                                                     double *__restrict__ xs, int n, int ntmp,
+                                                     int nxs, const int *__restrict__ run) {
+  if (run && *run == 0) return;
+  const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (r >= nrows) return;
+  b += (int64_t)blockIdx.y * n;
+  x += (int64_t)blockIdx.y * n;
+  tmp += (int64_t)blockIdx.y * ntmp;
+  xs += (int64_t)blockIdx.y * nxs;
+  const CoarseRow row = rows[r];
+  double s = 0.0;
+  for (int g = row.seg0; g < row.seg1; g++) {
+    const CoarseSeg sg = segs[g];
+    const TA *__restrict__ a = M + sg.a;
+    const int *__restrict__ ix = idx + sg.idx;
+    // eight entries per lane in flight (clamped to the segment, extra terms
+    // skipped)
+    for (int j0 = lane; j0 < sg.len; j0 += 8 * 64) {
+      double av[8], bv[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int j = min(j0 + 64 * k, sg.len - 1);
+        av[k] = (double)a[j];
+        const int i = ix[j];
+        bv[k] = STAGE == 1 ? (double)b[i] : STAGE == 2 ? tmp[i] : xs[i];
+      }
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        if (j0 + 64 * k < sg.len) s += av[k] * bv[k];
     }
   }
-  // L^-1: the diagonal blocks at once, then nblk - 1 right-looking steps
-  const int64_t tot = (int64_t)mp * mp;
-  hipLaunchKernelGGL(k_trtri_zero, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, mp, X);
-  hipLaunchKernelGGL(k_trtri_diag, dim3(nblk), dim3(DB), 0, st, W, X, mp);
-  for (int k = 0; k + 1 < nblk; k++)
-    hipLaunchKernelGGL(k_trtri_step, dim3((nblk - 1 - k) * (k + 1)), dim3(DT), 0, st, W, X, mp, k);
-  hipLaunchKernelGGL(k_gram, dim3(nblk * (nblk + 1) / 2), dim3(DT), 0, st, X, mp, nblk, m, out);
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+  if (lane != 0) return;
+  if (STAGE == 1) {
+    tmp[row.pos] = row.dof >= 0 ? (double)b[row.dof] - s : s;
+  } else if (STAGE == 2) {
+    xs[row.pos] = s;
+    x[row.dof] = (T)s;
+  } else {
+    x[row.dof] = (T)(tmp[row.pos] - s);
+  }
+}
+
+template <class T, class TA>
+static void coarse_stages(const CoarseBlocks &cb, const TA *M, const T *b, T *x, hipStream_t st,
+                          int nrhs) {
+#define TMRX_STAGE(S)                                                                             \
+  if (cb.nrow[S - 1])                                                                             \
+  hipLaunchKernelGGL((k_coarse_rows<T, TA, S>), dim3((cb.nrow[S - 1] + 3) / 4, nrhs), dim3(256),  \
+                     0, st, cb.nrow[S - 1], cb.row[S - 1], cb.seg, cb.idx, M, b, x, cb.tmp,       \
+                     cb.xs, cb.n, cb.ntmp, cb.nxs, cb.run)
+  TMRX_STAGE(1);
+  TMRX_STAGE(2);
+  TMRX_STAGE(3);
+#undef TMRX_STAGE
   TMRX_LAUNCH_CHECK();
 }
 
-void launch_bsr_to_dense(const int *brow, const int *col, const double *val, int n0, int n1,
-                         int k0, int k1, int mp, double *W, hipStream_t st) {
-  const int m = 3 * (n1 - n0);
-  const int64_t total = (int64_t)mp * mp;
-  hipLaunchKernelGGL(k_dense_fill, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, total,
-                     mp, m, W);
-  if (k1 > k0)
-    hipLaunchKernelGGL(k_bsr_scatter, dim3((k1 - k0 + 255) / 256), dim3(256), 0, st, col, val, n0,
-                       k0, k1, brow, mp, W);
-  TMRX_LAUNCH_CHECK();
+template <class T>
+void launch_coarse_schur(const CoarseBlocks &cb, const T *b, T *x, hipStream_t st, int nrhs) {
+  if (sizeof(T) == 4 && cb.Ainv32)
+    coarse_stages<T, float>(cb, cb.Ainv32, b, x, st, nrhs);
+  else
+    coarse_stages<T, double>(cb, cb.Ainv, b, x, st, nrhs);
 }
+template void launch_coarse_schur<float>(const CoarseBlocks &, const float *, float *, hipStream_t,
+                                         int);
+template void launch_coarse_schur<double>(const CoarseBlocks &, const double *, double *,
+                                          hipStream_t, int);
 
 }  // namespace tmrx

@@ -220,40 +220,65 @@ void launch_restrict(const TransferCSR &R, const uint8_t *bcmask_c, const T *rf,
 template <class T>
 void launch_cheb_first(int ndof, const T *b, const T *dinv, double c, T *d, T *x,
                        hipStream_t st, int nrhs = 1, const int *run = nullptr);
-// coarsest-level solve: block-diagonal explicit inverse (one block per
-// independent component), per row: first column, block size, row offset
+// one dense SPD matrix of a batched inversion: n rows padded to nblk blocks
+// of 64 (leading dimension 64 nblk), at `off` in both buffers
+struct GJProb {
+  int n, nblk;
+  int64_t off;
+};
+// C (M x N) = A (M x K) B^T (N x K), row-major at the given offsets; ct >= 0:
+// also C^T
+struct GemmProb {
+  int M, N, K;
+  int64_t a, b, c, ct;
+};
+// row of the substructured solve: segments [seg0, seg1), output dof and
+// position in the work vector
+struct CoarseRow {
+  int seg0, seg1, dof, pos;
+};
+struct CoarseSeg {
+  int64_t a;
+  int len, idx;
+};
+// coarsest-level solve: explicit inverses (per row of a whole component:
+// first column, block size (0: not such a row), row offset) and
+// substructured components (three stages of rows)
 struct CoarseBlocks {
   int n = 0;
+  bool direct = true;             // some rows have an explicit inverse
   const double *Ainv = nullptr;
   const float *Ainv32 = nullptr;  // the same in FP32 (FP32 V-cycles read it when set)
   const int *col0 = nullptr;
   const int *nb = nullptr;
   const int64_t *aoff = nullptr;
+  int nrow[3] = {0, 0, 0};
+  const CoarseRow *row[3] = {nullptr, nullptr, nullptr};
+  const CoarseSeg *seg = nullptr;
+  const int *idx = nullptr;
+  double *tmp = nullptr, *xs = nullptr;  // [nrhs][ntmp], [nrhs][nxs]
+  int ntmp = 0, nxs = 0;
   const int *run = nullptr;  // as Tiles::run
 };
 template <class T>
 void launch_dense_solve(const CoarseBlocks &cb, const T *b, T *x, hipStream_t st, int nrhs = 1);
-// rows and columns of the padded dense matrices of launch_dense_inverse
-int dense_padded(int m);
-// explicit inverse of an SPD matrix by blocked Cholesky on the device: W
-// holds the matrix row-major with dense_padded(m) rows and columns (identity
-// on the padding) and is overwritten by the factor; X (same size) receives
-// L^-1; out (m x m, row-major) receives A^-1; *bad |= 1 on a non-positive
-// pivot
-void launch_dense_inverse(double *W, double *X, int m, double *out, int *bad, hipStream_t st);
-// the same for m of at least 2048 over 256-wide super-blocks with the bulk in
-// FP64 GEMMs (rocBLAS handle from dense_blas_create, workspace of
-// dense_workspace(m) doubles); returns -1 if m is below that or a call fails
-int launch_dense_inverse_big(void *blas, double *W, double *X, double *ws, int m, double *out,
-                             int *bad, hipStream_t st);
-size_t dense_workspace(int m);
-void *dense_blas_create();
-void dense_blas_destroy(void *h);
-// W (mp x mp, row-major) = the BSR block rows [n0, n1) of a component
-// (blocks [k0, k1), block rows brow) as a dense matrix of its 3 (n1 - n0)
-// dofs, identity on the padding rows
-void launch_bsr_to_dense(const int *brow, const int *col, const double *val, int n0, int n1,
-                         int k0, int k1, int mp, double *W, hipStream_t st);
+// the substructured components' part of it
+template <class T>
+void launch_coarse_schur(const CoarseBlocks &cb, const T *b, T *x, hipStream_t st, int nrhs);
+// explicit inverses of nprob dense SPD matrices (largest first): matrix p
+// starts in A1 when its nblk is odd, else in A0, padding rows zero, and ends
+// in A0; both buffers are overwritten.  Step k works on the first active[k]
+// matrices, tiles[k] blocks; dinv: 2 x 64 x 64 words per matrix; *bad |= 1 on
+// a non-positive pivot
+void launch_gj_inverse(const GJProb *pr, const int *tile0, int nprob, const int *active,
+                       const int *tiles, int nsteps, double *A0, double *A1, double *dinv,
+                       int *bad, hipStream_t st);
+void launch_gemm_nt(int nprob, int ntiles, const GemmProb *pr, const int *tile0, const double *A,
+                    const double *B, double *C, double *Ct, hipStream_t st);
+void launch_coarse_scatter(int nnzb, const double *val, const uint8_t *which, const int64_t *dst,
+                           const int *ld, double *A0, double *A1, double *Et, hipStream_t st);
+void launch_schur_sum(int m, int lds, int nleaf, const int *loc, const int64_t *coff,
+                      const int *ldc, const double *C, double *S, hipStream_t st);
 
 // Galerkin coarse operator of one level: 3 x 3 blocks over the independent
 // nodes (block row i = node i), row-major blocks, clamped rows and columns

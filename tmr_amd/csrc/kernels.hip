@@ -582,6 +582,7 @@ __global__ __launch_bounds__(256) void k_dense_solve(int n, const TA *__restrict
   const TA *a = Ainv + aoff[row];
   const T *bb = b + col0[row];
   const int m = nb[row];
+  if (m == 0) return;  // a row of a substructured component
   // eight entries per lane in flight, added in the order of a one-at-a-time
   // loop (indices clamped to the row, extra terms skipped)
   for (int j0 = lane; j0 < m; j0 += 8 * 64) {
@@ -603,6 +604,8 @@ __global__ __launch_bounds__(256) void k_dense_solve(int n, const TA *__restrict
 template <class T>
 void launch_dense_solve(const CoarseBlocks &cb, const T *b, T *x, hipStream_t st, int nrhs) {
   if (cb.n == 0) return;
+  if (cb.nrow[0]) launch_coarse_schur<T>(cb, b, x, st, nrhs);
+  if (!cb.direct) return;
   if (sizeof(T) == 4 && cb.Ainv32)
     hipLaunchKernelGGL((k_dense_solve<T, float>), dim3((cb.n + 3) / 4, nrhs), dim3(256), 0, st,
                        cb.n, cb.Ainv32, cb.col0, cb.nb, cb.aoff, b, x, cb.run);
@@ -2542,6 +2545,7 @@ void launch_adjoint_grad(int n, const double *rho, const int16_t *lev, double q,
                                      const AsmArgs &, hipStream_t, int, int64_t);
 TMRX_INST(float)
 TMRX_INST(double)
+template void launch_fill<int>(int64_t, int, int *, hipStream_t);
 template void launch_convert<float, double>(int64_t, const float *, double *, hipStream_t);
 template void launch_convert<double, float>(int64_t, const double *, float *, hipStream_t);
 

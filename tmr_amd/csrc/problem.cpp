@@ -61,7 +61,6 @@ void Problem::drop_graphs() {
 
 Problem::~Problem() {
   drop_graphs();
-  dense_blas_destroy(blas_);
   for (int k = 0; k < 2; k++)
     if (gev_[k]) (void)hipEventDestroy(gev_[k]);
   if (cap_st_) (void)hipStreamDestroy(cap_st_);
@@ -1423,103 +1422,6 @@ int Problem::find_components() {
   return 0;
 }
 
-int Problem::coarse_factor() {
-  // K of the coarsest level (identity rows and columns on clamped dofs) as
-  // a BSR matrix assembled on the device from its element matrices (K_E of
-  // the Galerkin product, or the scaled element stiffness), then per
-  // independent component a dense block, its FP64 Cholesky and the explicit
-  // inverse for a one-GEMV coarse solve
-  const int last = (int)levels_.size() - 1;
-  Level &L = levels_[last];
-  const int n = (int)L.ndof;
-  const bool nodal = design_mode_ == 1;
-  const bool gal = galerkin_ && levels_.size() > 1;
-  if (!L.has_bsr && build_bsr(last)) return -1;
-  if (!gal) {
-    if ((L.KE.n < 576 * (size_t)L.n_elem && L.KE.alloc(576 * (size_t)L.n_elem)) ||
-        (nodal && Kgd_.n == 0 && Kgd_.upload(Kgh_))) {
-      last_error = "coarse: device allocation failed";
-      return -1;
-    }
-    launch_elem_matrices(L.n_elem, L.d_cls.p, nodal ? L.sg64.p : L.s64.p,
-                         nodal ? Kgd_.p : K0d_.p, nodal, L.KE.p, st_);
-  }
-  launch_bsr_assemble(bsr<double>(last), L.bt_ptr.p, L.bt_code.p, L.bt_w.p, L.bsr_row.p, L.KE.p,
-                      L.bsr64.p, st_);
-  std::vector<int> col0(n), nb(n);
-  std::vector<int64_t> aoff(n);
-  // component blocks of the inverse, one after the other
-  std::vector<size_t> base(nseg_ + 1, 0);
-  size_t wmax = 0, wsmax = 0;
-  for (int sg = 0; sg < nseg_; sg++) {
-    const size_t m = 3 * (size_t)(L.seg_node0[sg + 1] - L.seg_node0[sg]);
-    base[sg + 1] = base[sg] + m * m;
-    const size_t mp = (size_t)dense_padded((int)m);
-    wmax = std::max(wmax, mp * mp);
-    wsmax = std::max(wsmax, dense_workspace((int)m));
-  }
-  if ((Ainv_.n < base[nseg_] && Ainv_.alloc(base[nseg_])) ||
-      (cw_.n < wmax && (cw_.alloc(wmax) || cx_.alloc(wmax))) || (chk_.n == 0 && chk_.alloc(1)) ||
-      (cws_.n < wsmax && cws_.alloc(wsmax))) {
-    last_error = "coarse: device allocation failed";
-    return -1;
-  }
-  if (wsmax && !blas_ && !(blas_ = dense_blas_create())) {
-    last_error = "coarse: rocBLAS handle creation failed";
-    return -1;
-  }
-  HIPCHK(hipMemsetAsync(chk_.p, 0, sizeof(int), st_));
-  for (int sg = 0; sg < nseg_; sg++) {
-    const int n0 = L.seg_node0[sg], n1 = L.seg_node0[sg + 1];
-    const int d0 = 3 * n0, m = 3 * (n1 - n0);
-    const int mp = dense_padded(m);
-    launch_bsr_to_dense(L.bsr_row.p, L.bsr_col.p, L.bsr64.p, n0, n1, L.bsr_ptr_h[n0],
-                        L.bsr_ptr_h[n1], mp, cw_.p, st_);
-    if (dense_workspace(m)) {
-      if (launch_dense_inverse_big(blas_, cw_.p, cx_.p, cws_.p, m, Ainv_.p + base[sg], chk_.p,
-                                   st_)) {
-        last_error = "coarse: the super-block factorisation failed";
-        return -1;
-      }
-    } else {
-      launch_dense_inverse(cw_.p, cx_.p, m, Ainv_.p + base[sg], chk_.p, st_);
-    }
-    for (int i = 0; i < m; i++) {
-      col0[d0 + i] = d0;
-      nb[d0 + i] = m;
-      aoff[d0 + i] = (int64_t)(base[sg] + (size_t)i * m);
-    }
-  }
-  int bad = 0;
-  HIPCHK(hipMemcpyAsync(&bad, chk_.p, sizeof(int), hipMemcpyDeviceToHost, st_));
-  HIPCHK(hipStreamSynchronize(st_));
-  if (bad) {
-    last_error = "coarse Cholesky: the coarsest-level matrix is not positive definite "
-                 "(missing boundary conditions?)";
-    return -1;
-  }
-  if (cb_col0_.upload(col0) || cb_nb_.upload(nb) || cb_aoff_.upload(aoff)) {
-    last_error = "coarse: device allocation failed";
-    return -1;
-  }
-  coarse_.n = n;
-  coarse_.Ainv = Ainv_.p;
-  // FP32 V-cycles read an FP32 copy (half the bytes of every coarse solve)
-  coarse_.Ainv32 = nullptr;
-  if (setup_prec_pending_ == 1) {
-    if (Ainv32_.n < base[nseg_] && Ainv32_.alloc(base[nseg_])) {
-      last_error = "coarse: device allocation failed";
-      return -1;
-    }
-    launch_convert<double, float>((int64_t)base[nseg_], Ainv_.p, Ainv32_.p, st_);
-    coarse_.Ainv32 = Ainv32_.p;
-  }
-  coarse_.col0 = cb_col0_.p;
-  coarse_.nb = cb_nb_.p;
-  coarse_.aoff = cb_aoff_.p;
-  return 0;
-}
-
 int Problem::setup(const SolveOpts &o) {
   if (!have_design_) {
     last_error = "setup: set the design first";
@@ -1856,7 +1758,7 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
       last_error = "solve: device allocation failed";
       return -1;
     }
-  if (ensure_batch(nrhs)) return -1;
+  if (ensure_batch(nrhs) || (coarse_direct_ && ensure_coarse_work(nrhs))) return -1;
   fp32_valu_ = o.fp32_valu != 0;
   auto t0 = std::chrono::steady_clock::now();
   Level &L0 = levels_[0];

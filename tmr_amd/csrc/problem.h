@@ -197,6 +197,36 @@ struct Level {
   LevelVecs<double> v64;
 };
 
+// one batch of dense inversions: matrices (GJProb) largest first, their
+// blocks' offsets, and per step how many are still active and their blocks
+struct CoarseSet {
+  int nprob = 0;
+  DevArray<char> prob;
+  DevArray<int> tile0;
+  DevArray<double> dinv;  // two 64 x 64 diagonal-block inverses per matrix
+  std::vector<int> active, tiles;
+};
+
+// direct solve of the coarsest level (coarse.cpp): built once per hierarchy
+struct CoarsePlan {
+  bool built = false, any_direct = false, any_schur = false;
+  CoarseSet set[2];           // components and leaves; Schur complements
+  int64_t na = 0, nw = 0, net = 0;  // words of the inverses, of W, of E^T
+  int ng1 = 0, nt1 = 0, nt2 = 0;
+  DevArray<char> g1, g2, segs, rows[3];
+  DevArray<int> t1, t2, idx, loc, ldc, ld;
+  DevArray<int64_t> coff, dst;
+  DevArray<uint8_t> which;
+  DevArray<double> A1, Et, C;  // second inversion buffer, couplings, E^T W
+  DevArray<double> work;       // vectors of the substructured solve
+  struct Sum {
+    int m, ld, buf, nleaf;
+    int64_t off;
+    size_t loc0, leaf0;
+  };
+  std::vector<Sum> schur;
+};
+
 // race check of owner-tile schedules (schedule_check.cpp): 0 if the
 // records can accumulate without conflicts, else -1 with the reason in err
 int check_tile_schedule(int ntiles, const int *rec_ptr, const TileElem *recs, const int *nacc,
@@ -351,6 +381,8 @@ class Problem {
   T *first_target(int l, T *x, const SolveOpts &o);
   void precond(int nrhs, const SolveOpts &o);
   int coarse_factor();
+  int build_coarse_plan();
+  int ensure_coarse_work(int nrhs);
   int find_components();
   // batched FP64 flexible PCG from x = 0 on rhs ([nrhs][ndof], clamped rows
   // zeroed in place); work vectors r_, p_, q_, z_
@@ -390,9 +422,7 @@ class Problem {
   const uint8_t *state_mask() const { return has_ubc_ ? nomask_.p : levels_[0].d_bcmask.p; }
   DevArray<double> rho_;
   DevArray<double> Ainv_;
-  DevArray<double> cw_, cx_;  // coarse factorisation work (padded matrix, L^-1)
-  DevArray<double> cws_;      // workspace of the super-block factorisation
-  void *blas_ = nullptr;      // rocBLAS handle of the super-block factorisation
+  CoarsePlan cplan_;
   DevArray<int> cb_col0_, cb_nb_;
   DevArray<int64_t> cb_aoff_;
   CoarseBlocks coarse_;
