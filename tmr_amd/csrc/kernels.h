@@ -78,13 +78,15 @@ struct Tiles {
   int max_rec = 0, max_mrec = 0;  // records per tile (plain, matrix-core padded)
   int ncolors = 0;
   const int *node0 = nullptr;     // [n_tiles + 1]
-  // slots: owned, then the hanging ones (accumulated first) by their parents
-  // (a, b, c, d): two of weight 1/2 (c = -1) or four of weight 1/4, then the
-  // halo nodes
+  // slots: owned, then the hanging ones (accumulated first) by the LDS
+  // positions of their parents (four uint16: two parents of weight 1/2, third
+  // 0xffff, or four of 1/4), then the halo nodes (those corners and parents
+  // of the tile that it does not own), clamped dofs in the top three bits
   const int *extd_ptr = nullptr;  // [n_tiles + 1]
-  const int4 *extd = nullptr;
+  const uint2 *extd = nullptr;
   const int *ext_ptr = nullptr;   // [n_tiles + 1]
-  const int *ext = nullptr;       // global node
+  const uint32_t *ext = nullptr;
+  bool masked = true;             // false: every dof free (bcmask all zero)
   const int *nacc_dep = nullptr;  // [n_tiles] accumulated hanging slots
   const int *el_ptr = nullptr;    // [n_tiles + 1]
   const TileElem *el = nullptr;

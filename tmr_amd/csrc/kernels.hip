@@ -69,34 +69,6 @@ __device__ __forceinline__ void load_node(int e, const T *__restrict__ x,
   }
 }
 
-// Value of a hanging node from its packed parents (a, b, c, d): two parents
-// of weight 1/2 (c < 0) or four of weight 1/4, clamped dofs zero.  The four
-// loads go out together (the pair form loads its parents twice), so a hanging
-// node costs two dependent memory round trips, its record and its parents,
-// in place of the ten or so of the constraint-list loop of load_node; the
-// sums are the same, term by term.
-template <class T>
-__device__ __forceinline__ void load_dep(const int4 p, const T *__restrict__ x,
-                                         const uint8_t *__restrict__ bcmask, T v[3]) {
-  const bool two = p.z < 0;
-  const int g[4] = {p.x, p.y, two ? p.x : p.z, two ? p.y : p.w};
-  Vec3<T> u[4];
-  uint8_t m[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) u[k] = load_vec3(x + 3 * (size_t)g[k]);
-#pragma unroll
-  for (int k = 0; k < 4; k++) m[k] = bcmask[g[k]];
-  const T w = two ? T(0.5) : T(0.25);
-  v[0] = v[1] = v[2] = T(0);
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const bool on = k < 2 || !two;
-    if (on && !(m[k] & 1)) v[0] += w * u[k].a;
-    if (on && !(m[k] & 2)) v[1] += w * u[k].b;
-    if (on && !(m[k] & 4)) v[2] += w * u[k].c;
-  }
-}
-
 template <class T>
 __global__ __launch_bounds__(WG_ELEMS) void k_elem_apply(
     const int *__restrict__ wg_node_ptr, const int *__restrict__ wg_nodes,
@@ -1254,14 +1226,36 @@ void launch_dinv_dots(int64_t n, const double *dinv, double *y, const double *x,
 // ---------------------------------------------------------------------------
 // owner-tile apply: one pass, final values of the owned nodes, fused epilogue
 
-// stage x of the tile's slots into LDS (owned nodes in place, then the
-// hanging slots from their packed parents extd_l, then the halo nodes ext_l,
-// clamped dofs zero) and zero the accumulators; S values per node
+// halo entry of a tile: node index, clamped dofs in the top three bits
+__device__ __forceinline__ int halo_node(uint32_t e) { return (int)(e & 0x1fffffffu); }
+
+// LDS positions of a hanging slot's parents (four uint16; the third 0xffff:
+// two parents of weight 1/2, else four of 1/4)
+struct DepRec {
+  int q[4];
+  bool two;
+  __device__ __forceinline__ explicit DepRec(const uint2 r) {
+    q[0] = r.x & 0xffff;
+    q[1] = r.x >> 16;
+    q[2] = r.y & 0xffff;
+    q[3] = r.y >> 16;
+    two = q[2] == 0xffff;
+  }
+};
+
+// Stage x of the tile's slots into LDS (owned nodes in place, halo nodes
+// behind the hanging slots, clamped dofs zero), clear the accumulators, then
+// interpolate the hanging slots from their parents' slots; S values per node.
+// A tile of an adaptive forest holds about twice as many hanging slots as
+// owned nodes, and nearly all their parents are staged anyway (a 256-node
+// tile adds seven), so the parents are read from LDS: four node and mask
+// gathers from memory per hanging slot cost more than the element phase
+// (1.2M-hex FP32 Chebyshev step 78 -> 68 us, FP64 product 121 -> 110).
 template <class T, int S, int NT = TILE_THREADS, int SY = S>
-__device__ __forceinline__ void tile_stage(int n0, int nown, const int4 *__restrict__ extd_l,
-                                           int ndep, const int *__restrict__ ext_l, int nhalo,
+__device__ __forceinline__ void tile_stage(int n0, int nown, const uint2 *__restrict__ extd_l,
+                                           int ndep, const uint32_t *__restrict__ ext_l, int nhalo,
                                            int nacc, const uint8_t *__restrict__ bcmask,
-                                           const T *__restrict__ x, T *xs, T *ys) {
+                                           int maskall, const T *__restrict__ x, T *xs, T *ys) {
   const int tid = threadIdx.x;
   constexpr int VN = 2, VH = 2;
   auto put = [&](int pos, T a, T b, T c) {
@@ -1271,15 +1265,21 @@ __device__ __forceinline__ void tile_stage(int n0, int nown, const int4 *__restr
     xs[q + 2] = c;
   };
   const int h0 = nown + ndep;  // first halo slot
-  // First rounds: the halo node indices, then the owned values (one 12-byte
-  // load and one mask byte per node) and the halo values all go out before
-  // any is used; indices are clamped into the tile, so the loads are
-  // unconditional.
-  int gf[VH];
+  auto put_halo = [&](int i, uint32_t g, const Vec3<T> &v) {
+    const uint32_t m = (g >> 29) & (uint32_t)maskall;
+    put(h0 + i, (m & 1) ? T(0) : v.a, (m & 2) ? T(0) : v.b, (m & 4) ? T(0) : v.c);
+  };
+  // First rounds: the halo entries and the first hanging record, then the
+  // owned values (one 12-byte load and one mask byte per node) and the halo
+  // values all go out before any is used; indices are clamped into the tile,
+  // so the loads are unconditional.
+  uint32_t gf[VH];
 #pragma unroll
-  for (int k = 0; k < VH; k++) gf[k] = nhalo > 0 ? ext_l[min(tid + k * NT, nhalo - 1)] : 0;
+  for (int k = 0; k < VH; k++) gf[k] = nhalo > 0 ? ext_l[min(tid + k * NT, nhalo - 1)] : 0u;
+  uint2 rec = make_uint2(0u, 0u);
+  if (ndep > 0) rec = extd_l[min(tid, ndep - 1)];
   Vec3<T> vo[VN], vh[VH];
-  uint8_t mo[VN], mh[VH];
+  uint8_t mo[VN];
 #pragma unroll
   for (int k = 0; k < VN; k++) {
     const int j = min(tid + k * NT, nown - 1);
@@ -1287,10 +1287,7 @@ __device__ __forceinline__ void tile_stage(int n0, int nown, const int4 *__restr
     mo[k] = bcmask[n0 + j];
   }
 #pragma unroll
-  for (int k = 0; k < VH; k++) {
-    vh[k] = load_vec3(x + 3 * (size_t)gf[k]);
-    mh[k] = bcmask[gf[k]];
-  }
+  for (int k = 0; k < VH; k++) vh[k] = load_vec3(x + 3 * (size_t)halo_node(gf[k]));
 #pragma unroll
   for (int k = 0; k < VN; k++)
     if (tid + k * NT < nown)
@@ -1298,20 +1295,7 @@ __device__ __forceinline__ void tile_stage(int n0, int nown, const int4 *__restr
           (mo[k] & 4) ? T(0) : vo[k].c);
 #pragma unroll
   for (int k = 0; k < VH; k++)
-    if (tid + k * NT < nhalo)
-      put(h0 + tid + k * NT, (mh[k] & 1) ? T(0) : vh[k].a, (mh[k] & 2) ? T(0) : vh[k].b,
-          (mh[k] & 4) ? T(0) : vh[k].c);
-  // hanging slots; the next round's records load before this round's parents
-  if (ndep > 0) {
-    int4 pn = extd_l[min(tid, ndep - 1)];
-    for (int i = tid; i < ndep; i += NT) {
-      const int4 p = pn;
-      pn = extd_l[min(i + NT, ndep - 1)];
-      T v[3];
-      load_dep<T>(p, x, bcmask, v);
-      put(nown + i, v[0], v[1], v[2]);
-    }
-  }
+    if (tid + k * NT < nhalo) put_halo(tid + k * NT, gf[k], vh[k]);
   // further rounds (tiles of more than two nodes or halo slots per thread)
   for (int j0 = tid + VN * NT; j0 < nown; j0 += VN * NT) {
 #pragma unroll
@@ -1327,25 +1311,35 @@ __device__ __forceinline__ void tile_stage(int n0, int nown, const int4 *__restr
             (mo[k] & 4) ? T(0) : vo[k].c);
   }
   for (int i0 = tid + VH * NT; i0 < nhalo; i0 += VH * NT) {
-    int g[VH];
+    uint32_t g[VH];
 #pragma unroll
     for (int k = 0; k < VH; k++) g[k] = ext_l[min(i0 + k * NT, nhalo - 1)];
 #pragma unroll
-    for (int k = 0; k < VH; k++) {
-      vh[k] = load_vec3(x + 3 * (size_t)g[k]);
-      mh[k] = bcmask[g[k]];
-    }
+    for (int k = 0; k < VH; k++) vh[k] = load_vec3(x + 3 * (size_t)halo_node(g[k]));
 #pragma unroll
     for (int k = 0; k < VH; k++)
-      if (i0 + k * NT < nhalo)
-        put(h0 + i0 + k * NT, (mh[k] & 1) ? T(0) : vh[k].a, (mh[k] & 2) ? T(0) : vh[k].b,
-            (mh[k] & 4) ? T(0) : vh[k].c);
+      if (i0 + k * NT < nhalo) put_halo(i0 + k * NT, g[k], vh[k]);
   }
   // accumulators: SY * round8(nacc) values, a multiple of 16 bytes starting
   // 16-byte aligned, cleared 16 bytes at a time
   uint4 *y16 = reinterpret_cast<uint4 *>(ys);
   const int n16 = (int)((SY * ((nacc + 7) & ~7) * sizeof(T)) / 16);
   for (int i = tid; i < n16; i += NT) y16[i] = make_uint4(0u, 0u, 0u, 0u);
+  if (ndep > 0) {  // the same for every thread of the tile
+    __syncthreads();
+    for (int i = tid; i < ndep; i += NT) {
+      const DepRec p(rec);
+      rec = extd_l[min(i + NT, ndep - 1)];
+      const T w = p.two ? T(0.5) : T(0.25);
+      T v[3] = {T(0), T(0), T(0)};
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (k < 2 || !p.two)
+#pragma unroll
+          for (int c = 0; c < 3; c++) v[c] += w * xs[S * p.q[k] + c];
+      put(nown + i, v[0], v[1], v[2]);
+    }
+  }
 }
 
 // owned rows: add the hanging-node sums, then the mode's epilogue
@@ -1650,11 +1644,12 @@ __device__ __forceinline__ void lds_add3(T *p, T a, T b, T c) {
 
 template <class T, int MODE, bool SINGLE_CLASS, bool NODAL, int NT>
 __global__ __launch_bounds__(NT) void k_tile_apply(
-    const int *__restrict__ node0, const int *__restrict__ ext_ptr, const int *__restrict__ ext,
+    const int *__restrict__ node0, const int *__restrict__ ext_ptr,
+    const uint32_t *__restrict__ ext,
     const int *__restrict__ nacc_dep, const int *__restrict__ el_ptr,
     const uint2 *__restrict__ el, int ncolors, const int *__restrict__ comb_ptr,
     const uint4 *__restrict__ comb, const int *__restrict__ extd_ptr,
-    const int4 *__restrict__ extd, const uint8_t *__restrict__ bcmask,
+    const uint2 *__restrict__ extd, const uint8_t *__restrict__ bcmask, int maskall,
     const T *__restrict__ K0, const T *__restrict__ s_elem, const T *__restrict__ x,
     const T *__restrict__ b, T *__restrict__ y, T *__restrict__ x_out, T *__restrict__ d,
     const T *__restrict__ dinv, double ca, double cc, int cflags, double *__restrict__ partials,
@@ -1694,7 +1689,8 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
     w1 = el[3 * (size_t)(q0 + tid) + 1];
     w2 = el[3 * (size_t)(q0 + tid) + 2];
   }
-  tile_stage<T, SX, NT, S>(n0, nown, extd + d0, ndep, ext + e0, nhalo, nacc, bcmask, x, xs, ys);
+  tile_stage<T, SX, NT, S>(n0, nown, extd + d0, ndep, ext + e0, nhalo, nacc, bcmask, maskall, x,
+                           xs, ys);
   __syncthreads();
   for (int r0 = 0; r0 < nel; r0 += NT) {
     const int k = r0 + tid;
@@ -1816,10 +1812,10 @@ __device__ __forceinline__ void put_planes(uint2 *ph, int np, int pos, float vx,
 }
 
 __device__ __forceinline__ void tile_stage_planes(int n0, int nown,
-                                                  const int4 *__restrict__ extd_l, int ndep,
-                                                  const int *__restrict__ ext_l, int nhalo,
+                                                  const uint2 *__restrict__ extd_l, int ndep,
+                                                  const uint32_t *__restrict__ ext_l, int nhalo,
                                                   int nacc, int np,
-                                                  const uint8_t *__restrict__ bcmask,
+                                                  const uint8_t *__restrict__ bcmask, int maskall,
                                                   const float *__restrict__ x, uint2 *ph,
                                                   float *ys) {
   const int tid = threadIdx.x;
@@ -1842,29 +1838,38 @@ __device__ __forceinline__ void tile_stage_planes(int n0, int nown,
                    (mk[k] & 4) ? 0.0f : v[k][2]);
     }
   }
-  for (int i = tid; i < ndep; i += TILE_THREADS) {
-    float v[3];
-    load_dep<float>(extd_l[i], x, bcmask, v);
-    put_planes(ph, np, tile_pos(nown + i), v[0], v[1], v[2]);
-  }
   for (int i = tid; i < nhalo; i += TILE_THREADS) {
-    const int g = ext_l[i];
-    const Vec3<float> u = load_vec3(x + 3 * (size_t)g);
-    const uint8_t m = bcmask[g];
+    const uint32_t g = ext_l[i];
+    const Vec3<float> u = load_vec3(x + 3 * (size_t)halo_node(g));
+    const uint32_t m = (g >> 29) & (uint32_t)maskall;
     put_planes(ph, np, tile_pos(nown + ndep + i), (m & 1) ? 0.0f : u.a, (m & 2) ? 0.0f : u.b,
                (m & 4) ? 0.0f : u.c);
+  }
+  if (ndep > 0) {  // hanging slots from their parents' planes
+    __syncthreads();
+    for (int i = tid; i < ndep; i += TILE_THREADS) {
+      const DepRec p(extd_l[i]);
+      const float w = p.two ? 0.5f : 0.25f;
+      float v[3] = {0.0f, 0.0f, 0.0f};
+      for (int k = 0; k < (p.two ? 2 : 4); k++)
+        for (int c = 0; c < 3; c++)
+          v[c] += w * ((plane_get(ph[p.q[k]], c) + plane_get(ph[p.q[k] + np], c)) +
+                       plane_get(ph[p.q[k] + 2 * np], c));
+      put_planes(ph, np, tile_pos(nown + i), v[0], v[1], v[2]);
+    }
   }
   for (int i = tid; i < 4 * ((nacc + 7) & ~7); i += TILE_THREADS) ys[i] = 0.0f;
 }
 
 template <int MODE, bool SINGLE_CLASS>
 __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma(
-    const int *__restrict__ node0, const int *__restrict__ ext_ptr, const int *__restrict__ ext,
+    const int *__restrict__ node0, const int *__restrict__ ext_ptr,
+    const uint32_t *__restrict__ ext,
     const int *__restrict__ nacc_dep, const int *__restrict__ mb_ptr,
     const uint32_t *__restrict__ mel, int ncolors, const uint4 *__restrict__ afrag,
     const int *__restrict__ comb_ptr, const uint4 *__restrict__ comb,
-    const int *__restrict__ extd_ptr, const int4 *__restrict__ extd,
-    const uint8_t *__restrict__ bcmask, const float *__restrict__ s_elem,
+    const int *__restrict__ extd_ptr, const uint2 *__restrict__ extd,
+    const uint8_t *__restrict__ bcmask, int maskall, const float *__restrict__ s_elem,
     const float *__restrict__ x, const float *__restrict__ b, float *__restrict__ y,
     float *__restrict__ x_out, float *__restrict__ d, const float *__restrict__ dinv, double ca,
     double cc, int cflags, double *__restrict__ partials, int64_t vs,
@@ -1915,7 +1920,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma(
   if (bb0 < bb1) load_rec(bb0, r0);
   if (bb0 + 1 < bb1) load_rec(bb0 + 1, r1);
   if (bb0 + 2 < bb1) load_rec(bb0 + 2, r2);
-  tile_stage_planes(n0, nown, extd + d0, ndep, ext + e0, nhalo, nacc, np, bcmask, x, ph, ys);
+  tile_stage_planes(n0, nown, extd + d0, ndep, ext + e0, nhalo, nacc, np, bcmask, maskall, x, ph, ys);
   // A fragments of K0: [class][part hi, mid, lo][row block][lane]
   Frag a[3][2];
   if (SINGLE_CLASS) {
@@ -2029,12 +2034,13 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma(
 // those of k_tile_apply_mfma; products and sums are FP32 throughout.
 template <int MODE, bool SINGLE_CLASS>
 __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma32(
-    const int *__restrict__ node0, const int *__restrict__ ext_ptr, const int *__restrict__ ext,
+    const int *__restrict__ node0, const int *__restrict__ ext_ptr,
+    const uint32_t *__restrict__ ext,
     const int *__restrict__ nacc_dep, const int *__restrict__ mb_ptr,
     const uint32_t *__restrict__ mel, const float *__restrict__ afrag32,
     const int *__restrict__ comb_ptr, const uint4 *__restrict__ comb,
-    const int *__restrict__ extd_ptr, const int4 *__restrict__ extd,
-    const uint8_t *__restrict__ bcmask, const float *__restrict__ x, const float *__restrict__ b,
+    const int *__restrict__ extd_ptr, const uint2 *__restrict__ extd,
+    const uint8_t *__restrict__ bcmask, int maskall, const float *__restrict__ x, const float *__restrict__ b,
     float *__restrict__ y, float *__restrict__ x_out, float *__restrict__ d,
     const float *__restrict__ dinv, double ca, double cc, int cflags,
     double *__restrict__ partials, int64_t vs, const int *__restrict__ run) {
@@ -2085,7 +2091,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma32(
   if (bb0 + 1 < bb1) load_rec(bb0 + 1, r1);
   if (bb0 + 2 < bb1) load_rec(bb0 + 2, r2);
   tile_stage<float, 3, TILE_THREADS, 4>(n0, nown, extd + d0, ndep, ext + e0, nhalo, nacc,
-                                        bcmask, x, xs, ys);
+                                        bcmask, maskall, x, xs, ys);
   // A fragments: [class][row block][step][lane]
   float a[2][6];
   if (SINGLE_CLASS) {
@@ -2187,6 +2193,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
                        const AsmArgs &g, hipStream_t st, int nrhs, int64_t vs) {
   if (tl.n_tiles == 0) return;
   const dim3 grid(tl.n_tiles, nrhs);
+  const int maskall = tl.masked ? 7 : 0;  // the halo entries' clamp bits
   const size_t sh = ((size_t)tile_xstride<T>() * round8(tl.max_slots) +
                      (size_t)tile_stride<T>() * round8(tl.max_acc)) * sizeof(T);
   const T *b = (const T *)g.b;
@@ -2200,7 +2207,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
   hipLaunchKernelGGL((k_tile_apply_mfma32<M, S>), grid, dim3(TILE_THREADS), sh3, st, tl.node0,  \
                      tl.ext_ptr, tl.ext, tl.nacc_dep, tl.mb_ptr,                                \
                      reinterpret_cast<const uint32_t *>(tl.mel), tl.afrag32, tl.comb_ptr,       \
-                     tl.comb, tl.extd_ptr, tl.extd, tl.bcmask,     \
+                     tl.comb, tl.extd_ptr, tl.extd, tl.bcmask, maskall,     \
                      (const float *)x, (const float *)b, (float *)y, (float *)xo, (float *)d,    \
                      (const float *)dinv, g.ca, g.cc, g.cflags, g.partials, vs, tl.run)
 #define TMRX_MTILE32B(M)    \
@@ -2226,7 +2233,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
   hipLaunchKernelGGL((k_tile_apply_mfma<M, S>), grid, dim3(TILE_THREADS), sh4, st,               \
                      tl.node0, tl.ext_ptr, tl.ext, tl.nacc_dep, tl.mb_ptr,                       \
                      reinterpret_cast<const uint32_t *>(tl.mel), tl.ncolors, tl.afrag, tl.comb_ptr, \
-                     tl.comb, tl.extd_ptr, tl.extd, tl.bcmask,      \
+                     tl.comb, tl.extd_ptr, tl.extd, tl.bcmask, maskall,      \
                      (const float *)s_elem, (const float *)x, (const float *)b, (float *)y,      \
                      (float *)xo, (float *)d, (const float *)dinv, g.ca, g.cc, g.cflags,          \
                      g.partials, vs, tl.run)
@@ -2258,7 +2265,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
   hipLaunchKernelGGL((k_tile_apply<T, M, S, N, NTH>), grid, dim3(NTH), sh, st, tl.node0,          \
                      tl.ext_ptr, tl.ext, tl.nacc_dep, tl.el_ptr,                                  \
                      reinterpret_cast<const uint2 *>(recs), tl.ncolors, tl.comb_ptr,              \
-                     tl.comb, tl.extd_ptr, tl.extd, tl.bcmask, K0,   \
+                     tl.comb, tl.extd_ptr, tl.extd, tl.bcmask, maskall, K0,   \
                      s_elem, x, b, y, xo, d, dinv, g.ca, g.cc, g.cflags, g.partials, vs, tl.run)
 #define TMRX_TILE(M, S)                    \
   if (tl.threads == 512) {                 \

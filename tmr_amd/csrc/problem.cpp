@@ -641,11 +641,15 @@ int Problem::build_tiles(int l) {
   }
   tstart.push_back(n);
   const int ntiles = (int)tstart.size() - 1;
-  std::vector<int> node0(ntiles + 1), ext_ptr{0}, ext, extd_ptr{0}, extd, nacc(ntiles), el_ptr{0};
+  std::vector<int> node0(ntiles + 1), ext_ptr{0}, extd_ptr{0}, nacc(ntiles), el_ptr{0};
   std::vector<TileElem> els, mel;
   std::vector<int> mb_ptr((size_t)ntiles * (MFMA_WAVES + 1), 0);
   std::vector<int> comb_ptr(n + 1, 0);
-  std::vector<uint32_t> comb;
+  std::vector<uint32_t> comb, ext, extd;
+  if (n >= (1 << 29)) {
+    last_error = "problem: a level holds at most 2^29 - 1 nodes";
+    return -1;
+  }
   std::vector<int> stamp_n(n + nd, -1), slot(n + nd, 0), stamp_e(ne, -1);
   std::vector<uint32_t> col;
   int max_slots = 0, max_acc = 0, ncolors = 0, max_mrec = 0, max_rec = 0;
@@ -684,12 +688,6 @@ int Problem::build_tiles(int l) {
     for (int p = n0; p < n1; p++) add_elems(p);
     for (int d : rdeps) add_elems(n + d);
     std::sort(tel.begin(), tel.end());
-    auto put_dep = [&](int d) {
-      const int *p = &dconn[dptr[d]];
-      const bool two = dptr[d + 1] - dptr[d] == 2;
-      for (int k = 0; k < 4; k++) extd.push_back(two && k > 1 ? -1 : p[k]);
-    };
-    for (int d : rdeps) put_dep(d);
     int ns = na;
     // hanging slots first, so that a wave stages one kind of slot
     for (int e : tel)
@@ -698,8 +696,16 @@ int Problem::build_tiles(int l) {
         if (g >= 0 || stamp_n[xid(g)] == t) continue;
         stamp_n[xid(g)] = t;
         slot[xid(g)] = ns++;
-        put_dep(-g - 1);
+        rdeps.push_back(-g - 1);
       }
+    auto add_halo = [&](int g) {
+      if (stamp_n[g] == t) return;
+      stamp_n[g] = t;
+      slot[g] = ns++;
+      ext.push_back((uint32_t)g | (uint32_t)(L.bcmask[g] & 7) << 29);
+    };
+    for (int d : rdeps)
+      for (int j = dptr[d]; j < dptr[d + 1]; j++) add_halo(dconn[j]);
     const size_t el0 = els.size();
     for (int e : tel) {
       TileElem te{};
@@ -708,11 +714,7 @@ int Problem::build_tiles(int l) {
       for (int a = 0; a < 8; a++) {
         const int g = L.conn[8 * e + a];
         const int x = xid(g);
-        if (stamp_n[x] != t) {
-          stamp_n[x] = t;
-          slot[x] = ns++;
-          ext.push_back(g);
-        }
+        if (g >= 0) add_halo(g);
         if (slot[x] >= 65528) {
           last_error = "problem: tile slot index overflow";
           return -1;
@@ -721,6 +723,14 @@ int Problem::build_tiles(int l) {
         if (slot[x] < na) te.mask |= (uint8_t)(1u << a);
       }
       els.push_back(te);
+    }
+    for (int d : rdeps) {
+      const int *pn = &dconn[dptr[d]];
+      const bool two = dptr[d + 1] - dptr[d] == 2;
+      uint32_t q[4];
+      for (int k = 0; k < 4; k++) q[k] = two && k > 1 ? 0xffffu : (uint32_t)tile_pos(slot[pn[k]]);
+      extd.push_back(q[0] | q[1] << 16);
+      extd.push_back(q[2] | q[3] << 16);
     }
     // group equal corner masks (fewer divergent row blocks per wave), then
     // colour greedily over the accumulated slots
@@ -803,9 +813,9 @@ int Problem::build_tiles(int l) {
       }
       cp[MFMA_WAVES] = (int)(mel.size() / 16);
     }
-    nacc[t] = (int)rdeps.size();
+    nacc[t] = na - nown;
     ext_ptr.push_back((int)ext.size());
-    extd_ptr.push_back((int)(extd.size() / 4));
+    extd_ptr.push_back((int)(extd.size() / 2));
     el_ptr.push_back((int)els.size());
     max_slots = std::max(max_slots, ns);
     max_acc = std::max(max_acc, na);
@@ -837,8 +847,8 @@ int Problem::build_tiles(int l) {
     }
   }
   if (comb.empty()) comb.assign(4, 0u);
-  if (extd.empty()) extd.assign(4, 0);
-  if (ext.empty()) ext.push_back(0);
+  if (extd.empty()) extd.assign(2, 0u);
+  if (ext.empty()) ext.push_back(0u);
   if (L.t_node0.upload(node0) || L.t_ext_ptr.upload(ext_ptr) || L.t_ext.upload(ext) ||
       L.t_nacc.upload(nacc) || L.t_el_ptr.upload(el_ptr) || L.t_el.upload(els) ||
       L.t_extd_ptr.upload(extd_ptr) || L.t_extd.upload(extd) ||
@@ -875,7 +885,7 @@ int Problem::build_tiles(int l) {
   T.comb_ptr = L.t_comb_ptr.p;
   T.comb = reinterpret_cast<const uint4 *>(L.t_comb.p);
   T.extd_ptr = L.t_extd_ptr.p;
-  T.extd = reinterpret_cast<const int4 *>(L.t_extd.p);
+  T.extd = reinterpret_cast<const uint2 *>(L.t_extd.p);
   T.bcmask = L.d_bcmask.p;
   T.mb_ptr = L.t_mb_ptr.p;
   T.mel = L.t_mel.p;
@@ -1791,6 +1801,7 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
     HIPCHK(hipMemcpyAsync(lrhs_.p, rhs, m * sizeof(double), hipMemcpyDeviceToDevice, st_));
     Tiles tl = L0.tiles;
     tl.bcmask = nomask_.p;
+    tl.masked = false;
     tl.nodal = design_mode_ == 1;
     tl.use_mfma = false;
     AsmArgs a;

@@ -143,8 +143,8 @@ struct Level {
   DevArray<int> t_mb_ptr;
   DevArray<TileElem> t_mel;
   DevArray<int> t_mel_elem;
-  DevArray<int> t_node0, t_ext_ptr, t_ext, t_extd_ptr, t_extd, t_nacc, t_el_ptr, t_comb_ptr;
-  DevArray<uint32_t> t_comb;
+  DevArray<int> t_node0, t_ext_ptr, t_extd_ptr, t_nacc, t_el_ptr, t_comb_ptr;
+  DevArray<uint32_t> t_ext, t_extd, t_comb;
   DevArray<TileElem> t_el, t_el32;
   DevArray<int> t_el_elem;
   Tiles tiles;
