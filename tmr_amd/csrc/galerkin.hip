@@ -247,6 +247,8 @@ __global__ void __launch_bounds__(256)
     const bool bc = (msk >> c) & 1;
     if (MODE == ASM_STORE) {
       yo[c] = bc ? x[k3 + c] : a[c];
+    } else if (MODE == ASM_POWER) {
+      yo[c] = dinv[k3 + c] * (bc ? x[k3 + c] : a[c]);
     } else if (MODE == ASM_RESID) {
       yo[c] = bc ? T(0) : b[k3 + c] - a[c];
     } else {  // ASM_CHEB
@@ -289,6 +291,9 @@ void launch_bsr_apply(const BSR<T> &A, const T *x, int mode, const AsmArgs &g, h
                        A.val, A.bcmask, x, b, y, xo, d, dinv, ca, cc, g.cflags, A.run, vs);
   else if (mode == ASM_RESID)
     hipLaunchKernelGGL((k_bsr_apply<T, ASM_RESID>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
+                       A.val, A.bcmask, x, b, y, xo, d, dinv, ca, cc, g.cflags, A.run, vs);
+  else if (mode == ASM_POWER)
+    hipLaunchKernelGGL((k_bsr_apply<T, ASM_POWER>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
                        A.val, A.bcmask, x, b, y, xo, d, dinv, ca, cc, g.cflags, A.run, vs);
   else if (mode == ASM_CHEB)
     hipLaunchKernelGGL((k_bsr_apply<T, ASM_CHEB>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,

@@ -168,6 +168,8 @@ enum AsmMode {
   ASM_DIAG = 3,    // Dinv = 1 / diag(A)   (partials hold element diagonals)
   ASM_DOT = 4,     // y = A x and block partials of x . y
   ASM_GATHER = 5,  // y = sum of the slot partials (clamped rows zero): Z^T g
+  ASM_POWER = 6,   // y = Dinv A x (power iteration)
+  ASM_CHEBDOT = 7, // ASM_CHEB and per-tile partials of x_out . dr, x_out . dq
 };
 
 // Chebyshev-step flags: read the previous direction d, take d = x (the step
@@ -184,6 +186,7 @@ struct AsmArgs {
   double ca = 0.0, cc = 0.0;
   int cflags = CHEB_D_READ | CHEB_D_STORE;  // tile apply, ASM_CHEB
   double *partials = nullptr;
+  const double *dr = nullptr, *dq = nullptr;  // ASM_CHEBDOT
 };
 
 // single-pass apply with fused epilogue (modes as AsmMode, except ASM_DIAG);
@@ -423,7 +426,8 @@ struct SegPlan {
   const int *seg_blk = nullptr;  // [nseg + 1]
   const int *seg_tile = nullptr; // [nseg + 1] finest-level owner tiles of each segment
 };
-enum { FIN_BB = 0, FIN_RZ, FIN_PQ, FIN_RR, FIN_BETA, FIN_TRUE };
+// FIN_BETA sums the pairs of launch_b_dot2, FIN_BETA_TILE those of ASM_CHEBDOT
+enum { FIN_BB = 0, FIN_RZ, FIN_PQ, FIN_RR, FIN_BETA, FIN_TRUE, FIN_BETA_TILE };
 void launch_b_dot1(const SegPlan &pl, const double *a, const double *b, const int *act,
                    double *partials, hipStream_t st);
 // r -= alpha q, the FP32 copy r32 of r and, with x1, the finest level's
@@ -444,12 +448,13 @@ void launch_b_copy(const SegPlan &pl, const double *a, double *b, const int *act
                    hipStream_t st);
 // FIN_BB also sets the stop threshold max(rtol2 |b|^2, atol2) and the flags;
 // FIN_RR stops a segment at the threshold (itconv = iteration, negative on
-// breakdown); iter is the device iteration counter advanced by launch_b_tick
+// breakdown) and, with nact, its last block does launch_b_tick's work
 void launch_b_finalize(const SegPlan &pl, int mode, const double *partials, double *sc, int *act,
-                       double *thr2, const int *iter, int *itconv, double rtol2, double atol2,
-                       hipStream_t st);
-// advance the iteration counter and count the running segments into *nact
-void launch_b_tick(int *iter, const int *act, int nidx, int *nact, hipStream_t st);
+                       double *thr2, int *iter, int *itconv, double rtol2, double atol2,
+                       hipStream_t st, int *nact = nullptr, int *host = nullptr);
+// count the running segments into nact[0] and the pinned *host, advance the
+// iteration counter (nact[1]: arrival counter of FIN_RR, zero between launches)
+void launch_b_tick(int *iter, const int *act, int nidx, int *nact, int *host, hipStream_t st);
 
 // per-element compliance density and its design derivative (element mode)
 void launch_elem_energy(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,

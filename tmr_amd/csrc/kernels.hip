@@ -1363,12 +1363,14 @@ __device__ __forceinline__ EpiIn<T> epi_load(int node, const uint8_t *__restrict
                                              int cflags) {
   const size_t k3 = 3 * (size_t)node;
   EpiIn<T> e{{T(0), T(0), T(0)}, {T(0), T(0), T(0)}, {T(0), T(0), T(0)}, {T(0), T(0), T(0)}, 0};
-  if (MODE == ASM_RESID || MODE == ASM_CHEB) e.b = load_vec3(b + k3);
-  if (MODE == ASM_CHEB) {
+  constexpr bool CHEB = MODE == ASM_CHEB || MODE == ASM_CHEBDOT;
+  if (MODE == ASM_RESID || CHEB) e.b = load_vec3(b + k3);
+  if (MODE == ASM_POWER) e.w = load_vec3(dinv + k3);
+  if (CHEB) {
     if (cflags & CHEB_D_READ) e.d = load_vec3(d + k3);
     e.w = load_vec3(dinv + k3);
   }
-  if (MODE == ASM_STORE || MODE == ASM_DOT) e.x = load_vec3(x + k3);
+  if (MODE == ASM_STORE || MODE == ASM_DOT || MODE == ASM_POWER) e.x = load_vec3(x + k3);
   e.m = bcmask[node];
   return e;
 }
@@ -1379,7 +1381,9 @@ __device__ __forceinline__ void tile_finish(
     const uint8_t *__restrict__ bcmask, const T *xs, const T *ys,
     const T *__restrict__ x, const T *__restrict__ b, T *__restrict__ y, T *__restrict__ x_out,
     T *__restrict__ d, const T *__restrict__ dinv, double ca, double cc, int cflags,
-    double *__restrict__ partials, double *red, int pstride = 0, bool hang = true) {
+    double *__restrict__ partials, double *red, int pstride = 0, bool hang = true,
+    const double *__restrict__ dr = nullptr, const double *__restrict__ dq = nullptr) {
+  constexpr bool CHEB = MODE == ASM_CHEB || MODE == ASM_CHEBDOT;
   auto xat = [&](int pos, int c) -> T {
     if constexpr (SPLIT) {
       const uint2 *ph = reinterpret_cast<const uint2 *>(xs);
@@ -1389,7 +1393,7 @@ __device__ __forceinline__ void tile_finish(
       return xs[SX * pos + c];
     }
   };
-  double dot = 0.0;
+  double dot = 0.0, dot2 = 0.0;
   // two owned nodes per thread at a time: both nodes' loads (one per node
   // and vector, indices clamped into the tile) go out before either is used
   for (int i0 = threadIdx.x; i0 < nown; i0 += 2 * NT) {
@@ -1397,6 +1401,14 @@ __device__ __forceinline__ void tile_finish(
 #pragma unroll
     for (int u = 0; u < 2; u++)
       ein[u] = epi_load<T, MODE>(n0 + min(i0 + u * NT, nown - 1), bcmask, x, b, d, dinv, cflags);
+    Vec3<double> er[2], eq[2];
+    if (MODE == ASM_CHEBDOT)
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const size_t k3 = 3 * (size_t)(n0 + min(i0 + u * NT, nown - 1));
+        er[u] = load_vec3(dr + k3);
+        eq[u] = load_vec3(dq + k3);
+      }
     int cj[2][2] = {{0, 0}, {0, 0}};
     if (hang) {
 #pragma unroll
@@ -1440,6 +1452,8 @@ __device__ __forceinline__ void tile_finish(
         const bool bc = (m >> c) & 1;
         if (MODE == ASM_STORE) {
           yo[c] = bc ? xv[c] : a[c];
+        } else if (MODE == ASM_POWER) {
+          yo[c] = wv[c] * (bc ? xv[c] : a[c]);
         } else if (MODE == ASM_DOT) {
           const T xx = bc ? xv[c] : xat(ti, c);
           const T v = bc ? xx : a[c];
@@ -1447,7 +1461,7 @@ __device__ __forceinline__ void tile_finish(
           dot += (double)xx * (double)v;
         } else if (MODE == ASM_RESID) {
           yo[c] = bc ? T(0) : bv[c] - a[c];
-        } else if (MODE == ASM_CHEB) {
+        } else if (CHEB) {
           if (bc) {
             dno[c] = T(0);
             yo[c] = T(0);
@@ -1462,9 +1476,14 @@ __device__ __forceinline__ void tile_finish(
         }
       }
       // one store per node and vector
-      if (MODE == ASM_CHEB) {
+      if (CHEB) {
         if (cflags & CHEB_D_STORE) store_vec3(d + k3, dno);
         store_vec3(x_out + k3, yo);
+        if (MODE == ASM_CHEBDOT) {
+          const double z[3] = {(double)yo[0], (double)yo[1], (double)yo[2]};
+          dot += z[0] * er[u].a + z[1] * er[u].b + z[2] * er[u].c;
+          dot2 += z[0] * eq[u].a + z[1] * eq[u].b + z[2] * eq[u].c;
+        }
       } else {
         store_vec3(y + k3, yo);
       }
@@ -1473,6 +1492,15 @@ __device__ __forceinline__ void tile_finish(
   if (MODE == ASM_DOT) {
     const double sum = block_sum(dot, red);
     if (threadIdx.x == 0) partials[t] = sum;
+  }
+  if (MODE == ASM_CHEBDOT) {
+    const double sum = block_sum(dot, red);
+    __syncthreads();
+    const double sum2 = block_sum(dot2, red);
+    if (threadIdx.x == 0) {
+      partials[2 * (size_t)t] = sum;
+      partials[2 * (size_t)t + 1] = sum2;
+    }
   }
 }
 
@@ -1653,8 +1681,14 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
     const T *__restrict__ K0, const T *__restrict__ s_elem, const T *__restrict__ x,
     const T *__restrict__ b, T *__restrict__ y, T *__restrict__ x_out, T *__restrict__ d,
     const T *__restrict__ dinv, double ca, double cc, int cflags, double *__restrict__ partials,
-    int64_t vs, const int *__restrict__ run) {
-  if (run && *run == 0) return;
+    int64_t vs, const int *__restrict__ run, const double *__restrict__ dr,
+    const double *__restrict__ dq) {
+  // a grid that fills the chip tests the run flag first; in a small one its
+  // round trip to memory would precede every tile's loads, so it is tested
+  // once they are under way
+  const bool late = gridDim.x < 2048;
+  if (!late && run && *run == 0) return;
+  const int go = late && run ? *run : 1;
   constexpr int S = tile_stride<T>();
   constexpr int SX = tile_xstride<T>();
   // FP32 element-density products scale in the accumulation FMAs (24 fewer
@@ -1672,7 +1706,13 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
     if (y) y += off;
     if (x_out) x_out += off;
     if (d) d += off;
-    if (partials) partials += (int64_t)blockIdx.y * gridDim.x;
+    if (MODE == ASM_CHEBDOT) {
+      dr += off;
+      dq += off;
+      partials += 2 * (int64_t)blockIdx.y * gridDim.x;
+    } else if (partials) {
+      partials += (int64_t)blockIdx.y * gridDim.x;
+    }
   }
   const int n0 = node0[t], nown = node0[t + 1] - n0;
   const int e0 = ext_ptr[t], nhalo = ext_ptr[t + 1] - e0;
@@ -1691,6 +1731,7 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
   }
   tile_stage<T, SX, NT, S>(n0, nown, extd + d0, ndep, ext + e0, nhalo, nacc, bcmask, maskall, x,
                            xs, ys);
+  if (!go) return;  // the same for the whole grid
   __syncthreads();
   for (int r0 = 0; r0 < nel; r0 += NT) {
     const int k = r0 + tid;
@@ -1753,7 +1794,7 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
   }
   tile_finish<T, MODE, S, NT, false, SX>(t, n0, nown, comb_ptr, comb, bcmask, xs, ys, x, b, y,
                                          x_out, d, dinv, ca, cc, cflags, partials, red, 0,
-                                         nacc > nown);
+                                         nacc > nown, dr, dq);
 }
 
 // ---------------------------------------------------------------------------
@@ -2266,7 +2307,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
                      tl.ext_ptr, tl.ext, tl.nacc_dep, tl.el_ptr,                                  \
                      reinterpret_cast<const uint2 *>(recs), tl.ncolors, tl.comb_ptr,              \
                      tl.comb, tl.extd_ptr, tl.extd, tl.bcmask, maskall, K0,   \
-                     s_elem, x, b, y, xo, d, dinv, g.ca, g.cc, g.cflags, g.partials, vs, tl.run)
+                     s_elem, x, b, y, xo, d, dinv, g.ca, g.cc, g.cflags, g.partials, vs, tl.run, g.dr, g.dq)
 #define TMRX_TILE(M, S)                    \
   if (tl.threads == 512) {                 \
     if (tl.nodal)                          \
@@ -2290,6 +2331,13 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
     case ASM_RESID: TMRX_TILE2(ASM_RESID); break;
     case ASM_CHEB: TMRX_TILE2(ASM_CHEB); break;
     case ASM_DOT: TMRX_TILE2(ASM_DOT); break;
+    case ASM_CHEBDOT: TMRX_TILE2(ASM_CHEBDOT); break;
+    case ASM_POWER:
+      if constexpr (sizeof(T) == 8) {
+        TMRX_TILE2(ASM_POWER);
+        break;
+      }
+    default: note_launch(hipErrorInvalidValue);
   }
 #undef TMRX_TILE2
 #undef TMRX_TILE

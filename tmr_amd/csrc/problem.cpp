@@ -1066,16 +1066,17 @@ int Problem::ensure_batch(int nrhs) {
   const size_t n = (size_t)L0.ndof, m = n * (size_t)nrhs;
   const size_t nidx = (size_t)nrhs * nseg_;
   const size_t np = std::max({(size_t)2 * 2048, (size_t)assemble_num_blocks(L0.n_nodes),
-                              (size_t)L0.tiles.n_tiles * nrhs, (size_t)2 * plan_.nblk * nrhs,
+                              (size_t)2 * L0.tiles.n_tiles * nrhs, (size_t)2 * plan_.nblk * nrhs,
                               (size_t)(L0.n_elem + 255) / 256}) + 16;
   if (f_.alloc(m) || u_.alloc(m) || r_.alloc(m) || p_.alloc(m) || q_.alloc(m) || z_.alloc(m) ||
       parts_.alloc(np) || sc_.alloc(std::max(nidx * SC_N, (size_t)SC_N)) || act_.alloc(nidx) ||
-      itconv_.alloc(nidx) || thr_.alloc(nidx) || iter_.alloc(1) || nact_.alloc(1)) {
+      itconv_.alloc(nidx) || thr_.alloc(nidx) || iter_.alloc(1) || nact_.alloc(2)) {
     last_error = "problem: device allocation failed";
     return -1;
   }
   HIPCHK(hipMemset(u_.p, 0, m * sizeof(double)));
   HIPCHK(hipMemset(f_.p, 0, m * sizeof(double)));
+  HIPCHK(hipMemset(nact_.p, 0, 2 * sizeof(int)));
   if (!nact_host_) HIPCHK(hipHostMalloc((void **)&nact_host_, 2 * sizeof(int)));
   have_solution_ = false;
   batch_cap_ = nrhs;
@@ -1087,7 +1088,9 @@ int Problem::ensure_batch(int nrhs) {
 // component
 int Problem::build_plan() {
   const Level &L = levels_[0];
-  constexpr int CHUNK = 4096;  // dofs per reduction block
+  // dofs per reduction block: 4096 once that alone fills the chip, fewer (a
+  // shorter chain per thread) below
+  const int CHUNK = L.ndof >= 2048 * 4096 ? 4096 : 1024;
   std::vector<int> lo, bseg, sblk{0};
   for (int sg = 0; sg < nseg_; sg++) {
     const int d0 = 3 * L.seg_node0[sg], d1 = 3 * L.seg_node0[sg + 1];
@@ -1267,7 +1270,7 @@ template <class T>
 void Problem::apply_level(int l, const T *x, int mode, const AsmArgs &a, int nrhs) {
   Level &L = levels_[l];
   std::pair<hipEvent_t, hipEvent_t> *ev = nullptr;
-  if (l == 0 && ((timing_ >> mode) & 1)) {
+  if (l == 0 && ((timing_ >> (mode == ASM_POWER ? ASM_STORE : mode)) & 1)) {
     if (ev_used_ == ev_pool_.size()) {
       std::pair<hipEvent_t, hipEvent_t> e;
       if (hipEventCreate(&e.first) == hipSuccess && hipEventCreate(&e.second) == hipSuccess)
@@ -1313,11 +1316,16 @@ int Problem::estimate_eigs(int l, const SolveOpts &o, bool defer) {
   launch_start_vector(n, L.d_bcmask.p, 0x2545f4914f6cdd1dULL * (uint64_t)(l + 1), v.x.p, st_);
   double *a = v.x.p, *b = v.r.p;
   const int iters = std::max(1, o.eig_iters);
+  // Dinv rides in the product's epilogue; the norms are only needed once, so
+  // the last step keeps the separate pass that forms them (10 such passes
+  // were a tenth of a set-up: 4.2M hex 70 us each, 16^3 cube 4 us)
   for (int it = 0; it < iters; it++) {
+    const bool end = it + 1 == iters;
     AsmArgs g;
     g.y = b;
-    apply_level<double>(l, a, ASM_STORE, g);
-    launch_dinv_dots(n, v.dinv.p, b, a, parts_.p, st_);
+    g.dinv = v.dinv.p;
+    apply_level<double>(l, a, end ? ASM_STORE : ASM_POWER, g);
+    if (end) launch_dinv_dots(n, v.dinv.p, b, a, parts_.p, st_);
     std::swap(a, b);
   }
   double *slot = eig_sc_.p + (size_t)SC_N * l;
@@ -1521,7 +1529,7 @@ int Problem::setup(const SolveOpts &o) {
 // (tiles read halo values of x, so the update cannot be in place).
 template <class T>
 void Problem::cheb_step(int l, const T *b, const T *x_in, T *x_out, int k, const SolveOpts &o,
-                        int nrhs, int cflags) {
+                        int nrhs, int cflags, bool dots) {
   Level &L = levels_[l];
   LevelVecs<T> &v = vecs<T>(l);
   const double lmax = o.cheb_upper * L.lam_max, lmin = o.cheb_lower * L.lam_max;
@@ -1543,7 +1551,12 @@ void Problem::cheb_step(int l, const T *b, const T *x_in, T *x_out, int k, const
   a.ca = ca;
   a.cc = cc;
   a.cflags = k == 0 ? (cflags & CHEB_D_STORE) : cflags;  // step 0: no previous direction
-  apply_level<T>(l, x_in, ASM_CHEB, a, nrhs);
+  if (dots) {
+    a.dr = r_.p;
+    a.dq = q_.p;
+    a.partials = parts_.p;
+  }
+  apply_level<T>(l, x_in, dots ? ASM_CHEBDOT : ASM_CHEB, a, nrhs);
 }
 
 template <class T>
@@ -1647,7 +1660,8 @@ void Problem::vcycle(int l, const T *b, T *x, const SolveOpts &o, int nrhs, bool
   vcycle<T>(l + 1, c.b.p, c.x.p, o, nrhs, fuse);
   launch_prolong_add<T>(P, L.d_bcmask.p, c.x.p, cur, st_, nrhs, Lc.ndof, L.ndof);
   for (int k = 0; k < deg; k++) {
-    cheb_step<T>(l, b, cur, oth, k, o, nrhs, CHEB_D_READ | (k + 1 < deg ? CHEB_D_STORE : 0));
+    cheb_step<T>(l, b, cur, oth, k, o, nrhs, CHEB_D_READ | (k + 1 < deg ? CHEB_D_STORE : 0),
+                 l == 0 && k + 1 == deg && zdots_);
     std::swap(cur, oth);
   }
 }
@@ -1732,29 +1746,45 @@ void Problem::enqueue_iteration(const SegPlan &pl, int nrhs, double *xsol, const
   launch_b_update_xr(pl, r_.p, q_.p, r32, sc_.p, act_.p, parts_.p, st_,
                      fuse0 ? L0u.v32.dinv.p : nullptr, fuse0 ? cheb_c0<float>(0, o) : 0.0,
                      fuse0 ? first_target<float>(0, L0u.v32.x.p, o) : nullptr);
+  // its last block counts the segments still running (and advances the
+  // iteration counter) before the preconditioner: an iteration that converged
+  // skips it
   launch_b_finalize(pl, FIN_RR, parts_.p, sc_.p, act_.p, thr_.p, iter_.p, itconv_.p, rtol2, atol2,
-                    st_);
-  // count the segments still running (and advance the iteration counter)
-  // before the preconditioner: an iteration that converged skips it
-  launch_b_tick(iter_.p, act_.p, nidx, nact_.p, st_);
+                    st_, nact_.p, nact_host_ + slot);
   // z = M r; in mixed precision the FP64 updates read the FP32 result
   // directly (no FP64 copy of z)
   if (mixed) {
     Level &L0 = levels_[0];
+    const bool dots = vcycle_dots(o, nrhs);
+    zdots_ = dots;
     vcycle<float>(0, L0.v32.b.p, L0.v32.x.p, o, nrhs, fuse0);
-    launch_b_dot2<float>(pl, L0.v32.x.p, r_.p, q_.p, act_.p, parts_.p, st_);
-    launch_b_finalize(pl, FIN_BETA, parts_.p, sc_.p, act_.p, thr_.p, iter_.p, itconv_.p, rtol2,
+    zdots_ = false;
+    if (!dots) launch_b_dot2<float>(pl, L0.v32.x.p, r_.p, q_.p, act_.p, parts_.p, st_);
+    launch_b_finalize(pl, dots ? FIN_BETA_TILE : FIN_BETA, parts_.p, sc_.p, act_.p, thr_.p, iter_.p, itconv_.p, rtol2,
                       atol2, st_);
     launch_b_update_p<float>(pl, p_.p, L0.v32.x.p, sc_.p, act_.p, xsol, iter_.p, st_);
   } else {
+    const bool dots = vcycle_dots(o, nrhs);
+    zdots_ = dots;
     precond(nrhs, o);
-    launch_b_dot2<double>(pl, z_.p, r_.p, q_.p, act_.p, parts_.p, st_);
-    launch_b_finalize(pl, FIN_BETA, parts_.p, sc_.p, act_.p, thr_.p, iter_.p, itconv_.p, rtol2,
+    zdots_ = false;
+    if (!dots) launch_b_dot2<double>(pl, z_.p, r_.p, q_.p, act_.p, parts_.p, st_);
+    launch_b_finalize(pl, dots ? FIN_BETA_TILE : FIN_BETA, parts_.p, sc_.p, act_.p, thr_.p, iter_.p, itconv_.p, rtol2,
                       atol2, st_);
     launch_b_update_p<double>(pl, p_.p, z_.p, sc_.p, act_.p, xsol, iter_.p, st_);
   }
   run_ = nullptr;
-  (void)hipMemcpyAsync(nact_host_ + slot, nact_.p, sizeof(int), hipMemcpyDeviceToHost, st_);
+}
+
+// z.r and z.q ride in the finest level's last smoothing step (Chebyshev, on
+// the vector ALUs, of a level that is not also the coarsest) while the launch
+// saved counts: below 2048 tiles in flight.  16^3 cube: 9.7 us against 8.6 +
+// 6.0 for step and dots; 4.2M hex: 147 us against 93 + 47, the tiles read r
+// and q more slowly than the streaming pass.
+bool Problem::vcycle_dots(const SolveOpts &o, int nrhs) const {
+  const bool mfma = o.precision != 0 && fp32_mfma_ && !fp32_valu_ && design_mode_ == 0;
+  return levels_.size() > 1 && !sor_ && !mfma && timing_ == 0 &&
+         (int64_t)levels_[0].tiles.n_tiles * nrhs < 2048;
 }
 
 int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o,
@@ -1833,8 +1863,7 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
   launch_b_copy(pl, z_.p, p_.p, nullptr, st_);
   HIPCHK(hipMemsetAsync(iter_.p, 0, sizeof(int), st_));
   // count the running segments; iteration counter to 1
-  launch_b_tick(iter_.p, act_.p, nidx, nact_.p, st_);
-  HIPCHK(hipMemcpyAsync(nact_host_, nact_.p, sizeof(int), hipMemcpyDeviceToHost, st_));
+  launch_b_tick(iter_.p, act_.p, nidx, nact_.p, nact_host_, st_);
   HIPCHK(hipStreamSynchronize(st_));
   int running = nact_host_[0];
   // iterations: replayed graphs (or enqueued bodies), the stop count of
@@ -1880,17 +1909,33 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
   int launched = 0;
   while (running > 0 && launched < o.max_iters) {
     const int slot = launched & 1;
+    volatile int *count = nact_host_ + slot;
+    *count = -1;
     if (graphs)
       HIPCHK(hipGraphLaunch(gexec_[slot], st_));
     else
       enqueue_iteration(pl, nrhs, xsol, o, slot);
     HIPCHK(hipEventRecord(gev_[slot], st_));
     launched++;
-    if (o.monitor || launched >= 2) {
+    if (graphs) {
+      // the count reaches the pinned word before the iteration's V-cycle, so
+      // the next graph is launched in time and none is launched in vain (an
+      // iteration of empty launches costs 80 us); the event ends the wait
+      // whatever happens to the word
+      int spins = 0;
+      while (*count < 0)
+        if (++spins % 256 == 0 && hipEventQuery(gev_[slot]) != hipErrorNotReady) break;
+      if (*count < 0) HIPCHK(hipEventSynchronize(gev_[slot]));
+      running = *count;
+    } else if (o.monitor || launched >= 2) {
       const int prev = o.monitor ? slot : (slot ^ 1);
       HIPCHK(hipEventSynchronize(gev_[prev]));
       running = nact_host_[prev];
       if (o.monitor) fprintf(stderr, "[tmrx] pcg %3d  running %d of %d\n", launched, running, nidx);
+    }
+    if (running < 0) {
+      last_error = "solve: the device did not report its running count";
+      return -1;
     }
   }
   HIPCHK(hipStreamSynchronize(st_));
