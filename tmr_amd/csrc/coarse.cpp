@@ -449,6 +449,7 @@ int Problem::build_coarse_plan() {
   coarse_.nb = cb_nb_.p;
   coarse_.aoff = cb_aoff_.p;
   cp.built = true;
+  gen_++;
   return 0;
 }
 
@@ -525,9 +526,12 @@ int Problem::coarse_factor() {
   coarse_.Ainv32 = nullptr;
   if (setup_prec_pending_ == 1) {
     const size_t words = (size_t)(cp.na + 2 * cp.nw);
-    if (Ainv32_.n < words && Ainv32_.alloc(words)) {
-      last_error = "coarse: device allocation failed";
-      return -1;
+    if (Ainv32_.n < words) {
+      if (Ainv32_.alloc(words)) {
+        last_error = "coarse: device allocation failed";
+        return -1;
+      }
+      gen_++;
     }
     launch_convert<double, float>((int64_t)words, Ainv_.p, Ainv32_.p, st_);
     coarse_.Ainv32 = Ainv32_.p;

@@ -183,7 +183,9 @@ struct AsmArgs {
   void *x_out = nullptr;   // CHEB iterate output of the tile kernel
   void *d = nullptr;       // Chebyshev direction
   const void *dinv = nullptr;
-  double ca = 0.0, cc = 0.0;
+  // ASM_CHEB: device pair (a, c) of the step, so that a captured iteration
+  // outlives a new set-up's eigenvalue bounds
+  const double *cf = nullptr;
   int cflags = CHEB_D_READ | CHEB_D_STORE;  // tile apply, ASM_CHEB
   double *partials = nullptr;
   const double *dr = nullptr, *dq = nullptr;  // ASM_CHEBDOT
@@ -216,14 +218,14 @@ template <class T>
 void launch_prolong_add(const TransferCSR &P, const uint8_t *bcmask_f, const T *xc, T *xf,
                         hipStream_t st, int nrhs = 1, int64_t vsc = 0, int64_t vsf = 0);
 // rc = R rf (clamped rows zero); with x1, also the coarse level's first
-// Chebyshev step from zero, x1 = c0 Dinv_c rc
+// Chebyshev step from zero, x1 = *c0 Dinv_c rc
 template <class T>
 void launch_restrict(const TransferCSR &R, const uint8_t *bcmask_c, const T *rf, T *rc,
                      hipStream_t st, int nrhs = 1, int64_t vsf = 0, int64_t vsc = 0,
-                     const T *dinv_c = nullptr, double c0 = 0.0, T *x1 = nullptr);
-// x = c Dinv b (and d = x when d is not null)
+                     const T *dinv_c = nullptr, const double *c0 = nullptr, T *x1 = nullptr);
+// x = *c Dinv b (and d = x when d is not null)
 template <class T>
-void launch_cheb_first(int ndof, const T *b, const T *dinv, double c, T *d, T *x,
+void launch_cheb_first(int ndof, const T *b, const T *dinv, const double *c, T *d, T *x,
                        hipStream_t st, int nrhs = 1, const int *run = nullptr);
 // one dense SPD matrix of a batched inversion: n rows padded to nblk blocks
 // of 64 (leading dimension 64 nblk), at `off` in both buffers
@@ -337,6 +339,8 @@ void launch_sor_sweep(const BSR<T> &A, const int *nodes, const int *cptr, int nc
                       const T *b, T *x, double omega, hipStream_t st, int nrhs = 1,
                       int64_t vs = 0);
 
+// dst[0..n) = v (n <= 32), from kernel arguments
+void launch_set_words(int n, const double *v, double *dst, hipStream_t st);
 template <class TI, class TO>
 void launch_convert(int64_t n, const TI *a, TO *b, hipStream_t st);
 template <class T>
@@ -435,7 +439,8 @@ void launch_b_dot1(const SegPlan &pl, const double *a, const double *b, const in
 // the same iteration's p update, which reads p anyway)
 void launch_b_update_xr(const SegPlan &pl, double *r, const double *q, float *r32,
                         const double *sc, const int *act, double *partials, hipStream_t st,
-                        const float *dinv32 = nullptr, double c0 = 0.0, float *x1 = nullptr);
+                        const float *dinv32 = nullptr, const double *c0 = nullptr,
+                        float *x1 = nullptr);
 template <class TZ>
 void launch_b_dot2(const SegPlan &pl, const TZ *z, const double *r, const double *q,
                    const int *act, double *partials, hipStream_t st);

@@ -302,7 +302,8 @@ __global__ __launch_bounds__(NODE_BLOCK) void k_assemble(
     int n, const int *__restrict__ ptr, const int *__restrict__ slot, const float *__restrict__ w,
     const uint8_t *__restrict__ bcmask, const T *__restrict__ partial, const T *__restrict__ b,
     T *__restrict__ y, T *__restrict__ x, T *__restrict__ d, const T *__restrict__ dinv,
-    double ca, double cc, double *__restrict__ partials) {
+    const double *__restrict__ cf, double *__restrict__ partials) {
+  const double ca = MODE == ASM_CHEB ? cf[0] : 0.0, cc = MODE == ASM_CHEB ? cf[1] : 0.0;
   __shared__ double red[NODE_BLOCK / 64];
   const int i = xcd_block(blockIdx.x, gridDim.x) * NODE_BLOCK + threadIdx.x;
   double dot = 0.0;
@@ -365,7 +366,7 @@ void launch_assemble(const AsmCSR &a, const uint8_t *bcmask, const T *partial, i
   const T *dinv = (const T *)g.dinv;
 #define TMRX_ASM(M)                                                                           \
   hipLaunchKernelGGL((k_assemble<T, M>), dim3(nb), dim3(NODE_BLOCK), 0, st, a.n_nodes, a.ptr, \
-                     a.slot, a.w, bcmask, partial, b, y, x, d, dinv, g.ca, g.cc, g.partials)
+                     a.slot, a.w, bcmask, partial, b, y, x, d, dinv, g.cf, g.partials)
   switch (mode) {
     case ASM_STORE: TMRX_ASM(ASM_STORE); break;
     case ASM_RESID: TMRX_ASM(ASM_RESID); break;
@@ -432,7 +433,8 @@ __global__ __launch_bounds__(256) void k_restrict(int n, const int *__restrict__
                                                   const T *__restrict__ rf, T *__restrict__ rc,
                                                   int64_t vsf, int64_t vsc,
                                                   const int *__restrict__ run,
-                                                  const T *__restrict__ dinv_c, double c0,
+                                                  const T *__restrict__ dinv_c,
+                                                  const double *__restrict__ c0p,
                                                   T *__restrict__ x1,
                                                   const uint8_t *__restrict__ wexp) {
   if (run && *run == 0) return;
@@ -444,10 +446,14 @@ __global__ __launch_bounds__(256) void k_restrict(int n, const int *__restrict__
   T a0 = T(0), a1 = T(0), a2 = T(0);
   // the row's own inputs (mask, coarse diagonal) load before the gathers
   uint8_t m = 0;
+  double c0 = 0.0;
   Vec3<T> di{T(0), T(0), T(0)};
   if (i < n && sub == 0) {
     m = mask[i];
-    if (x1) di = load_vec3(dinv_c + 3 * (size_t)i);
+    if (x1) {
+      di = load_vec3(dinv_c + 3 * (size_t)i);
+      c0 = *c0p;
+    }
   }
   if (i < n) {
     const int j1 = ptr[i + 1];
@@ -501,7 +507,7 @@ void launch_prolong_add(const TransferCSR &P, const uint8_t *mask_f, const T *xc
 template <class T>
 void launch_restrict(const TransferCSR &R, const uint8_t *mask_c, const T *rf, T *rc,
                      hipStream_t st, int nrhs, int64_t vsf, int64_t vsc, const T *dinv_c,
-                     double c0, T *x1) {
+                     const double *c0, T *x1) {
   if (R.n_rows == 0) return;
   const int64_t threads = 8 * (int64_t)R.n_rows;
   hipLaunchKernelGGL(k_restrict<T>, dim3((unsigned)((threads + 255) / 256), nrhs), dim3(256), 0,
@@ -513,20 +519,21 @@ void launch_restrict(const TransferCSR &R, const uint8_t *mask_c, const T *rf, T
 // ---------------------------------------------------------------------------
 // Chebyshev first step from a zero guess: d = c Dinv b, x = d
 template <class T>
-__global__ void k_cheb_first(int n, const T *__restrict__ b, const T *__restrict__ dinv, double c,
+__global__ void k_cheb_first(int n, const T *__restrict__ b, const T *__restrict__ dinv,
+                             const double *__restrict__ c,
                              T *__restrict__ d, T *__restrict__ x, int64_t vs,
                              const int *__restrict__ run) {
   if (run && *run == 0) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int64_t off = (int64_t)blockIdx.y * vs;
-  const T v = (T)c * dinv[i] * b[off + i];
+  const T v = (T)*c * dinv[i] * b[off + i];
   if (d) d[off + i] = v;
   x[off + i] = v;
 }
 
 template <class T>
-void launch_cheb_first(int ndof, const T *b, const T *dinv, double c, T *d, T *x,
+void launch_cheb_first(int ndof, const T *b, const T *dinv, const double *c, T *d, T *x,
                        hipStream_t st, int nrhs, const int *run) {
   hipLaunchKernelGGL(k_cheb_first<T>, dim3((ndof + 255) / 256, nrhs), dim3(256), 0, st, ndof, b,
                      dinv, c, d, x, (int64_t)ndof, run);
@@ -584,6 +591,20 @@ void launch_dense_solve(const CoarseBlocks &cb, const T *b, T *x, hipStream_t st
   else
     hipLaunchKernelGGL((k_dense_solve<T, double>), dim3((cb.n + 3) / 4, nrhs), dim3(256), 0, st,
                        cb.n, cb.Ainv, cb.col0, cb.nb, cb.aoff, b, x, cb.run);
+  TMRX_LAUNCH_CHECK();
+}
+
+struct Words32 {
+  double v[32];
+};
+__global__ void k_set_words(int n, Words32 w, double *__restrict__ dst) {
+  const int i = threadIdx.x;
+  if (i < n) dst[i] = w.v[i];
+}
+void launch_set_words(int n, const double *v, double *dst, hipStream_t st) {
+  Words32 w{};
+  for (int i = 0; i < n && i < 32; i++) w.v[i] = v[i];
+  hipLaunchKernelGGL(k_set_words, dim3(1), dim3(32), 0, st, n, w, dst);
   TMRX_LAUNCH_CHECK();
 }
 
@@ -1680,8 +1701,8 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
     const uint2 *__restrict__ extd, const uint8_t *__restrict__ bcmask, int maskall,
     const T *__restrict__ K0, const T *__restrict__ s_elem, const T *__restrict__ x,
     const T *__restrict__ b, T *__restrict__ y, T *__restrict__ x_out, T *__restrict__ d,
-    const T *__restrict__ dinv, double ca, double cc, int cflags, double *__restrict__ partials,
-    int64_t vs, const int *__restrict__ run, const double *__restrict__ dr,
+    const T *__restrict__ dinv, const double *__restrict__ cf, int cflags,
+    double *__restrict__ partials, int64_t vs, const int *__restrict__ run, const double *__restrict__ dr,
     const double *__restrict__ dq) {
   // a grid that fills the chip tests the run flag first; in a small one its
   // round trip to memory would precede every tile's loads, so it is tested
@@ -1689,6 +1710,8 @@ __global__ __launch_bounds__(NT) void k_tile_apply(
   const bool late = gridDim.x < 2048;
   if (!late && run && *run == 0) return;
   const int go = late && run ? *run : 1;
+  constexpr bool CHEB = MODE == ASM_CHEB || MODE == ASM_CHEBDOT;
+  const double ca = CHEB ? cf[0] : 0.0, cc = CHEB ? cf[1] : 0.0;
   constexpr int S = tile_stride<T>();
   constexpr int SX = tile_xstride<T>();
   // FP32 element-density products scale in the accumulation FMAs (24 fewer
@@ -1912,9 +1935,10 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma(
     const int *__restrict__ extd_ptr, const uint2 *__restrict__ extd,
     const uint8_t *__restrict__ bcmask, int maskall, const float *__restrict__ s_elem,
     const float *__restrict__ x, const float *__restrict__ b, float *__restrict__ y,
-    float *__restrict__ x_out, float *__restrict__ d, const float *__restrict__ dinv, double ca,
-    double cc, int cflags, double *__restrict__ partials, int64_t vs,
+    float *__restrict__ x_out, float *__restrict__ d, const float *__restrict__ dinv,
+    const double *__restrict__ cf, int cflags, double *__restrict__ partials, int64_t vs,
     const int *__restrict__ run) {
+  const double ca = MODE == ASM_CHEB ? cf[0] : 0.0, cc = MODE == ASM_CHEB ? cf[1] : 0.0;
   if (run && *run == 0) return;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double red[TILE_THREADS / 64];
@@ -2083,9 +2107,10 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_apply_mfma32(
     const int *__restrict__ extd_ptr, const uint2 *__restrict__ extd,
     const uint8_t *__restrict__ bcmask, int maskall, const float *__restrict__ x, const float *__restrict__ b,
     float *__restrict__ y, float *__restrict__ x_out, float *__restrict__ d,
-    const float *__restrict__ dinv, double ca, double cc, int cflags,
+    const float *__restrict__ dinv, const double *__restrict__ cf, int cflags,
     double *__restrict__ partials, int64_t vs, const int *__restrict__ run) {
   if (run && *run == 0) return;
+  const double ca = MODE == ASM_CHEB ? cf[0] : 0.0, cc = MODE == ASM_CHEB ? cf[1] : 0.0;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double red[TILE_THREADS / 64];
   const int t = xcd_block(blockIdx.x, gridDim.x);
@@ -2250,7 +2275,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
                      reinterpret_cast<const uint32_t *>(tl.mel), tl.afrag32, tl.comb_ptr,       \
                      tl.comb, tl.extd_ptr, tl.extd, tl.bcmask, maskall,     \
                      (const float *)x, (const float *)b, (float *)y, (float *)xo, (float *)d,    \
-                     (const float *)dinv, g.ca, g.cc, g.cflags, g.partials, vs, tl.run)
+                     (const float *)dinv, g.cf, g.cflags, g.partials, vs, tl.run)
 #define TMRX_MTILE32B(M)    \
   if (single) {             \
     TMRX_MTILE32(M, true);  \
@@ -2276,7 +2301,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
                      reinterpret_cast<const uint32_t *>(tl.mel), tl.ncolors, tl.afrag, tl.comb_ptr, \
                      tl.comb, tl.extd_ptr, tl.extd, tl.bcmask, maskall,      \
                      (const float *)s_elem, (const float *)x, (const float *)b, (float *)y,      \
-                     (float *)xo, (float *)d, (const float *)dinv, g.ca, g.cc, g.cflags,          \
+                     (float *)xo, (float *)d, (const float *)dinv, g.cf, g.cflags,          \
                      g.partials, vs, tl.run)
 #define TMRX_MTILE2(M)    \
   if (single) {           \
@@ -2307,7 +2332,7 @@ void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x
                      tl.ext_ptr, tl.ext, tl.nacc_dep, tl.el_ptr,                                  \
                      reinterpret_cast<const uint2 *>(recs), tl.ncolors, tl.comb_ptr,              \
                      tl.comb, tl.extd_ptr, tl.extd, tl.bcmask, maskall, K0,   \
-                     s_elem, x, b, y, xo, d, dinv, g.ca, g.cc, g.cflags, g.partials, vs, tl.run, g.dr, g.dq)
+                     s_elem, x, b, y, xo, d, dinv, g.cf, g.cflags, g.partials, vs, tl.run, g.dr, g.dq)
 #define TMRX_TILE(M, S)                    \
   if (tl.threads == 512) {                 \
     if (tl.nodal)                          \
@@ -2591,8 +2616,9 @@ void launch_adjoint_grad(int n, const double *rho, const int16_t *lev, double q,
   template void launch_prolong_add<T>(const TransferCSR &, const uint8_t *, const T *, T *,     \
                                       hipStream_t, int, int64_t, int64_t);                      \
   template void launch_restrict<T>(const TransferCSR &, const uint8_t *, const T *, T *,        \
-                                   hipStream_t, int, int64_t, int64_t, const T *, double, T *); \
-  template void launch_cheb_first<T>(int, const T *, const T *, double, T *, T *,               \
+                                   hipStream_t, int, int64_t, int64_t, const T *, const double *,      \
+                                   T *); \
+  template void launch_cheb_first<T>(int, const T *, const T *, const double *, T *, T *,               \
                                      hipStream_t, int, const int *);                            \
   template void launch_dense_solve<T>(const CoarseBlocks &, const T *, T *, hipStream_t, int);  \
   template void launch_fill<T>(int64_t, T, T *, hipStream_t);                                 \

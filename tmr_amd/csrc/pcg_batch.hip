@@ -73,7 +73,8 @@ __global__ __launch_bounds__(BB) void k_b_update_xr(SegPlan pl, double *__restri
                                                     const double *__restrict__ sc,
                                                     const int *__restrict__ act,
                                                     double *__restrict__ partials,
-                                                    const float *__restrict__ dinv32, double c0,
+                                                    const float *__restrict__ dinv32,
+                                                    const double *__restrict__ c0p,
                                                     float *__restrict__ x1) {
   __shared__ double red[BB / 64];
   const int blk = blockIdx.x, rhs = blockIdx.y;
@@ -82,6 +83,7 @@ __global__ __launch_bounds__(BB) void k_b_update_xr(SegPlan pl, double *__restri
   const int64_t lo = pl.blk_lo[blk], hi = pl.blk_lo[blk + 1];
   const bool on = act[sidx] != 0;
   const double alpha = on ? sc[(int64_t)sidx * SC_N + SC_ALPHA] : 0.0;
+  const float c0 = x1 ? (float)*c0p : 0.0f;
   double s = 0.0;
   if (on || r32)
     for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += VU * BB) {
@@ -107,7 +109,7 @@ __global__ __launch_bounds__(BB) void k_b_update_xr(SegPlan pl, double *__restri
         if (r32) {
           const float rf = (float)rn;
           r32[off + i] = rf;
-          if (x1) x1[off + i] = (float)c0 * dv[k] * rf;
+          if (x1) x1[off + i] = c0 * dv[k] * rf;
         }
       }
     }
@@ -324,7 +326,7 @@ void launch_b_dot1(const SegPlan &pl, const double *a, const double *b, const in
 }
 void launch_b_update_xr(const SegPlan &pl, double *r, const double *q, float *r32,
                         const double *sc, const int *act, double *partials, hipStream_t st,
-                        const float *dinv32, double c0, float *x1) {
+                        const float *dinv32, const double *c0, float *x1) {
   hipLaunchKernelGGL(k_b_update_xr, dim3(pl.nblk, pl.nrhs), dim3(BB), 0, st, pl, r, q, r32, sc,
                      act, partials, dinv32, c0, x1);
   TMRX_LAUNCH_CHECK();

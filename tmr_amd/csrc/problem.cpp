@@ -50,13 +50,17 @@ static int default_tile_nodes(int n_nodes, bool hanging) {
   return n_nodes >= 500 * 128 ? 128 : 96;
 }
 
-void Problem::drop_graphs() {
+void Problem::drop_graph(IterGraph &g) {
   for (int k = 0; k < 2; k++)
-    if (gexec_[k]) {
-      (void)hipGraphExecDestroy(gexec_[k]);
-      gexec_[k] = nullptr;
+    if (g.exec[k]) {
+      (void)hipGraphExecDestroy(g.exec[k]);
+      g.exec[k] = nullptr;
     }
-  g_gen_ = -1;
+  g.gen = -1;
+}
+
+void Problem::drop_graphs() {
+  for (IterGraph &g : graphs_) drop_graph(g);
 }
 
 Problem::~Problem() {
@@ -1167,7 +1171,7 @@ int Problem::set_design(const double *rho, int n, bool on_device) {
   if (check_design_values(rho, n, on_device, "set_design")) return -1;
   HIPCHK(hipMemcpyAsync(rho_.p, rho, n * sizeof(double),
                         on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, st_));
-  design_mode_ = 0;
+  set_design_mode(0);
   launch_simp_scale(n, rho_.p, levels_[0].d_lev.p, mat_.q, mat_.k0, mat_.penalty_type,
                     levels_[0].s64.p, levels_[0].s32.p, st_);
   for (size_t l = 0; l + 1 < levels_.size(); l++) {
@@ -1234,13 +1238,19 @@ int Problem::set_design_nodal(const double *x, int n, bool on_device) {
                        L.d_lev.p, mat_.q, mat_.k0, mat_.penalty_type,
                        l == 0 ? rho_gp_.p : nullptr, L.sg64.p, L.sg32.p, st_);
   }
-  design_mode_ = 1;
+  set_design_mode(1);
   have_design_ = true;
   have_setup_ = false;
   return 0;
 oom:
   last_error = "set_design_nodal: device allocation failed";
   return -1;
+}
+
+// the captured iterations hold the kernels and tables of one design mode
+void Problem::set_design_mode(int mode) {
+  if (mode != design_mode_) gen_++;
+  design_mode_ = mode;
 }
 
 int Problem::design_size() const {
@@ -1518,7 +1528,6 @@ int Problem::setup(const SolveOpts &o) {
   HIPCHK(hipStreamSynchronize(st_));
   have_setup_ = true;
   setup_precision_ = prec;
-  gen_++;
   last_setup_ms_ = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   return 0;
 }
@@ -1532,24 +1541,13 @@ void Problem::cheb_step(int l, const T *b, const T *x_in, T *x_out, int k, const
                         int nrhs, int cflags, bool dots) {
   Level &L = levels_[l];
   LevelVecs<T> &v = vecs<T>(l);
-  const double lmax = o.cheb_upper * L.lam_max, lmin = o.cheb_lower * L.lam_max;
-  const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin);
-  const double sigma = theta / delta;
-  double rho_prev = 1.0 / sigma, ca = 0.0, cc = 1.0 / theta;
-  for (int j = 1; j <= k; j++) {
-    const double rho = 1.0 / (2.0 * sigma - rho_prev);
-    ca = rho * rho_prev;
-    cc = 2.0 * rho / delta;
-    rho_prev = rho;
-  }
   AsmArgs a;
   a.b = b;
   a.x = (void *)x_in;
   a.x_out = x_out;
   a.d = v.d.p;
   a.dinv = v.dinv.p;
-  a.ca = ca;
-  a.cc = cc;
+  a.cf = coef_.p + (size_t)l * coef_stride_ + 1 + 2 * (size_t)k;
   a.cflags = k == 0 ? (cflags & CHEB_D_STORE) : cflags;  // step 0: no previous direction
   if (dots) {
     a.dr = r_.p;
@@ -1568,11 +1566,46 @@ T *Problem::first_target(int l, T *x, const SolveOpts &o) {
   return (updates & 1) ? vecs<T>(l).x2.p : x;
 }
 
-template <class T>
-double Problem::cheb_c0(int l, const SolveOpts &o) const {
-  const Level &L = levels_[l];
-  const double lmax = o.cheb_upper * L.lam_max, lmin = o.cheb_lower * L.lam_max;
-  return 2.0 / (lmax + lmin);
+// The Chebyshev coefficients of every level on the device, for these options
+// and the eigenvalue bounds of the last set-up: per level c0 of the first
+// step from zero, then the pairs (a, c) of steps 0, 1, ...  The kernels read
+// them there, so an iteration captured once serves every later design.
+int Problem::upload_coefs(const SolveOpts &o) {
+  const int nl = (int)levels_.size();
+  const int deg = std::max(1, std::max(o.cheb_degree, o.cheb_pre_degree));
+  const size_t stride = 1 + 2 * (size_t)deg;
+  if (coef_.n < stride * nl || coef_stride_ != stride) {
+    if (coef_.n < stride * nl && coef_.alloc(stride * nl)) {
+      last_error = "solve: device allocation failed";
+      return -1;
+    }
+    coef_stride_ = stride;
+    coef_h_.clear();
+    gen_++;
+  }
+  std::vector<double> h(stride * nl, 0.0);
+  for (int l = 0; l < nl; l++) {
+    if (levels_[l].lam_max == 0.0) continue;  // a level that is not smoothed by Chebyshev
+    const double lmax = o.cheb_upper * levels_[l].lam_max, lmin = o.cheb_lower * levels_[l].lam_max;
+    const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin);
+    const double sigma = theta / delta;
+    double *c = &h[stride * l];
+    c[0] = 2.0 / (lmax + lmin);
+    double rho_prev = 1.0 / sigma, ca = 0.0, cc = 1.0 / theta;
+    for (int k = 0; k < deg; k++) {
+      c[1 + 2 * k] = ca;
+      c[2 + 2 * k] = cc;
+      const double rho = 1.0 / (2.0 * sigma - rho_prev);
+      ca = rho * rho_prev;
+      cc = 2.0 * rho / delta;
+      rho_prev = rho;
+    }
+  }
+  if (h == coef_h_) return 0;
+  for (size_t i = 0; i < h.size(); i += 32)
+    launch_set_words((int)std::min<size_t>(32, h.size() - i), &h[i], coef_.p + i, st_);
+  coef_h_ = std::move(h);
+  return 0;
 }
 
 template <class T>
@@ -1598,7 +1631,7 @@ void Problem::vcycle(int l, const T *b, T *x, const SolveOpts &o, int nrhs, bool
     T *cur = first_target<T>(l, x, o);
     T *oth = cur == x ? v.x2.p : x;
     if (!first_done)
-      launch_cheb_first<T>((int)L.ndof, b, v.dinv.p, cheb_c0<T>(l, o), nullptr, cur, st_, nrhs,
+      launch_cheb_first<T>((int)L.ndof, b, v.dinv.p, cheb_c0(l), nullptr, cur, st_, nrhs,
                            run_);
     for (int k = 1; k < deg; k++) {
       const int fl = (k == 1 ? CHEB_D_IS_X : CHEB_D_READ) | (k + 1 < deg ? CHEB_D_STORE : 0);
@@ -1622,8 +1655,7 @@ void Problem::vcycle(int l, const T *b, T *x, const SolveOpts &o, int nrhs, bool
     apply_level<T>(l, x, ASM_RESID, a, nrhs);
     TransferCSR R = L.R, P = L.P;
     R.run = P.run = run_;
-    launch_restrict<T>(R, Lc.d_bcmask.p, v.r.p, c.b.p, st_, nrhs, L.ndof, Lc.ndof, nullptr, 0.0,
-                       nullptr);
+    launch_restrict<T>(R, Lc.d_bcmask.p, v.r.p, c.b.p, st_, nrhs, L.ndof, Lc.ndof);
     vcycle<T>(l + 1, c.b.p, c.x.p, o, nrhs, false);
     launch_prolong_add<T>(P, L.d_bcmask.p, c.x.p, x, st_, nrhs, Lc.ndof, L.ndof);
     sor_smooth<T>(l, b, x, nrhs, false);
@@ -1638,7 +1670,7 @@ void Problem::vcycle(int l, const T *b, T *x, const SolveOpts &o, int nrhs, bool
   // the first step from a zero guess leaves d = x, so the second step reads
   // x for d; the last step of each sweep stores no direction
   if (!first_done)
-    launch_cheb_first<T>((int)L.ndof, b, v.dinv.p, cheb_c0<T>(l, o), nullptr, cur, st_, nrhs, run_);
+    launch_cheb_first<T>((int)L.ndof, b, v.dinv.p, cheb_c0(l), nullptr, cur, st_, nrhs, run_);
   for (int k = 1; k < pre; k++) {
     const int fl = (k == 1 ? CHEB_D_IS_X : CHEB_D_READ) | (k + 1 < pre ? CHEB_D_STORE : 0);
     cheb_step<T>(l, b, cur, oth, k, o, nrhs, fl);
@@ -1655,7 +1687,7 @@ void Problem::vcycle(int l, const T *b, T *x, const SolveOpts &o, int nrhs, bool
   // level is solved directly
   const bool fuse = l + 1 < last || !coarse_direct_;
   launch_restrict<T>(R, Lc.d_bcmask.p, v.r.p, c.b.p, st_, nrhs, L.ndof, Lc.ndof,
-                     fuse ? c.dinv.p : nullptr, fuse ? cheb_c0<T>(l + 1, o) : 0.0,
+                     fuse ? c.dinv.p : nullptr, fuse ? cheb_c0(l + 1) : nullptr,
                      fuse ? first_target<T>(l + 1, c.x.p, o) : nullptr);
   vcycle<T>(l + 1, c.b.p, c.x.p, o, nrhs, fuse);
   launch_prolong_add<T>(P, L.d_bcmask.p, c.x.p, cur, st_, nrhs, Lc.ndof, L.ndof);
@@ -1744,7 +1776,7 @@ void Problem::enqueue_iteration(const SegPlan &pl, int nrhs, double *xsol, const
   Level &L0u = levels_[0];
   const bool fuse0 = mixed && !sor_;
   launch_b_update_xr(pl, r_.p, q_.p, r32, sc_.p, act_.p, parts_.p, st_,
-                     fuse0 ? L0u.v32.dinv.p : nullptr, fuse0 ? cheb_c0<float>(0, o) : 0.0,
+                     fuse0 ? L0u.v32.dinv.p : nullptr, fuse0 ? cheb_c0(0) : nullptr,
                      fuse0 ? first_target<float>(0, L0u.v32.x.p, o) : nullptr);
   // its last block counts the segments still running (and advances the
   // iteration counter) before the preconditioner: an iteration that converged
@@ -1799,6 +1831,7 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
       return -1;
     }
   if (ensure_batch(nrhs) || (coarse_direct_ && ensure_coarse_work(nrhs))) return -1;
+  if (upload_coefs(o)) return -1;
   fp32_valu_ = o.fp32_valu != 0;
   auto t0 = std::chrono::steady_clock::now();
   Level &L0 = levels_[0];
@@ -1869,15 +1902,18 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
   // iterations: replayed graphs (or enqueued bodies), the stop count of
   // iteration k read while iteration k + 1 runs
   const bool graphs = !o.no_graph && !o.monitor && timing_ == 0;
+  IterGraph *ig = nullptr;
   if (graphs && running > 0) {
-    const bool same = g_gen_ == gen_ && g_nrhs_ == nrhs && g_xsol_ == xsol &&
-                      g_opts_.precision == o.precision &&
-                      g_opts_.fp32_valu == o.fp32_valu && g_opts_.cheb_degree == o.cheb_degree &&
-                      g_opts_.cheb_pre_degree == o.cheb_pre_degree &&
-                      g_opts_.cheb_lower == o.cheb_lower && g_opts_.cheb_upper == o.cheb_upper &&
-                      g_opts_.rtol == o.rtol && g_opts_.atol == o.atol;
-    if (!same || !gexec_[0] || !gexec_[1]) {
-      drop_graphs();
+    for (IterGraph &g : graphs_)
+      if (g.exec[0] && g.gen == gen_ && g.nrhs == nrhs && g.xsol == xsol &&
+          g.o.precision == o.precision && g.o.fp32_valu == o.fp32_valu &&
+          g.o.cheb_degree == o.cheb_degree && g.o.cheb_pre_degree == o.cheb_pre_degree &&
+          g.o.rtol == o.rtol && g.o.atol == o.atol)
+        ig = &g;
+    if (!ig) {
+      // the set used longest ago makes room
+      ig = graphs_[0].used < graphs_[1].used ? &graphs_[0] : &graphs_[1];
+      drop_graph(*ig);
       if (!cap_st_) HIPCHK(hipStreamCreateWithFlags(&cap_st_, hipStreamNonBlocking));
       hipStream_t keep = st_;
       for (int k = 0; k < 2; k++) {
@@ -1890,19 +1926,20 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
         }
         st_ = keep;
         if (e == hipSuccess) e = take_launch_error();
-        if (e == hipSuccess) e = hipGraphInstantiate(&gexec_[k], g, nullptr, nullptr, 0);
+        if (e == hipSuccess) e = hipGraphInstantiate(&ig->exec[k], g, nullptr, nullptr, 0);
         if (g) (void)hipGraphDestroy(g);
         if (e != hipSuccess) {
-          drop_graphs();
+          drop_graph(*ig);
           last_error = std::string("solve: graph capture failed: ") + hipGetErrorString(e);
           return -1;
         }
       }
-      g_gen_ = gen_;
-      g_nrhs_ = nrhs;
-      g_xsol_ = xsol;
-      g_opts_ = o;
+      ig->gen = gen_;
+      ig->nrhs = nrhs;
+      ig->xsol = xsol;
+      ig->o = o;
     }
+    ig->used = ++graph_clock_;
   }
   for (int k = 0; k < 2; k++)
     if (!gev_[k]) HIPCHK(hipEventCreateWithFlags(&gev_[k], hipEventDisableTiming));
@@ -1912,7 +1949,7 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
     volatile int *count = nact_host_ + slot;
     *count = -1;
     if (graphs)
-      HIPCHK(hipGraphLaunch(gexec_[slot], st_));
+      HIPCHK(hipGraphLaunch(ig->exec[slot], st_));
     else
       enqueue_iteration(pl, nrhs, xsol, o, slot);
     HIPCHK(hipEventRecord(gev_[slot], st_));
@@ -2243,7 +2280,7 @@ int Problem::mg_op_t(int op, int l, const double *x, double *y, bool on_device,
       // the V-cycle's pre-smoothing: c0 Dinv b, then pre - 1 ping-pong steps
       const int pre = o.cheb_pre_degree > 0 ? o.cheb_pre_degree : std::max(1, o.cheb_degree);
       T *cur = vo.x.p, *oth = vo.x2.p;
-      launch_cheb_first<T>((int)Lo.ndof, in, vo.dinv.p, cheb_c0<T>(l, o), nullptr, cur, st_, 1);
+      launch_cheb_first<T>((int)Lo.ndof, in, vo.dinv.p, cheb_c0(l), nullptr, cur, st_, 1);
       for (int k = 1; k < pre; k++) {
         const int fl = (k == 1 ? CHEB_D_IS_X : CHEB_D_READ) | (k + 1 < pre ? CHEB_D_STORE : 0);
         cheb_step<T>(l, in, cur, oth, k, o, 1, fl);
@@ -2308,6 +2345,7 @@ int Problem::mg_op(int op, int l, const double *x, double *y, bool on_device,
   if (!have_setup_ || setup_precision_ != prec) {
     if (setup(o)) return -1;
   }
+  if (upload_coefs(o)) return -1;
   fp32_valu_ = o.fp32_valu != 0;
   if (lam) *lam = levels_[l].lam_max;
   return prec ? mg_op_t<float>(op, l, x, y, on_device, o)
@@ -2479,6 +2517,15 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
   }
   Level &L0 = levels_[0];
   const int64_t n = L0.ndof;
+  if (coef_.n < 2 && coef_.alloc(2)) {
+    last_error = "autotune: allocation failed";
+    return -1;
+  }
+  {
+    const double cf[2] = {0.5, 0.25};
+    launch_set_words(2, cf, coef_.p, st_);
+    coef_h_.clear();
+  }
   // inputs of the timed launches in the V-cycle's scratch vectors
   // (Chebyshev steps and residuals need b, x, d and a diagonal, r standing
   // in for it; the values only have to be finite; the set-up Dinv is not
@@ -2525,8 +2572,7 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
     ac.x_out = L0.v32.x2.p;
     ac.d = L0.v32.d.p;
     ac.dinv = L0.v32.r.p;
-    ac.ca = 0.5;
-    ac.cc = 0.25;
+    ac.cf = coef_.p;
     ac.cflags = CHEB_D_READ | CHEB_D_STORE;
     ar.b = L0.v32.b.p;
     ar.y = L0.v32.d.p;

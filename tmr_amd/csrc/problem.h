@@ -376,8 +376,12 @@ class Problem {
   // first_done: the first smoothing step from zero (c0 Dinv b) is already
   // in the level's spare buffer (written by the restriction or the PCG update)
   void vcycle(int l, const T *b, T *x, const SolveOpts &o, int nrhs = 1, bool first_done = false);
-  template <class T>
-  double cheb_c0(int l, const SolveOpts &o) const;
+  const double *cheb_c0(int l) const { return coef_.p + (size_t)l * coef_stride_; }
+  int upload_coefs(const SolveOpts &o);
+  void set_design_mode(int mode);
+  DevArray<double> coef_;       // Chebyshev coefficients, coef_stride_ per level
+  size_t coef_stride_ = 0;
+  std::vector<double> coef_h_;  // what coef_ holds
   // buffer of level l that the first smoothing step writes (x or its spare)
   template <class T>
   T *first_target(int l, T *x, const SolveOpts &o);
@@ -442,15 +446,22 @@ class Problem {
   DevArray<int> chk_;  // flag of the design-value check
   DevArray<double> thr_;
   int *nact_host_ = nullptr;  // pinned, two slots (iterations alternate)
-  // PCG iteration bodies captured as HIP graphs (two: they write alternate
-  // stop-count slots), valid for one (nrhs, options, buffers, setup)
-  hipGraphExec_t gexec_[2] = {nullptr, nullptr};
+  // PCG iteration bodies captured as HIP graphs (two each: they write
+  // alternate stop-count slots), valid for one (nrhs, solution vector,
+  // options, gen_); two sets, for a forward and an adjoint solve in turn
+  struct IterGraph {
+    hipGraphExec_t exec[2] = {nullptr, nullptr};
+    int nrhs = 0, gen = -1;
+    double *xsol = nullptr;
+    SolveOpts o;
+    int64_t used = 0;
+  };
+  IterGraph graphs_[2];
+  int64_t graph_clock_ = 0;
+  void drop_graph(IterGraph &g);
   hipEvent_t gev_[2] = {nullptr, nullptr};
   hipStream_t cap_st_ = nullptr;
-  int g_nrhs_ = 0, g_gen_ = -1;
-  double *g_xsol_ = nullptr;
-  SolveOpts g_opts_;
-  int gen_ = 0;  // bumped whenever buffers move or setup reruns
+  int gen_ = 0;  // bumped whenever buffers move or the iteration's kernels change
   // while a PCG iteration is enqueued: the device count of running segments;
   // the operator, transfer and smoother launches return at once when it is 0
   // (the iteration launched after the one that converged)

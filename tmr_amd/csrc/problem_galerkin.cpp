@@ -233,6 +233,7 @@ int Problem::build_bsr(int l) {
     return -1;
   }
   L.has_bsr = true;
+  gen_++;
   return 0;
 }
 
@@ -373,6 +374,7 @@ int Problem::build_sor(int l) {
   L.sor_cptr = cptr;
   L.sor_nodes_h = nodes;
   L.has_sor = true;
+  gen_++;
   return 0;
 }
 
