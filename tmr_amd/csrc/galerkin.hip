@@ -208,9 +208,9 @@ __global__ void __launch_bounds__(256)
                 const T *__restrict__ val, const uint8_t *__restrict__ bcmask,
                 const T *__restrict__ x, const T *__restrict__ b, T *__restrict__ y,
                 T *__restrict__ x_out, T *__restrict__ d, const T *__restrict__ dinv,
-                const double *__restrict__ cf, int cflags, const int *__restrict__ run, int64_t vs) {
+                const T *__restrict__ cf, int cflags, const int *__restrict__ run, int64_t vs) {
   if (run && *run == 0) return;
-  const T ca = MODE == ASM_CHEB ? (T)cf[0] : T(0), cc = MODE == ASM_CHEB ? (T)cf[1] : T(0);
+  const T ca = MODE == ASM_CHEB ? cf[0] : T(0), cc = MODE == ASM_CHEB ? cf[1] : T(0);
   const int64_t off = (int64_t)blockIdx.y * vs;
   x += off;
   if (b) b += off;
@@ -288,16 +288,16 @@ void launch_bsr_apply(const BSR<T> &A, const T *x, int mode, const AsmArgs &g, h
   const T *dinv = (const T *)g.dinv;
   if (mode == ASM_STORE)
     hipLaunchKernelGGL((k_bsr_apply<T, ASM_STORE>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
-                       A.val, A.bcmask, x, b, y, xo, d, dinv, g.cf, g.cflags, A.run, vs);
+                       A.val, A.bcmask, x, b, y, xo, d, dinv, (const T *)g.cf, g.cflags, A.run, vs);
   else if (mode == ASM_RESID)
     hipLaunchKernelGGL((k_bsr_apply<T, ASM_RESID>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
-                       A.val, A.bcmask, x, b, y, xo, d, dinv, g.cf, g.cflags, A.run, vs);
+                       A.val, A.bcmask, x, b, y, xo, d, dinv, (const T *)g.cf, g.cflags, A.run, vs);
   else if (mode == ASM_POWER)
     hipLaunchKernelGGL((k_bsr_apply<T, ASM_POWER>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
-                       A.val, A.bcmask, x, b, y, xo, d, dinv, g.cf, g.cflags, A.run, vs);
+                       A.val, A.bcmask, x, b, y, xo, d, dinv, (const T *)g.cf, g.cflags, A.run, vs);
   else if (mode == ASM_CHEB)
     hipLaunchKernelGGL((k_bsr_apply<T, ASM_CHEB>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
-                       A.val, A.bcmask, x, b, y, xo, d, dinv, g.cf, g.cflags, A.run, vs);
+                       A.val, A.bcmask, x, b, y, xo, d, dinv, (const T *)g.cf, g.cflags, A.run, vs);
   else
     note_launch(hipErrorInvalidValue);
   TMRX_LAUNCH_CHECK();

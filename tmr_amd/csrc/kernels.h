@@ -183,9 +183,9 @@ struct AsmArgs {
   void *x_out = nullptr;   // CHEB iterate output of the tile kernel
   void *d = nullptr;       // Chebyshev direction
   const void *dinv = nullptr;
-  // ASM_CHEB: device pair (a, c) of the step, so that a captured iteration
-  // outlives a new set-up's eigenvalue bounds
-  const double *cf = nullptr;
+  // ASM_CHEB: device pair (a, c) of the step in the vectors' type, so that a
+  // captured iteration outlives a new set-up's eigenvalue bounds
+  const void *cf = nullptr;
   int cflags = CHEB_D_READ | CHEB_D_STORE;  // tile apply, ASM_CHEB
   double *partials = nullptr;
   const double *dr = nullptr, *dq = nullptr;  // ASM_CHEBDOT
@@ -339,8 +339,8 @@ void launch_sor_sweep(const BSR<T> &A, const int *nodes, const int *cptr, int nc
                       const T *b, T *x, double omega, hipStream_t st, int nrhs = 1,
                       int64_t vs = 0);
 
-// dst[0..n) = v (n <= 32), from kernel arguments
-void launch_set_words(int n, const double *v, double *dst, hipStream_t st);
+// dst[0..n) = dst32[0..n) = v (n <= 32), from kernel arguments
+void launch_set_words(int n, const double *v, double *dst, float *dst32, hipStream_t st);
 template <class TI, class TO>
 void launch_convert(int64_t n, const TI *a, TO *b, hipStream_t st);
 template <class T>

@@ -173,6 +173,14 @@ __global__ __launch_bounds__(BB) void k_b_update_p(SegPlan pl, double *__restric
   if (!upx && !upp) return;
   const double alpha = s[SC_ALPHA], beta = s[SC_BETA];
   const int64_t off = (int64_t)rhs * pl.n;
+  if (VU == 1) {
+    for (int64_t i = pl.blk_lo[blk] + threadIdx.x; i < pl.blk_lo[blk + 1]; i += BB) {
+      const double pv = p[off + i];
+      if (upx) x[off + i] += alpha * pv;
+      if (upp) p[off + i] = (double)z[off + i] + beta * pv;
+    }
+    return;
+  }
   const int64_t lo = pl.blk_lo[blk], hi = pl.blk_lo[blk + 1];
   for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += VU * BB) {
     double pv[VU], xv[VU], zv[VU];

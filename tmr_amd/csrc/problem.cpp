@@ -1547,7 +1547,8 @@ void Problem::cheb_step(int l, const T *b, const T *x_in, T *x_out, int k, const
   a.x_out = x_out;
   a.d = v.d.p;
   a.dinv = v.dinv.p;
-  a.cf = coef_.p + (size_t)l * coef_stride_ + 1 + 2 * (size_t)k;
+  const size_t ck = (size_t)l * coef_stride_ + 1 + 2 * (size_t)k;
+  a.cf = sizeof(T) == 4 ? (const void *)(coef32_.p + ck) : (const void *)(coef_.p + ck);
   a.cflags = k == 0 ? (cflags & CHEB_D_STORE) : cflags;  // step 0: no previous direction
   if (dots) {
     a.dr = r_.p;
@@ -1575,7 +1576,7 @@ int Problem::upload_coefs(const SolveOpts &o) {
   const int deg = std::max(1, std::max(o.cheb_degree, o.cheb_pre_degree));
   const size_t stride = 1 + 2 * (size_t)deg;
   if (coef_.n < stride * nl || coef_stride_ != stride) {
-    if (coef_.n < stride * nl && coef_.alloc(stride * nl)) {
+    if (coef_.n < stride * nl && (coef_.alloc(stride * nl) || coef32_.alloc(stride * nl))) {
       last_error = "solve: device allocation failed";
       return -1;
     }
@@ -1603,7 +1604,7 @@ int Problem::upload_coefs(const SolveOpts &o) {
   }
   if (h == coef_h_) return 0;
   for (size_t i = 0; i < h.size(); i += 32)
-    launch_set_words((int)std::min<size_t>(32, h.size() - i), &h[i], coef_.p + i, st_);
+    launch_set_words((int)std::min<size_t>(32, h.size() - i), &h[i], coef_.p + i, coef32_.p + i, st_);
   coef_h_ = std::move(h);
   return 0;
 }
@@ -2517,13 +2518,13 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
   }
   Level &L0 = levels_[0];
   const int64_t n = L0.ndof;
-  if (coef_.n < 2 && coef_.alloc(2)) {
+  if (coef_.n < 2 && (coef_.alloc(2) || coef32_.alloc(2))) {
     last_error = "autotune: allocation failed";
     return -1;
   }
   {
     const double cf[2] = {0.5, 0.25};
-    launch_set_words(2, cf, coef_.p, st_);
+    launch_set_words(2, cf, coef_.p, coef32_.p, st_);
     coef_h_.clear();
   }
   // inputs of the timed launches in the V-cycle's scratch vectors
@@ -2572,7 +2573,7 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
     ac.x_out = L0.v32.x2.p;
     ac.d = L0.v32.d.p;
     ac.dinv = L0.v32.r.p;
-    ac.cf = coef_.p;
+    ac.cf = coef32_.p;
     ac.cflags = CHEB_D_READ | CHEB_D_STORE;
     ar.b = L0.v32.b.p;
     ar.y = L0.v32.d.p;

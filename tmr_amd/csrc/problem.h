@@ -380,6 +380,7 @@ class Problem {
   int upload_coefs(const SolveOpts &o);
   void set_design_mode(int mode);
   DevArray<double> coef_;       // Chebyshev coefficients, coef_stride_ per level
+  DevArray<float> coef32_;
   size_t coef_stride_ = 0;
   std::vector<double> coef_h_;  // what coef_ holds
   // buffer of level l that the first smoothing step writes (x or its spare)
