@@ -197,12 +197,11 @@ void launch_bsr_dinv(int n, const int *diag, const double *val, T *dinv, hipStre
 }
 
 // ---------------------------------------------------------------------------
-// BSR operator with the epilogues of the tile apply (ASM_STORE, ASM_RESID,
-// ASM_CHEB): BSR_LANES lanes per block row, each summing every BSR_LANES-th
-// block of the row, then a butterfly over the group in a fixed order.
-constexpr int BSR_LANES = 4;
-
-template <class T, int MODE>
+// BSR operator with the epilogues of the tile apply: LANES lanes per block
+// row, each summing every LANES-th block of the row two at a time, then a
+// butterfly over the group in a fixed order.  32 lanes while they fit the
+// chip (the loop over a row is a chain of dependent loads), else 8.
+template <class T, int MODE, int LANES>
 __global__ void __launch_bounds__(256)
     k_bsr_apply(int n, const int *__restrict__ ptr, const int *__restrict__ col,
                 const T *__restrict__ val, const uint8_t *__restrict__ bcmask,
@@ -218,22 +217,38 @@ __global__ void __launch_bounds__(256)
   if (x_out) x_out += off;
   if (d) d += off;
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  const int row = g / BSR_LANES, sub = g % BSR_LANES;
+  const int row = g / LANES, sub = g % LANES;
   const bool valid = row < n;
   T a0 = T(0), a1 = T(0), a2 = T(0);
   if (valid) {
     const int k1 = ptr[row + 1];
-    for (int k = ptr[row] + sub; k < k1; k += BSR_LANES) {
-      const int j = col[k];
-      const T *v = val + 9 * (size_t)k;
-      const T x0 = x[3 * (size_t)j], x1 = x[3 * (size_t)j + 1], x2 = x[3 * (size_t)j + 2];
-      a0 += v[0] * x0 + v[1] * x1 + v[2] * x2;
-      a1 += v[3] * x0 + v[4] * x1 + v[5] * x2;
-      a2 += v[6] * x0 + v[7] * x1 + v[8] * x2;
+    for (int k = ptr[row] + sub; k < k1; k += 2 * LANES) {
+      const int kb = min(k + LANES, k1 - 1);
+      const bool second = k + LANES < k1;
+      const int ja = col[k], jb = col[kb];
+      T va[9], vb[9], xa[3], xb[3];
+#pragma unroll
+      for (int e = 0; e < 9; e++) va[e] = val[9 * (size_t)k + e];
+      if (second)
+#pragma unroll
+        for (int e = 0; e < 9; e++) vb[e] = val[9 * (size_t)kb + e];
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        xa[c] = x[3 * (size_t)ja + c];
+        xb[c] = x[3 * (size_t)jb + c];
+      }
+      a0 += va[0] * xa[0] + va[1] * xa[1] + va[2] * xa[2];
+      a1 += va[3] * xa[0] + va[4] * xa[1] + va[5] * xa[2];
+      a2 += va[6] * xa[0] + va[7] * xa[1] + va[8] * xa[2];
+      if (second) {
+        a0 += vb[0] * xb[0] + vb[1] * xb[1] + vb[2] * xb[2];
+        a1 += vb[3] * xb[0] + vb[4] * xb[1] + vb[5] * xb[2];
+        a2 += vb[6] * xb[0] + vb[7] * xb[1] + vb[8] * xb[2];
+      }
     }
   }
 #pragma unroll
-  for (int m = 1; m < BSR_LANES; m <<= 1) {
+  for (int m = 1; m < LANES; m <<= 1) {
     a0 += __shfl_xor(a0, m);
     a1 += __shfl_xor(a1, m);
     a2 += __shfl_xor(a2, m);
@@ -278,28 +293,33 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+template <class T, int MODE>
+static void bsr_launch(const BSR<T> &A, const T *x, const AsmArgs &g, hipStream_t st, int nrhs,
+                       int64_t vs) {
+  const bool wide = (int64_t)A.n * nrhs * 32 <= 256 * 8 * 256;
+  const int lanes = wide ? 32 : 8;
+  const dim3 grid((unsigned)(((int64_t)A.n * lanes + 255) / 256), (unsigned)nrhs);
+  if (wide)
+    hipLaunchKernelGGL((k_bsr_apply<T, MODE, 32>), grid, dim3(256), 0, st, A.n, A.ptr, A.col, A.val,
+                       A.bcmask, x, (const T *)g.b, (T *)g.y, (T *)g.x_out, (T *)g.d,
+                       (const T *)g.dinv, (const T *)g.cf, g.cflags, A.run, vs);
+  else
+    hipLaunchKernelGGL((k_bsr_apply<T, MODE, 8>), grid, dim3(256), 0, st, A.n, A.ptr, A.col, A.val,
+                       A.bcmask, x, (const T *)g.b, (T *)g.y, (T *)g.x_out, (T *)g.d,
+                       (const T *)g.dinv, (const T *)g.cf, g.cflags, A.run, vs);
+}
+
 template <class T>
 void launch_bsr_apply(const BSR<T> &A, const T *x, int mode, const AsmArgs &g, hipStream_t st,
                       int nrhs, int64_t vs) {
   if (A.n == 0) return;
-  const dim3 grid((unsigned)(((int64_t)A.n * BSR_LANES + 255) / 256), (unsigned)nrhs);
-  const T *b = (const T *)g.b;
-  T *y = (T *)g.y, *xo = (T *)g.x_out, *d = (T *)g.d;
-  const T *dinv = (const T *)g.dinv;
-  if (mode == ASM_STORE)
-    hipLaunchKernelGGL((k_bsr_apply<T, ASM_STORE>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
-                       A.val, A.bcmask, x, b, y, xo, d, dinv, (const T *)g.cf, g.cflags, A.run, vs);
-  else if (mode == ASM_RESID)
-    hipLaunchKernelGGL((k_bsr_apply<T, ASM_RESID>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
-                       A.val, A.bcmask, x, b, y, xo, d, dinv, (const T *)g.cf, g.cflags, A.run, vs);
-  else if (mode == ASM_POWER)
-    hipLaunchKernelGGL((k_bsr_apply<T, ASM_POWER>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
-                       A.val, A.bcmask, x, b, y, xo, d, dinv, (const T *)g.cf, g.cflags, A.run, vs);
-  else if (mode == ASM_CHEB)
-    hipLaunchKernelGGL((k_bsr_apply<T, ASM_CHEB>), grid, dim3(256), 0, st, A.n, A.ptr, A.col,
-                       A.val, A.bcmask, x, b, y, xo, d, dinv, (const T *)g.cf, g.cflags, A.run, vs);
-  else
-    note_launch(hipErrorInvalidValue);
+  switch (mode) {
+    case ASM_STORE: bsr_launch<T, ASM_STORE>(A, x, g, st, nrhs, vs); break;
+    case ASM_RESID: bsr_launch<T, ASM_RESID>(A, x, g, st, nrhs, vs); break;
+    case ASM_POWER: bsr_launch<T, ASM_POWER>(A, x, g, st, nrhs, vs); break;
+    case ASM_CHEB: bsr_launch<T, ASM_CHEB>(A, x, g, st, nrhs, vs); break;
+    default: note_launch(hipErrorInvalidValue);
+  }
   TMRX_LAUNCH_CHECK();
 }
 
@@ -309,17 +329,21 @@ void launch_bsr_apply(const BSR<T> &A, const T *x, int mode, const AsmArgs &g, h
 // src/TMR_RefinementTools.cpp:93-94).  The matrix is the level's BSR with
 // its rows in the sweep's colour-major node order (row k holds node
 // nodes[k]; columns are node indices), so a colour's rows are contiguous.
-// Every node of the colour takes
-// SOR_LANES lanes: they sum the row's off-diagonal blocks (consecutive
-// lanes on consecutive blocks, which read x of other colours only, so the
-// nodes of a colour update side by side) and a butterfly combines them;
-// then the node's three dofs update one after another through the diagonal
-// block, 0, 1, 2 (BACK: 2, 1, 0), each
+// Every node of the colour takes LANES lanes: they sum the row's
+// off-diagonal blocks (consecutive lanes on consecutive blocks, which read x
+// of other colours only, so the nodes of a colour update side by side) and a
+// butterfly combines them; then the node's three dofs update one after
+// another through the diagonal block, 0, 1, 2 (backward: 2, 1, 0), each
 // x_p <- (1 - omega) x_p + omega (b_p - sum_{q != p} a_pq x_q) / a_pp --
 // the point SOR of the dofs in colour-major node order.
-constexpr int SOR_LANES = 8;
-
-template <class T, bool BACK>
+// DIR 0: forward, 1: backward, 2: forward then backward, the turn of a
+// symmetric sweep (the last colour's neighbours do not change in between).
+// A colour is a chain of dependent loads (row, columns, x): with 8 lanes a
+// row of 27 to 60 blocks goes round that chain four to eight times, with 32
+// once or twice.  32 lanes are taken until they fill the chip (32,858-node
+// adaptive level, 2,200 rows a colour: 6.9 -> 4.9 us a launch; one colour of
+// 3,058 nodes 5.3 -> 4.1); beyond, 8 lanes leave fewer idle.
+template <class T, int DIR, int LANES>
 __global__ __launch_bounds__(256) void k_sor_colour(int cnt, const int *__restrict__ nodes,
                                                     const int *__restrict__ ptr,
                                                     const int *__restrict__ col,
@@ -327,46 +351,78 @@ __global__ __launch_bounds__(256) void k_sor_colour(int cnt, const int *__restri
                                                     const T *__restrict__ b, T *__restrict__ x,
                                                     T omega, const int *__restrict__ run,
                                                     int64_t vs) {
-  if (run && *run == 0) return;
+  const int go = run ? *run : 1;
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  const int k = g / SOR_LANES, sub = g % SOR_LANES;
+  const int k = g / LANES, sub = g % LANES;
   const bool valid = k < cnt;
   const int64_t off = (int64_t)blockIdx.y * vs;
   x += off;
   b += off;
-  const int i = valid ? nodes[k] : 0;
+  const int kk = valid ? k : 0;
+  const int i = nodes[kk], q0 = ptr[kk], q1 = ptr[kk + 1];
+  if (go == 0) return;
+  const size_t i3 = 3 * (size_t)i;
+  T xi[3] = {T(0), T(0), T(0)}, bi[3] = {T(0), T(0), T(0)};
+  if (valid && sub == 0) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      xi[c] = x[i3 + c];
+      bi[c] = b[i3 + c];
+    }
+  }
   T s0 = T(0), s1 = T(0), s2 = T(0);
   int kd = -1;
   if (valid) {
-    const int q1 = ptr[k + 1];
-    for (int q = ptr[k] + sub; q < q1; q += SOR_LANES) {
-      const int j = col[q];
-      if (j == i) {
-        kd = q;
-        continue;
+    // two blocks per lane at a time, loads issued together (the second index
+    // clamped to the row, its term skipped past the end)
+    for (int q = q0 + sub; q < q1; q += 2 * LANES) {
+      const int qb = min(q + LANES, q1 - 1);
+      const bool second = q + LANES < q1;
+      const int ja = col[q], jb = col[qb];
+      T va[9], vb[9], xa[3], xb[3];
+#pragma unroll
+      for (int e = 0; e < 9; e++) va[e] = val[9 * (size_t)q + e];
+      if (second)
+#pragma unroll
+        for (int e = 0; e < 9; e++) vb[e] = val[9 * (size_t)qb + e];
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        xa[c] = x[3 * (size_t)ja + c];
+        xb[c] = x[3 * (size_t)jb + c];
       }
-      const T *v = val + 9 * (size_t)q;
-      const T x0 = x[3 * (size_t)j], x1 = x[3 * (size_t)j + 1], x2 = x[3 * (size_t)j + 2];
-      s0 += v[0] * x0 + v[1] * x1 + v[2] * x2;
-      s1 += v[3] * x0 + v[4] * x1 + v[5] * x2;
-      s2 += v[6] * x0 + v[7] * x1 + v[8] * x2;
+      if (ja == i) {
+        kd = q;
+      } else {
+        s0 += va[0] * xa[0] + va[1] * xa[1] + va[2] * xa[2];
+        s1 += va[3] * xa[0] + va[4] * xa[1] + va[5] * xa[2];
+        s2 += va[6] * xa[0] + va[7] * xa[1] + va[8] * xa[2];
+      }
+      if (second) {
+        if (jb == i) {
+          kd = qb;
+        } else {
+          s0 += vb[0] * xb[0] + vb[1] * xb[1] + vb[2] * xb[2];
+          s1 += vb[3] * xb[0] + vb[4] * xb[1] + vb[5] * xb[2];
+          s2 += vb[6] * xb[0] + vb[7] * xb[1] + vb[8] * xb[2];
+        }
+      }
     }
   }
 #pragma unroll
-  for (int m = 1; m < SOR_LANES; m <<= 1) {
+  for (int m = 1; m < LANES; m <<= 1) {
     s0 += __shfl_xor(s0, m);
     s1 += __shfl_xor(s1, m);
     s2 += __shfl_xor(s2, m);
     kd = max(kd, __shfl_xor(kd, m));
   }
   if (!valid || sub != 0 || kd < 0) return;
-  const T *D = val + 9 * (size_t)kd;
-  const size_t i3 = 3 * (size_t)i;
-  T xi[3] = {x[i3], x[i3 + 1], x[i3 + 2]};
-  const T r[3] = {b[i3] - s0, b[i3 + 1] - s1, b[i3 + 2] - s2};
+  T D[9];
 #pragma unroll
-  for (int t = 0; t < 3; t++) {
-    const int p = BACK ? 2 - t : t;
+  for (int e = 0; e < 9; e++) D[e] = val[9 * (size_t)kd + e];
+  const T r[3] = {bi[0] - s0, bi[1] - s1, bi[2] - s2};
+#pragma unroll
+  for (int t = 0; t < (DIR == 2 ? 6 : 3); t++) {
+    const int p = DIR == 1 ? 2 - t : t < 3 ? t : 5 - t;
     T acc = r[p];
 #pragma unroll
     for (int q = 0; q < 3; q++)
@@ -394,29 +450,41 @@ void launch_bsr_gather(int nnzb, const int *map, const double *val, double *out,
   TMRX_LAUNCH_CHECK();
 }
 
-template <class T>
-void launch_sor_sweep(const BSR<T> &A, const int *nodes, const int *cptr, int ncolors, bool back,
-                      const T *b, T *x, double omega, hipStream_t st, int nrhs, int64_t vs) {
-  for (int t = 0; t < ncolors; t++) {
-    const int c = back ? ncolors - 1 - t : t;
-    const int c0 = cptr[c], cnt = cptr[c + 1] - c0;
-    if (cnt == 0) continue;
-    const dim3 grid((unsigned)(((int64_t)cnt * SOR_LANES + 255) / 256), (unsigned)nrhs);
-    if (back)
-      hipLaunchKernelGGL((k_sor_colour<T, true>), grid, dim3(256), 0, st, cnt, nodes + c0,
-                         A.ptr + c0, A.col, A.val, b, x, (T)omega, A.run, vs);
-    else
-      hipLaunchKernelGGL((k_sor_colour<T, false>), grid, dim3(256), 0, st, cnt, nodes + c0,
-                         A.ptr + c0, A.col, A.val, b, x, (T)omega, A.run, vs);
-    TMRX_LAUNCH_CHECK();
-  }
+template <class T, int DIR>
+static void sor_colour(const BSR<T> &A, const int *nodes, int c0, int cnt, const T *b, T *x,
+                       double omega, hipStream_t st, int nrhs, int64_t vs) {
+  if (cnt == 0) return;
+  // 32 lanes per row until they fill the 256 CUs with 8 workgroups each
+  const bool wide = (int64_t)cnt * nrhs * 32 <= 256 * 8 * 256;
+  const int lanes = wide ? 32 : 8;
+  const dim3 grid((unsigned)(((int64_t)cnt * lanes + 255) / 256), (unsigned)nrhs);
+  if (wide)
+    hipLaunchKernelGGL((k_sor_colour<T, DIR, 32>), grid, dim3(256), 0, st, cnt, nodes + c0,
+                       A.ptr + c0, A.col, A.val, b, x, (T)omega, A.run, vs);
+  else
+    hipLaunchKernelGGL((k_sor_colour<T, DIR, 8>), grid, dim3(256), 0, st, cnt, nodes + c0,
+                       A.ptr + c0, A.col, A.val, b, x, (T)omega, A.run, vs);
+  TMRX_LAUNCH_CHECK();
 }
 
-template void launch_sor_sweep<float>(const BSR<float> &, const int *, const int *, int, bool,
-                                      const float *, float *, double, hipStream_t, int, int64_t);
-template void launch_sor_sweep<double>(const BSR<double> &, const int *, const int *, int, bool,
-                                       const double *, double *, double, hipStream_t, int,
-                                       int64_t);
+template <class T>
+void launch_sor_symmetric(const BSR<T> &A, const int *nodes, const int *cptr, int ncolors,
+                          const T *b, T *x, double omega, hipStream_t st, int nrhs, int64_t vs) {
+  for (int c = 0; c + 1 < ncolors; c++)
+    sor_colour<T, 0>(A, nodes, cptr[c], cptr[c + 1] - cptr[c], b, x, omega, st, nrhs, vs);
+  if (ncolors > 0)
+    sor_colour<T, 2>(A, nodes, cptr[ncolors - 1], cptr[ncolors] - cptr[ncolors - 1], b, x, omega,
+                     st, nrhs, vs);
+  for (int c = ncolors - 2; c >= 0; c--)
+    sor_colour<T, 1>(A, nodes, cptr[c], cptr[c + 1] - cptr[c], b, x, omega, st, nrhs, vs);
+}
+
+template void launch_sor_symmetric<float>(const BSR<float> &, const int *, const int *, int,
+                                          const float *, float *, double, hipStream_t, int,
+                                          int64_t);
+template void launch_sor_symmetric<double>(const BSR<double> &, const int *, const int *, int,
+                                           const double *, double *, double, hipStream_t, int,
+                                           int64_t);
 template void launch_bsr_dinv<float>(int, const int *, const double *, float *, hipStream_t);
 template void launch_bsr_dinv<double>(int, const int *, const double *, double *, hipStream_t);
 template void launch_bsr_apply<float>(const BSR<float> &, const float *, int, const AsmArgs &,

@@ -328,16 +328,16 @@ template <class T>
 void launch_bsr_apply(const BSR<T> &A, const T *x, int mode, const AsmArgs &g, hipStream_t st,
                       int nrhs = 1, int64_t vs = 0);
 
-// One point SOR sweep (forward, or BACK in reverse) over the colours of a
-// node colouring of A's graph: nodes[cptr[c] .. cptr[c + 1]) hold colour c
-// (cptr on the host, ncolors + 1 entries) and A's block row k is node
-// nodes[k] (colour-major rows, node-index columns); x updated in place
 // out[k] = val[map[k]] per 3 x 3 block
 void launch_bsr_gather(int nnzb, const int *map, const double *val, double *out, hipStream_t st);
+// One symmetric point SOR sweep (forward, then in reverse) over the colours
+// of a node colouring of A's graph: nodes[cptr[c] .. cptr[c + 1]) hold colour
+// c (cptr on the host, ncolors + 1 entries) and A's block row k is node
+// nodes[k] (colour-major rows, node-index columns); x updated in place
 template <class T>
-void launch_sor_sweep(const BSR<T> &A, const int *nodes, const int *cptr, int ncolors, bool back,
-                      const T *b, T *x, double omega, hipStream_t st, int nrhs = 1,
-                      int64_t vs = 0);
+void launch_sor_symmetric(const BSR<T> &A, const int *nodes, const int *cptr, int ncolors,
+                          const T *b, T *x, double omega, hipStream_t st, int nrhs = 1,
+                          int64_t vs = 0);
 
 // dst[0..n) = dst32[0..n) = v (n <= 32), from kernel arguments
 void launch_set_words(int n, const double *v, double *dst, float *dst32, hipStream_t st);

@@ -418,10 +418,7 @@ void Problem::sor_smooth(int l, const T *b, T *x, int nrhs, bool from_zero) {
     A.val = L.sor_val32.p;
   A.run = run_;
   const int nc = (int)L.sor_cptr.size() - 1;
-  launch_sor_sweep<T>(A, L.sor_nodes.p, L.sor_cptr.data(), nc, false, b, x, omega_, st_, nrhs,
-                      L.ndof);
-  launch_sor_sweep<T>(A, L.sor_nodes.p, L.sor_cptr.data(), nc, true, b, x, omega_, st_, nrhs,
-                      L.ndof);
+  launch_sor_symmetric<T>(A, L.sor_nodes.p, L.sor_cptr.data(), nc, b, x, omega_, st_, nrhs, L.ndof);
 }
 
 template void Problem::sor_smooth<float>(int, const float *, float *, int, bool);
