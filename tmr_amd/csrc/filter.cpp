@@ -144,7 +144,8 @@ int Filter::init(Forest *f, int kind, double r, int nterms) {
   if (ptr_.upload(ptr) || col_.upload(col) || mval_.upload(mv) || aval_.upload(av) ||
       dinv_.upload(dinv) || ascale_.upload(a) || bscale_.upload(b) || tinv_.alloc(n_) ||
       w1_.alloc(n_) || w2_.alloc(n_) || w3_.alloc(n_) || w4_.alloc(n_) || w5_.alloc(n_) ||
-      in_.alloc(n_) || out_.alloc(n_) || parts_.alloc(filter_reduce_blocks(n_) + 1)) {
+      in_.alloc(n_) || out_.alloc(n_) || parts_.alloc(filter_cg_parts()) ||
+      sc_.alloc(3) || flag_.alloc(2)) {
     last_error = "filter: device allocation failed";
     return -1;
   }
@@ -256,47 +257,32 @@ int Filter::horner(const double *x, double *y, bool transpose) {
   return 0;
 }
 
-double Filter::dot(const double *a, const double *b) {
-  const int nb = filter_reduce_blocks(n_);
-  launch_filter_dot(n_, a, b, parts_.p, st_);
-  std::vector<double> h(nb);
-  if (hipMemcpyAsync(h.data(), parts_.p, nb * sizeof(double), hipMemcpyDeviceToHost, st_) !=
-          hipSuccess ||
-      hipStreamSynchronize(st_) != hipSuccess)
-    return std::nan("");
-  double s = 0.0;
-  for (double v : h) s += v;
-  return s;
-}
-
-// (M + r^2 K) x = rhs by Jacobi-preconditioned CG from zero to rtol 1e-12
+// (M + r^2 K) x = rhs by Jacobi-preconditioned CG from zero to rtol 1e-12;
+// the stop flag is read every eight iterations, the launches behind a
+// convergence return at once
 int Filter::helmholtz_solve(const double *rhs, double *x) {
-  double *r = w1_.p, *z = w2_.p, *p = w3_.p, *q = w4_.p;
-  launch_filter_fill(n_, 0.0, x, st_);
-  launch_filter_copy(n_, rhs, r, st_);
-  const double bb = dot(rhs, rhs);
-  if (!(bb == bb)) {
+  double *r = w1_.p, *p = w3_.p, *q = w4_.p;
+  launch_filter_cg_init(n_, rhs, dinv_.p, x, r, p, parts_.p, 1e-24, sc_.p, flag_.p, st_);
+  int h[2] = {0, 0};
+  double tol2 = 0.0;
+  if (hipMemcpyAsync(&tol2, sc_.p + 2, sizeof(double), hipMemcpyDeviceToHost, st_) != hipSuccess ||
+      hipStreamSynchronize(st_) != hipSuccess || !(tol2 == tol2)) {
     last_error = "filter: device error";
     return -1;
   }
   iters_ = 0;
-  if (bb == 0.0) return 0;
-  launch_filter_mul(n_, dinv_.p, r, z, st_);
-  launch_filter_copy(n_, z, p, st_);
-  double rz = dot(r, z);
-  const double tol2 = 1e-24 * bb;
-  for (int it = 1; it <= 2000; it++) {
-    launch_filter_spmv(n_, ptr_.p, col_.p, aval_.p, p, q, st_);
-    const double alpha = rz / dot(p, q);
-    launch_filter_axpy(n_, alpha, p, x, st_);
-    launch_filter_axpy(n_, -alpha, q, r, st_);
-    const double rr = dot(r, r);
-    iters_ = it;
-    if (rr <= tol2) return 0;
-    launch_filter_mul(n_, dinv_.p, r, z, st_);
-    const double rzn = dot(r, z);
-    launch_filter_xpby(n_, z, rzn / rz, p, st_);  // p = z + beta p
-    rz = rzn;
+  if (tol2 == 0.0) return 0;
+  for (int it = 1; it <= 2000;) {
+    for (int k = 0; k < 8 && it <= 2000; k++, it++)
+      launch_filter_cg_iteration(n_, it, ptr_.p, col_.p, aval_.p, dinv_.p, x, r, p, q, parts_.p,
+                                 sc_.p, flag_.p, st_);
+    if (hipMemcpyAsync(h, flag_.p, sizeof(h), hipMemcpyDeviceToHost, st_) != hipSuccess ||
+        hipStreamSynchronize(st_) != hipSuccess) {
+      last_error = "filter: device error";
+      return -1;
+    }
+    iters_ = h[1];
+    if (h[0]) return 0;
   }
   last_error = "filter: the Helmholtz solve did not converge";
   return -1;
@@ -308,16 +294,19 @@ int Filter::apply(int nv, const double *in, double *out, bool on_device, bool tr
     return -1;
   }
   const size_t n = (size_t)n_ * nv;
-  DevArray<double> din, dout;
   const double *xin = in;
   double *xout = out;
   if (!on_device) {
-    if (din.upload(in, n) || dout.alloc(n)) {
+    if (hin_.n < n && (hin_.alloc(n) || hout_.alloc(n))) {
       last_error = "filter: device allocation failed";
       return -1;
     }
-    xin = din.p;
-    xout = dout.p;
+    if (hipMemcpyAsync(hin_.p, in, n * sizeof(double), hipMemcpyHostToDevice, st_) != hipSuccess) {
+      last_error = "filter: copy failed";
+      return -1;
+    }
+    xin = hin_.p;
+    xout = hout_.p;
   }
   for (int v = 0; v < nv; v++) {
     launch_filter_gather(n_, nv, v, xin, in_.p, st_);
@@ -333,7 +322,7 @@ int Filter::apply(int nv, const double *in, double *out, bool on_device, bool tr
     launch_filter_scatter(n_, nv, v, out_.p, xout, st_);
   }
   if (!on_device &&
-      hipMemcpyAsync(out, dout.p, n * sizeof(double), hipMemcpyDeviceToHost, st_) != hipSuccess) {
+      hipMemcpyAsync(out, hout_.p, n * sizeof(double), hipMemcpyDeviceToHost, st_) != hipSuccess) {
     last_error = "filter: copy failed";
     return -1;
   }

@@ -26,7 +26,6 @@ class Filter {
  private:
   int horner(const double *x, double *y, bool transpose);
   int helmholtz_solve(const double *rhs, double *x);
-  double dot(const double *a, const double *b);
 
   int kind_ = 0, nterms_ = 0, n_ = 0, iters_ = 0;
   double r_ = 0.0;
@@ -34,11 +33,12 @@ class Filter {
   DevArray<int> ptr_, col_, tptr_, tcol_;  // t*: the transpose (kind 2, B not symmetric)
   DevArray<double> tval_;
   DevArray<double> mval_, aval_, dinv_, ascale_, bscale_, tinv_;
-  DevArray<double> w1_, w2_, w3_, w4_, w5_, in_, out_, parts_;
+  DevArray<double> w1_, w2_, w3_, w4_, w5_, in_, out_, parts_, sc_;
+  DevArray<double> hin_, hout_;  // device copies of host vectors
+  DevArray<int> flag_;
 };
 
 // kernels (filter.hip)
-int filter_reduce_blocks(int n);
 void launch_filter_spmv(int n, const int *ptr, const int *col, const double *val,
                         const double *x, double *y, hipStream_t st);
 void launch_filter_fill(int n, double v, double *x, hipStream_t st);
@@ -49,13 +49,17 @@ void launch_filter_mul(int n, const double *a, const double *x, double *y, hipSt
 void launch_filter_mul_add(int n, const double *a, const double *u, const double *t, double *y,
                            hipStream_t st);
 void launch_filter_add(int n, const double *t, double *y, hipStream_t st);
-void launch_filter_axpy(int n, double alpha, const double *x, double *y, hipStream_t st);
-// p = z + beta p
-void launch_filter_xpby(int n, const double *z, double beta, double *p, hipStream_t st);
 // y[i] = 1 / x[i] (0 where x is 0)
 void launch_filter_recip(int n, const double *x, double *y, hipStream_t st);
-// per-block partial sums of a o b
-void launch_filter_dot(int n, const double *a, const double *b, double *parts, hipStream_t st);
+// conjugate gradients on the device (parts: filter_cg_parts() words, sc: 3,
+// flag: converged, iterations)
+int filter_cg_parts();
+void launch_filter_cg_init(int n, const double *rhs, const double *dinv, double *x, double *r,
+                           double *p, double *parts, double rtol2, double *sc, int *flag,
+                           hipStream_t st);
+void launch_filter_cg_iteration(int n, int it, const int *ptr, const int *col, const double *val,
+                                const double *dinv, double *x, double *r, double *p, double *q,
+                                double *parts, double *sc, int *flag, hipStream_t st);
 // component v of an interleaved nv-vector to/from a plain one
 void launch_filter_gather(int n, int nv, int v, const double *x, double *y, hipStream_t st);
 void launch_filter_scatter(int n, int nv, int v, const double *x, double *y, hipStream_t st);
