@@ -39,9 +39,7 @@ struct ElemBatches {
   const int *wg_class = nullptr;     // [n_wg]
   const uint16_t *lconn = nullptr;   // [n_elem * 8]
   const uint8_t *color = nullptr;    // [n_elem]
-  const int *dep_ptr = nullptr;      // hanging-node constraints
-  const int *dep_conn = nullptr;
-  const float *dep_w = nullptr;
+  const int4 *dep4 = nullptr;        // hanging nodes' parents (load_node)
   const uint8_t *bcmask = nullptr;   // [n_nodes], bit d set = dof d clamped
 };
 
@@ -197,9 +195,6 @@ struct AsmArgs {
 template <class T>
 void launch_tile_apply(const Tiles &tl, const T *K0, const T *s_elem, const T *x, int mode,
                        const AsmArgs &args, hipStream_t st, int nrhs = 1, int64_t vs = 0);
-template <class T>
-void launch_elem_apply(const ElemBatches &eb, const T *K0, const T *s_elem, const T *x,
-                       T *partial, hipStream_t st);
 template <class T>
 void launch_elem_diag(const ElemBatches &eb, const T *K0, const T *s_elem, T *partial,
                       hipStream_t st, bool nodal = false);
@@ -379,8 +374,7 @@ void launch_restrict_scale(int nc, const int *ptr, const int *child, const float
 // every element from its corner values (hanging corners interpolated from
 // their parents), s = penalty(rho) * 2^-level per point; rho_gp (may be null)
 // receives the point densities
-void launch_nodal_scale(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                        const float *dep_w, const double *xn, const int16_t *level, double q,
+void launch_nodal_scale(int nelem, const int *conn, const int4 *dep4, const double *xn, const int16_t *level, double q,
                         double k0, int penalty_type, double *rho_gp, double *s64, float *s32,
                         hipStream_t st);
 // design vector to the next coarser level: x_c = (R x_f) / (R 1), R = P^T
@@ -388,8 +382,7 @@ void launch_nodal_scale(int nelem, const int *conn, const int *dep_ptr, const in
 // src/topology/TMRConformFilter.cpp:154-167)
 void launch_weight_restrict(const TransferCSR &R, const double *xf, double *xc, hipStream_t st);
 // v_e^T K_g u_e at every Gauss point of every element (full-block tables)
-void launch_nodal_energy(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                         const float *dep_w, const uint8_t *bcmask, const int *cls,
+void launch_nodal_energy(int nelem, const int *conn, const int4 *dep4, const uint8_t *bcmask, const int *cls,
                          const double *G, const double *u, const double *v, double *out,
                          hipStream_t st);
 // nodal design gradient into slot partials (element batches, component 0):
@@ -462,23 +455,21 @@ void launch_b_finalize(const SegPlan &pl, int mode, const double *partials, doub
 void launch_b_tick(int *iter, const int *act, int nidx, int *nact, int *host, hipStream_t st);
 
 // per-element compliance density and its design derivative (element mode)
-void launch_elem_energy(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                        const float *dep_w, const uint8_t *bcmask, const int *cls,
+// K: the REFL_TABLE blocks of every class
+void launch_elem_energy(int nelem, const int *conn, const int4 *dep4, const uint8_t *bcmask, const int *cls,
                         const double *K0, const double *u, double *energy, hipStream_t st);
 // p-norm of the relaxed von Mises failure (TMROctConstitutive::evalFailure,
 // src/topology/TMROctConstitutive.cpp:1056-1104; TACS "pnorm-continuous"
-// aggregation): S = sum_e sum_g (V_e / 8) (r(rho_e) vm(C0 B_g u_e) / ys)^P.
-// CB: per class, the 8 Gauss-point stress operators C0 B_g (6 x 24) of the
-// full-block element; vol: per class block volume.
+// aggregation): S = sum_e sum_g (V_e / 8) (r(rho_e) vm(C0 B_g u_e) / ys)^P,
+// the stress formed from grad u at the point; vol: per class block volume.
 struct StressArgs {
   double P = 8.0, eps = 0.3, ys = 1.0;
-  const double *CB = nullptr;
+  const double *G = nullptr;    // NODAL_TABLE tables
   const double *vol = nullptr;
 };
 // rho_gp (nodal design, may be null): densities at the Gauss points, used
 // in place of the element densities rho
-void launch_stress_sum(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                       const float *dep_w, const uint8_t *bcmask, const int *cls,
+void launch_stress_sum(int nelem, const int *conn, const int4 *dep4, const uint8_t *bcmask, const int *cls,
                        const int16_t *lev, const double *rho, const double *rho_gp,
                        const double *u, const StressArgs &sa, double *partials, hipStream_t st);
 // element dfdu into slot partials (element batches) and the explicit
@@ -489,8 +480,7 @@ void launch_stress_grad(const ElemBatches &eb, const int16_t *lev, const int *cl
                         const StressArgs &sa, const double *sc, double *partial,
                         double *dfdrho, hipStream_t st);
 // psi_e^T K0 u_e per element (adjoint-residual product without the factor)
-void launch_elem_energy2(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                         const float *dep_w, const uint8_t *bcmask, const int *cls,
+void launch_elem_energy2(int nelem, const int *conn, const int4 *dep4, const uint8_t *bcmask, const int *cls,
                          const double *K0, const double *u, const double *v, double *out,
                          hipStream_t st);
 // g = dfdrho_explicit - dpenalty(rho) 2^-level * prod

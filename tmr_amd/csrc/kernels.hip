@@ -42,11 +42,12 @@ __device__ __forceinline__ void store_vec3(T *__restrict__ p, const T v[3]) {
   *reinterpret_cast<Vec3<T> *>(p) = Vec3<T>{v[0], v[1], v[2]};
 }
 
+// value of node e (>= 0 independent, < 0 hanging -e - 1), clamped dofs zero.
+// dep4: the parents (a, b, c, d) of every hanging node, two of weight 1/2
+// (c < 0) or four of 1/4: one record and one round of loads per node
 template <class T>
 __device__ __forceinline__ void load_node(int e, const T *__restrict__ x,
-                                          const int *__restrict__ dep_ptr,
-                                          const int *__restrict__ dep_conn,
-                                          const float *__restrict__ dep_w,
+                                          const int4 *__restrict__ dep4,
                                           const uint8_t *__restrict__ bcmask, T v[3]) {
   if (e >= 0) {
     const uint8_t m = bcmask[e];
@@ -54,88 +55,27 @@ __device__ __forceinline__ void load_node(int e, const T *__restrict__ x,
     v[0] = (m & 1) ? T(0) : u.a;
     v[1] = (m & 2) ? T(0) : u.b;
     v[2] = (m & 4) ? T(0) : u.c;
-  } else {
-    const int d = -e - 1;
-    v[0] = v[1] = v[2] = T(0);
-    for (int j = dep_ptr[d]; j < dep_ptr[d + 1]; j++) {
-      const int p = dep_conn[j];
-      const T w = (T)dep_w[j];
-      const uint8_t m = bcmask[p];
-      const Vec3<T> u = load_vec3(x + 3 * (size_t)p);
-      if (!(m & 1)) v[0] += w * u.a;
-      if (!(m & 2)) v[1] += w * u.b;
-      if (!(m & 4)) v[2] += w * u.c;
-    }
+    return;
   }
-}
-
-template <class T>
-__global__ __launch_bounds__(WG_ELEMS) void k_elem_apply(
-    const int *__restrict__ wg_node_ptr, const int *__restrict__ wg_nodes,
-    const int *__restrict__ wg_elem_ptr, const int *__restrict__ wg_class,
-    const uint4 *__restrict__ lconn, const uint8_t *__restrict__ color, int ncolors,
-    const int *__restrict__ dep_ptr, const int *__restrict__ dep_conn,
-    const float *__restrict__ dep_w, const uint8_t *__restrict__ bcmask,
-    const T *__restrict__ K0, const T *__restrict__ s_elem, const T *__restrict__ x,
-    T *__restrict__ partial) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int wg = xcd_block(blockIdx.x, gridDim.x);
-  const int tid = threadIdx.x;
-  const int nb = wg_node_ptr[wg];
-  const int nn = wg_node_ptr[wg + 1] - nb;
-  T *xs = reinterpret_cast<T *>(smem_raw);
-  T *ys = xs + 3 * nn;
-  for (int i = tid; i < nn; i += WG_ELEMS) {
-    T v[3];
-    load_node<T>(wg_nodes[nb + i], x, dep_ptr, dep_conn, dep_w, bcmask, v);
-    xs[3 * i] = v[0];
-    xs[3 * i + 1] = v[1];
-    xs[3 * i + 2] = v[2];
-    ys[3 * i] = ys[3 * i + 1] = ys[3 * i + 2] = T(0);
+  const int4 p = dep4[-e - 1];
+  const bool two = p.z < 0;
+  const int g[4] = {p.x, p.y, two ? p.x : p.z, two ? p.y : p.w};
+  Vec3<T> u[4];
+  uint8_t m[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    u[k] = load_vec3(x + 3 * (size_t)g[k]);
+    m[k] = bcmask[g[k]];
   }
-  __syncthreads();
-  const int e0 = wg_elem_ptr[wg];
-  const int ne = wg_elem_ptr[wg + 1] - e0;
-  const int cls = __builtin_amdgcn_readfirstlane(wg_class[wg]);
-  const T *__restrict__ K = K0 + 576 * cls;
-  T ye[24];
-  int lc[8];
-  int col = -1;
-  if (tid < ne) {
-    const uint4 q = lconn[e0 + tid];
-    lc[0] = q.x & 0xffff; lc[1] = q.x >> 16;
-    lc[2] = q.y & 0xffff; lc[3] = q.y >> 16;
-    lc[4] = q.z & 0xffff; lc[5] = q.z >> 16;
-    lc[6] = q.w & 0xffff; lc[7] = q.w >> 16;
-    col = color[e0 + tid];
-    const T s = s_elem[e0 + tid];
-    T xe[24];
+  const T w = two ? T(0.5) : T(0.25);
+  v[0] = v[1] = v[2] = T(0);
 #pragma unroll
-    for (int a = 0; a < 8; a++) {
-      xe[3 * a] = xs[3 * lc[a]];
-      xe[3 * a + 1] = xs[3 * lc[a] + 1];
-      xe[3 * a + 2] = xs[3 * lc[a] + 2];
-    }
-#pragma unroll
-    for (int i = 0; i < 24; i++) {
-      T acc = T(0);
-#pragma unroll
-      for (int j = 0; j < 24; j++) acc += K[24 * i + j] * xe[j];
-      ye[i] = s * acc;
-    }
+  for (int k = 0; k < 4; k++) {
+    const bool on = k < 2 || !two;
+    if (on && !(m[k] & 1)) v[0] += w * u[k].a;
+    if (on && !(m[k] & 2)) v[1] += w * u[k].b;
+    if (on && !(m[k] & 4)) v[2] += w * u[k].c;
   }
-  for (int c = 0; c < ncolors; c++) {
-    if (col == c) {
-#pragma unroll
-      for (int a = 0; a < 8; a++) {
-        ys[3 * lc[a]] += ye[3 * a];
-        ys[3 * lc[a] + 1] += ye[3 * a + 1];
-        ys[3 * lc[a] + 2] += ye[3 * a + 2];
-      }
-    }
-    __syncthreads();
-  }
-  for (int i = tid; i < 3 * nn; i += WG_ELEMS) partial[3 * nb + i] = ys[i];
 }
 
 template <class T, bool NODAL>
@@ -201,18 +141,6 @@ __global__ __launch_bounds__(WG_ELEMS) void k_elem_diag(
 }
 
 template <class T>
-void launch_elem_apply(const ElemBatches &eb, const T *K0, const T *s_elem, const T *x,
-                       T *partial, hipStream_t st) {
-  if (eb.n_wg == 0) return;
-  size_t sh = 2 * 3 * (size_t)eb.max_wg_nodes * sizeof(T);
-  hipLaunchKernelGGL(k_elem_apply<T>, dim3(eb.n_wg), dim3(WG_ELEMS), sh, st, eb.wg_node_ptr,
-                     eb.wg_nodes, eb.wg_elem_ptr, eb.wg_class,
-                     reinterpret_cast<const uint4 *>(eb.lconn), eb.color, eb.ncolors,
-                     eb.dep_ptr, eb.dep_conn, eb.dep_w, eb.bcmask, K0, s_elem, x, partial);
-  TMRX_LAUNCH_CHECK();
-}
-
-template <class T>
 void launch_elem_diag(const ElemBatches &eb, const T *K0, const T *s_elem, T *partial,
                       hipStream_t st, bool nodal) {
   if (eb.n_wg == 0) return;
@@ -230,17 +158,17 @@ void launch_elem_diag(const ElemBatches &eb, const T *K0, const T *s_elem, T *pa
   TMRX_LAUNCH_CHECK();
 }
 
-// corner-pair diagonal terms (elements with hanging corners), one thread
-// per node that has them; records in a fixed order, so the sums are too
+// corner-pair diagonal terms (elements with hanging corners), eight lanes per
+// node that has them (1.2M adaptive hex: one thread 516 us, now 102);
+// records and lanes in a fixed order, so the sums are too
 template <bool NODAL>
 __global__ __launch_bounds__(256) void k_diag_cross(
     int n, const int *__restrict__ ptr, const int *__restrict__ node, const int *__restrict__ code,
     const double *__restrict__ w, const int *__restrict__ cls, const double *__restrict__ K0,
     const double *__restrict__ s, const uint8_t *__restrict__ bcmask, double *__restrict__ dinv) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const int i = (blockIdx.x * 256 + threadIdx.x) / 8, sub = threadIdx.x % 8;
   double c[3] = {0.0, 0.0, 0.0};
-  for (int j = ptr[i]; j < ptr[i + 1]; j++) {
+  for (int j = i < n ? ptr[i] + sub : 0, j1 = i < n ? ptr[i + 1] : 0; j < j1; j += 8) {
     const int cd = code[j], e = cd >> 6, a = (cd >> 3) & 7, b = cd & 7;
     const double wj = w[j];
     if (NODAL) {
@@ -259,6 +187,11 @@ __global__ __launch_bounds__(256) void k_diag_cross(
       for (int d = 0; d < 3; d++) c[d] += se * K[(3 * a + d) * 24 + 3 * b + d];
     }
   }
+#pragma unroll
+  for (int k = 1; k < 8; k <<= 1)
+#pragma unroll
+    for (int d = 0; d < 3; d++) c[d] += __shfl_xor(c[d], k);
+  if (i >= n || sub != 0) return;
   const int nd = node[i];
   const uint8_t m = bcmask[nd];
   for (int d = 0; d < 3; d++)
@@ -273,10 +206,10 @@ void launch_diag_cross(int n, const int *ptr, const int *node, const int *code, 
                        const uint8_t *bcmask, double *dinv, hipStream_t st) {
   if (n == 0) return;
   if (nodal)
-    hipLaunchKernelGGL(k_diag_cross<true>, dim3((n + 255) / 256), dim3(256), 0, st, n, ptr, node,
+    hipLaunchKernelGGL(k_diag_cross<true>, dim3((n + 31) / 32), dim3(256), 0, st, n, ptr, node,
                        code, w, cls, K0, s, bcmask, dinv);
   else
-    hipLaunchKernelGGL(k_diag_cross<false>, dim3((n + 255) / 256), dim3(256), 0, st, n, ptr, node,
+    hipLaunchKernelGGL(k_diag_cross<false>, dim3((n + 31) / 32), dim3(256), 0, st, n, ptr, node,
                        code, w, cls, K0, s, bcmask, dinv);
   TMRX_LAUNCH_CHECK();
 }
@@ -812,13 +745,18 @@ __device__ __forceinline__ double gauss_N(int a, int g) {
 }
 
 __device__ __forceinline__ double node_value(int g, const double *__restrict__ xn,
-                                             const int *__restrict__ dep_ptr,
-                                             const int *__restrict__ dep_conn,
-                                             const float *__restrict__ dep_w) {
+                                             const int4 *__restrict__ dep4) {
   if (g >= 0) return xn[g];
-  const int d = -g - 1;
+  const int4 p = dep4[-g - 1];
   double v = 0.0;
-  for (int j = dep_ptr[d]; j < dep_ptr[d + 1]; j++) v += (double)dep_w[j] * xn[dep_conn[j]];
+  const bool two = p.z < 0;
+  const double w = two ? 0.5 : 0.25;
+  v += w * xn[p.x];
+  v += w * xn[p.y];
+  if (!two) {
+    v += w * xn[p.z];
+    v += w * xn[p.w];
+  }
   return v;
 }
 
@@ -832,8 +770,7 @@ __device__ __forceinline__ double dpenalty_of(double r, double q, int ptype) {
   return (q + 1.0) / (t * t);
 }
 
-__global__ void k_nodal_scale(int ne, const int *__restrict__ conn, const int *__restrict__ dep_ptr,
-                              const int *__restrict__ dep_conn, const float *__restrict__ dep_w,
+__global__ void k_nodal_scale(int ne, const int *__restrict__ conn, const int4 *__restrict__ dep4,
                               const double *__restrict__ xn, const int16_t *__restrict__ lev,
                               double q, double k0, int ptype, double *__restrict__ rho_gp,
                               double *__restrict__ s64, float *__restrict__ s32) {
@@ -841,7 +778,7 @@ __global__ void k_nodal_scale(int ne, const int *__restrict__ conn, const int *_
   if (e >= ne) return;
   double xa[8];
 #pragma unroll
-  for (int a = 0; a < 8; a++) xa[a] = node_value(conn[8 * (size_t)e + a], xn, dep_ptr, dep_conn, dep_w);
+  for (int a = 0; a < 8; a++) xa[a] = node_value(conn[8 * (size_t)e + a], xn, dep4);
   const int l = lev[e];
 #pragma unroll
   for (int g = 0; g < 8; g++) {
@@ -856,13 +793,12 @@ __global__ void k_nodal_scale(int ne, const int *__restrict__ conn, const int *_
   }
 }
 
-void launch_nodal_scale(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                        const float *dep_w, const double *xn, const int16_t *level, double q,
+void launch_nodal_scale(int nelem, const int *conn, const int4 *dep4, const double *xn, const int16_t *level, double q,
                         double k0, int penalty_type, double *rho_gp, double *s64, float *s32,
                         hipStream_t st) {
   if (nelem == 0) return;
   hipLaunchKernelGGL(k_nodal_scale, dim3((nelem + 255) / 256), dim3(256), 0, st, nelem, conn,
-                     dep_ptr, dep_conn, dep_w, xn, level, q, k0, penalty_type, rho_gp, s64, s32);
+                     dep4, xn, level, q, k0, penalty_type, rho_gp, s64, s32);
   TMRX_LAUNCH_CHECK();
 }
 
@@ -890,15 +826,18 @@ void launch_weight_restrict(const TransferCSR &R, const double *xf, double *xc, 
 // grad u at Gauss point g of an element (H[3 c + d] = du_c / dx_d)
 __device__ __forceinline__ void grad_at(const double *__restrict__ G, const double ue[24],
                                         double H[9]) {
+#pragma unroll
   for (int i = 0; i < 9; i++) H[i] = 0.0;
+#pragma unroll
   for (int a = 0; a < 8; a++)
+#pragma unroll
     for (int c = 0; c < 3; c++)
+#pragma unroll
       for (int d = 0; d < 3; d++) H[3 * c + d] += ue[3 * a + c] * G[3 * a + d];
 }
 
 __global__ void k_nodal_energy(int ne, const int *__restrict__ conn,
-                               const int *__restrict__ dep_ptr, const int *__restrict__ dep_conn,
-                               const float *__restrict__ dep_w, const uint8_t *__restrict__ bcmask,
+                               const int4 *__restrict__ dep4, const uint8_t *__restrict__ bcmask,
                                const int *__restrict__ cls, const double *__restrict__ Gtab,
                                const double *__restrict__ u, const double *__restrict__ v,
                                double *__restrict__ out) {
@@ -907,11 +846,11 @@ __global__ void k_nodal_energy(int ne, const int *__restrict__ conn,
   double ue[24], ve[24];
   for (int a = 0; a < 8; a++) {
     double t[3];
-    load_node<double>(conn[8 * (size_t)e + a], u, dep_ptr, dep_conn, dep_w, bcmask, t);
+    load_node<double>(conn[8 * (size_t)e + a], u, dep4, bcmask, t);
     ue[3 * a] = t[0];
     ue[3 * a + 1] = t[1];
     ue[3 * a + 2] = t[2];
-    load_node<double>(conn[8 * (size_t)e + a], v, dep_ptr, dep_conn, dep_w, bcmask, t);
+    load_node<double>(conn[8 * (size_t)e + a], v, dep4, bcmask, t);
     ve[3 * a] = t[0];
     ve[3 * a + 1] = t[1];
     ve[3 * a + 2] = t[2];
@@ -932,13 +871,12 @@ __global__ void k_nodal_energy(int ne, const int *__restrict__ conn,
   }
 }
 
-void launch_nodal_energy(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                         const float *dep_w, const uint8_t *bcmask, const int *cls,
+void launch_nodal_energy(int nelem, const int *conn, const int4 *dep4, const uint8_t *bcmask, const int *cls,
                          const double *G, const double *u, const double *v, double *out,
                          hipStream_t st) {
   if (nelem == 0) return;
   hipLaunchKernelGGL(k_nodal_energy, dim3((nelem + 255) / 256), dim3(256), 0, st, nelem, conn,
-                     dep_ptr, dep_conn, dep_w, bcmask, cls, G, u, v, out);
+                     dep4, bcmask, cls, G, u, v, out);
   TMRX_LAUNCH_CHECK();
 }
 
@@ -1157,38 +1095,20 @@ void launch_finalize(int nparts, const double *partials, int mode, double *sc, h
 // ---------------------------------------------------------------------------
 // element strain energy u_e^T K0 u_e (unscaled) for the adjoint / compliance
 // sensitivities (src/topology/TMROctConstitutive.cpp:557-654 restricted to
-// element-constant density).
-__global__ void k_elem_energy(int ne, const int *__restrict__ conn, const int *__restrict__ dep_ptr,
-                              const int *__restrict__ dep_conn, const float *__restrict__ dep_w,
+// element-constant density), or v_e^T K0 u_e, through the reflection blocks
+// (refl_elem: 45 multiply-adds against 576 and 45 table reads against 576;
+// 1.2M adaptive hex 348 -> 138 us)
+template <bool TWO>
+__global__ void k_elem_energy(int ne, const int *__restrict__ conn, const int4 *__restrict__ dep4,
                               const uint8_t *__restrict__ bcmask, const int *__restrict__ cls,
-                              const double *__restrict__ K0, const double *__restrict__ u,
-                              double *__restrict__ energy) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
-  double ue[24];
-  for (int a = 0; a < 8; a++) {
-    double v[3];
-    load_node<double>(conn[8 * e + a], u, dep_ptr, dep_conn, dep_w, bcmask, v);
-    ue[3 * a] = v[0];
-    ue[3 * a + 1] = v[1];
-    ue[3 * a + 2] = v[2];
-  }
-  const double *K = K0 + 576 * cls[e];
-  double s = 0.0;
-  for (int i = 0; i < 24; i++) {
-    double t = 0.0;
-    for (int j = 0; j < 24; j++) t += K[24 * i + j] * ue[j];
-    s += ue[i] * t;
-  }
-  energy[e] = s;
-}
+                              const double *__restrict__ R, const double *__restrict__ u,
+                              const double *__restrict__ v, double *__restrict__ energy);
 
-void launch_elem_energy(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                        const float *dep_w, const uint8_t *bcmask, const int *cls,
+void launch_elem_energy(int nelem, const int *conn, const int4 *dep4, const uint8_t *bcmask, const int *cls,
                         const double *K0, const double *u, double *energy, hipStream_t st) {
   if (nelem == 0) return;
-  hipLaunchKernelGGL(k_elem_energy, dim3((nelem + 255) / 256), dim3(256), 0, st, nelem, conn,
-                     dep_ptr, dep_conn, dep_w, bcmask, cls, K0, u, energy);
+  hipLaunchKernelGGL(k_elem_energy<false>, dim3((nelem + 255) / 256), dim3(256), 0, st, nelem, conn,
+                     dep4, bcmask, cls, K0, u, u, energy);
   TMRX_LAUNCH_CHECK();
 }
 
@@ -1594,6 +1514,32 @@ __device__ __forceinline__ void refl_elem(const T *__restrict__ M, T sc, const T
     ye[3 * a + 1] = Y1[a];
     ye[3 * a + 2] = Y2[a];
   }
+}
+
+template <bool TWO>
+__global__ void k_elem_energy(int ne, const int *__restrict__ conn, const int4 *__restrict__ dep4,
+                              const uint8_t *__restrict__ bcmask, const int *__restrict__ cls,
+                              const double *__restrict__ R, const double *__restrict__ u,
+                              const double *__restrict__ v, double *__restrict__ energy) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= ne) return;
+  double ue[24], ye[24];
+#pragma unroll
+  for (int a = 0; a < 8; a++)
+    load_node<double>(conn[8 * (size_t)e + a], u, dep4, bcmask, ue + 3 * a);
+  refl_elem<double, false>(R + REFL_TABLE * (size_t)cls[e], 1.0, ue, ye);
+  double s = 0.0;
+#pragma unroll
+  for (int a = 0; a < 8; a++) {
+    if (TWO) {
+      double ve[3];
+      load_node<double>(conn[8 * (size_t)e + a], v, dep4, bcmask, ve);
+      s += ve[0] * ye[3 * a] + ve[1] * ye[3 * a + 1] + ve[2] * ye[3 * a + 2];
+    } else {
+      s += ue[3 * a] * ye[3 * a] + ue[3 * a + 1] * ye[3 * a + 1] + ue[3 * a + 2] * ye[3 * a + 2];
+    }
+  }
+  energy[e] = s;
 }
 
 // Nodal-design element product y_e = sum_g s_g K_g x_e in gradient form: at
@@ -2399,13 +2345,27 @@ __device__ __forceinline__ void vm_terms(const double s[6], double ys, double *J
   (void)ys;
 }
 
+// stress (xx, yy, zz, yz, xz, xy) at a Gauss point from grad u (72
+// multiply-adds and 24 table reads against the 144 of a 6 x 24 operator)
+__device__ __forceinline__ void point_stress(const double *__restrict__ G, const double ue[24],
+                                             double lam, double mu, double sg[6]) {
+  double H[9];
+  grad_at(G, ue, H);
+  const double tr = lam * (H[0] + H[4] + H[8]);
+  sg[0] = tr + 2.0 * mu * H[0];
+  sg[1] = tr + 2.0 * mu * H[4];
+  sg[2] = tr + 2.0 * mu * H[8];
+  sg[3] = mu * (H[5] + H[7]);
+  sg[4] = mu * (H[2] + H[6]);
+  sg[5] = mu * (H[1] + H[3]);
+}
+
 __global__ __launch_bounds__(256) void k_stress_sum(
-    int ne, const int *__restrict__ conn, const int *__restrict__ dep_ptr,
-    const int *__restrict__ dep_conn, const float *__restrict__ dep_w,
+    int ne, const int *__restrict__ conn, const int4 *__restrict__ dep4,
     const uint8_t *__restrict__ bcmask, const int *__restrict__ cls,
     const int16_t *__restrict__ lev, const double *__restrict__ rho,
     const double *__restrict__ rho_gp, const double *__restrict__ u, double P, double eps,
-    double ys, const double *__restrict__ CB, const double *__restrict__ vol,
+    double ys, const double *__restrict__ Gtab, const double *__restrict__ vol,
     double *__restrict__ partials) {
   __shared__ double red[4];
   const int e = blockIdx.x * 256 + threadIdx.x;
@@ -2414,7 +2374,7 @@ __global__ __launch_bounds__(256) void k_stress_sum(
     double ue[24];
     for (int a = 0; a < 8; a++) {
       double v[3];
-      load_node<double>(conn[8 * e + a], u, dep_ptr, dep_conn, dep_w, bcmask, v);
+      load_node<double>(conn[8 * e + a], u, dep4, bcmask, v);
       ue[3 * a] = v[0];
       ue[3 * a + 1] = v[1];
       ue[3 * a + 2] = v[2];
@@ -2423,16 +2383,13 @@ __global__ __launch_bounds__(256) void k_stress_sum(
     const double hs = ldexp(1.0, l);  // B scales as 1/h
     const double Ve = ldexp(vol[c], -3 * l);
     const double re = rho_gp ? 0.0 : rho[e];
-    const double *G = CB + 8 * 144 * (size_t)c;
+    const double *__restrict__ Gt = Gtab + NODAL_TABLE * (size_t)c;
+    const double lam = Gt[192] * 8.0 / vol[c], mu = Gt[193] * 8.0 / vol[c];
     for (int g = 0; g < 8; g++) {
       const double rh = rho_gp ? rho_gp[8 * (size_t)e + g] : re;
       const double r = rh / (eps * (1.0 - rh) + rh);
       double sg[6];
-      for (int i = 0; i < 6; i++) {
-        double t = 0.0;
-        for (int j = 0; j < 24; j++) t += G[144 * g + 24 * i + j] * ue[j];
-        sg[i] = hs * t;
-      }
+      point_stress(Gt + 24 * g, ue, hs * lam, hs * mu, sg);
       double J, dJ[6];
       vm_terms(sg, ys, &J, dJ);
       const double fail = r * sqrt(J) / ys;
@@ -2443,14 +2400,13 @@ __global__ __launch_bounds__(256) void k_stress_sum(
   if (threadIdx.x == 0) partials[blockIdx.x] = sum;
 }
 
-void launch_stress_sum(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                       const float *dep_w, const uint8_t *bcmask, const int *cls,
+void launch_stress_sum(int nelem, const int *conn, const int4 *dep4, const uint8_t *bcmask, const int *cls,
                        const int16_t *lev, const double *rho, const double *rho_gp,
                        const double *u, const StressArgs &sa, double *partials, hipStream_t st) {
   if (nelem == 0) return;
   hipLaunchKernelGGL(k_stress_sum, dim3((nelem + 255) / 256), dim3(256), 0, st, nelem, conn,
-                     dep_ptr, dep_conn, dep_w, bcmask, cls, lev, rho, rho_gp, u, sa.P, sa.eps,
-                     sa.ys, sa.CB, sa.vol, partials);
+                     dep4, bcmask, cls, lev, rho, rho_gp, u, sa.P, sa.eps,
+                     sa.ys, sa.G, sa.vol, partials);
   TMRX_LAUNCH_CHECK();
 }
 
@@ -2460,12 +2416,11 @@ void launch_stress_sum(int nelem, const int *conn, const int *dep_ptr, const int
 __global__ __launch_bounds__(WG_ELEMS) void k_stress_grad(
     const int *__restrict__ wg_node_ptr, const int *__restrict__ wg_nodes,
     const int *__restrict__ wg_elem_ptr, const uint4 *__restrict__ lconn,
-    const uint8_t *__restrict__ color, int ncolors, const int *__restrict__ dep_ptr,
-    const int *__restrict__ dep_conn, const float *__restrict__ dep_w,
+    const uint8_t *__restrict__ color, int ncolors, const int4 *__restrict__ dep4,
     const uint8_t *__restrict__ bcmask, const int16_t *__restrict__ lev,
     const int *__restrict__ cls, const double *__restrict__ rho,
     const double *__restrict__ rho_gp, const double *__restrict__ u, double P, double eps,
-    double ys, const double *__restrict__ CB, const double *__restrict__ vol,
+    double ys, const double *__restrict__ Gtab, const double *__restrict__ vol,
     const double *__restrict__ sc, double *__restrict__ partial, double *__restrict__ dfdrho) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int wg = blockIdx.x, tid = threadIdx.x;
@@ -2474,7 +2429,7 @@ __global__ __launch_bounds__(WG_ELEMS) void k_stress_grad(
   double *ys_acc = xs + 3 * nn;
   for (int i = tid; i < nn; i += WG_ELEMS) {
     double v[3];
-    load_node<double>(wg_nodes[nb + i], u, dep_ptr, dep_conn, dep_w, bcmask, v);
+    load_node<double>(wg_nodes[nb + i], u, dep4, bcmask, v);
     xs[3 * i] = v[0];
     xs[3 * i + 1] = v[1];
     xs[3 * i + 2] = v[2];
@@ -2502,18 +2457,15 @@ __global__ __launch_bounds__(WG_ELEMS) void k_stress_grad(
     const double hs = ldexp(1.0, l);
     const double Ve = ldexp(vol[c], -3 * l);
     const double re = rho_gp ? 0.0 : rho[e];
-    const double *G = CB + 8 * 144 * (size_t)c;
+    const double *__restrict__ Gt = Gtab + NODAL_TABLE * (size_t)c;
+    const double lam = Gt[192] * 8.0 / vol[c], mu = Gt[193] * 8.0 / vol[c];
     double sum_vmP = 0.0;
     for (int g = 0; g < 8; g++) {
       const double rh = rho_gp ? rho_gp[8 * (size_t)e + g] : re;
       const double den = eps * (1.0 - rh) + rh;
       const double r = rh / den, dr = eps / (den * den);
       double sg[6];
-      for (int i = 0; i < 6; i++) {
-        double t = 0.0;
-        for (int j = 0; j < 24; j++) t += G[144 * g + 24 * i + j] * ue[j];
-        sg[i] = hs * t;
-      }
+      point_stress(Gt + 24 * g, ue, hs * lam, hs * mu, sg);
       double J, dJ[6];
       vm_terms(sg, ys, &J, dJ);
       const double vm = sqrt(J) / ys;
@@ -2521,10 +2473,18 @@ __global__ __launch_bounds__(WG_ELEMS) void k_stress_grad(
       if (rho_gp) dfdrho[8 * (size_t)e + g] = coef * 0.125 * Ve * pow(r, P - 1.0) * dr * pow(vm, P);
       // coef (V/8) r^P vm^(P-2) / (2 ys^2) * dJ^T CB_g (with the 1/h factor)
       const double w = coef * 0.125 * Ve * pow(r, P) * pow(vm, P - 2.0) / (2.0 * ys * ys) * hs;
-      for (int i = 0; i < 6; i++) {
-        const double wi = w * dJ[i];
-        for (int j = 0; j < 24; j++) ge[j] += wi * G[144 * g + 24 * i + j];
-      }
+      // (C0 dJ) : grad N_a
+      const double tr = w * lam * (dJ[0] + dJ[1] + dJ[2]), m2 = 2.0 * w * mu, m1 = w * mu;
+      const double S[9] = {tr + m2 * dJ[0], m1 * dJ[5],      m1 * dJ[4],
+                           m1 * dJ[5],      tr + m2 * dJ[1], m1 * dJ[3],
+                           m1 * dJ[4],      m1 * dJ[3],      tr + m2 * dJ[2]};
+      const double *__restrict__ G = Gt + 24 * g;
+#pragma unroll
+      for (int a = 0; a < 8; a++)
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+          ge[3 * a + d] += S[3 * d] * G[3 * a] + S[3 * d + 1] * G[3 * a + 1] +
+                           S[3 * d + 2] * G[3 * a + 2];
     }
     if (!rho_gp) {
       const double den = eps * (1.0 - re) + re;
@@ -2550,48 +2510,18 @@ void launch_stress_grad(const ElemBatches &eb, const int16_t *lev, const int *cl
   const size_t sh = 2 * 3 * (size_t)eb.max_wg_nodes * sizeof(double);
   hipLaunchKernelGGL(k_stress_grad, dim3(eb.n_wg), dim3(WG_ELEMS), sh, st, eb.wg_node_ptr,
                      eb.wg_nodes, eb.wg_elem_ptr, reinterpret_cast<const uint4 *>(eb.lconn),
-                     eb.color, eb.ncolors, eb.dep_ptr, eb.dep_conn, eb.dep_w, eb.bcmask, lev,
-                     cls, rho, rho_gp, u, sa.P, sa.eps, sa.ys, sa.CB, sa.vol, sc, partial,
+                     eb.color, eb.ncolors, eb.dep4, eb.bcmask, lev,
+                     cls, rho, rho_gp, u, sa.P, sa.eps, sa.ys, sa.G, sa.vol, sc, partial,
                      dfdrho);
   TMRX_LAUNCH_CHECK();
 }
 
-__global__ void k_elem_energy2(int ne, const int *__restrict__ conn, const int *__restrict__ dep_ptr,
-                               const int *__restrict__ dep_conn, const float *__restrict__ dep_w,
-                               const uint8_t *__restrict__ bcmask, const int *__restrict__ cls,
-                               const double *__restrict__ K0, const double *__restrict__ u,
-                               const double *__restrict__ v, double *__restrict__ out) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
-  double ue[24], ve[24];
-  for (int a = 0; a < 8; a++) {
-    double t[3];
-    load_node<double>(conn[8 * e + a], u, dep_ptr, dep_conn, dep_w, bcmask, t);
-    ue[3 * a] = t[0];
-    ue[3 * a + 1] = t[1];
-    ue[3 * a + 2] = t[2];
-    load_node<double>(conn[8 * e + a], v, dep_ptr, dep_conn, dep_w, bcmask, t);
-    ve[3 * a] = t[0];
-    ve[3 * a + 1] = t[1];
-    ve[3 * a + 2] = t[2];
-  }
-  const double *K = K0 + 576 * cls[e];
-  double s = 0.0;
-  for (int i = 0; i < 24; i++) {
-    double t = 0.0;
-    for (int j = 0; j < 24; j++) t += K[24 * i + j] * ue[j];
-    s += ve[i] * t;
-  }
-  out[e] = s;
-}
-
-void launch_elem_energy2(int nelem, const int *conn, const int *dep_ptr, const int *dep_conn,
-                         const float *dep_w, const uint8_t *bcmask, const int *cls,
+void launch_elem_energy2(int nelem, const int *conn, const int4 *dep4, const uint8_t *bcmask, const int *cls,
                          const double *K0, const double *u, const double *v, double *out,
                          hipStream_t st) {
   if (nelem == 0) return;
-  hipLaunchKernelGGL(k_elem_energy2, dim3((nelem + 255) / 256), dim3(256), 0, st, nelem, conn,
-                     dep_ptr, dep_conn, dep_w, bcmask, cls, K0, u, v, out);
+  hipLaunchKernelGGL(k_elem_energy<true>, dim3((nelem + 255) / 256), dim3(256), 0, st, nelem, conn,
+                     dep4, bcmask, cls, K0, u, v, out);
   TMRX_LAUNCH_CHECK();
 }
 
@@ -2622,8 +2552,6 @@ void launch_adjoint_grad(int n, const double *rho, const int16_t *lev, double q,
 
 // explicit instantiations
 #define TMRX_INST(T)                                                                            \
-  template void launch_elem_apply<T>(const ElemBatches &, const T *, const T *, const T *, T *, \
-                                     hipStream_t);                                              \
   template void launch_elem_diag<T>(const ElemBatches &, const T *, const T *, T *,             \
                                     hipStream_t, bool);                                         \
   template void launch_assemble<T>(const AsmCSR &, const uint8_t *, const T *, int,             \

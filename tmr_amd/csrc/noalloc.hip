@@ -18,7 +18,7 @@
 
 namespace tmrx {
 
-StressArgs Problem_stress_args(const Material &m, double P, const double *CB, const double *vol);
+StressArgs Problem_stress_args(const Material &m, double P, const double *G, const double *vol);
 
 // partial sums of 256-element blocks: up to NOALLOC_MAX_BLOCKS * 256 =
 // 16,777,216 elements; the PCG scalar slots in front (SC_N doubles)
@@ -81,8 +81,8 @@ int Problem::stress_pnorm_noalloc(double P, double *f) {
   double *scr = nullptr;
   if (scratch_address(dev, &scr, last_error)) return -1;
   double *sc = scr, *parts = scr + SC_N;
-  const StressArgs sa = Problem_stress_args(mat_, P, CB_.p, cvol_.p);
-  launch_stress_sum(L.n_elem, L.d_conn.p, L.dep_ptr.p, L.dep_conn.p, L.dep_w.p, state_mask(),
+  const StressArgs sa = Problem_stress_args(mat_, P, G64_.p, cvol_.p);
+  launch_stress_sum(L.n_elem, L.d_conn.p, L.dep4(), state_mask(),
                     L.d_cls.p, L.d_lev.p, rho_.p, design_mode_ == 1 ? rho_gp_.p : nullptr, u_.p,
                     sa, parts, st_);
   launch_finalize(nb, parts, 4, sc, st_);

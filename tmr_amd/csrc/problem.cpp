@@ -254,26 +254,11 @@ int Problem::init(int nlevels, Forest **forests, const Material &mat, int nbcs,
       return -1;
     }
   }
-  // Gauss-point stress operators C0 B_g (6 x 24, 8 points) and volumes of the
-  // full-block element of every class (p-norm stress functional)
+  // block volumes (p-norm stress functional)
   {
-    std::vector<double> cb(8 * 144 * (size_t)nclasses_), vol(nclasses_);
-    const double gp = 1.0 / std::sqrt(3.0);
-    for (int c = 0; c < nclasses_; c++) {
-      vol[c] = ext[c][0] * ext[c][1] * ext[c][2];
-      for (int g = 0; g < 8; g++) {
-        const double pt[3] = {(g & 1) ? gp : -gp, (g & 2) ? gp : -gp, (g & 4) ? gp : -gp};
-        double B[144], N[8];
-        hex8_box_B(ext[c][0], ext[c][1], ext[c][2], pt, B, N);
-        for (int i = 0; i < 6; i++)
-          for (int j = 0; j < 24; j++) {
-            double t = 0.0;
-            for (int k = 0; k < 6; k++) t += C[6 * i + k] * B[24 * k + j];
-            cb[144 * (8 * (size_t)c + g) + 24 * i + j] = t;
-          }
-      }
-    }
-    if (CB_.upload(cb) || cvol_.upload(vol)) {
+    std::vector<double> vol(nclasses_);
+    for (int c = 0; c < nclasses_; c++) vol[c] = ext[c][0] * ext[c][1] * ext[c][2];
+    if (cvol_.upload(vol)) {
       last_error = "problem: device allocation failed";
       return -1;
     }
@@ -558,13 +543,25 @@ int Problem::build_level(int l, int nbcs, const char **names, const int *masks) 
       return -1;
     }
   }
-  std::vector<int> dp(dptr.begin(), dptr.end());
-  if (dp.empty()) dp.push_back(0);
-  std::vector<float> dwf(dw.begin(), dw.end());
+  // A hanging node of a trilinear mesh sits in the middle of a coarser edge
+  // (two parents, 1/2) or face (four, 1/4); the kernels' packed records hold
+  // nothing else.
+  std::vector<int> dep4;
+  for (int d = 0; d < L.n_dep; d++) {
+    const int np = dptr[d + 1] - dptr[d];
+    bool ok = np == 2 || np == 4;
+    for (int j = dptr[d]; ok && j < dptr[d + 1]; j++) ok = dw[j] * np == 1.0 && dconn[j] >= 0;
+    if (!ok) {
+      last_error = "problem: a hanging node is not the mean of two or four nodes";
+      return -1;
+    }
+    for (int k = 0; k < 4; k++) dep4.push_back(k < np ? dconn[dptr[d] + k] : -1);
+  }
+  if (dep4.empty()) dep4.assign(4, 0);
   if (L.wg_node_ptr.upload(wg_node_ptr) || L.wg_nodes.upload(wg_nodes) ||
       L.wg_elem_ptr.upload(wg_elem_ptr) || L.wg_class.upload(wg_class) ||
       L.lconn.upload(lconn) || L.color.upload(color) || L.d_bcmask.upload(L.bcmask) ||
-      L.dep_ptr.upload(dp) || L.dep_conn.upload(dconn) || L.dep_w.upload(dwf) ||
+      L.d_dep4.upload(dep4) ||
       L.asm_ptr.upload(aptr) || L.asm_slot.upload(aslot) || L.asm_w.upload(aw) ||
       L.d_conn.upload(L.conn) || L.d_cls.upload(L.cls) || L.d_lev.upload(L.lev) ||
       L.s64.alloc(ne) || L.s32.alloc(ne)) {
@@ -582,9 +579,7 @@ int Problem::build_level(int l, int nbcs, const char **names, const int *masks) 
   eb.wg_class = L.wg_class.p;
   eb.lconn = L.lconn.p;
   eb.color = L.color.p;
-  eb.dep_ptr = L.dep_ptr.p;
-  eb.dep_conn = L.dep_conn.p;
-  eb.dep_w = L.dep_w.p;
+  eb.dep4 = L.dep4();
   eb.bcmask = L.d_bcmask.p;
   L.asmc.n_nodes = L.n_nodes;
   L.asmc.ptr = L.asm_ptr.p;
@@ -615,19 +610,8 @@ int Problem::build_tiles(int l) {
     for (int e = 0; e < ne; e++)
       for (int a = 0; a < 8; a++) iel[fill[xid(L.conn[8 * e + a])]++] = e;
   }
-  // parent -> hanging nodes.  A hanging node of a trilinear mesh sits in the
-  // middle of a coarser edge (two parents, 1/2) or face (four, 1/4); the
-  // kernels' packed records hold nothing else.
+  // parent -> hanging nodes
   std::vector<int> pptr(n + 1, 0), pdep;
-  for (int d = 0; d < nd; d++) {
-    const int np = dptr[d + 1] - dptr[d];
-    bool ok = np == 2 || np == 4;
-    for (int j = dptr[d]; ok && j < dptr[d + 1]; j++) ok = dw[j] * np == 1.0 && dconn[j] >= 0;
-    if (!ok) {
-      last_error = "problem: a hanging node is not the mean of two or four nodes";
-      return -1;
-    }
-  }
   for (int j = 0; j < (nd ? dptr[nd] : 0); j++) pptr[dconn[j] + 1]++;
   for (int i = 0; i < n; i++) pptr[i + 1] += pptr[i];
   pdep.resize(pptr[n]);
@@ -1234,7 +1218,7 @@ int Problem::set_design_nodal(const double *x, int n, bool on_device) {
     launch_weight_restrict(levels_[l].R, levels_[l].xn.p, levels_[l + 1].xn.p, st_);
   for (size_t l = 0; l < levels_.size(); l++) {
     Level &L = levels_[l];
-    launch_nodal_scale(L.n_elem, L.d_conn.p, L.dep_ptr.p, L.dep_conn.p, L.dep_w.p, L.xn.p,
+    launch_nodal_scale(L.n_elem, L.d_conn.p, L.dep4(), L.xn.p,
                        L.d_lev.p, mat_.q, mat_.k0, mat_.penalty_type,
                        l == 0 ? rho_gp_.p : nullptr, L.sg64.p, L.sg32.p, st_);
   }
@@ -2089,12 +2073,12 @@ int Problem::compliance_grad(double *g, bool on_device) {
   }
   Level &L = levels_[0];
   if (design_mode_ == 1) {
-    launch_nodal_energy(L.n_elem, L.d_conn.p, L.dep_ptr.p, L.dep_conn.p, L.dep_w.p, state_mask(),
+    launch_nodal_energy(L.n_elem, L.d_conn.p, L.dep4(), state_mask(),
                         L.d_cls.p, G64_.p, u_.p, u_.p, egp_.p, st_);
     return nodal_gather(nullptr, g, on_device);
   }
-  launch_elem_energy(L.n_elem, L.d_conn.p, L.dep_ptr.p, L.dep_conn.p, L.dep_w.p, state_mask(),
-                     L.d_cls.p, K0d_.p, u_.p, energy_.p, st_);
+  launch_elem_energy(L.n_elem, L.d_conn.p, L.dep4(), state_mask(),
+                     L.d_cls.p, R64_.p, u_.p, energy_.p, st_);
   double *out = g;
   DevArray<double> tmp;
   if (!on_device) {
@@ -2144,12 +2128,12 @@ int Problem::nodal_gather(const double *ex_gp, double *g, bool on_device) {
   return 0;
 }
 
-StressArgs Problem_stress_args(const Material &m, double P, const double *CB, const double *vol) {
+StressArgs Problem_stress_args(const Material &m, double P, const double *G, const double *vol) {
   StressArgs sa;
   sa.P = P;
   sa.eps = m.eps;
   sa.ys = m.ys;
-  sa.CB = CB;
+  sa.G = G;
   sa.vol = vol;
   return sa;
 }
@@ -2164,13 +2148,13 @@ int Problem::stress_pnorm(double P, double *f) {
     return -1;
   }
   Level &L = levels_[0];
-  const StressArgs sa = Problem_stress_args(mat_, P, CB_.p, cvol_.p);
+  const StressArgs sa = Problem_stress_args(mat_, P, G64_.p, cvol_.p);
   const int nb = (L.n_elem + 255) / 256;
   if ((size_t)nb > parts_.n) {
     last_error = "stress_pnorm: reduction buffer too small";
     return -1;
   }
-  launch_stress_sum(L.n_elem, L.d_conn.p, L.dep_ptr.p, L.dep_conn.p, L.dep_w.p, state_mask(),
+  launch_stress_sum(L.n_elem, L.d_conn.p, L.dep4(), state_mask(),
                     L.d_cls.p, L.d_lev.p, rho_.p, design_mode_ == 1 ? rho_gp_.p : nullptr, u_.p,
                     sa, parts_.p, st_);
   launch_finalize(nb, parts_.p, 4, sc_.p, st_);
@@ -2187,7 +2171,7 @@ int Problem::stress_pnorm_grad(double P, double *g, bool on_device, const SolveO
   double fval;
   if (stress_pnorm(P, &fval)) return -1;
   Level &L = levels_[0];
-  const StressArgs sa = Problem_stress_args(mat_, P, CB_.p, cvol_.p);
+  const StressArgs sa = Problem_stress_args(mat_, P, G64_.p, cvol_.p);
   // coef = S^(1/P - 1) into the scalar slot the gradient kernel reads
   const double coef = std::pow(last_stress_sum_, 1.0 / P - 1.0);
   HIPCHK(hipMemcpyAsync(sc_.p + SC_ZQ, &coef, sizeof(double), hipMemcpyHostToDevice, st_));
@@ -2209,12 +2193,12 @@ int Problem::stress_pnorm_grad(double P, double *g, bool on_device, const SolveO
   last_true_residual = tr;
   if (r != 0) return r < 0 ? -1 : 1;
   if (nodal) {
-    launch_nodal_energy(L.n_elem, L.d_conn.p, L.dep_ptr.p, L.dep_conn.p, L.dep_w.p, state_mask(),
+    launch_nodal_energy(L.n_elem, L.d_conn.p, L.dep4(), state_mask(),
                         L.d_cls.p, G64_.p, u_.p, psi_.p, egp_.p, st_);
     return nodal_gather(exgp_.p, g, on_device);
   }
-  launch_elem_energy2(L.n_elem, L.d_conn.p, L.dep_ptr.p, L.dep_conn.p, L.dep_w.p, state_mask(),
-                      L.d_cls.p, K0d_.p, u_.p, psi_.p, energy_.p, st_);
+  launch_elem_energy2(L.n_elem, L.d_conn.p, L.dep4(), state_mask(),
+                      L.d_cls.p, R64_.p, u_.p, psi_.p, energy_.p, st_);
   double *out = g;
   DevArray<double> tmp;
   if (!on_device) {

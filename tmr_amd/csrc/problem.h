@@ -134,8 +134,9 @@ struct Level {
   DevArray<int> wg_node_ptr, wg_nodes, wg_elem_ptr, wg_class;
   DevArray<uint16_t> lconn;
   DevArray<uint8_t> color, d_bcmask;
-  DevArray<int> dep_ptr, dep_conn, asm_ptr, asm_slot, d_conn, d_cls;
-  DevArray<float> dep_w, asm_w;
+  DevArray<int> d_dep4, asm_ptr, asm_slot, d_conn, d_cls;
+  DevArray<float> asm_w;
+  const int4 *dep4() const { return reinterpret_cast<const int4 *>(d_dep4.p); }
   DevArray<int16_t> d_lev;
   ElemBatches eb;
   AsmCSR asmc;
@@ -472,7 +473,7 @@ class Problem {
   int last_nrhs_ = 0;
   std::vector<double> seg_sc_;
   std::vector<int> seg_itc_, seg_act_;
-  DevArray<double> energy_, psi_, adjf_, dfdrho_, CB_, cvol_;
+  DevArray<double> energy_, psi_, adjf_, dfdrho_, cvol_;
   bool have_design_ = false, have_setup_ = false, have_solution_ = false;
   int setup_precision_ = -1;
   double last_setup_ms_ = 0.0;
