@@ -44,3 +44,22 @@ def test_product_over_tile_sizes_and_forms(name, tile, meshes):
         print("  form %d precision %d: %.2e" % (form, precision, e), flush=True)
         assert e < bound
     prob.set_fp32_form(0)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_product_in_place_and_overlapping_vectors(precision, meshes):
+    """Device vectors are used in place; y on top of x, or overlapping it,
+    gives the same values."""
+    import torch
+    prob, x, ref = meshes["adaptive"]
+    n = prob.ndof
+    buf = torch.zeros(2 * n, dtype=torch.float64, device="cuda")
+    want = torch.from_numpy(prob.apply(x, precision=precision)).cuda()
+    for a, b in ((0, n), (n, 0), (0, 0), (0, n // 2), (n // 2 + 1, 0)):
+        buf.zero_()
+        src, dst = buf[a:a + n], buf[b:b + n]
+        src.copy_(torch.from_numpy(x))
+        prob.apply(src, precision=precision, y=dst)
+        assert torch.equal(dst, want), (a, b)
+        if a + n <= b or b + n <= a:
+            assert np.array_equal(src.cpu().numpy(), x)

@@ -2348,23 +2348,44 @@ int Problem::apply(const double *x, double *y, bool on_device, int precision) {
     last_error = "apply: allocation failed";
     return -1;
   }
-  HIPCHK(hipMemcpyAsync(p_.p, x, n * sizeof(double),
-                        on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, st_));
+  // vectors on this device that do not overlap are read and written in place
+  // (3.0M dofs FP64 84 -> 68 us).  The tiles read neighbours' x, so an overlap
+  // goes through copies, and so does memory of another device, which only a
+  // copy may reach.
+  const uintptr_t xa = (uintptr_t)x, ya = (uintptr_t)y, bytes = n * sizeof(double);
+  int device = 0;
+  HIPCHK(hipGetDevice(&device));
+  auto own = [&](const void *v) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, v) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == device &&
+           (uintptr_t)v % alignof(double) == 0;
+  };
+  const bool direct = on_device && (xa + bytes <= ya || ya + bytes <= xa) && own(x) && own(y);
+  const double *in = direct ? x : p_.p;
+  double *out = direct ? y : q_.p;
+  if (!direct)
+    HIPCHK(hipMemcpyAsync(p_.p, x, n * sizeof(double),
+                          on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, st_));
   AsmArgs a;
   if (precision) {
     const bool keep = fp32_valu_;
     fp32_valu_ = precision == 2;
-    launch_convert<double, float>(n, p_.p, L.v32.b.p, st_);
+    launch_convert<double, float>(n, in, L.v32.b.p, st_);
     a.y = L.v32.r.p;
     apply_level<float>(0, L.v32.b.p, ASM_STORE, a);
     fp32_valu_ = keep;
-    launch_convert<float, double>(n, L.v32.r.p, q_.p, st_);
+    launch_convert<float, double>(n, L.v32.r.p, out, st_);
   } else {
-    a.y = q_.p;
-    apply_level<double>(0, p_.p, ASM_STORE, a);
+    a.y = out;
+    apply_level<double>(0, in, ASM_STORE, a);
   }
-  HIPCHK(hipMemcpyAsync(y, q_.p, n * sizeof(double),
-                        on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, st_));
+  if (!direct)
+    HIPCHK(hipMemcpyAsync(y, q_.p, n * sizeof(double),
+                          on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, st_));
   HIPCHK(hipStreamSynchronize(st_));
   return 0;
 }
