@@ -201,7 +201,7 @@ int Problem::build_coarse_plan() {
       m.off = na;
       pr.push_back({m.n, nb, na});
       na += (int64_t)padded(m.n) * padded(m.n);
-      tile0.push_back(tile0.back() + nb * nb);
+      tile0.push_back(tile0.back() + nb * (nb + 1) / 2);
     }
     cs.nprob = (int)pr.size();
     cs.active.clear();

@@ -9,10 +9,14 @@
 // of the Cholesky factorisation of an SPD matrix.  A step is one launch over
 // all blocks of all matrices, from one buffer to the other, and the
 // workgroup that produces block (k + 1, k + 1) also inverts it, so that a
-// matrix of nb blocks takes nb + 1 launches.  What bounds it at the sizes of
-// a coarse level is that chain: the 64 dependent pivots of a block (in
-// registers, one barrier each) and the launch, not the arithmetic (FP64
-// matrix cores).  It replaced blocked Cholesky, L^-1 and L^-T L^-1 (about
+// matrix of nb blocks takes nb + 1 launches.  On the way the block (j, i) is
+// the transpose of (i, j), or its negative where k lies between them, so only
+// the blocks of the lower triangle are computed and each is stored twice (a
+// step of 37 x 37 blocks 70 -> 51 us, of 31 x 31 blocks 53 -> 42), the next
+// pivot block in the first workgroup.  What bounds it at the sizes of a
+// coarse level is that chain: the 64 dependent pivots of a block (in
+// registers, one barrier each, 23 us) and the launch, not the arithmetic
+// (FP64 matrix cores).  It replaced blocked Cholesky, L^-1 and L^-T L^-1 (about
 // five launches a block column, 54 us of them for the diagonal factor in
 // LDS).
 //
@@ -173,12 +177,27 @@ __global__ __launch_bounds__(DT) void k_gj_step(int k, int nprob, const GJProb *
   __shared__ double sa[DB * LDA], sb[DB * LDB];
   const int q = find_prob(tile0, nprob, blockIdx.x);
   const GJProb p = pr[q];
-  const int nb = p.nblk, t = blockIdx.x - tile0[q], i = t / nb, j = t % nb;
+  const int nb = p.nblk;
+  // the block that goes on to the next inversion starts with the first wave
+  // of workgroups
+  int t = blockIdx.x - tile0[q];
+  if (k + 1 < nb) {
+    const int next = (k + 1) * (k + 4) / 2;
+    t = t == 0 ? next : t == next ? 0 : t;
+  }
+  int i = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
+  i += (i + 1) * (i + 2) / 2 <= t;
+  i -= i * (i + 1) / 2 > t;
+  const int j = t - i * (i + 1) / 2;
   const int64_t ld = DB * nb;
   const double *src = (((nb - k) & 1) ? A1 : A0) + p.off;
   double *dst = (((nb - k - 1) & 1) ? A1 : A0) + p.off;
   const double *P = dinv + (size_t)DB * DB * (2 * q + (k & 1));
   double *out = dst + (int64_t)DB * i * ld + DB * j;
+  // block (j, i) of the result: the negative of the transpose where one of
+  // the two block rows has been through its step and the other has not
+  double *mir = dst + (int64_t)DB * j * ld + DB * i;
+  const double sign = (i <= k) == (j <= k) ? 1.0 : -1.0;
   if (i == k && j == k) {
     for (int s = threadIdx.x; s < DB * DB; s += DT) out[(s >> 6) * ld + (s & 63)] = P[s];
     return;
@@ -201,8 +220,11 @@ __global__ __launch_bounds__(DT) void k_gj_step(int k, int nprob, const GJProb *
 #pragma unroll
       for (int v = 0; v < 2; v++)
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-          out[quad_row(u, e) * ld + quad_col(v)] = i == k ? acc[u][v][e] : -acc[u][v][e];
+        for (int e = 0; e < 4; e++) {
+          const double w = i == k ? acc[u][v][e] : -acc[u][v][e];
+          out[quad_row(u, e) * ld + quad_col(v)] = w;
+          mir[quad_col(v) * ld + quad_row(u, e)] = sign * w;
+        }
     return;
   }
   // A_ij - A_ik (P A_kj)
@@ -231,7 +253,10 @@ __global__ __launch_bounds__(DT) void k_gj_step(int k, int nprob, const GJProb *
 #pragma unroll
     for (int v = 0; v < 2; v++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) out[quad_row(u, e) * ld + quad_col(v)] = o[u][v][e];
+      for (int e = 0; e < 4; e++) {
+        out[quad_row(u, e) * ld + quad_col(v)] = o[u][v][e];
+        if (i != j) mir[quad_col(v) * ld + quad_row(u, e)] = sign * o[u][v][e];
+      }
   if (i != k + 1 || j != k + 1) return;
   __syncthreads();
 #pragma unroll
