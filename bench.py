@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark: solves/s and MDOF*iter/s of the multigrid-preconditioned FP64
 PCG on the 2 x 1 x 1 box cantilever (256 x 128 x 128 = 4,194,304 hex8,
-12,830,211 dofs, 6-level hierarchy, coarsest 8 x 4 x 4 by FP64 Cholesky),
+12,830,211 dofs, 6-level hierarchy, coarsest 8 x 4 x 4 by FP64 inverse),
 FP32 V-cycle (value) and FP64 V-cycle (comparison), to a 1e-8 relative
 residual.  One step = one solve K(rho) u = f from u = 0 with f and u resident
 in HBM; the density-dependent multigrid setup is timed separately.

@@ -337,7 +337,7 @@ void tmrx_problem_free(tmrx_problem *p);
      colour updates in parallel), not in TACS's row order: the smoother is
      the same SOR, its iterates follow that order.
    use_coarse_direct_solve: 1 solves the coarsest level directly (FP64
-     Cholesky, TACSMg's direct solve, :83-86); 0 smooths it like the other
+     inverse, TACSMg's direct solve, :83-86); 0 smooths it like the other
      levels, one Chebyshev sweep of cheb_degree steps from zero (the
      smoother TMR hands TACSMg there, :87-102).
    omega: the SOR relaxation factor, in (0, 2) (unused by Chebyshev).
@@ -392,7 +392,7 @@ int tmrx_problem_level_design(tmrx_problem *p, int level, double *x);
    gradient then use the full u (-u^T dK/drho u, as TMR's compliance branch). */
 int tmrx_problem_set_bc_values(tmrx_problem *p, const double *ubc, int n, int on_device);
 /* Density-dependent multigrid setup (diagonals, eigenvalue bounds, coarse
-   Cholesky): mg->assembleJacobian + mg->factor
+   inverse): mg->assembleJacobian + mg->factor
    (src/topology/TMRTopoProblem.cpp:1000-1001). */
 int tmrx_problem_setup(tmrx_problem *p, const tmrx_solve_opts *opts);
 /* K(rho) u = f by FP64 flexible PCG with one multigrid V-cycle as the

@@ -204,9 +204,8 @@ void launch_elem_diag(const ElemBatches &eb, const T *K0, const T *s_elem, T *pa
 void launch_diag_cross(int n, const int *ptr, const int *node, const int *code, const double *w,
                        const int *cls, const double *K0, const double *s, bool nodal,
                        const uint8_t *bcmask, double *dinv, hipStream_t st);
-template <class T>
-void launch_assemble(const AsmCSR &a, const uint8_t *bcmask, const T *partial, int mode,
-                     const AsmArgs &args, hipStream_t st);
+void launch_assemble(const AsmCSR &a, const uint8_t *bcmask, const double *partial, int mode,
+                     double *y, hipStream_t st);
 int assemble_num_blocks(int n_nodes);
 
 template <class T>
@@ -397,14 +396,8 @@ void launch_take_comp0(int n, const double *in, double *out, hipStream_t st);
 // SC_XIT: the iteration whose alpha p is still to be added to x (-1: none)
 enum { SC_RZ = 0, SC_PQ, SC_ALPHA, SC_RR, SC_ZQ, SC_BETA, SC_BB, SC_RZNEW, SC_TRR, SC_XIT, SC_N };
 int reduce_blocks(int64_t n);
-void launch_pcg_update_xr(int64_t ndof, double *x, double *r, const double *p, const double *q,
-                          const double *sc, double *partials, float *r32, hipStream_t st);
-void launch_dot2(int64_t ndof, const double *z, const double *r, const double *q,
-                 double *partials, hipStream_t st);
 void launch_dot1(int64_t ndof, const double *a, const double *b, double *partials,
                  hipStream_t st);
-void launch_pcg_update_p(int64_t ndof, double *p, const double *z, const double *sc,
-                         hipStream_t st);
 void launch_dinv_dots(int64_t n, const double *dinv, double *y, const double *x,
                       double *partials, hipStream_t st);
 // finalize: mode 0 rz, 1 pq->alpha, 2 rr, 3 (zr, zq)->beta, 4 bb,

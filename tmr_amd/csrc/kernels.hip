@@ -215,7 +215,8 @@ void launch_diag_cross(int n, const int *ptr, const int *node, const int *code, 
 }
 
 // ---------------------------------------------------------------------------
-// assembly pass: node-parallel weighted gather of slot partials + epilogue
+// assembly pass: node-parallel weighted gather of slot partials (ASM_GATHER)
+// or the inverse of the diagonal (ASM_DIAG, weights squared)
 constexpr int NODE_BLOCK = 256;
 
 __device__ __forceinline__ double block_sum(double v, double *red) {
@@ -230,85 +231,37 @@ __device__ __forceinline__ double block_sum(double v, double *red) {
   return s;
 }
 
-template <class T, int MODE>
+template <int MODE>
 __global__ __launch_bounds__(NODE_BLOCK) void k_assemble(
     int n, const int *__restrict__ ptr, const int *__restrict__ slot, const float *__restrict__ w,
-    const uint8_t *__restrict__ bcmask, const T *__restrict__ partial, const T *__restrict__ b,
-    T *__restrict__ y, T *__restrict__ x, T *__restrict__ d, const T *__restrict__ dinv,
-    const double *__restrict__ cf, double *__restrict__ partials) {
-  const double ca = MODE == ASM_CHEB ? cf[0] : 0.0, cc = MODE == ASM_CHEB ? cf[1] : 0.0;
-  __shared__ double red[NODE_BLOCK / 64];
+    const uint8_t *__restrict__ bcmask, const double *__restrict__ partial,
+    double *__restrict__ y) {
   const int i = xcd_block(blockIdx.x, gridDim.x) * NODE_BLOCK + threadIdx.x;
-  double dot = 0.0;
-  if (i < n) {
-    T a0 = T(0), a1 = T(0), a2 = T(0);
-    for (int j = ptr[i]; j < ptr[i + 1]; j++) {
-      const int s = slot[j];
-      T ww = (T)w[j];
-      if (MODE == ASM_DIAG) ww = ww * ww;
-      a0 += ww * partial[3 * s];
-      a1 += ww * partial[3 * s + 1];
-      a2 += ww * partial[3 * s + 2];
-    }
-    const uint8_t m = bcmask[i];
-    const T acc[3] = {a0, a1, a2};
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      const int k = 3 * i + c;
-      const bool bc = (m >> c) & 1;
-      if (MODE == ASM_STORE) {
-        y[k] = bc ? x[k] : acc[c];
-      } else if (MODE == ASM_DOT) {
-        const T v = bc ? x[k] : acc[c];
-        y[k] = v;
-        dot += (double)x[k] * (double)v;
-      } else if (MODE == ASM_RESID) {
-        y[k] = bc ? T(0) : b[k] - acc[c];
-      } else if (MODE == ASM_CHEB) {
-        if (bc) {
-          d[k] = T(0);
-          x[k] = T(0);
-        } else {
-          const T r = b[k] - acc[c];
-          const T dn = (T)ca * d[k] + (T)cc * dinv[k] * r;
-          d[k] = dn;
-          x[k] += dn;
-        }
-      } else if (MODE == ASM_DIAG) {
-        y[k] = bc ? T(1) : T(1) / acc[c];
-      } else if (MODE == ASM_GATHER) {
-        y[k] = bc ? T(0) : acc[c];
-      }
-    }
+  if (i >= n) return;
+  double acc[3] = {};
+  for (int j = ptr[i]; j < ptr[i + 1]; j++) {
+    const int s = slot[j];
+    double ww = w[j];
+    if (MODE == ASM_DIAG) ww = ww * ww;
+    for (int c = 0; c < 3; c++) acc[c] += ww * partial[3 * s + c];
   }
-  if (MODE == ASM_DOT) {
-    const double s = block_sum(dot, red);
-    if (threadIdx.x == 0) partials[blockIdx.x] = s;
+  const uint8_t m = bcmask[i];
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    const bool bc = (m >> c) & 1;
+    y[3 * i + c] = MODE == ASM_DIAG ? (bc ? 1.0 : 1.0 / acc[c]) : (bc ? 0.0 : acc[c]);
   }
 }
 
 int assemble_num_blocks(int n_nodes) { return (n_nodes + NODE_BLOCK - 1) / NODE_BLOCK; }
 
-template <class T>
-void launch_assemble(const AsmCSR &a, const uint8_t *bcmask, const T *partial, int mode,
-                     const AsmArgs &g, hipStream_t st) {
+void launch_assemble(const AsmCSR &a, const uint8_t *bcmask, const double *partial, int mode,
+                     double *y, hipStream_t st) {
   const int nb = assemble_num_blocks(a.n_nodes);
   if (nb == 0) return;
-  const T *b = (const T *)g.b;
-  T *y = (T *)g.y, *x = (T *)g.x, *d = (T *)g.d;
-  const T *dinv = (const T *)g.dinv;
-#define TMRX_ASM(M)                                                                           \
-  hipLaunchKernelGGL((k_assemble<T, M>), dim3(nb), dim3(NODE_BLOCK), 0, st, a.n_nodes, a.ptr, \
-                     a.slot, a.w, bcmask, partial, b, y, x, d, dinv, (const double *)g.cf, g.partials)
-  switch (mode) {
-    case ASM_STORE: TMRX_ASM(ASM_STORE); break;
-    case ASM_RESID: TMRX_ASM(ASM_RESID); break;
-    case ASM_CHEB: TMRX_ASM(ASM_CHEB); break;
-    case ASM_DIAG: TMRX_ASM(ASM_DIAG); break;
-    case ASM_DOT: TMRX_ASM(ASM_DOT); break;
-    case ASM_GATHER: TMRX_ASM(ASM_GATHER); break;
-  }
-#undef TMRX_ASM
+  const auto kern = mode == ASM_DIAG ? k_assemble<ASM_DIAG> : k_assemble<ASM_GATHER>;
+  hipLaunchKernelGGL(kern, dim3(nb), dim3(NODE_BLOCK), 0, st, a.n_nodes, a.ptr, a.slot, a.w, bcmask,
+                     partial, y);
   TMRX_LAUNCH_CHECK();
 }
 
@@ -962,62 +915,6 @@ int reduce_blocks(int64_t n) {
   return (int)(b < RED_MAX_BLOCKS ? (b < 1 ? 1 : b) : RED_MAX_BLOCKS);
 }
 
-__global__ __launch_bounds__(RED_BLOCK) void k_pcg_update_xr(int64_t n, double *__restrict__ x,
-                                                             double *__restrict__ r,
-                                                             const double *__restrict__ p,
-                                                             const double *__restrict__ q,
-                                                             const double *__restrict__ sc,
-                                                             double *__restrict__ partials,
-                                                             float *__restrict__ r32) {
-  __shared__ double red[RED_BLOCK / 64];
-  const double alpha = sc[SC_ALPHA];
-  double acc = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * RED_BLOCK + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * RED_BLOCK) {
-    x[i] += alpha * p[i];
-    const double rn = r[i] - alpha * q[i];
-    r[i] = rn;
-    if (r32) r32[i] = (float)rn;
-    acc += rn * rn;
-  }
-  const double s = block_sum(acc, red);
-  if (threadIdx.x == 0) partials[blockIdx.x] = s;
-}
-
-void launch_pcg_update_xr(int64_t ndof, double *x, double *r, const double *p, const double *q,
-                          const double *sc, double *partials, float *r32, hipStream_t st) {
-  hipLaunchKernelGGL(k_pcg_update_xr, dim3(reduce_blocks(ndof)), dim3(RED_BLOCK), 0, st, ndof, x, r,
-                     p, q, sc, partials, r32);
-  TMRX_LAUNCH_CHECK();
-}
-
-__global__ __launch_bounds__(RED_BLOCK) void k_dot2(int64_t n, const double *__restrict__ z,
-                                                    const double *__restrict__ r,
-                                                    const double *__restrict__ q,
-                                                    double *__restrict__ partials) {
-  __shared__ double red[RED_BLOCK / 64];
-  double a = 0.0, b = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * RED_BLOCK + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * RED_BLOCK) {
-    a += z[i] * r[i];
-    b += z[i] * q[i];
-  }
-  const double sa = block_sum(a, red);
-  __syncthreads();
-  const double sb = block_sum(b, red);
-  if (threadIdx.x == 0) {
-    partials[2 * blockIdx.x] = sa;
-    partials[2 * blockIdx.x + 1] = sb;
-  }
-}
-
-void launch_dot2(int64_t ndof, const double *z, const double *r, const double *q,
-                 double *partials, hipStream_t st) {
-  hipLaunchKernelGGL(k_dot2, dim3(reduce_blocks(ndof)), dim3(RED_BLOCK), 0, st, ndof, z, r, q,
-                     partials);
-  TMRX_LAUNCH_CHECK();
-}
-
 __global__ __launch_bounds__(RED_BLOCK) void k_dot1(int64_t n, const double *__restrict__ a,
                                                     const double *__restrict__ b,
                                                     double *__restrict__ partials) {
@@ -1034,21 +931,6 @@ void launch_dot1(int64_t ndof, const double *a, const double *b, double *partial
                  hipStream_t st) {
   hipLaunchKernelGGL(k_dot1, dim3(reduce_blocks(ndof)), dim3(RED_BLOCK), 0, st, ndof, a, b,
                      partials);
-  TMRX_LAUNCH_CHECK();
-}
-
-__global__ void k_pcg_update_p(int64_t n, double *__restrict__ p, const double *__restrict__ z,
-                               const double *__restrict__ sc) {
-  const double beta = sc[SC_BETA];
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = z[i] + beta * p[i];
-}
-
-void launch_pcg_update_p(int64_t ndof, double *p, const double *z, const double *sc,
-                         hipStream_t st) {
-  hipLaunchKernelGGL(k_pcg_update_p, dim3(reduce_blocks(ndof)), dim3(RED_BLOCK), 0, st, ndof, p, z,
-                     sc);
   TMRX_LAUNCH_CHECK();
 }
 
@@ -2554,8 +2436,6 @@ void launch_adjoint_grad(int n, const double *rho, const int16_t *lev, double q,
 #define TMRX_INST(T)                                                                            \
   template void launch_elem_diag<T>(const ElemBatches &, const T *, const T *, T *,             \
                                     hipStream_t, bool);                                         \
-  template void launch_assemble<T>(const AsmCSR &, const uint8_t *, const T *, int,             \
-                                   const AsmArgs &, hipStream_t);                               \
   template void launch_prolong_add<T>(const TransferCSR &, const uint8_t *, const T *, T *,     \
                                       hipStream_t, int, int64_t, int64_t);                      \
   template void launch_restrict<T>(const TransferCSR &, const uint8_t *, const T *, T *,        \

@@ -1492,9 +1492,7 @@ int Problem::setup(const SolveOpts &o) {
       launch_elem_diag<double>(L.eb, G64_.p, L.sg64.p, L.v64.partial.p, st_, true);
     else
       launch_elem_diag<double>(L.eb, K0d_.p, L.s64.p, L.v64.partial.p, st_);
-    AsmArgs a;
-    a.y = L.v64.dinv.p;
-    launch_assemble<double>(L.asmc, L.d_bcmask.p, L.v64.partial.p, ASM_DIAG, a, st_);
+    launch_assemble(L.asmc, L.d_bcmask.p, L.v64.partial.p, ASM_DIAG, L.v64.dinv.p, st_);
     launch_diag_cross(L.n_xd, L.xd_ptr.p, L.xd_node.p, L.xd_code.p, L.xd_w.p, L.d_cls.p,
                       design_mode_ == 1 ? G64_.p : K0d_.p,
                       design_mode_ == 1 ? L.sg64.p : L.s64.p, design_mode_ == 1,
@@ -2109,9 +2107,7 @@ int Problem::nodal_gather(const double *ex_gp, double *g, bool on_device) {
   }
   launch_nodal_grad(L.eb, L.d_lev.p, rho_gp_.p, mat_.q, mat_.penalty_type, egp_.p, ex_gp,
                     L.v64.partial.p, st_);
-  AsmArgs a;
-  a.y = gtmp_.p;
-  launch_assemble<double>(L.asmc, nomask_.p, L.v64.partial.p, ASM_GATHER, a, st_);
+  launch_assemble(L.asmc, nomask_.p, L.v64.partial.p, ASM_GATHER, gtmp_.p, st_);
   double *out = g;
   DevArray<double> tmp;
   if (!on_device) {
@@ -2180,9 +2176,7 @@ int Problem::stress_pnorm_grad(double P, double *g, bool on_device, const SolveO
   eb.bcmask = state_mask();
   launch_stress_grad(eb, L.d_lev.p, L.d_cls.p, rho_.p, nodal ? rho_gp_.p : nullptr, u_.p, sa,
                      sc_.p, L.v64.partial.p, nodal ? exgp_.p : dfdrho_.p, st_);
-  AsmArgs a;
-  a.y = adjf_.p;
-  launch_assemble<double>(L.asmc, L.d_bcmask.p, L.v64.partial.p, ASM_GATHER, a, st_);
+  launch_assemble(L.asmc, L.d_bcmask.p, L.v64.partial.p, ASM_GATHER, adjf_.p, st_);
   HIPCHK(hipStreamSynchronize(st_));
   // adjoint K psi = df/du (K symmetric); u_ and f_ are left untouched
   const double tr = last_true_residual;

@@ -322,7 +322,7 @@ class Mg:
     smoother is TMR's default symmetric SOR with relaxation ``omega`` on
     the assembled level matrices (``use_chebyshev_smoother=False``, swept in
     colour-major node order), or Chebyshev on the Jacobi-scaled operator;
-    the coarsest level is a direct FP64 Cholesky solve, or with
+    the coarsest level is a direct FP64 solve, or with
     ``use_coarse_direct_solve=False`` the level's smoother once (TMR hands
     TACSMg the smoother there, src/TMR_RefinementTools.cpp:87-102)."""
 
