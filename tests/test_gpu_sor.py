@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import pyoracle as po
-from tmr_amd import solver, workloads
+from tmr_amd import TMR, solver, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -106,6 +106,36 @@ def test_sor_rediscretised_finest(hier):
     assert es < 1e-12
     with pytest.raises(Exception):
         prob.smoother_order(len(forests) - 1)  # the coarsest level is solved directly
+
+
+# node grids 3^3, 7 x 7 x 3, 7 x 5 x 5 and 7^3: every colour (8 and 32 nodes
+# at most), all but the first (27 after 36) or only the last one (27 after 36)
+# runs in the one-workgroup tail of the sweep
+@pytest.mark.parametrize("blocks", [(1, 1, 1), (3, 3, 1), (3, 2, 2), (3, 3, 3)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_sor_small_last_colours(blocks, precision):
+    f = TMR.createBoxForest(*blocks, tuple(float(b) for b in blocks),
+                            face_names=workloads.FACES)
+    f.createTrees(1)
+    forests = workloads.hierarchy(f, 2)
+    rho = np.random.default_rng(2).uniform(0.1, 1.0, len(forests[0].getOctants()))
+    orc = po.from_forest(forests[0], BCS)
+    orc.assemble(rho ** Q + K0)
+    mg = po.Multigrid(orc, forests, BCS)
+    mg.setup("sor", omega=0.9)
+    free = _free(mg.masks[0])
+    prob = solver.Problem(forests, q=Q, k0=K0, bcs=BCS)
+    prob.set_multigrid(use_chebyshev_smoother=False, omega=0.9)
+    prob.set_design(rho)
+    opts = solver.default_opts(precision=precision)
+    prob.mg_op("apply", 0, np.zeros(len(free)), opts)
+    nodes, cptr = prob.smoother_order(0)
+    print("colours of %s nodes" % np.diff(cptr), flush=True)
+    mg.set_order(0, nodes)
+    b = np.where(free, np.random.default_rng(7).standard_normal(len(free)), 0.0)
+    y, _ = prob.mg_op("smooth", 0, b, opts)
+    # two sweeps of at most 81 products a row, rounding of the precision each
+    assert _rel(y, mg.op("smooth", 0, b)) < (1e-12 if precision == 0 else 1e-5)
 
 
 @pytest.mark.parametrize("galerkin", [False, True])

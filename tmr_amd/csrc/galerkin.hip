@@ -327,6 +327,8 @@ void launch_bsr_apply(const BSR<T> &A, const T *x, int mode, const AsmArgs &g, h
 }
 
 // ---------------------------------------------------------------------------
+constexpr int SOR_TAIL_MAX = 8, SOR_TAIL_ROWS = 32;
+
 // One colour of a point SOR sweep on the BSR matrix (TACSGaussSeidel's
 // smoother, symmetric SOR with relaxation omega; TMR_CreateTACSMg,
 // src/TMR_RefinementTools.cpp:93-94).  The matrix is the level's BSR with
@@ -346,24 +348,12 @@ void launch_bsr_apply(const BSR<T> &A, const T *x, int mode, const AsmArgs &g, h
 // once or twice.  32 lanes are taken until they fill the chip (32,858-node
 // adaptive level, 2,200 rows a colour: 6.9 -> 4.9 us a launch; one colour of
 // 3,058 nodes 5.3 -> 4.1); beyond, 8 lanes leave fewer idle.
+
+// row i (blocks q0 .. q1) on lane `sub` of its LANES
 template <class T, int DIR, int LANES>
-__global__ __launch_bounds__(256) void k_sor_colour(int cnt, const int *__restrict__ nodes,
-                                                    const int *__restrict__ ptr,
-                                                    const int *__restrict__ col,
-                                                    const T *__restrict__ val,
-                                                    const T *__restrict__ b, T *__restrict__ x,
-                                                    T omega, const int *__restrict__ run,
-                                                    int64_t vs) {
-  const int go = run ? *run : 1;
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  const int k = g / LANES, sub = g % LANES;
-  const bool valid = k < cnt;
-  const int64_t off = (int64_t)blockIdx.y * vs;
-  x += off;
-  b += off;
-  const int kk = valid ? k : 0;
-  const int i = nodes[kk], q0 = ptr[kk], q1 = ptr[kk + 1];
-  if (go == 0) return;
+__device__ __forceinline__ void sor_row(bool valid, int sub, int i, int q0, int q1,
+                                        const int *__restrict__ col, const T *__restrict__ val,
+                                        const T *__restrict__ b, T *x, T omega) {
   const size_t i3 = 3 * (size_t)i;
   T xi[3] = {T(0), T(0), T(0)}, bi[3] = {T(0), T(0), T(0)};
   if (valid && sub == 0) {
@@ -436,6 +426,63 @@ __global__ __launch_bounds__(256) void k_sor_colour(int cnt, const int *__restri
   for (int c = 0; c < 3; c++) x[i3 + c] = xi[c];
 }
 
+template <class T, int DIR, int LANES>
+__global__ __launch_bounds__(256) void k_sor_colour(int cnt, const int *__restrict__ nodes,
+                                                    const int *__restrict__ ptr,
+                                                    const int *__restrict__ col,
+                                                    const T *__restrict__ val,
+                                                    const T *__restrict__ b, T *__restrict__ x,
+                                                    T omega, const int *__restrict__ run,
+                                                    int64_t vs) {
+  const int go = run ? *run : 1;
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = g / LANES, sub = g % LANES;
+  const bool valid = k < cnt;
+  const int64_t off = (int64_t)blockIdx.y * vs;
+  const int kk = valid ? k : 0;
+  const int i = nodes[kk], q0 = ptr[kk], q1 = ptr[kk + 1];
+  if (go == 0) return;
+  sor_row<T, DIR, LANES>(valid, sub, i, q0, q1, col, val, b + off, x + off, omega);
+}
+
+// The last colours of a sweep, forward, the turn and backward, in one
+// workgroup per right-hand side with a barrier in place of a launch between
+// colours.  Greedy colouring leaves a few colours of a few nodes at the end
+// (hanging corners make cliques), and each was a launch of 4.3 us for one or
+// two rounds of loads.  SOR_TAIL_ROWS is one round of 32 lanes a row: a round
+// takes about 2.3 us, so a second one costs what the launch did (adaptive
+// 50k hex, 22 iterations: 22.8 ms with launches alone, 22.1 with 32 or 64
+// rows, 22.5 with 96).
+struct SorTail {
+  int n, ptr[SOR_TAIL_MAX + 1];  // rows of the n last colours
+};
+template <class T, int DIR>
+__device__ __forceinline__ void sor_tail_colour(int r0, int r1, const int *__restrict__ nodes,
+                                                const int *__restrict__ ptr,
+                                                const int *__restrict__ col,
+                                                const T *__restrict__ val,
+                                                const T *__restrict__ b, T *x, T omega) {
+  for (int r = r0 + (threadIdx.x >> 5); r < r1; r += 32)
+    sor_row<T, DIR, 32>(true, threadIdx.x & 31, nodes[r], ptr[r], ptr[r + 1], col, val, b, x, omega);
+  __syncthreads();
+}
+template <class T>
+__global__ __launch_bounds__(1024) void k_sor_tail(SorTail t, const int *__restrict__ nodes,
+                                                   const int *__restrict__ ptr,
+                                                   const int *__restrict__ col,
+                                                   const T *__restrict__ val,
+                                                   const T *__restrict__ b, T *x, T omega,
+                                                   const int *__restrict__ run, int64_t vs) {
+  if (run && *run == 0) return;
+  b += (int64_t)blockIdx.y * vs;
+  x += (int64_t)blockIdx.y * vs;
+  for (int c = 0; c + 1 < t.n; c++)
+    sor_tail_colour<T, 0>(t.ptr[c], t.ptr[c + 1], nodes, ptr, col, val, b, x, omega);
+  sor_tail_colour<T, 2>(t.ptr[t.n - 1], t.ptr[t.n], nodes, ptr, col, val, b, x, omega);
+  for (int c = t.n - 2; c >= 0; c--)
+    sor_tail_colour<T, 1>(t.ptr[c], t.ptr[c + 1], nodes, ptr, col, val, b, x, omega);
+}
+
 // val_out[k] = val[map[k]] for every 3 x 3 block (the colour-major copy)
 __global__ void k_bsr_gather(int nnzb, const int *__restrict__ map, const double *__restrict__ val,
                              double *__restrict__ out) {
@@ -473,12 +520,23 @@ static void sor_colour(const BSR<T> &A, const int *nodes, int c0, int cnt, const
 template <class T>
 void launch_sor_symmetric(const BSR<T> &A, const int *nodes, const int *cptr, int ncolors,
                           const T *b, T *x, double omega, hipStream_t st, int nrhs, int64_t vs) {
-  for (int c = 0; c + 1 < ncolors; c++)
+  if (ncolors == 0) return;
+  // colours from t0 on go to the one-workgroup form
+  int t0 = ncolors;
+  while (t0 > 0 && ncolors - t0 < SOR_TAIL_MAX && cptr[t0] - cptr[t0 - 1] <= SOR_TAIL_ROWS) t0--;
+  if (t0 > ncolors - 2) t0 = ncolors - 1;  // the turn alone
+  for (int c = 0; c < t0; c++)
     sor_colour<T, 0>(A, nodes, cptr[c], cptr[c + 1] - cptr[c], b, x, omega, st, nrhs, vs);
-  if (ncolors > 0)
-    sor_colour<T, 2>(A, nodes, cptr[ncolors - 1], cptr[ncolors] - cptr[ncolors - 1], b, x, omega,
-                     st, nrhs, vs);
-  for (int c = ncolors - 2; c >= 0; c--)
+  if (t0 == ncolors - 1) {
+    sor_colour<T, 2>(A, nodes, cptr[t0], cptr[t0 + 1] - cptr[t0], b, x, omega, st, nrhs, vs);
+  } else {
+    SorTail t{ncolors - t0, {}};
+    for (int c = 0; c <= t.n; c++) t.ptr[c] = cptr[t0 + c];
+    hipLaunchKernelGGL(k_sor_tail<T>, dim3(1, (unsigned)nrhs), dim3(1024), 0, st, t, nodes, A.ptr,
+                       A.col, A.val, b, x, (T)omega, A.run, vs);
+    TMRX_LAUNCH_CHECK();
+  }
+  for (int c = t0 - 1; c >= 0; c--)
     sor_colour<T, 1>(A, nodes, cptr[c], cptr[c + 1] - cptr[c], b, x, omega, st, nrhs, vs);
 }
 
