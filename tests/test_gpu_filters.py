@@ -75,6 +75,28 @@ def test_filter_matches_oracle(adapt, kind, r, N):
     free()
 
 
+# the squared tolerance of the conjugate gradients underflows for the smaller
+# two, |rhs|^2 does not
+@pytest.mark.parametrize("norm", [1e-100, 1e-151, 1e-153])
+def test_helmholtz_of_tiny_vectors(adapt, norm):
+    """The filter is linear: a tiny right-hand side gives a tiny solution,
+    not zero; a zero one gives zero."""
+    forest, M, K = adapt
+    run, iters, free = _native(forest, 0, 0.1)
+    y = np.random.default_rng(3).standard_normal(M.shape[0])
+    y *= norm / np.linalg.norm(y)          # the transpose's right-hand side
+    ref = po.helmholtz_filter(M, K, 0.1, y / norm, transpose=True)
+    out = run(y, transpose=True) / norm
+    e = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    print("|rhs| %.0e: rel err %.2e, CG its %d" % (norm, e, iters()), flush=True)
+    # a residual below 1.6e-162 squares to zero and stops the iteration; 1e3
+    # for the condition number between residual and error
+    assert e < max(1e-10, 1e3 * 1.6e-162 / norm)
+    assert iters() > 0
+    assert not run(np.zeros_like(y)).any() and iters() == 0
+    free()
+
+
 def _mfilter(assemblers, filters):
     mf = TopOptUtils.Mfilter(4, assemblers, filters, dim=3, r=0.15)
     mf.initialize()

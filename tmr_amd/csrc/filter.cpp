@@ -266,12 +266,15 @@ int Filter::helmholtz_solve(const double *rhs, double *x) {
   int h[2] = {0, 0};
   double tol2 = 0.0;
   if (hipMemcpyAsync(&tol2, sc_.p + 2, sizeof(double), hipMemcpyDeviceToHost, st_) != hipSuccess ||
+      hipMemcpyAsync(h, flag_.p, sizeof(h), hipMemcpyDeviceToHost, st_) != hipSuccess ||
       hipStreamSynchronize(st_) != hipSuccess || !(tol2 == tol2)) {
     last_error = "filter: device error";
     return -1;
   }
   iters_ = 0;
-  if (tol2 == 0.0) return 0;
+  // set for a zero right-hand side only (the tolerance underflows to zero
+  // from |rhs| of about 1e-150, whose solution is not zero)
+  if (h[0]) return 0;
   for (int it = 1; it <= 2000;) {
     for (int k = 0; k < 8 && it <= 2000; k++, it++)
       launch_filter_cg_iteration(n_, it, ptr_.p, col_.p, aval_.p, dinv_.p, x, r, p, q, parts_.p,
