@@ -97,6 +97,29 @@ def test_helmholtz_of_tiny_vectors(adapt, norm):
     free()
 
 
+@pytest.mark.parametrize("blocks,level", [((1, 1, 1), 1), ((3, 2, 2), 3), ((3, 1, 1), 5)])
+def test_helmholtz_over_grid_sizes(blocks, level):
+    """One workgroup with most of its threads idle, a few, and more rows than
+    the grid holds at once: the stop of an iteration reaches every block, so
+    repeated solves agree bit for bit with equal iteration counts."""
+    forest = TMR.createBoxForest(*blocks, tuple(float(b) for b in blocks), face_names=FACES)
+    forest.createTrees(level)
+    forest.balance(1)
+    forest.createNodes()
+    M, K = po.scalar_mass_laplacian(forest)
+    run, iters, free = _native(forest, 0, 0.1)
+    x = np.random.default_rng(level).random(M.shape[0])
+    out = run(x)
+    its = iters()
+    rhs = M @ x
+    e = np.linalg.norm(M @ out + 0.01 * (K @ out) - rhs) / np.linalg.norm(rhs)
+    print("%d nodes, CG its %d, residual %.2e" % (len(x), its, e), flush=True)
+    assert e < 1e-11  # stops at 1e-12 of the recursive residual
+    for _ in range(5):
+        assert np.array_equal(run(x), out) and iters() == its
+    free()
+
+
 def _mfilter(assemblers, filters):
     mf = TopOptUtils.Mfilter(4, assemblers, filters, dim=3, r=0.15)
     mf.initialize()

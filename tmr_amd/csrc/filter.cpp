@@ -145,7 +145,7 @@ int Filter::init(Forest *f, int kind, double r, int nterms) {
       dinv_.upload(dinv) || ascale_.upload(a) || bscale_.upload(b) || tinv_.alloc(n_) ||
       w1_.alloc(n_) || w2_.alloc(n_) || w3_.alloc(n_) || w4_.alloc(n_) || w5_.alloc(n_) ||
       in_.alloc(n_) || out_.alloc(n_) || parts_.alloc(filter_cg_parts()) ||
-      sc_.alloc(3) || flag_.alloc(2)) {
+      sc_.alloc(3) || flag_.alloc(3)) {
     last_error = "filter: device allocation failed";
     return -1;
   }

@@ -52,7 +52,7 @@ void launch_filter_add(int n, const double *t, double *y, hipStream_t st);
 // y[i] = 1 / x[i] (0 where x is 0)
 void launch_filter_recip(int n, const double *x, double *y, hipStream_t st);
 // conjugate gradients on the device (parts: filter_cg_parts() words, sc: 3,
-// flag: converged, iterations)
+// flag: 3 words, converged, iterations, one of the kernels' own)
 int filter_cg_parts();
 void launch_filter_cg_init(int n, const double *rhs, const double *dinv, double *x, double *r,
                            double *p, double *parts, double rtol2, double *sc, int *flag,

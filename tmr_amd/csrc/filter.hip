@@ -61,7 +61,10 @@ void launch_filter_spmv(int n, const int *ptr, const int *col, const double *val
 // back, an iteration took three round trips (9,537 nodes: 130 us, now 12).
 // At most FCG_BLOCKS blocks, each over a contiguous chunk, so that the sums
 // stay short; st: [0..1] r.z of the iterations in turn, [2] tolerance;
-// flag[0] set when converged, flag[1] the iterations done.
+// flag[0] set when converged, flag[1] the iterations done, flag[2] what
+// flag[0] was before the direction launch.  That launch sets flag[0] in one
+// block and tests flag[2]: blocks that tested the word it sets could lose some
+// of their waves before a barrier that the others wait at.
 constexpr int FCG_BLOCKS = 1024;
 int filter_cg_blocks(int n) {
   const int64_t b = ((int64_t)n + FB - 1) / FB;
@@ -120,6 +123,7 @@ __global__ __launch_bounds__(FB) void k_fcg_start(int np, const double *__restri
     st[2] = rtol2 * bb;
     flag[0] = bb == 0.0 ? 1 : 0;
     flag[1] = 0;
+    flag[2] = 0;
   }
 }
 
@@ -156,9 +160,11 @@ __global__ __launch_bounds__(FB) void k_fcg_step(int n, int chunk, int it, int n
                                                  double *__restrict__ x, double *__restrict__ r,
                                                  const double *__restrict__ st,
                                                  double *__restrict__ parts,
-                                                 const int *__restrict__ flag) {
+                                                 int *__restrict__ flag) {
   __shared__ double red[FB / 64];
-  if (flag[0]) return;
+  const bool stop = flag[0] != 0;
+  if (stop && blockIdx.x == 0 && threadIdx.x == 0) flag[2] = 1;
+  if (stop) return;
   const double alpha = st[it & 1] / fparts(npq, pq, 1, 0, red);
   const int lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
   double a = 0.0, b = 0.0;
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(FB) void k_fcg_direction(int n, int chunk, int it, 
                                                       double *__restrict__ st,
                                                       int *__restrict__ flag) {
   __shared__ double red[FB / 64];
-  if (flag[0]) return;
+  if (flag[2]) return;
   const double rr = fparts(np, parts, 2, 0, red), rz = fparts(np, parts, 2, 1, red);
   const bool done = rr <= st[2];
   const double beta = rz / st[it & 1];
