@@ -48,6 +48,40 @@ def test_multi_rhs_bit_identical_to_single(adapt, precision, no_graph):
         assert prob.true_residual() < 1e-9
 
 
+# 65,536 hex, 70,785 nodes.  64-node tiles (1,107): above the finest level's
+# rule for fused dot products alone and with more cases; 128-node tiles (554):
+# below it alone, four cases beyond it together
+@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_batch_does_not_change_a_case(box65k, precision, tile):
+    _batch_against_single(box65k, precision, tile)
+
+
+@pytest.fixture(scope="module")
+def box65k():
+    forests, rho, L = workloads.box(level=5, nlevels=4, seed=3)
+    prob = solver.Problem(forests, q=Q, k0=K0, bcs=BCS)
+    prob.set_design(rho)
+    return prob
+
+
+def _batch_against_single(prob, precision, tile):
+    prob.set_tiling(tile)
+    F = _loads(prob, 4)
+    opts = solver.default_opts(rtol=1e-9, precision=precision)
+    single = [prob.solve(f, opts=opts) for f in F]
+    for n in (2, 4):
+        U = prob.solve_multi(F[:n], opts=opts)
+        print("tiles", prob.tile_info(0), "cases", n, [i.iters for i in prob.infos], flush=True)
+        for k in range(n):
+            assert np.array_equal(U[k], single[k]), (n, k)
+    # timed launches do the same arithmetic
+    prob.kernel_timing()
+    u = prob.solve(F[0], opts=opts)
+    prob.kernel_timing(False)
+    assert np.array_equal(u, single[0])
+
+
 def test_multi_rhs_state_is_case_zero(adapt):
     forests, rho, prob = adapt
     F = _loads(prob, 3)

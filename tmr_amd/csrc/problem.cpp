@@ -1264,7 +1264,8 @@ template <class T>
 void Problem::apply_level(int l, const T *x, int mode, const AsmArgs &a, int nrhs) {
   Level &L = levels_[l];
   std::pair<hipEvent_t, hipEvent_t> *ev = nullptr;
-  if (l == 0 && ((timing_ >> (mode == ASM_POWER ? ASM_STORE : mode)) & 1)) {
+  const int timed = mode == ASM_POWER ? ASM_STORE : mode == ASM_CHEBDOT ? ASM_CHEB : mode;
+  if (l == 0 && ((timing_ >> timed) & 1)) {
     if (ev_used_ == ev_pool_.size()) {
       std::pair<hipEvent_t, hipEvent_t> e;
       if (hipEventCreate(&e.first) == hipSuccess && hipEventCreate(&e.second) == hipSuccess)
@@ -1770,7 +1771,7 @@ void Problem::enqueue_iteration(const SegPlan &pl, int nrhs, double *xsol, const
   // directly (no FP64 copy of z)
   if (mixed) {
     Level &L0 = levels_[0];
-    const bool dots = vcycle_dots(o, nrhs);
+    const bool dots = vcycle_dots(o);
     zdots_ = dots;
     vcycle<float>(0, L0.v32.b.p, L0.v32.x.p, o, nrhs, fuse0);
     zdots_ = false;
@@ -1779,7 +1780,7 @@ void Problem::enqueue_iteration(const SegPlan &pl, int nrhs, double *xsol, const
                       atol2, st_);
     launch_b_update_p<float>(pl, p_.p, L0.v32.x.p, sc_.p, act_.p, xsol, iter_.p, st_);
   } else {
-    const bool dots = vcycle_dots(o, nrhs);
+    const bool dots = vcycle_dots(o);
     zdots_ = dots;
     precond(nrhs, o);
     zdots_ = false;
@@ -1793,13 +1794,18 @@ void Problem::enqueue_iteration(const SegPlan &pl, int nrhs, double *xsol, const
 
 // z.r and z.q ride in the finest level's last smoothing step (Chebyshev, on
 // the vector ALUs, of a level that is not also the coarsest) while the launch
-// saved counts: below 2048 tiles in flight.  16^3 cube: 9.7 us against 8.6 +
-// 6.0 for step and dots; 4.2M hex: 147 us against 93 + 47, the tiles read r
-// and q more slowly than the streaming pass.
-bool Problem::vcycle_dots(const SolveOpts &o, int nrhs) const {
+// saved counts: levels below DOTS_TILES tiles.  Per iteration, fused against
+// separate: 16^3 cube (52 tiles) 9.7 us against 8.6 + 6.0 for step and dots;
+// 245,760 hex (1,008 tiles) 246 us against 250 in all; adaptive 236k hex (1,308
+// tiles) 346 against 349 with one load case, 1,793 against 1,760 with sixteen;
+// 4.2M hex (4,177 tiles) 147 against 93 + 47: the tiles read r and q more
+// slowly than the streaming pass.  The two forms add in different orders, so
+// the rule looks at the level alone: a load case takes the same form in a
+// batch as by itself, and whether or not launches are timed.
+static constexpr int DOTS_TILES = 1024;
+bool Problem::vcycle_dots(const SolveOpts &o) const {
   const bool mfma = o.precision != 0 && fp32_mfma_ && !fp32_valu_ && design_mode_ == 0;
-  return levels_.size() > 1 && !sor_ && !mfma && timing_ == 0 &&
-         (int64_t)levels_[0].tiles.n_tiles * nrhs < 2048;
+  return levels_.size() > 1 && !sor_ && !mfma && levels_[0].tiles.n_tiles < DOTS_TILES;
 }
 
 int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o,

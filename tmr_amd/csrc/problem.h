@@ -369,7 +369,7 @@ class Problem {
   template <class T>
   void cheb_step(int l, const T *b, const T *x_in, T *x_out, int k, const SolveOpts &o,
                  int nrhs = 1, int cflags = CHEB_D_READ | CHEB_D_STORE, bool dots = false);
-  bool vcycle_dots(const SolveOpts &o, int nrhs) const;
+  bool vcycle_dots(const SolveOpts &o) const;
   bool zdots_ = false;  // this V-cycle's last step also forms z.r and z.q
   template <class T>
   int mg_op_t(int op, int l, const double *x, double *y, bool on_device, const SolveOpts &o);
