@@ -82,6 +82,19 @@ def _batch_against_single(prob, precision, tile):
     assert np.array_equal(u, single[0])
 
 
+# the same hierarchy: coarse levels of 9,537 nodes and fewer, colours of 8,848
+# nodes and fewer, within the 16,384 rows of the 32-lane form by themselves
+# and beyond it two cases together
+@pytest.mark.parametrize("mg", [{"use_galerkin": True}, {"use_chebyshev_smoother": False}])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_batch_does_not_change_a_case_on_assembled_levels(box65k, precision, mg):
+    box65k.set_multigrid(**mg)
+    try:
+        _batch_against_single(box65k, precision, 128)
+    finally:
+        box65k.set_multigrid()
+
+
 def test_multi_rhs_state_is_case_zero(adapt):
     forests, rho, prob = adapt
     F = _loads(prob, 3)

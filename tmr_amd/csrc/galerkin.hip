@@ -202,8 +202,10 @@ void launch_bsr_dinv(int n, const int *diag, const double *val, T *dinv, hipStre
 // ---------------------------------------------------------------------------
 // BSR operator with the epilogues of the tile apply: LANES lanes per block
 // row, each summing every LANES-th block of the row two at a time, then a
-// butterfly over the group in a fixed order.  32 lanes while they fit the
-// chip (the loop over a row is a chain of dependent loads), else 8.
+// butterfly over the group in a fixed order.  32 lanes while one right-hand
+// side's rows fit the chip (the loop over a row is a chain of dependent
+// loads), else 8; the number of right-hand sides does not count, so that a
+// load case is summed in the same order in a batch as by itself.
 template <class T, int MODE, int LANES>
 __global__ void __launch_bounds__(256)
     k_bsr_apply(int n, const int *__restrict__ ptr, const int *__restrict__ col,
@@ -296,10 +298,13 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// rows of 32 lanes that fill the 256 CUs with at most 8 workgroups each
+static bool wide_rows(int n) { return (int64_t)n * 32 <= 256 * 8 * 256; }
+
 template <class T, int MODE>
 static void bsr_launch(const BSR<T> &A, const T *x, const AsmArgs &g, hipStream_t st, int nrhs,
                        int64_t vs) {
-  const bool wide = (int64_t)A.n * nrhs * 32 <= 256 * 8 * 256;
+  const bool wide = wide_rows(A.n);
   const int lanes = wide ? 32 : 8;
   const dim3 grid((unsigned)(((int64_t)A.n * lanes + 255) / 256), (unsigned)nrhs);
   if (wide)
@@ -504,8 +509,7 @@ template <class T, int DIR>
 static void sor_colour(const BSR<T> &A, const int *nodes, int c0, int cnt, const T *b, T *x,
                        double omega, hipStream_t st, int nrhs, int64_t vs) {
   if (cnt == 0) return;
-  // 32 lanes per row until they fill the 256 CUs with 8 workgroups each
-  const bool wide = (int64_t)cnt * nrhs * 32 <= 256 * 8 * 256;
+  const bool wide = wide_rows(cnt);
   const int lanes = wide ? 32 : 8;
   const dim3 grid((unsigned)(((int64_t)cnt * lanes + 255) / 256), (unsigned)nrhs);
   if (wide)
