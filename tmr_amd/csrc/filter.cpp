@@ -300,7 +300,7 @@ int Filter::apply(int nv, const double *in, double *out, bool on_device, bool tr
   const double *xin = in;
   double *xout = out;
   if (!on_device) {
-    if (hin_.n < n && (hin_.alloc(n) || hout_.alloc(n))) {
+    if (alloc_all(n, hin_, hout_)) {
       last_error = "filter: device allocation failed";
       return -1;
     }

@@ -1035,6 +1035,7 @@ int Problem::ensure_vecs(int l, int precision, int nrhs) {
     }
     if (v.cap >= nrhs) return 0;
     const size_t m = n * (size_t)nrhs;
+    v.cap = 0;
     if (v.b.alloc(m) || v.x.alloc(m) || v.x2.alloc(m) || v.r.alloc(m) || v.d.alloc(m)) return -1;
     if (hipMemset(v.d.p, 0, m * sizeof(T)) != hipSuccess ||
         hipMemset(v.x.p, 0, m * sizeof(T)) != hipSuccess ||
@@ -1056,6 +1057,8 @@ int Problem::ensure_batch(int nrhs) {
   const size_t np = std::max({(size_t)2 * 2048, (size_t)assemble_num_blocks(L0.n_nodes),
                               (size_t)2 * L0.tiles.n_tiles * nrhs, (size_t)2 * plan_.nblk * nrhs,
                               (size_t)(L0.n_elem + 255) / 256}) + 16;
+  batch_cap_ = 0;
+  have_solution_ = false;
   if (f_.alloc(m) || u_.alloc(m) || r_.alloc(m) || p_.alloc(m) || q_.alloc(m) || z_.alloc(m) ||
       parts_.alloc(np) || sc_.alloc(std::max(nidx * SC_N, (size_t)SC_N)) || act_.alloc(nidx) ||
       itconv_.alloc(nidx) || thr_.alloc(nidx) || iter_.alloc(1) || nact_.alloc(2)) {
@@ -1066,7 +1069,6 @@ int Problem::ensure_batch(int nrhs) {
   HIPCHK(hipMemset(f_.p, 0, m * sizeof(double)));
   HIPCHK(hipMemset(nact_.p, 0, 2 * sizeof(int)));
   if (!nact_host_) HIPCHK(hipHostMalloc((void **)&nact_host_, 2 * sizeof(int)));
-  have_solution_ = false;
   batch_cap_ = nrhs;
   gen_++;
   return 0;
@@ -1197,8 +1199,7 @@ int Problem::set_design_nodal(const double *x, int n, bool on_device) {
   if (check_design_values(x, n, on_device, "set_design_nodal")) return -1;
   for (auto &L : levels_) {
     if (L.xn.n < (size_t)L.n_nodes && L.xn.alloc(L.n_nodes)) goto oom;
-    if (L.sg64.n < 8 * (size_t)L.n_elem && (L.sg64.alloc(8 * (size_t)L.n_elem) ||
-                                            L.sg32.alloc(8 * (size_t)L.n_elem)))
+    if (alloc_all(8 * (size_t)L.n_elem, L.sg64, L.sg32))
       goto oom;
   }
   {
@@ -1455,6 +1456,7 @@ int Problem::setup(const SolveOpts &o) {
   }
   auto t0 = std::chrono::steady_clock::now();
   const int prec = o.precision ? 1 : 0;
+  if (ensure_batch(1)) return -1;
   for (size_t l = 0; l < levels_.size(); l++) {
     if (ensure_vecs((int)l, 0) || (prec == 1 && ensure_vecs((int)l, 1))) {
       last_error = "setup: device allocation failed";
@@ -1559,7 +1561,8 @@ int Problem::upload_coefs(const SolveOpts &o) {
   const int deg = std::max(1, std::max(o.cheb_degree, o.cheb_pre_degree));
   const size_t stride = 1 + 2 * (size_t)deg;
   if (coef_.n < stride * nl || coef_stride_ != stride) {
-    if (coef_.n < stride * nl && (coef_.alloc(stride * nl) || coef32_.alloc(stride * nl))) {
+    coef_stride_ = 0;
+    if (alloc_all(stride * nl, coef_, coef32_)) {
       last_error = "solve: device allocation failed";
       return -1;
     }
@@ -2044,6 +2047,7 @@ int Problem::set_state(const double *f, const double *u, bool on_device) {
     last_error = "set_state: null load or displacement";
     return -1;
   }
+  if (ensure_batch(1)) return -1;
   Level &L = levels_[0];
   const int64_t n = L.ndof;
   const hipMemcpyKind k = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
@@ -2344,7 +2348,7 @@ int Problem::apply(const double *x, double *y, bool on_device, int precision) {
   }
   Level &L = levels_[0];
   const int64_t n = L.ndof;
-  if (ensure_vecs(0, 0) || (precision && ensure_vecs(0, 1))) {
+  if (ensure_batch(1) || ensure_vecs(0, 0) || (precision && ensure_vecs(0, 1))) {
     last_error = "apply: allocation failed";
     return -1;
   }
@@ -2523,7 +2527,7 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
   }
   Level &L0 = levels_[0];
   const int64_t n = L0.ndof;
-  if (coef_.n < 2 && (coef_.alloc(2) || coef32_.alloc(2))) {
+  if (alloc_all(2, coef_, coef32_)) {
     last_error = "autotune: allocation failed";
     return -1;
   }

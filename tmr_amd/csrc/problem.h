@@ -61,6 +61,16 @@ struct DevArray {
   int upload(const std::vector<T> &v) { return upload(v.data(), v.size()); }
 };
 
+// All of the arrays hold at least `count` entries, or (-1) none of them any:
+// one that had kept its new size would pass for all of them in a later call.
+template <class... A>
+int alloc_all(size_t count, A &...a) {
+  if (((a.n >= count) && ...)) return 0;
+  if (!(a.alloc(count) || ...)) return 0;
+  (a.release(), ...);
+  return -1;
+}
+
 struct Material {
   double E = 1.0, nu = 0.3, ys = 1.0;
   double q = 3.0, k0 = 1e-6, eps = 0.3;
