@@ -63,3 +63,24 @@ def test_product_in_place_and_overlapping_vectors(precision, meshes):
         assert torch.equal(dst, want), (a, b)
         if a + n <= b or b + n <= a:
             assert np.array_equal(src.cpu().numpy(), x)
+
+
+@pytest.mark.parametrize("tile", [0, 200])
+def test_failed_autotune_keeps_the_tiles(tile):
+    """Candidates that do not fit in LDS (4096 owned nodes take 196 KB for x
+    and the accumulators alone): the tiles, the operator form and the solution
+    stay what they were."""
+    from tmr_amd._lib import TmrxError
+    forests, rho, _ = workloads.box(level=4, nlevels=3, seed=1)
+    prob = solver.Problem(forests, q=Q, k0=K0, bcs=[("fixed", 7)])
+    prob.set_design(rho)
+    if tile:
+        prob.set_tiling(tile)
+    keep = [prob.tile_info(l) for l in range(3)], prob.tuning()
+    f = prob.traction_load("load", [0.0, 0.2, -1.0])
+    u = prob.solve(f)
+    for call in (lambda: prob.autotune((4096, 4000)), lambda: prob.set_tiling(4096)):
+        with pytest.raises(TmrxError, match="fit"):
+            call()
+        assert ([prob.tile_info(l) for l in range(3)], prob.tuning()) == keep
+        assert np.array_equal(prob.solve(f), u)

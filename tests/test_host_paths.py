@@ -48,6 +48,7 @@ def _child(lib, *args):
 
 
 @pytest.mark.parametrize("call", [
-    "solve", "FP64 solve", "three cases", "degree", "nodal design", "Galerkin", "SOR", "filter"])
+    "solve", "FP64 solve", "three cases", "degree", "nodal design", "Galerkin", "SOR",
+    "matrix cores", "tiling", "autotune", "filter"])
 def test_failed_allocations(fake_lib, call):
     _child(fake_lib, call)

@@ -324,9 +324,15 @@ int Problem::init(int nlevels, Forest **forests, const Material &mat, int nbcs,
     L.cls.resize(octs.size());
     for (size_t e = 0; e < octs.size(); e++) L.cls[e] = block_cls[l][octs[e].block];
     if (build_level(l, nbcs, names, dof_masks)) return -1;
-    L.tile_nodes = l > 0 ? coarse_tile_nodes(TILE_NODES, L.n_nodes)
-                         : default_tile_nodes(L.n_nodes, L.n_dep > 0);
-    if (build_tiles(l)) return -1;
+    TileSet ts;
+    if (make_tiles(l, l > 0 ? coarse_tile_nodes(TILE_NODES, L.n_nodes)
+                            : default_tile_nodes(L.n_nodes, L.n_dep > 0), false, ts))
+      return -1;
+    if (!ts.fits) {
+      last_error = "the tiles of level " + std::to_string(l) + " do not fit in LDS";
+      return -1;
+    }
+    install_tiles(l, std::move(ts));
   }
   for (int l = 0; l + 1 < nlevels; l++)
     if (build_transfer(l)) return -1;
@@ -588,11 +594,11 @@ int Problem::build_level(int l, int nbcs, const char **names, const int *masks) 
   return 0;
 }
 
-// Owner tiles: contiguous ranges of L.tile_nodes independent nodes; every
+// Owner tiles: contiguous ranges of tile_nodes independent nodes; every
 // element touching an owned node, or a hanging node with an owned parent, is
 // staged with its corners in LDS slots [owned | accumulated hanging | halo].
-int Problem::build_tiles(int l) {
-  Level &L = levels_[l];
+int Problem::make_tiles(int l, int tile_nodes, bool mfma, TileSet &out) const {
+  const Level &L = levels_[l];
   Forest *f = L.forest;
   const int n = L.n_nodes, nd = L.n_dep, ne = L.n_elem;
   const auto &dptr = f->dep_ptr();
@@ -622,10 +628,11 @@ int Problem::build_tiles(int l) {
   }
   // tiles never straddle two independent components
   std::vector<int> tstart;
-  L.seg_tile.assign(1, 0);
+  out.tile_nodes = tile_nodes;
+  out.seg_tile.assign(1, 0);
   for (size_t sg = 0; sg + 1 < L.seg_node0.size(); sg++) {
-    for (int a = L.seg_node0[sg]; a < L.seg_node0[sg + 1]; a += L.tile_nodes) tstart.push_back(a);
-    L.seg_tile.push_back((int)tstart.size());
+    for (int a = L.seg_node0[sg]; a < L.seg_node0[sg + 1]; a += tile_nodes) tstart.push_back(a);
+    out.seg_tile.push_back((int)tstart.size());
   }
   tstart.push_back(n);
   const int ntiles = (int)tstart.size() - 1;
@@ -646,7 +653,7 @@ int Problem::build_tiles(int l) {
     if (L.cls[e] != L.cls[0]) single = false;
   std::vector<int> tel, rdeps, rdep_wave;
   for (int t = 0; t < ntiles; t++) {
-    const int n0 = tstart[t], n1 = std::min(tstart[t + 1], n0 + L.tile_nodes), nown = n1 - n0;
+    const int n0 = tstart[t], n1 = std::min(tstart[t + 1], n0 + tile_nodes), nown = n1 - n0;
     node0[t] = n0;
     rdeps.clear();
     rdep_wave.clear();
@@ -746,11 +753,12 @@ int Problem::build_tiles(int l) {
       return a.color != b.color ? a.color < b.color : a.mask > b.mask;
     });
     // matrix-core batches (when a matrix-core form has been asked for): each
-    // of the MFMA_WAVES waves owns a contiguous share of the owned nodes (and the hanging nodes whose first owned
-    // parent it owns) and takes every element touching them, with the rows
-    // of those corners only; per wave, records are coloured over its
-    // corners and (colour, class) groups are padded to 16 records
-    if (mfma_tiles_) {
+    // of the MFMA_WAVES waves owns a contiguous share of the owned nodes (and
+    // the hanging nodes whose first owned parent it owns) and takes every
+    // element touching them, with the rows of those corners only; per wave,
+    // records are coloured over its corners and (colour, class) groups are
+    // padded to 16 records
+    if (mfma) {
       auto wave_of = [&](int pos) {
         const int sl = tile_pos(pos);  // tile_pos is an involution
         return sl < nown ? sl / qw : (sl < na ? rdep_wave[sl - nown] : -1);
@@ -808,7 +816,7 @@ int Problem::build_tiles(int l) {
     max_slots = std::max(max_slots, ns);
     max_acc = std::max(max_acc, na);
     max_rec = std::max(max_rec, (int)(els.size() - el0));
-    if (mfma_tiles_) {
+    if (mfma) {
       const int *cp = &mb_ptr[(size_t)t * (MFMA_WAVES + 1)];
       max_mrec = std::max(max_mrec, 16 * (cp[MFMA_WAVES] - cp[0]));
     }
@@ -829,67 +837,114 @@ int Problem::build_tiles(int l) {
     for (int t = 0; t < ntiles; t++) na_t[t] = node0[t + 1] - node0[t] + nacc[t];
     std::string err;
     if (check_tile_schedule(ntiles, el_ptr.data(), els.data(), na_t.data(),
-                            mfma_tiles_ ? MFMA_WAVES : 0, mb_ptr.data(), mel.data(), err)) {
+                            mfma ? MFMA_WAVES : 0, mb_ptr.data(), mel.data(), err)) {
       last_error = "problem: tile schedule check failed: " + err;
       return -1;
     }
   }
+  {
+    // slots and accumulators of the largest tile, FP64 (FP32 matrix-core
+    // planes take no more), and the kernels' static words
+    int dev = 0, max_lds = 0;
+    HIPCHK(hipGetDevice(&dev));
+    HIPCHK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    const size_t lds = 24 * (size_t)(round8(max_slots) + round8(max_acc));
+    out.fits = lds + 64 <= (size_t)max_lds;
+    if (!out.fits) return 0;
+  }
   if (comb.empty()) comb.assign(4, 0u);
   if (extd.empty()) extd.assign(2, 0u);
   if (ext.empty()) ext.push_back(0u);
-  if (L.t_node0.upload(node0) || L.t_ext_ptr.upload(ext_ptr) || L.t_ext.upload(ext) ||
-      L.t_nacc.upload(nacc) || L.t_el_ptr.upload(el_ptr) || L.t_el.upload(els) ||
-      L.t_extd_ptr.upload(extd_ptr) || L.t_extd.upload(extd) ||
-      L.t_comb_ptr.upload(comb_ptr) || L.t_comb.upload(comb) || L.t_mb_ptr.upload(mb_ptr) || L.t_mel.upload(mel)) {
+  std::vector<int> me(mel.size()), ee(els.size());
+  for (size_t k = 0; k < mel.size(); k++) me[k] = mel[k].elem;
+  for (size_t k = 0; k < els.size(); k++) ee[k] = els[k].elem;
+  if (out.node0.upload(node0) || out.ext_ptr.upload(ext_ptr) || out.ext.upload(ext) ||
+      out.nacc.upload(nacc) || out.el_ptr.upload(el_ptr) || out.el.upload(els) ||
+      out.extd_ptr.upload(extd_ptr) || out.extd.upload(extd) || out.comb_ptr.upload(comb_ptr) ||
+      out.comb.upload(comb) || out.mb_ptr.upload(mb_ptr) || out.mel.upload(mel) ||
+      out.mel_elem.upload(me) || out.el32.upload(els) || out.el_elem.upload(ee)) {
     last_error = "problem: device allocation failed";
     return -1;
   }
-  {
-    std::vector<int> me(mel.size()), ee(els.size());
-    for (size_t k = 0; k < mel.size(); k++) me[k] = mel[k].elem;
-    for (size_t k = 0; k < els.size(); k++) ee[k] = els[k].elem;
-    if (L.t_mel_elem.upload(me) || L.t_el32.upload(els) || L.t_el_elem.upload(ee)) {
-      last_error = "problem: device allocation failed";
-      return -1;
-    }
-  }
-  Tiles &T = L.tiles;
+  Tiles &T = out.tiles;
   T.n_tiles = ntiles;
   // large tiles take 512 threads on the vector ALUs, so that the LDS they
   // need (4 tiles per CU) still fills the CU with waves
-  T.threads = L.tile_nodes >= 768 ? 512 : TILE_THREADS;
+  T.threads = tile_nodes >= 768 ? 512 : TILE_THREADS;
   T.single_class = single;
   T.max_slots = max_slots;
   T.max_mrec = max_mrec;
   T.max_rec = max_rec;
   T.max_acc = max_acc;
   T.ncolors = ncolors;
-  T.node0 = L.t_node0.p;
-  T.ext_ptr = L.t_ext_ptr.p;
-  T.ext = L.t_ext.p;
-  T.nacc_dep = L.t_nacc.p;
-  T.el_ptr = L.t_el_ptr.p;
-  T.el = L.t_el.p;
-  T.comb_ptr = L.t_comb_ptr.p;
-  T.comb = reinterpret_cast<const uint4 *>(L.t_comb.p);
-  T.extd_ptr = L.t_extd_ptr.p;
-  T.extd = reinterpret_cast<const uint2 *>(L.t_extd.p);
+  T.node0 = out.node0.p;
+  T.ext_ptr = out.ext_ptr.p;
+  T.ext = out.ext.p;
+  T.nacc_dep = out.nacc.p;
+  T.el_ptr = out.el_ptr.p;
+  T.el = out.el.p;
+  T.comb_ptr = out.comb_ptr.p;
+  T.comb = reinterpret_cast<const uint4 *>(out.comb.p);
+  T.extd_ptr = out.extd_ptr.p;
+  T.extd = reinterpret_cast<const uint2 *>(out.extd.p);
   T.bcmask = L.d_bcmask.p;
-  T.mb_ptr = L.t_mb_ptr.p;
-  T.mel = L.t_mel.p;
-  T.mel_elem = L.t_mel_elem.p;
+  T.mb_ptr = out.mb_ptr.p;
+  T.mel = out.mel.p;
+  T.mel_elem = out.mel_elem.p;
   T.n_mrec = (int)mel.size();
-  T.el32 = L.t_el32.p;
-  T.el_elem = L.t_el_elem.p;
+  T.el32 = out.el32.p;
+  T.el_elem = out.el_elem.p;
   T.n_rec = (int)els.size();
+  T.afrag = reinterpret_cast<const uint4 *>(afrag_.p);
+  T.afrag32 = afrag32_.p;
+  T.use_mfma = mfma;
+  return 0;
+}
+
+void Problem::install_tiles(int l, TileSet &&ts) {
+  Level &L = levels_[l];
+  L.ts = std::move(ts);
+  const Tiles &T = L.ts.tiles;
   if (have_design_) {
     launch_rec_scale(T.n_mrec, T.mel_elem, L.s32.p, reinterpret_cast<uint32_t *>(T.mel), st_);
     launch_rec_scale(T.n_rec, T.el_elem, L.s32.p, reinterpret_cast<uint32_t *>(T.el32), st_);
   }
-  T.afrag = reinterpret_cast<const uint4 *>(afrag_.p);
-  T.afrag32 = afrag32_.p;
-  T.use_mfma = mfma_tiles_;
+  gen_++;
+}
+
+int Problem::retile(const std::vector<int> &tile_nodes, bool mfma, bool *fits) {
+  std::vector<TileSet> ts(levels_.size());
+  if (fits) *fits = true;
+  for (size_t l = 0; l < levels_.size(); l++) {
+    if (make_tiles((int)l, tile_nodes[l], mfma, ts[l])) return -1;
+    if (ts[l].fits) continue;
+    if (fits) {
+      *fits = false;
+      return 0;
+    }
+    last_error = "the tiles of level " + std::to_string(l) + " do not fit in LDS";
+    return -1;
+  }
+  DevArray<int> seg;
+  if (seg.upload(ts[0].seg_tile)) {
+    last_error = "problem: device allocation failed";
+    return -1;
+  }
+  for (size_t l = 0; l < levels_.size(); l++) install_tiles((int)l, std::move(ts[l]));
+  mfma_tiles_ = mfma;
+  // the reduction plan follows the finest level's tiles
+  pl_seg_tile_ = std::move(seg);
+  plan_.seg_tile = pl_seg_tile_.p;
+  plan_.ntiles = levels_[0].ts.tiles.n_tiles;
+  drop_graphs();
   return 0;
+}
+
+// the partial sums for the tiles in use; the solution is given up
+int Problem::follow_tiles() {
+  const int cap = std::max(1, batch_cap_);
+  batch_cap_ = 0;
+  return ensure_batch(cap);
 }
 
 int Problem::build_transfer(int l) {
@@ -1055,7 +1110,7 @@ int Problem::ensure_batch(int nrhs) {
   const size_t n = (size_t)L0.ndof, m = n * (size_t)nrhs;
   const size_t nidx = (size_t)nrhs * nseg_;
   const size_t np = std::max({(size_t)2 * 2048, (size_t)assemble_num_blocks(L0.n_nodes),
-                              (size_t)2 * L0.tiles.n_tiles * nrhs, (size_t)2 * plan_.nblk * nrhs,
+                              (size_t)2 * L0.ts.tiles.n_tiles * nrhs, (size_t)2 * plan_.nblk * nrhs,
                               (size_t)(L0.n_elem + 255) / 256}) + 16;
   batch_cap_ = 0;
   have_solution_ = false;
@@ -1093,14 +1148,14 @@ int Problem::build_plan() {
   lo.push_back((int)L.ndof);
   if (bseg.empty()) bseg.push_back(0);
   if (pl_blk_lo_.upload(lo) || pl_blk_seg_.upload(bseg) || pl_seg_blk_.upload(sblk) ||
-      pl_seg_tile_.upload(L.seg_tile)) {
+      pl_seg_tile_.upload(L.ts.seg_tile)) {
     last_error = "problem: device allocation failed";
     return -1;
   }
   plan_.nrhs = 1;
   plan_.nseg = nseg_;
   plan_.nblk = (int)lo.size() - 1;
-  plan_.ntiles = L.tiles.n_tiles;
+  plan_.ntiles = L.ts.tiles.n_tiles;
   plan_.n = L.ndof;
   plan_.blk_lo = pl_blk_lo_.p;
   plan_.blk_seg = pl_blk_seg_.p;
@@ -1167,10 +1222,10 @@ int Problem::set_design(const double *rho, int n, bool on_device) {
   }
   for (auto &L : levels_) {
     if (fp32_mfma_)
-      launch_rec_scale(L.tiles.n_mrec, L.tiles.mel_elem, L.s32.p,
-                       reinterpret_cast<uint32_t *>(L.tiles.mel), st_);
-    launch_rec_scale(L.tiles.n_rec, L.tiles.el_elem, L.s32.p,
-                     reinterpret_cast<uint32_t *>(L.tiles.el32), st_);
+      launch_rec_scale(L.ts.tiles.n_mrec, L.ts.tiles.mel_elem, L.s32.p,
+                       reinterpret_cast<uint32_t *>(L.ts.tiles.mel), st_);
+    launch_rec_scale(L.ts.tiles.n_rec, L.ts.tiles.el_elem, L.s32.p,
+                     reinterpret_cast<uint32_t *>(L.ts.tiles.el32), st_);
   }
   have_design_ = true;
   have_setup_ = false;
@@ -1283,7 +1338,7 @@ void Problem::apply_level(int l, const T *x, int mode, const AsmArgs &a, int nrh
     launch_bsr_apply<T>(A, x, mode, g, st_, nrhs, L.ndof);
     return;
   }
-  Tiles tl = L.tiles;
+  Tiles tl = L.ts.tiles;
   tl.run = run_;
   tl.nodal = design_mode_ == 1;
   tl.use_mfma = tl.use_mfma && !fp32_valu_ && fp32_mfma_ && !tl.nodal;
@@ -1808,7 +1863,7 @@ void Problem::enqueue_iteration(const SegPlan &pl, int nrhs, double *xsol, const
 static constexpr int DOTS_TILES = 1024;
 bool Problem::vcycle_dots(const SolveOpts &o) const {
   const bool mfma = o.precision != 0 && fp32_mfma_ && !fp32_valu_ && design_mode_ == 0;
-  return levels_.size() > 1 && !sor_ && !mfma && levels_[0].tiles.n_tiles < DOTS_TILES;
+  return levels_.size() > 1 && !sor_ && !mfma && levels_[0].ts.tiles.n_tiles < DOTS_TILES;
 }
 
 int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o,
@@ -1854,7 +1909,7 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
       return -1;
     }
     HIPCHK(hipMemcpyAsync(lrhs_.p, rhs, m * sizeof(double), hipMemcpyDeviceToDevice, st_));
-    Tiles tl = L0.tiles;
+    Tiles tl = L0.ts.tiles;
     tl.bcmask = nomask_.p;
     tl.masked = false;
     tl.nodal = design_mode_ == 1;
@@ -2451,38 +2506,25 @@ int Problem::set_tiling(int tile_nodes) {
     last_error = "set_tiling: tile sizes must lie in [64, 4096]";
     return -1;
   }
-  int dev = 0, max_lds = 0;
-  HIPCHK(hipGetDevice(&dev));
-  HIPCHK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-  for (size_t l = 0; l < levels_.size(); l++) {
-    Level &L = levels_[l];
-    L.tile_nodes = l == 0 ? tile_nodes : coarse_tile_nodes(tile_nodes, L.n_nodes);
-    if (build_tiles((int)l)) return -1;
-    const Tiles &tl = L.tiles;
-    const size_t lds64 = 3 * (size_t)(round8(tl.max_slots) + round8(tl.max_acc)) * sizeof(double);
-    const size_t lds32 = 24 * (size_t)round8(tl.max_slots) + 16 * (size_t)round8(tl.max_acc);
-    if (std::max(lds64, lds32) + 64 > (size_t)max_lds) {
-      last_error = "set_tiling: the tiles of level " + std::to_string(l) + " do not fit in LDS";
-      return -1;
-    }
+  if (retile(tile_sizes(tile_nodes), mfma_tiles_)) {
+    last_error = "set_tiling: " + last_error;
+    return -1;
   }
-  if (build_plan()) return -1;
-  const int cap = std::max(1, batch_cap_);
-  batch_cap_ = 0;
-  if (ensure_batch(cap)) return -1;
-  drop_graphs();
-  gen_++;
-  return 0;
+  return follow_tiles();
 }
 
-// The matrix-core batches of every level's tiles are only built once a
-// matrix-core form is asked for.
-int Problem::ensure_mfma_tiles() {
-  if (mfma_tiles_) return 0;
-  mfma_tiles_ = true;
+// tile_nodes at the finest level, the rule's sizes below it
+std::vector<int> Problem::tile_sizes(int tile_nodes) const {
+  std::vector<int> t;
   for (size_t l = 0; l < levels_.size(); l++)
-    if (build_tiles((int)l)) return -1;
-  return 0;
+    t.push_back(l == 0 ? tile_nodes : coarse_tile_nodes(tile_nodes, levels_[l].n_nodes));
+  return t;
+}
+
+std::vector<int> Problem::tile_sizes() const {
+  std::vector<int> t;
+  for (const Level &L : levels_) t.push_back(L.ts.tile_nodes);
+  return t;
 }
 
 int Problem::set_fp32_form(int form) {
@@ -2492,12 +2534,13 @@ int Problem::set_fp32_form(int form) {
     return -1;
   }
   if (form != 0) {
-    if (ensure_mfma_tiles()) return -1;
+    // the matrix-core batches are only built once such a form is asked for
+    if (!mfma_tiles_ && retile(tile_sizes(), true)) return -1;
     // set_design keeps their scales current only while a matrix-core form is on
     if (have_design_ && design_mode_ == 0)
       for (auto &L : levels_)
-        launch_rec_scale(L.tiles.n_mrec, L.tiles.mel_elem, L.s32.p,
-                         reinterpret_cast<uint32_t *>(L.tiles.mel), st_);
+        launch_rec_scale(L.ts.tiles.n_mrec, L.ts.tiles.mel_elem, L.s32.p,
+                         reinterpret_cast<uint32_t *>(L.ts.tiles.mel), st_);
   }
   fp32_mfma_ = form != 0;
   fp32_mfma_in32_ = form == 2;
@@ -2550,27 +2593,26 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   const bool keep_valu = fp32_valu_, keep_mfma = fp32_mfma_, keep_in32 = fp32_mfma_in32_;
+  const bool keep_tiles = mfma_tiles_;
+  const std::vector<int> keep = tile_sizes();
   fp32_valu_ = false;
-  mfma_tiles_ = true;  // every form is timed
-  int dev = 0, max_lds = 0;
-  HIPCHK(hipGetDevice(&dev));
-  HIPCHK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  // what the call found, for every way out but the last
+  auto give_up = [&](std::string why) {
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    fp32_valu_ = keep_valu;
+    fp32_mfma_ = keep_mfma;
+    fp32_mfma_in32_ = keep_in32;
+    // (tiles that cannot be made again: those of the last candidate serve)
+    if (retile(keep, keep_tiles)) (void)follow_tiles();
+    last_error = why;
+    return -1;
+  };
   int best = -1, best_form = 1;
   double best_ms = 0.0;
   for (int c = 0; c < ncand; c++) {
     bool fits = true;
-    for (size_t l = 0; l < levels_.size(); l++) {
-      levels_[l].tile_nodes = l == 0 ? cands[c] : coarse_tile_nodes(cands[c], levels_[l].n_nodes);
-      if (build_tiles((int)l)) {
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        return -1;
-      }
-      const Tiles &tl = levels_[l].tiles;
-      const size_t lds64 = 3 * (size_t)(round8(tl.max_slots) + round8(tl.max_acc)) * sizeof(double);
-      const size_t lds32 = 24 * (size_t)round8(tl.max_slots) + 16 * (size_t)round8(tl.max_acc);
-      if (std::max(lds64, lds32) + 64 > (size_t)max_lds) fits = false;
-    }
+    if (retile(tile_sizes(cands[c]), true, &fits)) return give_up(last_error);  // every form is timed
     if (!fits) {  // the tiles would not fit in LDS
       if (ms_out) ms_out[c] = -1.0;
       continue;
@@ -2617,14 +2659,8 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
     const double tm = design_mode_ == 1 ? tv : time_op(0);
     const double tm32 = design_mode_ == 1 ? tv : time_op(3);
     if (tm < 0 || tm32 < 0 || tv < 0 || t64 < 0) {
-      (void)hipEventDestroy(e0);
-      (void)hipEventDestroy(e1);
-      fp32_valu_ = keep_valu;
-      fp32_mfma_ = keep_mfma;
-      fp32_mfma_in32_ = keep_in32;
-      HIPCHK(hipGetLastError());
-      last_error = "autotune: timing failed";
-      return -1;
+      (void)hipGetLastError();
+      return give_up("autotune: timing failed");
     }
     int form = 1;
     double tf = tv;
@@ -2647,34 +2683,16 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
   fp32_valu_ = keep_valu;
   fp32_mfma_ = keep_mfma;
   fp32_mfma_in32_ = keep_in32;
-  if (best < 0) {
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    last_error = "autotune: no candidate tile size fits in LDS";
-    best = -1;
-    for (size_t l = 0; l < levels_.size(); l++) {
-      levels_[l].tile_nodes = l == 0 ? TILE_NODES : coarse_tile_nodes(TILE_NODES, levels_[l].n_nodes);
-      if (build_tiles((int)l)) return -1;
-    }
-    if (build_plan()) return -1;
-    const int cap0 = std::max(1, batch_cap_);
-    batch_cap_ = 0;
-    if (ensure_batch(cap0)) return -1;
-    return -1;
-  }
-  for (size_t l = 0; l < levels_.size(); l++) {
-    levels_[l].tile_nodes = l == 0 ? cands[best] : coarse_tile_nodes(cands[best], levels_[l].n_nodes);
-    if (build_tiles((int)l)) return -1;
-  }
+  if (best < 0) return give_up("autotune: no candidate tile size fits in LDS");
+  if (retile(tile_sizes(cands[best]), true)) return give_up(last_error);
   // coarse levels large enough to fill the GPU: their own tile size, by the
   // time of the FP32 product on the vector ALUs at that level
   for (size_t l = 1; l + 1 < levels_.size(); l++) {
     Level &Lc = levels_[l];
     if (Lc.n_nodes < 65536) break;
-    if (ensure_vecs((int)l, 1)) return -1;
+    if (ensure_vecs((int)l, 1)) return give_up("autotune: allocation failed");
     launch_fill<float>(Lc.ndof, 1.0f, Lc.v32.b.p, st_);
-    const int keep = Lc.tile_nodes;
-    int bsz = keep;
+    int bsz = Lc.ts.tile_nodes;
     double bms = -1.0;
     AsmArgs ac;
     ac.y = Lc.v32.r.p;
@@ -2682,22 +2700,18 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
     fp32_valu_ = true;
     for (int cand : {128, 256, 512, 1024}) {
       if ((Lc.n_nodes + cand - 1) / cand < 256) continue;  // at least one tile per CU
-      Lc.tile_nodes = cand;
-      if (build_tiles((int)l)) return -1;
-      const Tiles &tl = Lc.tiles;
-      const size_t lds64 = 3 * (size_t)(round8(tl.max_slots) + round8(tl.max_acc)) * sizeof(double);
-      if (lds64 + 64 > (size_t)max_lds) continue;
+      TileSet ts;
+      if (make_tiles((int)l, cand, true, ts)) return give_up(last_error);
+      if (!ts.fits) continue;
+      install_tiles((int)l, std::move(ts));
       apply_level<float>((int)l, Lc.v32.b.p, ASM_STORE, ac);
       (void)hipEventRecord(e0, st_);
       for (int r = 0; r < reps; r++) apply_level<float>((int)l, Lc.v32.b.p, ASM_STORE, ac);
       (void)hipEventRecord(e1, st_);
       float ms = 0.0f;
       if (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-        fp32_valu_ = kv;
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        last_error = "autotune: timing failed";
-        return -1;
+        (void)hipGetLastError();
+        return give_up("autotune: timing failed");
       }
       if (bms < 0 || ms < bms) {
         bms = ms;
@@ -2705,19 +2719,16 @@ int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double
       }
     }
     fp32_valu_ = kv;
-    Lc.tile_nodes = bsz;
-    if (build_tiles((int)l)) return -1;
+    if (bsz == Lc.ts.tile_nodes) continue;
+    TileSet ts;
+    if (make_tiles((int)l, bsz, true, ts)) return give_up(last_error);
+    install_tiles((int)l, std::move(ts));
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  // tiles moved: reduction plan, partial buffers and captured graphs follow
-  if (build_plan()) return -1;
-  const int cap = std::max(1, batch_cap_);
-  batch_cap_ = 0;
-  if (ensure_batch(cap)) return -1;
-  gen_++;
   fp32_mfma_ = best_form != 1;
   fp32_mfma_in32_ = best_form == 3;
+  if (follow_tiles()) return -1;
   if (chosen) *chosen = cands[best];
   return 0;
 }

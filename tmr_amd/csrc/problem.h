@@ -123,6 +123,17 @@ struct LevelVecs {
   int cap = 0;  // right-hand sides the per-rhs vectors hold
 };
 
+// owner tiles of one level and their device tables
+struct TileSet {
+  int tile_nodes = 0;         // nodes per tile
+  std::vector<int> seg_tile;  // tiles [seg_tile[s], seg_tile[s+1]) hold component s
+  bool fits = true;           // a tile fits in LDS (else there are no tables)
+  DevArray<int> node0, ext_ptr, extd_ptr, nacc, el_ptr, comb_ptr, el_elem, mb_ptr, mel_elem;
+  DevArray<uint32_t> ext, extd, comb;
+  DevArray<TileElem> el, el32, mel;
+  Tiles tiles;
+};
+
 struct Level {
   Forest *forest = nullptr;
   // the next coarser level is a coarsen() of this one (same blocks); else
@@ -131,10 +142,8 @@ struct Level {
   int n_nodes = 0, n_dep = 0, n_elem = 0;
   int64_t ndof = 0;
   // independent components (separate problems sharing the hierarchy):
-  // nodes [seg_node0[s], seg_node0[s+1]) belong to component s, owner
-  // tiles [seg_tile[s], seg_tile[s+1]) hold them
-  std::vector<int> seg_node0, seg_tile;
-  int tile_nodes = TILE_NODES;  // owner-tile size
+  // nodes [seg_node0[s], seg_node0[s+1]) belong to component s
+  std::vector<int> seg_node0;
   // host copies
   std::vector<int16_t> lev;
   std::vector<int> cls;
@@ -150,15 +159,7 @@ struct Level {
   DevArray<int16_t> d_lev;
   ElemBatches eb;
   AsmCSR asmc;
-  // owner tiles (single-pass apply)
-  DevArray<int> t_mb_ptr;
-  DevArray<TileElem> t_mel;
-  DevArray<int> t_mel_elem;
-  DevArray<int> t_node0, t_ext_ptr, t_extd_ptr, t_nacc, t_el_ptr, t_comb_ptr;
-  DevArray<uint32_t> t_ext, t_extd, t_comb;
-  DevArray<TileElem> t_el, t_el32;
-  DevArray<int> t_el_elem;
-  Tiles tiles;
+  TileSet ts;  // owner tiles (single-pass apply)
   // transfer to the next coarser level (P: rows = this level's nodes)
   DevArray<int> P_ptr, P_col, R_ptr, R_col;
   DevArray<float> P_w, R_w;
@@ -270,12 +271,12 @@ class Problem {
   int num_segments() const { return nseg_; }
   // owner-tile size autotuner (ms per candidate, chosen size)
   int autotune(const int *cands, int ncand, int reps, int *chosen, double *ms);
-  int tile_nodes() const { return levels_.empty() ? 0 : levels_[0].tile_nodes; }
+  int tile_nodes() const { return levels_.empty() ? 0 : levels_[0].ts.tile_nodes; }
   // owner tiles of level l: count and nominal size
   int tile_info(int l, int *ntiles, int *tile_nodes) const {
     if (l < 0 || l >= (int)levels_.size()) return -1;
-    if (ntiles) *ntiles = levels_[l].tiles.n_tiles;
-    if (tile_nodes) *tile_nodes = levels_[l].tile_nodes;
+    if (ntiles) *ntiles = levels_[l].ts.tiles.n_tiles;
+    if (tile_nodes) *tile_nodes = levels_[l].ts.tile_nodes;
     return 0;
   }
   bool fp32_matrix_cores() const { return fp32_mfma_; }
@@ -339,7 +340,15 @@ class Problem {
  private:
   int build_level(int l, int nbcs, const char **names, const int *masks);
   int build_transfer(int l);
-  int build_tiles(int l);
+  // the owner tiles of a level are made beside those in use and put in their
+  // place whole, so that a failure changes nothing
+  int make_tiles(int l, int tile_nodes, bool mfma, TileSet &out) const;
+  void install_tiles(int l, TileSet &&ts);
+  // every level's; *fits (may be null: an error): whether all fit in LDS
+  int retile(const std::vector<int> &tile_nodes, bool mfma, bool *fits = nullptr);
+  int follow_tiles();
+  std::vector<int> tile_sizes(int tile_nodes) const;
+  std::vector<int> tile_sizes() const;  // those in use
   int ensure_vecs(int l, int precision, int nrhs = 1);
   int ensure_batch(int nrhs);
   int build_plan();
@@ -496,7 +505,6 @@ class Problem {
   // 202 us; adaptive 1.2M hex 106 / 175 us for the first two).
   bool fp32_mfma_ = false;
   bool mfma_tiles_ = false;      // tiles carry matrix-core batches
-  int ensure_mfma_tiles();
   bool fp32_mfma_in32_ = false;  // ... with FP32 inputs (else bf16 three-way split)
   int timing_ = 0;  // mask of the timed launch modes (bit m = AsmMode m)
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_pool_;
