@@ -132,5 +132,18 @@ def allocation_failures(only):
         assert failed > 0
 
 
+def small_lds():
+    """The default tiles get smaller until they fit."""
+    forests, rho, _ = workloads.cube_l4(2)
+    p = solver.Problem(forests, q=3.0, k0=1e-6, bcs=[("fixed", 7)])
+    assert p.tile_info(0)[1] == 96
+    L.fake_max_lds(8 * 1024)  # 96 nodes and their halo take more, 64 less
+    p = solver.Problem(forests, q=3.0, k0=1e-6, bcs=[("fixed", 7)])
+    assert p.tile_info(0)[1] == 64
+    p.set_design(rho)
+    use(p)
+    expect_clean("tiles in 8 KB")
+
+
 if __name__ == "__main__":
-    allocation_failures(sys.argv[1:])
+    small_lds() if sys.argv[1:] == ["LDS"] else allocation_failures(sys.argv[1:])

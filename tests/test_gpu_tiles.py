@@ -84,3 +84,26 @@ def test_failed_autotune_keeps_the_tiles(tile):
             call()
         assert ([prob.tile_info(l) for l in range(3)], prob.tuning()) == keep
         assert np.array_equal(prob.solve(f), u)
+
+
+def test_default_tiles_of_rows_of_single_element_blocks():
+    """2.2M nodes numbered row by row: the 1,024-node tiles of large uniform
+    levels do not fit in LDS there."""
+    from tmr_amd import TMR
+    f = TMR.createBoxForest(1100, 44, 44, (1100.0, 44.0, 44.0), face_names=workloads.FACES)
+    f.createTrees(0)
+    f.createNodes()
+    prob = solver.Problem([f], q=Q, k0=K0, bcs=[("fixed", 7)])
+    tiles, size = prob.tile_info(0)
+    print("%d tiles of %d nodes" % (tiles, size), flush=True)
+    assert size == 512
+    rng = np.random.default_rng(6)
+    prob.set_design(rng.uniform(0.1, 1.0, prob.nelem))
+    x = rng.standard_normal(prob.ndof)
+    y = prob.apply(x, precision=0)
+    y32 = prob.apply(x, precision=1)
+    prob.set_tiling(200)
+    ref = prob.apply(x, precision=0)
+    # sums of about 80 terms a row in another order; FP32 operands and sums
+    assert np.linalg.norm(y - ref) < 1e-14 * np.linalg.norm(ref)
+    assert np.linalg.norm(y32 - ref) < 1e-5 * np.linalg.norm(ref)

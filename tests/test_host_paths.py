@@ -52,3 +52,7 @@ def _child(lib, *args):
     "matrix cores", "tiling", "autotune", "filter"])
 def test_failed_allocations(fake_lib, call):
     _child(fake_lib, call)
+
+
+def test_default_tiles_fit_in_lds(fake_lib):
+    _child(fake_lib, "LDS")

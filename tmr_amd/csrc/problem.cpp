@@ -324,12 +324,19 @@ int Problem::init(int nlevels, Forest **forests, const Material &mat, int nbcs,
     L.cls.resize(octs.size());
     for (size_t e = 0; e < octs.size(); e++) L.cls[e] = block_cls[l][octs[e].block];
     if (build_level(l, nbcs, names, dof_masks)) return -1;
+    // halved where the halo is long for the nodes owned (blocks of a single
+    // element, numbered row by row: 1,024-node tiles of 1100 x 44 x 44 take
+    // 246 KB of LDS, 512-node tiles 123 KB)
     TileSet ts;
-    if (make_tiles(l, l > 0 ? coarse_tile_nodes(TILE_NODES, L.n_nodes)
-                            : default_tile_nodes(L.n_nodes, L.n_dep > 0), false, ts))
-      return -1;
+    int t = l > 0 ? coarse_tile_nodes(TILE_NODES, L.n_nodes)
+                  : default_tile_nodes(L.n_nodes, L.n_dep > 0);
+    while (true) {
+      if (make_tiles(l, t, false, ts)) return -1;
+      if (ts.fits || t <= 64) break;
+      t = std::max(64, t / 2);
+    }
     if (!ts.fits) {
-      last_error = "the tiles of level " + std::to_string(l) + " do not fit in LDS";
+      last_error = "problem: the tiles of level " + std::to_string(l) + " do not fit in LDS";
       return -1;
     }
     install_tiles(l, std::move(ts));
