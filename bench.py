@@ -452,7 +452,7 @@ def main():
                     help="skip the oracle's residual check of the solution")
     ap.add_argument("--cpu-level", type=int, default=5)
     ap.add_argument("--fp32-valu", action="store_true",
-                    help="FP32 operator on the vector ALUs instead of the matrix cores")
+                    help="FP32 operator on the vector ALUs whatever the autotuner chose")
     ap.add_argument("--fp32-form", type=int, choices=(0, 1, 2), default=None,
                     help="pin the FP32 operator form after the autotuner: 0 vector ALUs, 1 matrix "
                          "cores (bf16 split), 2 matrix cores (FP32 operands)")

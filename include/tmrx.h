@@ -294,7 +294,8 @@ typedef struct {
                        entry, the PCG solves for the correction and rtol is
                        relative to the initial residual |f - K u0| (the Krylov
                        convention of TACS's GMRES) */
-  int fp32_valu;    /* FP32 operator on the vector ALUs instead of the matrix cores */
+  int fp32_valu;    /* 1: FP32 operator on the vector ALUs whatever tmrx_problem_set_fp32_form
+                       or the autotuner chose (they are the default) */
   int no_graph;     /* enqueue each PCG iteration instead of replaying a captured HIP graph */
   int cheb_pre_degree; /* pre-smoothing degree (0: cheb_degree); post-smoothing uses cheb_degree */
 } tmrx_solve_opts;
@@ -511,8 +512,9 @@ int tmrx_problem_stress_pnorm_grad(tmrx_problem *p, double P, double *g, int on_
    up first if the design changed. */
 int tmrx_problem_mg_op(tmrx_problem *p, int op, int level, const double *x, double *y,
                        int on_device, const tmrx_solve_opts *opts, double *lam_max);
-/* y = K(rho) x on the finest level (precision 0 FP64, 1 FP32 on the matrix
-   cores, 2 FP32 on the vector ALUs). */
+/* y = K(rho) x on the finest level (precision 0 FP64, 1 FP32 in the form of
+   tmrx_problem_tuning, by default the vector ALUs, 2 FP32 on the vector
+   ALUs). */
 int tmrx_problem_apply(tmrx_problem *p, const double *x, double *y, int on_device, int precision);
 /* Consistent nodal load of a constant traction tr[3] on the faces named
    `name`: TopOptUtils.compute3DTractionLoad (tmr/TopOptUtils.py:241-267).

@@ -1,5 +1,7 @@
 """GPU parity of the hex8 apply, the MG-PCG solve, compliance and its
 gradient against the FP64 CPU oracle (oracle/fe_oracle.c)."""
+import contextlib
+
 import numpy as np
 import pytest
 
@@ -39,6 +41,18 @@ def adapt():
     return forests, rho, prob
 
 
+@contextlib.contextmanager
+def _form(prob, form):
+    """The FP32 operator in the given form (1: matrix cores, bf16 split)."""
+    keep = prob.tuning()[1]
+    prob.set_fp32_form(form)
+    assert prob.tuning()[1] == form
+    try:
+        yield
+    finally:
+        prob.set_fp32_form(keep)
+
+
 @pytest.mark.parametrize("which", ["cube", "adapt"])
 def test_apply_parity(which, cube, adapt):
     forests, rho, prob = cube if which == "cube" else adapt
@@ -49,8 +63,12 @@ def test_apply_parity(which, cube, adapt):
     # identity rows on clamped dofs in both operators
     y_ref = orc.matvec(x)
     y64 = prob.apply(x, precision=0)
-    y32 = prob.apply(x, precision=1)   # matrix cores, bf16 hi/lo split products
-    y32v = prob.apply(x, precision=2)  # vector ALUs, FP32 products
+    with _form(prob, 1):
+        y32 = prob.apply(x, precision=1)   # matrix cores, bf16 split products
+        y32v = prob.apply(x, precision=2)  # vector ALUs, FP32 products
+    # the two forms round differently: both ran
+    assert not np.array_equal(y32, y32v)
+    assert np.array_equal(prob.apply(x, precision=1), y32v)  # the default form
     e64 = np.linalg.norm(y64 - y_ref) / np.linalg.norm(y_ref)
     e32 = np.linalg.norm(y32 - y_ref) / np.linalg.norm(y_ref)
     e32v = np.linalg.norm(y32v - y_ref) / np.linalg.norm(y_ref)
@@ -64,9 +82,8 @@ def test_apply_parity(which, cube, adapt):
 
 @pytest.mark.parametrize("nlevels", [1, 2])
 def test_large_coarse_direct_solve(nlevels):
-    """A coarsest level of at least 2048 dofs takes the super-block Cholesky
-    and explicit inverse (256-wide blocks, the bulk in FP64 GEMMs): with one
-    level it is the whole 16 x 8 x 8 box (4,131 dofs), so the coarse solve
+    """A coarsest level of at least 2048 dofs is substructured (inverses of
+    leaves and of a separator's Schur complement): with one level it is the whole 16 x 8 x 8 box (4,131 dofs), so the coarse solve
     must match the oracle's operator and one PCG step solves the problem;
     with two levels (Galerkin) the coarse solve of the 32 x 16 x 16 box's
     coarse level must match the oracle multigrid's own Cholesky solve."""
@@ -142,8 +159,8 @@ def test_fp32_matrix_cores_fp32_operands(which, cube, adapt):
 @pytest.mark.parametrize("precision", [0, 1, 2])
 @pytest.mark.parametrize("which", ["cube", "adapt"])
 def test_solve_compliance_parity(which, precision, cube, adapt):
-    """precision 0: FP64 V-cycle; 1: FP32 V-cycle on the matrix cores;
-    2: FP32 V-cycle on the vector ALUs."""
+    """precision 0: FP64 V-cycle; 1: FP32 V-cycle on the matrix cores (bf16
+    split); 2: FP32 V-cycle on the vector ALUs."""
     forests, rho, prob = cube if which == "cube" else adapt
     print("solve parity", which, "precision", precision, flush=True)
     f = _load(prob)
@@ -152,9 +169,10 @@ def test_solve_compliance_parity(which, precision, cube, adapt):
     c_ref = float(f @ u_ref)
     opts = solver.default_opts(rtol=1e-10, precision=min(precision, 1),
                                fp32_valu=int(precision == 2))
-    u = prob.solve(f, opts=opts)
-    c = prob.compliance()
-    tr = prob.true_residual()
+    with _form(prob, 1) if precision == 1 else contextlib.nullcontext():
+        u = prob.solve(f, opts=opts)
+        c = prob.compliance()
+        tr = prob.true_residual()
     print("iters", prob.info.iters, "true res %.3e" % tr, "c %.12g ref %.12g" % (c, c_ref), flush=True)
     assert prob.info.converged
     assert tr < 1e-8
@@ -212,9 +230,8 @@ def test_asymmetric_cycles_converge(pre, post, cube):
 @pytest.mark.parametrize("level", [2, 3])
 def test_single_level_is_a_direct_solve(level):
     """With one level the preconditioner is the coarsest-level solve alone:
-    the explicit inverse from the GPU's blocked Cholesky (375 dofs in 6
-    blocks of 64 at level 2, 2,187 dofs in 35 blocks at level 3, padding
-    included), so PCG converges in one iteration to the oracle's solution."""
+    the explicit inverse at level 2 (375 dofs in 6 blocks of 64, padding
+    included), the substructured solve at level 3 (2,187 dofs), so PCG converges in one iteration to the oracle's solution."""
     from tmr_amd import TMR
     f0 = TMR.createBoxForest(1, 1, 1, (1.0, 1.0, 1.0), face_names=workloads.FACES)
     f0.createTrees(level)

@@ -92,7 +92,7 @@ struct SolveOpts {
   int eig_iters = 10;
   int monitor = 0;
   int zero_guess = 1;
-  int fp32_valu = 0;  // FP32 operator on the vector ALUs (else matrix cores)
+  int fp32_valu = 0;  // FP32 operator on the vector ALUs (else in the form set or tuned)
   int no_graph = 0;   // enqueue every PCG iteration instead of replaying a HIP graph
   int cheb_pre_degree = 0;  // pre-smoothing degree (0: cheb_degree)
 };
