@@ -128,14 +128,20 @@ int Problem::build_coarse_plan() {
     std::vector<int> all(n1 - n0);
     for (int i = n0; i < n1; i++) all[i - n0] = i;
     // the depth of least time: what the solves of one set-up read (about 25
-    // V-cycles) at 4 TB/s, and the inversion steps at 20 us and 40 ns a block
-    auto inverse_s = [](int64_t d, int64_t largest) {
-      const double nb = (double)(padded((int)d) / DB);
-      return nb * nb * (padded((int)largest) / DB) * 40e-9;
+    // V-cycles) at 4 TB/s, the inversion steps at 20 us and 48 ns a block (of
+    // the lower triangle, over a matrix's own steps) and the products with the
+    // couplings at 10 ns a block product, zero ones counted.  Set-up in ms at
+    // depths 2 to 5 (the rest of it included): 4,131 dofs 1.54, 1.28, 1.47,
+    // 2.22; 9,441 dofs 7.9, 5.8, 7.0, 11.0; 13,923 dofs 16.2, 5.9, 7.2, 13.1;
+    // 35,067 dofs 209, 65, 50, 109.  The model takes depths 3, 3, 3 and 4.
+    auto blocks = [](int64_t d) { return (double)(padded((int)d) / DB); };
+    auto inverse_s = [&](int64_t d) {
+      const double nb = blocks(d);
+      return 0.5 * nb * (nb + 1.0) * nb * 48e-9;
     };
-    auto steps_s = [](int64_t largest) { return (padded((int)largest) / DB) * 20e-6; };
+    auto steps_s = [&](int64_t largest) { return blocks(largest) * 20e-6; };
     const double word_s = 25.0 * 8.0 / 4e12;
-    double best = word_s * (double)m * (double)m + inverse_s(m, m) + steps_s(m);
+    double best = word_s * (double)m * (double)m + inverse_s(m) + steps_s(m);
     Partition keep;
     for (int depth = 1; depth <= 8 && (m >> depth) >= DB; depth++) {
       Partition p;
@@ -155,12 +161,12 @@ int Problem::build_coarse_plan() {
         }
       }
       const int64_t ms = 3 * (int64_t)p.sep.size();
-      double words = (double)ms * (double)ms, s = inverse_s(ms, ms) + steps_s(ms);
+      double words = (double)ms * (double)ms, s = inverse_s(ms) + steps_s(ms);
       int64_t nmax = 0;
       for (size_t k = 0; k < p.leaves.size(); k++) {
         const int64_t ni = 3 * (int64_t)p.leaves[k].size();
         words += (double)ni * (double)(ni + 2 * nb[k]);
-        s += inverse_s(ni, ni);
+        s += inverse_s(ni) + blocks(nb[k]) * blocks(ni) * (blocks(ni) + blocks(nb[k])) * 10e-9;
         nmax = std::max(nmax, ni);
       }
       s += steps_s(nmax) + word_s * words;
