@@ -257,7 +257,7 @@ int Problem::build_coarse_plan() {
     std::vector<int> bnd;  // separator nodes, in separator order
     std::vector<int> loc;  // [separator node] -> place in bnd
     int np, mq;
-    int64_t et, wt, w, c;
+    int64_t et, wt, c;
     const Mat *m;
   };
   std::vector<std::vector<Leaf>> leaves(schur.size());
@@ -291,7 +291,6 @@ int Problem::build_coarse_plan() {
   }
   for (auto &lv : leaves)
     for (Leaf &lf : lv) {
-      lf.w = nw + lf.wt;
       if (lf.mq == 0) continue;
       // W^T = E^T D^-1 (and W), C = E^T W
       g1.push_back({lf.mq, lf.np, lf.np, lf.et, lf.m->off, lf.wt, lf.wt});

@@ -242,7 +242,7 @@ void launch_filter_fill(int n, double v, double *x, hipStream_t st) {
   TMRX_LAUNCH_CHECK();
 }
 
-__global__ void k_filter_lin(int n, int op, double alpha, const double *a, const double *x,
+__global__ void k_filter_lin(int n, int op, const double *a, const double *x,
                              const double *t, double *y) {
   const int i = blockIdx.x * FB + threadIdx.x;
   if (i >= n) return;
@@ -251,30 +251,30 @@ __global__ void k_filter_lin(int n, int op, double alpha, const double *a, const
     case 1: y[i] = a[i] * x[i]; break;                // elementwise product
     case 2: y[i] = a[i] * x[i] + t[i]; break;         // product plus t
     case 3: y[i] += t[i]; break;                      // add
-    case 6: y[i] = x[i] != 0.0 ? 1.0 / x[i] : 0.0; break;  // reciprocal
+    case 4: y[i] = x[i] != 0.0 ? 1.0 / x[i] : 0.0; break;  // reciprocal
   }
 }
-static void lin(int n, int op, double alpha, const double *a, const double *x, const double *t,
+static void lin(int n, int op, const double *a, const double *x, const double *t,
                 double *y, hipStream_t st) {
   if (n == 0) return;
-  hipLaunchKernelGGL(k_filter_lin, grid_of(n), dim3(FB), 0, st, n, op, alpha, a, x, t, y);
+  hipLaunchKernelGGL(k_filter_lin, grid_of(n), dim3(FB), 0, st, n, op, a, x, t, y);
   TMRX_LAUNCH_CHECK();
 }
 void launch_filter_copy(int n, const double *x, double *y, hipStream_t st) {
-  lin(n, 0, 0.0, nullptr, x, nullptr, y, st);
+  lin(n, 0, nullptr, x, nullptr, y, st);
 }
 void launch_filter_mul(int n, const double *a, const double *x, double *y, hipStream_t st) {
-  lin(n, 1, 0.0, a, x, nullptr, y, st);
+  lin(n, 1, a, x, nullptr, y, st);
 }
 void launch_filter_mul_add(int n, const double *a, const double *u, const double *t, double *y,
                            hipStream_t st) {
-  lin(n, 2, 0.0, a, u, t, y, st);
+  lin(n, 2, a, u, t, y, st);
 }
 void launch_filter_add(int n, const double *t, double *y, hipStream_t st) {
-  lin(n, 3, 0.0, nullptr, nullptr, t, y, st);
+  lin(n, 3, nullptr, nullptr, t, y, st);
 }
 void launch_filter_recip(int n, const double *x, double *y, hipStream_t st) {
-  lin(n, 6, 0.0, nullptr, x, nullptr, y, st);
+  lin(n, 4, nullptr, x, nullptr, y, st);
 }
 
 __global__ void k_filter_stride(int n, int nv, int v, int dir, const double *x, double *y) {

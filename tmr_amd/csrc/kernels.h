@@ -400,9 +400,10 @@ void launch_dot1(int64_t ndof, const double *a, const double *b, double *partial
                  hipStream_t st);
 void launch_dinv_dots(int64_t n, const double *dinv, double *y, const double *x,
                       double *partials, hipStream_t st);
-// finalize: mode 0 rz, 1 pq->alpha, 2 rr, 3 (zr, zq)->beta, 4 bb,
-// 5 (|y|^2, |x|^2) of the power iteration
-void launch_finalize(int nparts, const double *partials, int mode, double *sc, hipStream_t st);
+// sc[SC_BB] = sum of the partials; or of the pairs of launch_dinv_dots,
+// |y|^2 into sc[SC_ZQ] and |x|^2 into sc[SC_RZNEW]
+void launch_finalize(int nparts, const double *partials, double *sc, hipStream_t st);
+void launch_finalize_pairs(int nparts, const double *partials, double *sc, hipStream_t st);
 
 // Batched PCG over nrhs right-hand sides (vectors [nrhs][n]) whose dofs split
 // into independent segments (components) with their own scalars

@@ -934,43 +934,32 @@ void launch_dot1(int64_t ndof, const double *a, const double *b, double *partial
   TMRX_LAUNCH_CHECK();
 }
 
-// one block sums the partials (fixed order) and updates the PCG scalars
+// one block sums the partials (fixed order): single sums into SC_BB, or (PAIR)
+// the pairs of the power iteration, |Dinv A x|^2 and |x|^2, into SC_ZQ and
+// SC_RZNEW
+template <bool PAIR>
 __global__ __launch_bounds__(256) void k_finalize(int np, const double *__restrict__ part,
-                                                  int mode, double *__restrict__ sc) {
+                                                  double *__restrict__ sc) {
   __shared__ double red[4];
-  const int stride = (mode == 3 || mode == 5) ? 2 : 1;
   double a = 0.0, b = 0.0;
   for (int i = threadIdx.x; i < np; i += 256) {
-    a += part[stride * i];
-    if (mode == 3 || mode == 5) b += part[2 * i + 1];
+    a += part[(PAIR ? 2 : 1) * i];
+    if (PAIR) b += part[2 * i + 1];
   }
   const double sa = block_sum(a, red);
   __syncthreads();
-  const double sb = block_sum(b, red);
+  const double sb = PAIR ? block_sum(b, red) : 0.0;
   if (threadIdx.x != 0) return;
-  switch (mode) {
-    case 0: sc[SC_RZ] = sa; break;
-    case 1:
-      sc[SC_PQ] = sa;
-      sc[SC_ALPHA] = sc[SC_RZ] / sa;
-      break;
-    case 2: sc[SC_RR] = sa; break;
-    case 3:  // flexible (Polak-Ribiere) beta = z_{k+1}.(r_{k+1}-r_k) / z_k.r_k
-      sc[SC_RZNEW] = sa;
-      sc[SC_ZQ] = sb;
-      sc[SC_BETA] = -sc[SC_ALPHA] * sb / sc[SC_RZ];
-      sc[SC_RZ] = sa;
-      break;
-    case 4: sc[SC_BB] = sa; break;
-    case 5:  // power iteration: |Dinv A x|^2 and |x|^2
-      sc[SC_ZQ] = sa;
-      sc[SC_RZNEW] = sb;
-      break;
-  }
+  sc[PAIR ? SC_ZQ : SC_BB] = sa;
+  if (PAIR) sc[SC_RZNEW] = sb;
 }
 
-void launch_finalize(int nparts, const double *partials, int mode, double *sc, hipStream_t st) {
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, st, nparts, partials, mode, sc);
+void launch_finalize(int nparts, const double *partials, double *sc, hipStream_t st) {
+  hipLaunchKernelGGL(k_finalize<false>, dim3(1), dim3(256), 0, st, nparts, partials, sc);
+  TMRX_LAUNCH_CHECK();
+}
+void launch_finalize_pairs(int nparts, const double *partials, double *sc, hipStream_t st) {
+  hipLaunchKernelGGL(k_finalize<true>, dim3(1), dim3(256), 0, st, nparts, partials, sc);
   TMRX_LAUNCH_CHECK();
 }
 

@@ -85,7 +85,7 @@ int Problem::stress_pnorm_noalloc(double P, double *f) {
   launch_stress_sum(L.n_elem, L.d_conn.p, L.dep4(), state_mask(),
                     L.d_cls.p, L.d_lev.p, rho_.p, design_mode_ == 1 ? rho_gp_.p : nullptr, u_.p,
                     sa, parts, st_);
-  launch_finalize(nb, parts, 4, sc, st_);
+  launch_finalize(nb, parts, sc, st_);
   double h = 0.0;
   hipError_t e = take_launch_error();
   if (e == hipSuccess)

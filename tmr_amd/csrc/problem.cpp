@@ -1387,7 +1387,7 @@ int Problem::estimate_eigs(int l, const SolveOpts &o, bool defer) {
     std::swap(a, b);
   }
   double *slot = eig_sc_.p + (size_t)SC_N * l;
-  launch_finalize(reduce_blocks(n), parts_.p, 5, slot, st_);
+  launch_finalize_pairs(reduce_blocks(n), parts_.p, slot, st_);
   if (defer) return 0;
   double hsc[SC_N];
   HIPCHK(hipMemcpyAsync(hsc, slot, SC_N * sizeof(double), hipMemcpyDeviceToHost, st_));
@@ -2128,7 +2128,7 @@ int Problem::compliance(double *c) {
   }
   const int64_t n = levels_[0].ndof;
   launch_dot1(n, f_.p, u_.p, parts_.p, st_);
-  launch_finalize(reduce_blocks(n), parts_.p, 4, sc_.p, st_);
+  launch_finalize(reduce_blocks(n), parts_.p, sc_.p, st_);
   double h[SC_N];
   HIPCHK(hipMemcpyAsync(h, sc_.p, SC_N * sizeof(double), hipMemcpyDeviceToHost, st_));
   HIPCHK(hipStreamSynchronize(st_));
@@ -2225,7 +2225,7 @@ int Problem::stress_pnorm(double P, double *f) {
   launch_stress_sum(L.n_elem, L.d_conn.p, L.dep4(), state_mask(),
                     L.d_cls.p, L.d_lev.p, rho_.p, design_mode_ == 1 ? rho_gp_.p : nullptr, u_.p,
                     sa, parts_.p, st_);
-  launch_finalize(nb, parts_.p, 4, sc_.p, st_);
+  launch_finalize(nb, parts_.p, sc_.p, st_);
   double h[SC_N];
   HIPCHK(hipMemcpyAsync(h, sc_.p, SC_N * sizeof(double), hipMemcpyDeviceToHost, st_));
   HIPCHK(hipStreamSynchronize(st_));
