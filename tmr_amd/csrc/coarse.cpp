@@ -220,7 +220,7 @@ int Problem::build_coarse_plan() {
     }
     if (pr.empty()) pr.push_back({0, 0, 0});
     if (cs.prob.upload(reinterpret_cast<const char *>(pr.data()), pr.size() * sizeof(GJProb)) ||
-        cs.tile0.upload(tile0) || cs.dinv.alloc((size_t)2 * DB * DB * std::max(1, cs.nprob))) {
+        cs.tile0.upload(tile0) || cs.fac.alloc((size_t)4 * DB * DB * std::max(1, cs.nprob))) {
       last_error = "coarse: device allocation failed";
       return -1;
     }
@@ -504,7 +504,7 @@ int Problem::coarse_factor() {
   launch_coarse_scatter(L.nnzb, L.bsr64.p, cp.which.p, cp.dst.p, cp.ld.p, A0, A1, cp.Et.p, st_);
   auto invert = [&](CoarseSet &cs) {
     launch_gj_inverse(reinterpret_cast<const GJProb *>(cs.prob.p), cs.tile0.p, cs.nprob,
-                      cs.active.data(), cs.tiles.data(), (int)cs.active.size(), A0, A1, cs.dinv.p,
+                      cs.active.data(), cs.tiles.data(), (int)cs.active.size(), A0, A1, cs.fac.p,
                       chk_.p, st_);
   };
   invert(cp.set[0]);

@@ -3,24 +3,30 @@
 //
 // Explicit inverses of dense SPD matrices, many at once, by blocked
 // Gauss-Jordan: step k turns every 64 x 64 block of A into
-//   A_kk <- P = A_kk^-1,  A_kj <- P A_kj,  A_ik <- -A_ik P,
-//   A_ij <- A_ij - A_ik (P A_kj),
-// and after the last block A holds A^-1.  No pivoting: the pivots are those
-// of the Cholesky factorisation of an SPD matrix.  A step is one launch over
-// all blocks of all matrices, from one buffer to the other, and the
-// workgroup that produces block (k + 1, k + 1) also inverts it, so that a
-// matrix of nb blocks takes nb + 1 launches.  On the way the block (j, i) is
-// the transpose of (i, j), or its negative where k lies between them, so only
-// the blocks of the lower triangle are computed and each is stored twice (a
-// step of 37 x 37 blocks 70 -> 51 us, of 31 x 31 blocks 53 -> 42), the next
-// pivot block in the first workgroup.  What bounds it at the sizes of a
-// coarse level is that chain: the 64 dependent pivots of a block (in
-// registers, one barrier each, 23 us) and the launch, not the arithmetic
-// (FP64 matrix cores).  It replaced blocked Cholesky, L^-1 and L^-T L^-1 (about
-// five launches a block column, 54 us of them for the diagonal factor in
+//   A_kk <- A_kk^-1,  A_kj <- A_kk^-1 A_kj,  A_ik <- -A_ik A_kk^-1,
+//   A_ij <- A_ij - A_ik A_kk^-1 A_kj,
+// and after the last block A holds A^-1.  A_kk^-1 is never multiplied as such:
+// with A_kk = L D L^T, M = D^-1/2 L^-1 and Y_j = M A_kj the products are M^T M,
+// M^T Y_j and Y_i^T Y_j, whose terms stay of the size of A as those of a Cholesky
+// factorisation do.  (With the explicit A_kk^-1, entries of 1 / k0 meet small
+// couplings: islands of material in void of 1e-8 times the stiffness gave
+// residuals of 1e-3 |A| |x|, of 1e-9 a negative pivot; now 6e-17 at 1e-12.)  No
+// pivoting: the pivots are those of the Cholesky factorisation of an SPD
+// matrix.  A step is one launch over all blocks of all matrices, from one
+// buffer to the other, and the workgroup that produces block (k + 1, k + 1)
+// also factors it, so that a matrix of nb blocks takes nb + 1 launches.  On the
+// way the block (j, i) is the transpose of (i, j), or its negative where k lies
+// between them, so only the blocks of the lower triangle are computed and each
+// is stored twice, the next pivot block in the first workgroup.  What bounds it
+// at the sizes of a coarse level is that chain: the 64 dependent pivots of a
+// block (in registers, one barrier each, about 20 us) and the launch, not the
+// arithmetic (FP64 matrix cores; three products a block): set-up of 1.2M
+// adaptive hex, whose coarsest level takes 16 + 37 steps, 5.9 ms, of the 16^3
+// cube with 6 steps 0.48 ms.  It replaced blocked Cholesky, L^-1 and L^-T L^-1
+// (about five launches a block column, 54 us of them for the diagonal factor in
 // LDS).
 //
-// Matrices of coarse_schur_min dofs and more are first split by
+// Matrices of SCHUR_MIN dofs and more are first split by
 // substructuring (coarse.cpp): leaves D_i, separator S,
 //   W_i^T = E_i^T D_i^-1,  S <- S - sum_i E_i^T W_i,
 // all products through k_gemm_nt, and the solve goes through D_i^-1, W_i and
@@ -43,8 +49,8 @@ constexpr int LDB = 80;  // read as [k][col]
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 // wave w of four takes the 32 x 32 quadrant (w / 2, w % 2) of a 64 x 64
-// product over 64 inner indices: acc += A B, A[row][k] with leading dimension
-// LDA, B[k][col] with LDB, or (NT) B[col][k] with LDA
+// product over 64 inner indices: acc += A^T B, A[k][row] and B[k][col] with
+// leading dimension LDB, or (NT) A B^T, A[row][k] and B[col][k] with LDA
 template <bool NT>
 __device__ __forceinline__ void quad_product(const double *A, const double *B, f64x4 acc[2][2]) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -54,7 +60,7 @@ __device__ __forceinline__ void quad_product(const double *A, const double *B, f
     double a[2], b[2];
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-      a[u] = A[(r + 16 * u) * LDA + k + g];
+      a[u] = NT ? A[(r + 16 * u) * LDA + k + g] : A[(k + g) * LDB + r + 16 * u];
       b[u] = NT ? B[(c + 16 * u) * LDA + k + g] : B[(k + g) * LDB + c + 16 * u];
     }
 #pragma unroll
@@ -79,14 +85,15 @@ __device__ __forceinline__ void stage_block(const double *__restrict__ src, int6
   for (int t = threadIdx.x; t < DB * DB; t += DT) dst[(t >> 6) * LD + (t & 63)] = src[(t >> 6) * ld + (t & 63)];
 }
 
-// in-place inverse of the SPD block in `blk` (LDS, leading dimension LDA),
-// written to out (row-major 64 x 64): a 4 x 4 piece per thread in registers,
-// the pivot row and column through LDS (buf: 256 doubles, two sets in turn,
-// so one barrier a pivot)
-__device__ __forceinline__ void invert_block(const double *blk, double *buf, double *__restrict__ out,
+// M = D^-1/2 L^-1 of the SPD block in `blk` (LDS, leading dimension LDA), A = L
+// D L^T, so that A^-1 = M^T M: written to out row by row, and its transpose
+// behind.  A 4 x 4 piece per thread in registers, L^-1 growing where the
+// eliminated columns were, the pivot row and column through LDS (buf: 256
+// doubles, two sets in turn, so one barrier a pivot).
+__device__ __forceinline__ void factor_block(const double *blk, double *buf, double *__restrict__ out,
                                              int *bad) {
   const int tr = threadIdx.x >> 4, tc = threadIdx.x & 15;
-  double a[4][4];
+  double a[4][4], di[4] = {1.0, 1.0, 1.0, 1.0};  // 1 / d of the piece's rows
 #pragma unroll
   for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -111,31 +118,37 @@ __device__ __forceinline__ void invert_block(const double *blk, double *buf, dou
       for (int i = 0; i < 4; i++) cv[i] = col[4 * tr + i];
       if (!(p > 0.0)) neg = true;
       // 1 / p by two Newton steps from the hardware estimate: the division's
-      // range scaling would lengthen every pivot's chain
+      // range scaling would lengthen every pivot's chain (neither the estimate
+      // nor a step leaves the range for p within 2^-1022 .. 2^1022)
       double d = __builtin_amdgcn_rcp(p);
       d = __builtin_fma(__builtin_fma(-p, d, 1.0), d, d);
       d = __builtin_fma(__builtin_fma(-p, d, 1.0), d, d);
+      // rows below the pivot
 #pragma unroll
-      for (int j = 0; j < 4; j++) rv[j] *= d;
+      for (int i = 0; i < 4; i++) cv[i] = tr > kb || (tr == kb && i > q) ? -d * cv[i] : 0.0;
+      if (tr == kb) di[q] = d;
 #pragma unroll
       for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) a[i][j] = __builtin_fma(-cv[i], rv[j], a[i][j]);
-      if (tr == kb)
+        for (int j = 0; j < 4; j++) a[i][j] = __builtin_fma(cv[i], rv[j], a[i][j]);
+      if (tc == kb)
 #pragma unroll
-        for (int j = 0; j < 4; j++) a[q][j] = rv[j];
-      if (tc == kb) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) a[i][q] = -d * cv[i];
-        if (tr == kb) a[q][q] = d;
-      }
+        for (int i = 0; i < 4; i++)
+          if (tr > kb || (tr == kb && i > q)) a[i][q] = cv[i];
     }
   }
   if (neg && threadIdx.x == 0) atomicOr(bad, 1);
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < 4; i++) {
+    const double w = sqrt(di[i]);
 #pragma unroll
-    for (int j = 0; j < 4; j++) out[(4 * tr + i) * DB + 4 * tc + j] = a[i][j];
+    for (int j = 0; j < 4; j++) {
+      const int r = 4 * tr + i, c = 4 * tc + j;
+      const double m = r > c ? w * a[i][j] : r == c ? w : 0.0;
+      out[DB * r + c] = m;
+      out[DB * DB + DB * c + r] = m;
+    }
+  }
 }
 
 // problem of block b: last p with tile0[p] <= b
@@ -161,25 +174,39 @@ __global__ void k_gj_pad(const GJProb *__restrict__ pr, double *A0, double *A1) 
   if (i < ld) A[(size_t)i * ld + i] = 1.0;
 }
 
+// words of a pivot block's factors (M and its transpose), two sets in turn
+constexpr int FAC = 2 * DB * DB;
+
 __global__ __launch_bounds__(DT) void k_gj_first(const GJProb *__restrict__ pr, const double *A0,
-                                                 const double *A1, double *__restrict__ dinv,
+                                                 const double *A1, double *__restrict__ fac,
                                                  int *bad) {
   __shared__ double blk[DB * LDA], buf[256];
   const GJProb p = pr[blockIdx.x];
   stage_block<LDA>(((p.nblk & 1) ? A1 : A0) + p.off, DB * p.nblk, blk);
   __syncthreads();
-  invert_block(blk, buf, dinv + (size_t)2 * DB * DB * blockIdx.x, bad);
+  factor_block(blk, buf, fac + (size_t)2 * FAC * blockIdx.x, bad);
+}
+
+// w x (the quadrants of a product) into LDS, leading dimension LD
+template <int LD>
+__device__ __forceinline__ void stage_quads(const f64x4 x[2][2], double w, double *dst) {
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) dst[quad_row(u, e) * LD + quad_col(v)] = w * x[u][v][e];
 }
 
 __global__ __launch_bounds__(DT) void k_gj_step(int k, int nprob, const GJProb *__restrict__ pr,
                                                 const int *__restrict__ tile0, double *A0,
-                                                double *A1, double *dinv, int *bad) {
-  __shared__ double sa[DB * LDA], sb[DB * LDB];
+                                                double *A1, double *fac, int *bad) {
+  __shared__ double sa[DB * LDB], sb[DB * LDB];
   const int q = find_prob(tile0, nprob, blockIdx.x);
   const GJProb p = pr[q];
   const int nb = p.nblk;
-  // the block that goes on to the next inversion starts with the first wave
-  // of workgroups
+  // the block that goes on to the next factorisation starts with the first
+  // wave of workgroups
   int t = blockIdx.x - tile0[q];
   if (k + 1 < nb) {
     const int next = (k + 1) * (k + 4) / 2;
@@ -192,60 +219,66 @@ __global__ __launch_bounds__(DT) void k_gj_step(int k, int nprob, const GJProb *
   const int64_t ld = DB * nb;
   const double *src = (((nb - k) & 1) ? A1 : A0) + p.off;
   double *dst = (((nb - k - 1) & 1) ? A1 : A0) + p.off;
-  const double *P = dinv + (size_t)DB * DB * (2 * q + (k & 1));
+  const double *M = fac + (size_t)FAC * (2 * q + (k & 1)), *Mt = M + DB * DB;
   double *out = dst + (int64_t)DB * i * ld + DB * j;
   // block (j, i) of the result: the negative of the transpose where one of
   // the two block rows has been through its step and the other has not
   double *mir = dst + (int64_t)DB * j * ld + DB * i;
   const double sign = (i <= k) == (j <= k) ? 1.0 : -1.0;
-  if (i == k && j == k) {
-    for (int s = threadIdx.x; s < DB * DB; s += DT) out[(s >> 6) * ld + (s & 63)] = P[s];
-    return;
-  }
-  const double *Aik = src + (int64_t)DB * i * ld + DB * k;
-  const double *Akj = src + (int64_t)DB * k * ld + DB * j;
-  f64x4 acc[2][2] = {};
-  if (j == k) {
-    stage_block<LDA>(Aik, ld, sa);
-    stage_block<LDB>(P, DB, sb);
-  } else {
-    stage_block<LDA>(P, DB, sa);
-    stage_block<LDB>(Akj, ld, sb);
-  }
-  __syncthreads();
-  quad_product<false>(sa, sb, acc);
+  f64x4 yj[2][2] = {}, o[2][2] = {};
   if (i == k || j == k) {
+    // block row k: M^T (M A_kc), c the other index, or M^T M
+    const int c = i == k ? j : i;
+    if (c == k) {
+      stage_block<LDB>(M, DB, sb);
+    } else {
+      stage_block<LDB>(Mt, DB, sa);
+      stage_block<LDB>(src + (int64_t)DB * k * ld + DB * c, ld, sb);
+      __syncthreads();
+      quad_product<false>(sa, sb, yj);
+      __syncthreads();
+      stage_quads<LDB>(yj, 1.0, sb);
+    }
+    stage_block<LDB>(M, DB, sa);
+    __syncthreads();
+    quad_product<false>(sa, sb, o);
+    double *Nkc = i == k ? out : mir, *Nck = i == k ? mir : out;
 #pragma unroll
     for (int u = 0; u < 2; u++)
 #pragma unroll
       for (int v = 0; v < 2; v++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          const double w = i == k ? acc[u][v][e] : -acc[u][v][e];
-          out[quad_row(u, e) * ld + quad_col(v)] = w;
-          mir[quad_col(v) * ld + quad_row(u, e)] = sign * w;
+          Nkc[quad_row(u, e) * ld + quad_col(v)] = o[u][v][e];
+          if (c != k) Nck[quad_col(v) * ld + quad_row(u, e)] = sign * o[u][v][e];
         }
     return;
   }
-  // A_ij - A_ik (P A_kj)
+  // A_ij - A_ik A_kk^-1 A_kj = A_ij -+ Y_i^T Y_j, Y = M A_k. (A_ik is the
+  // transpose of A_ki, or its negative where i has been through its step)
+  stage_block<LDB>(Mt, DB, sa);
+  stage_block<LDB>(src + (int64_t)DB * k * ld + DB * j, ld, sb);
+  __syncthreads();
+  quad_product<false>(sa, sb, yj);
+  __syncthreads();
+  if (i != j) {
+    f64x4 yi[2][2] = {};
+    stage_block<LDB>(src + (int64_t)DB * k * ld + DB * i, ld, sb);
+    __syncthreads();
+    quad_product<false>(sa, sb, yi);
+    __syncthreads();
+    stage_quads<LDB>(yi, i < k ? 1.0 : -1.0, sa);
+  } else {
+    stage_quads<LDB>(yj, i < k ? 1.0 : -1.0, sa);
+  }
+  stage_quads<LDB>(yj, 1.0, sb);
   const double *Aij = src + (int64_t)DB * i * ld + DB * j;
-  f64x4 o[2][2];
 #pragma unroll
   for (int u = 0; u < 2; u++)
 #pragma unroll
     for (int v = 0; v < 2; v++)
 #pragma unroll
       for (int e = 0; e < 4; e++) o[u][v][e] = Aij[quad_row(u, e) * ld + quad_col(v)];
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < 2; u++)
-#pragma unroll
-    for (int v = 0; v < 2; v++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        sb[quad_row(u, e) * LDB + quad_col(v)] = -acc[u][v][e];
-      }
-  stage_block<LDA>(Aik, ld, sa);
   __syncthreads();
   quad_product<false>(sa, sb, o);
 #pragma unroll
@@ -259,25 +292,20 @@ __global__ __launch_bounds__(DT) void k_gj_step(int k, int nprob, const GJProb *
       }
   if (i != k + 1 || j != k + 1) return;
   __syncthreads();
-#pragma unroll
-  for (int u = 0; u < 2; u++)
-#pragma unroll
-    for (int v = 0; v < 2; v++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) sa[quad_row(u, e) * LDA + quad_col(v)] = o[u][v][e];
+  stage_quads<LDA>(o, 1.0, sa);
   __syncthreads();
-  invert_block(sa, sb, dinv + (size_t)DB * DB * (2 * q + ((k + 1) & 1)), bad);
+  factor_block(sa, sb, fac + (size_t)FAC * (2 * q + ((k + 1) & 1)), bad);
 }
 
 void launch_gj_inverse(const GJProb *pr, const int *tile0, int nprob, const int *active,
-                       const int *tiles, int nsteps, double *A0, double *A1, double *dinv,
+                       const int *tiles, int nsteps, double *A0, double *A1, double *fac,
                        int *bad, hipStream_t st) {
   if (nprob == 0) return;
   hipLaunchKernelGGL(k_gj_pad, dim3(nprob), dim3(DB), 0, st, pr, A0, A1);
-  hipLaunchKernelGGL(k_gj_first, dim3(nprob), dim3(DT), 0, st, pr, A0, A1, dinv, bad);
+  hipLaunchKernelGGL(k_gj_first, dim3(nprob), dim3(DT), 0, st, pr, A0, A1, fac, bad);
   for (int k = 0; k < nsteps; k++)
     hipLaunchKernelGGL(k_gj_step, dim3(tiles[k]), dim3(DT), 0, st, k, active[k], pr, tile0, A0, A1,
-                       dinv, bad);
+                       fac, bad);
   TMRX_LAUNCH_CHECK();
 }
 

@@ -269,10 +269,10 @@ void launch_coarse_schur(const CoarseBlocks &cb, const T *b, T *x, hipStream_t s
 // explicit inverses of nprob dense SPD matrices (largest first): matrix p
 // starts in A1 when its nblk is odd, else in A0, padding rows zero, and ends
 // in A0; both buffers are overwritten.  Step k works on the first active[k]
-// matrices, tiles[k] blocks; dinv: 2 x 64 x 64 words per matrix; *bad |= 1 on
-// a non-positive pivot
+// matrices, tiles[k] blocks; fac: 4 x 64 x 64 words per matrix; *bad |= 1 on a
+// non-positive pivot
 void launch_gj_inverse(const GJProb *pr, const int *tile0, int nprob, const int *active,
-                       const int *tiles, int nsteps, double *A0, double *A1, double *dinv,
+                       const int *tiles, int nsteps, double *A0, double *A1, double *fac,
                        int *bad, hipStream_t st);
 void launch_gemm_nt(int nprob, int ntiles, const GemmProb *pr, const int *tile0, const double *A,
                     const double *B, double *C, double *Ct, hipStream_t st);

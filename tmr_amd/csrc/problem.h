@@ -215,7 +215,7 @@ struct CoarseSet {
   int nprob = 0;
   DevArray<char> prob;
   DevArray<int> tile0;
-  DevArray<double> dinv;  // two 64 x 64 diagonal-block inverses per matrix
+  DevArray<double> fac;  // two sets of a 64 x 64 diagonal block's factors per matrix
   std::vector<int> active, tiles;
 };
 
