@@ -1803,9 +1803,9 @@ int Problem::solve_multi(int nrhs, const double *f, double *u, bool on_device, c
 }
 
 // one flexible-PCG iteration for every running (right-hand side, component):
-// q = A p, alpha, r, stop test, z = M r, beta, x and p; then the running
-// count into pinned slot `slot` and the iteration counter advanced.  Kernels
-// and one copy only, so that it can be captured.
+// q = A p, alpha, r, stop test (which also writes the running count into
+// pinned slot `slot` and advances the iteration counter), z = M r, beta, x and
+// p.  Kernels only, so that it can be captured.
 void Problem::enqueue_iteration(const SegPlan &pl, int nrhs, double *xsol, const SolveOpts &o,
                                 int slot) {
   const bool mixed = o.precision != 0;
@@ -1953,8 +1953,9 @@ int Problem::solve_batch(int nrhs, double *rhs, double *xsol, const SolveOpts &o
   launch_b_tick(iter_.p, act_.p, nidx, nact_.p, nact_host_, st_);
   HIPCHK(hipStreamSynchronize(st_));
   int running = nact_host_[0];
-  // iterations: replayed graphs (or enqueued bodies), the stop count of
-  // iteration k read while iteration k + 1 runs
+  // iterations: replayed graphs, each launched once the one before has
+  // reported its running count, or enqueued bodies, the count of iteration k
+  // read after iteration k + 1 is enqueued
   const bool graphs = !o.no_graph && !o.monitor && timing_ == 0;
   IterGraph *ig = nullptr;
   if (graphs && running > 0) {
@@ -2490,10 +2491,6 @@ int Problem::traction_load(const char *name, const double tr[3], double *f) {
   return 0;
 }
 
-// Owner-tile size autotuner: for each candidate size, rebuild the tiles of
-// every level and time the finest-level operator (FP32 product on the matrix
-// cores 4x, as in a V-cycle's smoothing and residual, plus one FP64 product,
-// as in a PCG iteration); keep the fastest.  Needs a design.
 int Problem::set_coarse_direct(bool on) {
   if (on != coarse_direct_) {
     coarse_direct_ = on;
@@ -2556,6 +2553,10 @@ int Problem::set_fp32_form(int form) {
   return 0;
 }
 
+// Owner-tile size autotuner: for each candidate size, rebuild the tiles of
+// every level and time the finest-level operator (three FP32 Chebyshev steps
+// and a residual in each of the three forms, as in a V-cycle, plus one FP64
+// product, as in a PCG iteration); keep the fastest.  Needs a design.
 int Problem::autotune(const int *cands, int ncand, int reps, int *chosen, double *ms_out) {
   if (!have_design_) {
     last_error = "autotune: set the design first";
