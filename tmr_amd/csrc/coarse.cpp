@@ -128,16 +128,16 @@ int Problem::build_coarse_plan() {
     std::vector<int> all(n1 - n0);
     for (int i = n0; i < n1; i++) all[i - n0] = i;
     // the depth of least time: what the solves of one set-up read (about 25
-    // V-cycles) at 4 TB/s, the inversion steps at 20 us and 48 ns a block (of
+    // V-cycles) at 4 TB/s, the inversion steps at 20 us and 52 ns a block (of
     // the lower triangle, over a matrix's own steps) and the products with the
     // couplings at 10 ns a block product, zero ones counted.  Set-up in ms at
-    // depths 2 to 5 (the rest of it included): 4,131 dofs 1.54, 1.28, 1.47,
-    // 2.22; 9,441 dofs 7.9, 5.8, 7.0, 11.0; 13,923 dofs 16.2, 5.9, 7.2, 13.1;
-    // 35,067 dofs 209, 65, 50, 109.  The model takes depths 3, 3, 3 and 4.
+    // depths 2 to 5 (the rest of it included): 4,131 dofs 1.50, 1.26, 1.45,
+    // 2.27; 9,441 dofs 7.9, 5.9, 7.1, 11.4; 13,923 dofs 16.4, 6.1, 7.3, 13.7;
+    // 35,067 dofs 226, 68, 52, 118.  The model takes depths 3, 3, 3 and 4.
     auto blocks = [](int64_t d) { return (double)(padded((int)d) / DB); };
     auto inverse_s = [&](int64_t d) {
       const double nb = blocks(d);
-      return 0.5 * nb * (nb + 1.0) * nb * 48e-9;
+      return 0.5 * nb * (nb + 1.0) * nb * 52e-9;
     };
     auto steps_s = [&](int64_t largest) { return blocks(largest) * 20e-6; };
     const double word_s = 25.0 * 8.0 / 4e12;
