@@ -94,6 +94,8 @@ def test_helmholtz_of_tiny_vectors(adapt, norm):
     assert e < max(1e-10, 1e3 * 1.6e-162 / norm)
     assert iters() > 0
     assert not run(np.zeros_like(y)).any() and iters() == 0
+    with pytest.raises(RuntimeError, match="device error"):
+        run(np.full_like(y, np.nan), transpose=True)
     free()
 
 

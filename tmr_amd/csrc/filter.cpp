@@ -264,10 +264,8 @@ int Filter::helmholtz_solve(const double *rhs, double *x) {
   double *r = w1_.p, *p = w3_.p, *q = w4_.p;
   launch_filter_cg_init(n_, rhs, dinv_.p, x, r, p, parts_.p, 1e-24, sc_.p, flag_.p, st_);
   int h[2] = {0, 0};
-  double tol2 = 0.0;
-  if (hipMemcpyAsync(&tol2, sc_.p + 2, sizeof(double), hipMemcpyDeviceToHost, st_) != hipSuccess ||
-      hipMemcpyAsync(h, flag_.p, sizeof(h), hipMemcpyDeviceToHost, st_) != hipSuccess ||
-      hipStreamSynchronize(st_) != hipSuccess || !(tol2 == tol2)) {
+  if (hipMemcpyAsync(h, flag_.p, sizeof(h), hipMemcpyDeviceToHost, st_) != hipSuccess ||
+      hipStreamSynchronize(st_) != hipSuccess || h[0] == 2) {
     last_error = "filter: device error";
     return -1;
   }

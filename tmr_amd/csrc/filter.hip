@@ -61,7 +61,8 @@ void launch_filter_spmv(int n, const int *ptr, const int *col, const double *val
 // back, an iteration took three round trips (9,537 nodes: 130 us, now 12).
 // At most FCG_BLOCKS blocks, each over a contiguous chunk, so that the sums
 // stay short; st: [0..1] r.z of the iterations in turn, [2] tolerance;
-// flag[0] set when converged, flag[1] the iterations done, flag[2] what
+// flag[0] set when converged (2: |rhs|^2 is not a number), flag[1] the
+// iterations done, flag[2] what
 // flag[0] was before the direction launch.  That launch sets flag[0] in one
 // block and tests flag[2]: blocks that tested the word it sets could lose some
 // of their waves before a barrier that the others wait at.
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(FB) void k_fcg_start(int np, const double *__restri
   if (threadIdx.x == 0) {
     st[1] = rz;
     st[2] = rtol2 * bb;
-    flag[0] = bb == 0.0 ? 1 : 0;
+    flag[0] = bb != bb ? 2 : bb == 0.0 ? 1 : 0;
     flag[1] = 0;
     flag[2] = 0;
   }
@@ -160,11 +161,12 @@ __global__ __launch_bounds__(FB) void k_fcg_step(int n, int chunk, int it, int n
                                                  double *__restrict__ x, double *__restrict__ r,
                                                  const double *__restrict__ st,
                                                  double *__restrict__ parts,
-                                                 int *__restrict__ flag) {
+                                                 const int *__restrict__ flag, int *publish) {
   __shared__ double red[FB / 64];
-  const bool stop = flag[0] != 0;
-  if (stop && blockIdx.x == 0 && threadIdx.x == 0) flag[2] = 1;
-  if (stop) return;
+  if (flag[0]) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *publish = 1;
+    return;
+  }
   const double alpha = st[it & 1] / fparts(npq, pq, 1, 0, red);
   const int lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
   double a = 0.0, b = 0.0;
@@ -189,9 +191,10 @@ __global__ __launch_bounds__(FB) void k_fcg_direction(int n, int chunk, int it, 
                                                       const double *__restrict__ r,
                                                       double *__restrict__ p,
                                                       double *__restrict__ st,
+                                                      const int *__restrict__ before,
                                                       int *__restrict__ flag) {
   __shared__ double red[FB / 64];
-  if (flag[2]) return;
+  if (*before) return;
   const double rr = fparts(np, parts, 2, 0, red), rz = fparts(np, parts, 2, 1, red);
   const bool done = rr <= st[2];
   const double beta = rz / st[it & 1];
@@ -225,9 +228,9 @@ void launch_filter_cg_iteration(int n, int it, const int *ptr, const int *col, c
   hipLaunchKernelGGL(k_fcg_product, dim3(nq), dim3(FB), 0, st, n, qchunk, ptr, col, val, p, q, pq,
                      flag);
   hipLaunchKernelGGL(k_fcg_step, dim3(nb), dim3(FB), 0, st, n, chunk, it, nq, pq, p, q, dinv, x, r,
-                     sc, parts, flag);
+                     sc, parts, flag, flag + 2);
   hipLaunchKernelGGL(k_fcg_direction, dim3(nb), dim3(FB), 0, st, n, chunk, it, nb, parts, dinv, r,
-                     p, sc, flag);
+                     p, sc, flag + 2, flag);
   TMRX_LAUNCH_CHECK();
 }
 int filter_cg_parts() { return 3 * FCG_BLOCKS; }
